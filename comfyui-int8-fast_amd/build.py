@@ -48,8 +48,24 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found; install ROCm or set HIPCC")
 
 
-def sources() -> list[str]:
-    return sorted(glob.glob(os.path.join(CSRC, "*.hip")))
+# gemm_i8_tiles.hip is compiled once per tile configuration and output type (names of csrc/gemm_i8_impl.hpp)
+GEMM_CFGS = ("CfgBig", "CfgB192", "CfgTall", "CfgWide", "CfgMid", "CfgW96", "CfgMidDeep", "CfgM96Deep", "CfgS64Deep", "CfgT64Deep")
+GEMM_GROUPED = ("CfgBig", "CfgB192", "CfgTall", "CfgWide")
+GEMM_OUTS = ("OUT_BF16", "OUT_F16", "OUT_F32", "OUT_I32")
+
+
+def units() -> list[tuple[str, str, list[str]]]:
+    """(source, name of the object file, extra flags) of every compilation, the longest first."""
+    out = []
+    tiles = os.path.join(CSRC, "gemm_i8_tiles.hip")
+    for cfg in GEMM_CFGS:
+        for o in GEMM_OUTS:
+            grouped = int(cfg in GEMM_GROUPED and o != "OUT_I32")
+            out.append((tiles, f"gemm_i8_tiles_{cfg}_{o}.o", [f"-DI8F_TU_CFG={cfg}", f"-DI8F_TU_OUT={o}", f"-DI8F_TU_GROUPED={grouped}"]))
+    for src in sorted(glob.glob(os.path.join(CSRC, "*.hip"))):
+        if src != tiles:
+            out.append((src, os.path.basename(src)[:-4] + ".o", []))
+    return out
 
 
 def _stale(target: str, deps: list[str]) -> bool:
@@ -65,11 +81,11 @@ def build(force: bool = False, keep_temps: bool = False, verbose: bool = True) -
     headers = glob.glob(os.path.join(CSRC, "*.hpp")) + glob.glob(os.path.join(HERE, "..", "include", "*.h"))
     jobs = []
     objs = []
-    for src in sources():
-        obj = os.path.join(OBJ, os.path.basename(src)[:-4] + ".o")
+    for src, name, extra in units():
+        obj = os.path.join(OBJ, name)
         objs.append(obj)
         if force or _stale(obj, [src] + headers):
-            cmd = [cc, *FLAGS, "-c", src, "-o", obj]
+            cmd = [cc, *FLAGS, *extra, "-c", src, "-o", obj]
             if keep_temps:
                 cmd += ["-save-temps=obj"]
             jobs.append(cmd)

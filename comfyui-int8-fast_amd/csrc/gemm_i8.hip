@@ -148,7 +148,7 @@ extern "C" int i8f_gemm_tile(int64_t M, int64_t N, int64_t K, int *bm, int *bn, 
     using namespace i8f;
     using namespace i8f::gemm;
     if (M <= 0 || N <= 0 || K < 0 || !bm || !bn || !stages) return I8F_ERR_INVALID;
-    if (K % 16 || N % 8 || N * K >= (1ll << 31)) {  // such shapes take the one-thread-per-output kernel
+    if (K % 16 || N % 8 || N * K >= (1ll << 31)) {  // such shapes take the kernel of gemm_ragged.hpp
         *bm = *bn = 1, *stages = 0;
         return I8F_OK;
     }

@@ -991,50 +991,11 @@ __global__ __launch_bounds__(C::NT) void gemm_i8_grouped_kernel(int gN, int gK, 
                                 gg.gate_rows[grp]);
 }
 
-// ---- slow but shape-agnostic kernel: one thread per output -----------------------------
-template <int OUT>
-__global__ __launch_bounds__(256) void gemm_i8_generic_kernel(const GemmArgs g) {
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (int64_t)g.M * g.N) return;
-    const int m = (int)(idx / g.N), n = (int)(idx % g.N);
-    const int8_t *xr = g.x + (int64_t)m * g.K;
-    const int8_t *wr = g.w + (int64_t)n * g.K;
-    int acc = 0;
-    for (int k = 0; k < g.K; ++k) acc += (int)xr[k] * (int)wr[k];
-    if constexpr (OUT == OUT_I32) {
-        ((int *)g.out)[idx] = acc;
-    } else {
-        constexpr int DT = OUT == OUT_BF16 ? I8F_BF16 : (OUT == OUT_F16 ? I8F_F16 : I8F_F32);
-        const float xs = g.xs[m];
-        const float ws = g.ws ? g.ws[g.row_scale ? n : 0] : g.ws_host;
-        const float a = (float)acc;
-        float b = 0.0f;
-        if (g.bias) {
-            if (g.bias_dtype == I8F_F32) b = ((const float *)g.bias)[n];
-            else if (g.bias_dtype == I8F_BF16) b = bf16_bits_to_f32(((const uint16_t *)g.bias)[n]);
-            else b = f16_bits_to_f32(((const uint16_t *)g.bias)[n]);
-        }
-        float t;
-        if (g.order == I8F_EPI_TORCH) {
-            if (g.row_scale) {
-                t = a * xs;
-                t = t * ws;
-            } else {
-                const float sc = ws * xs;
-                t = a * sc;
-            }
-            t = round_to_dtype<DT>(t);
-            if (g.bias) t = t + round_to_dtype<DT>(b);
-        } else {
-            const float sc = xs * ws;
-            t = a * sc;
-            if (g.bias) t = t + b;
-        }
-        if (g.gate) t = round_to_dtype<DT>(t) * load_as_f32<DT>(g.gate, (int64_t)(m / g.gate_rows) * g.N + n);
-        if (g.addend) t = round_to_dtype<DT>(t) + load_as_f32<DT>(g.addend, idx);
-        store_from_f32<DT>(g.out, idx, t);
-    }
-}
+}  // namespace gemm
+}  // namespace i8f
+#include "gemm_ragged.hpp"
+namespace i8f {
+namespace gemm {
 
 // tile configurations.  The one-workgroup-per-CU tiles run on v_mfma_i32_16x16x64_i8: on realistic operands the chip is at
 // its power limit, and the same multiply-accumulates cost less energy in that form than as v_mfma_i32_32x32x32_i8 (with
@@ -1100,6 +1061,17 @@ int launch_cfg(GemmArgs &g, hipStream_t st) {
                            g.tiles_m, g.tiles_n, g.xs, g.ws, g.bias, flags, g);
     return check_launch();
 }
+
+// Every tile configuration is compiled once per output type in a translation unit of its own (gemm_i8_tiles.hip, built
+// once for each pair), so that they compile side by side.
+#define I8F_GEMM_CFGS(X) X(CfgBig) X(CfgB192) X(CfgMid) X(CfgTall) X(CfgWide) X(CfgW96) X(CfgMidDeep) X(CfgM96Deep) X(CfgS64Deep) X(CfgT64Deep)
+#define I8F_EXTERN_CFG(C)                                                                                        \
+    extern template int launch_cfg<C, OUT_BF16>(GemmArgs &, hipStream_t);                                        \
+    extern template int launch_cfg<C, OUT_F16>(GemmArgs &, hipStream_t);                                         \
+    extern template int launch_cfg<C, OUT_F32>(GemmArgs &, hipStream_t);                                         \
+    extern template int launch_cfg<C, OUT_I32>(GemmArgs &, hipStream_t);
+I8F_GEMM_CFGS(I8F_EXTERN_CFG)
+#undef I8F_EXTERN_CFG
 
 enum Tile { TILE_BIG, TILE_B192, TILE_MID, TILE_TALL, TILE_WIDE, TILE_W96, TILE_MID_DEEP, TILE_M96_DEEP, TILE_S64_DEEP, TILE_T64_DEEP };
 
@@ -1248,9 +1220,7 @@ int launch(GemmArgs &g, hipStream_t st) {
     const bool fast = aligned && ((int64_t)g.M * g.K < (1ll << 31));
     if (g.side_t && (!fast || g.K % 128 || (uintptr_t)g.side_t % 16 || (uintptr_t)g.side_b % 16)) return I8F_ERR_UNSUPPORTED;
     if (!fast) {
-        const int64_t total = (int64_t)g.M * g.N;
-        hipLaunchKernelGGL((gemm_i8_generic_kernel<OUT>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, g);
-        return check_launch();
+        return launch_ragged<OUT>(g, st);
     }
     Tile t = choose_tile(g.M, g.N);
     int splits = 1;
@@ -1282,6 +1252,13 @@ int launch_cfg_grouped(const GemmArgs *gs, int n, hipStream_t st) {
     hipLaunchKernelGGL((gemm_i8_grouped_kernel<C, OUT>), dim3((unsigned)first), dim3(C::NT), 0, st, gs[0].N, gs[0].K, tiles_n, flags, gg, gs[0]);
     return check_launch();
 }
+
+#define I8F_EXTERN_GROUPED(C)                                                                                    \
+    extern template int launch_cfg_grouped<C, OUT_BF16>(const GemmArgs *, int, hipStream_t);                     \
+    extern template int launch_cfg_grouped<C, OUT_F16>(const GemmArgs *, int, hipStream_t);                      \
+    extern template int launch_cfg_grouped<C, OUT_F32>(const GemmArgs *, int, hipStream_t);
+I8F_EXTERN_GROUPED(CfgBig) I8F_EXTERN_GROUPED(CfgB192) I8F_EXTERN_GROUPED(CfgTall) I8F_EXTERN_GROUPED(CfgWide)
+#undef I8F_EXTERN_GROUPED
 
 // Estimated shader cycles of one launch, for the choice between one launch for a group of problems and one launch per
 // problem; the constants are this kernel's measured figures.  A one-workgroup-per-CU tile costs its rounds over the 256

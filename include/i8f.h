@@ -284,8 +284,8 @@ int i8f_gemm_i32(const int8_t *a, const int8_t *w, int64_t M, int64_t N, int64_t
 /*
  * The tile configuration i8f_gemm_i32 / i8f_linear_w8a8 use for an aligned M x N x K
  * problem: rows and columns of the output tile one workgroup computes and the number
- * of K-tile stages it keeps in LDS (1 x 1, 0 stages for shapes that take the
- * one-thread-per-output kernel).  No counterpart in the reference; for benchmarks
+ * of K-tile stages it keeps in LDS (1 x 1, 0 stages for shapes that fit no tile:
+ * K % 16 != 0, N % 8 != 0, or a weight of 2^31 bytes and more, which a kernel of their own takes).  No counterpart in the reference; for benchmarks
  * and profiles that have to name the kernel variant they measured.
  */
 int i8f_gemm_tile(int64_t M, int64_t N, int64_t K, int *bm, int *bn, int *stages);

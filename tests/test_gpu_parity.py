@@ -519,6 +519,28 @@ def test_gemm_i32_misaligned_operands_use_the_generic_kernel(L, dev):
     assert np.array_equal(acc.cpu().numpy(), O.gemm_i32(np.ascontiguousarray(a.numpy()[:, :160]), np.ascontiguousarray(w.numpy()[:, :160])))
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 1), (3, 65, 15), (64, 64, 17), (65, 63, 127), (63, 129, 129), (70, 9, 263), (129, 1001, 1160),   # edges of tiles and of 16-byte chunks
+    (2050, 2047, 40), (2048, 2049, 143),                                                                    # 128 x 128 tiles
+])
+def test_linear_w8a8_of_any_width_bit_exact(L, dev, M, N, K):
+    """Widths and row counts that fit no tile (K % 16 != 0 or N % 8 != 0): integers, both epilogue orders and the gated
+    residual are the oracle's bit for bit."""
+    x, wq = acts(M, K), i8(N, K)
+    ws = torch.rand(N, generator=G) * 0.002 + 0.0005
+    bias = (torch.randn(N, generator=G) * 0.01).bfloat16()
+    xa, code = O.from_torch(x)
+    q, s = L.quant_rowwise(x.to(dev))
+    wd = wq.to(dev)
+    assert np.array_equal(L.gemm_i32(q, wd).cpu().numpy(), O.gemm_i32(q.cpu().numpy(), wq.numpy()))
+    for order, odt in ((0, torch.bfloat16), (1, torch.float16)):
+        want = O.linear_w8a8(xa, code, wq.numpy(), ws.numpy(), O.from_torch(bias)[0], O.BF16, O.BF16 if odt == torch.bfloat16 else O.F16, 0, order)
+        got = L.linear_w8a8(q, s, wd, ws.to(dev), bias.to(dev), odt, order)
+        assert np.array_equal(bits(got), want)
+    gate, res = torch.randn(1, N, generator=G).half().to(dev), torch.randn(M, N, generator=G).half().to(dev)
+    assert torch.equal(L.linear_w8a8(q, s, wd, ws.to(dev), bias.to(dev), odt, order, addend=res, gate=gate), res + gate * got)
+
+
 # ------------------------------------------------------------------ fused linear (a6, a7)
 LIN_CASES = [
     # M, N, K, row, bias dtype or None, out dtype, order
