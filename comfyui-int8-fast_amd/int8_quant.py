@@ -366,7 +366,11 @@ class INT8LoRAPatchAdapter(LoRAAdapter):
 
 class INT8MergedLoRAPatchAdapter(LoRAAdapter):
     """Sums several LoRA deltas in float and applies ONE stochastic rounding step
-    (int8_quant.py:325-408).  `patches` is a list of (adapter, strength)."""
+    (int8_quant.py:325-408).  `patches` is a list of (adapter, strength).  A stack of plain LoRAs is one product of
+    the factors side by side, each `down` times its LoRA's multiplier, and goes through the fused kernel like a single
+    LoRA; other stacks are reconstructed and summed in float first."""
+
+    fuse_low_rank = True  # False: build the summed delta with torch like the reference, then merge
 
     def __init__(self, patches, weight_scale, seed=0):
         first = patches[0][0]
@@ -379,12 +383,38 @@ class INT8MergedLoRAPatchAdapter(LoRAAdapter):
         rows = delta_f if isinstance(delta_f, int) else delta_f.shape[0]
         return _slice_scale_mismatch_only(self.weight_scale, rows, offset)
 
+    def _stacked_factors(self, weight, dev):
+        """(up [N,R], down [R,K]) in float32 with up @ down the summed delta of the stack, or None where the patches are
+        not all plain LoRAs of this weight or their ranks and widths are not those of the fused kernel's matrix-core form."""
+        parts, rank = [], 0
+        for adapter, strength in self.patches:
+            plain = _plain_lora(adapter.weights)
+            if plain is None or weight.dim() != 2 or plain[0].shape[0] != weight.shape[0] or plain[1].shape[1] != weight.shape[1]:
+                return None
+            alpha, r = adapter.weights[2], plain[1].shape[0]
+            parts.append((*plain, (alpha / r) * strength if alpha is not None else strength))
+            rank += r
+        if weight.shape[1] % 16 or rank % 4 or rank > 256:
+            return None
+        up = torch.cat([u.to(dev, torch.float32) for u, _, _ in parts], dim=1)
+        down = torch.cat([d.to(dev, torch.float32) * m for _, d, m in parts], dim=0)
+        return up, down
+
     def calculate_weight(self, weight, key, strength, strength_model, offset, function,
                          intermediate_dtype=torch.float32, original_weight=None):
         if intermediate_dtype == torch.int8:
             intermediate_dtype = torch.float32
         home = weight.device
         dev = compute_device() if weight.dtype == torch.int8 else home
+        if weight.dtype == torch.int8 and intermediate_dtype == torch.float32 and self.fuse_low_rank:
+            stacked = self._stacked_factors(weight, dev)
+            if stacked is not None:
+                up, down = stacked
+                if _quarot_applies(weight):   # rotating the rows of up @ down is rotating the rows of down
+                    down = _lib.rotate128(down)
+                eff = self._get_effective_scale(weight.shape[0], offset)
+                noise = _draw_noise(tuple(weight.shape), self.seed, dev)
+                return _lib.lora_merge_sr(weight.to(dev), eff, noise, up=up, down=down).to(home)
         total = None
         for adapter, lora_strength in self.patches:  # ComfyUI's own `strength` is ignored here, as in the reference
             diff, mult = reconstruct_lora_diff(adapter.weights, weight.shape, dev, intermediate_dtype, lora_strength)

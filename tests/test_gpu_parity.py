@@ -1139,6 +1139,19 @@ def test_lora_merge_bit_exact(L, dev, N, K, r, row):
     assert np.array_equal(dq.cpu().numpy(), O.sr_delta(delta, ws.numpy(), noise.numpy()))
 
 
+@pytest.mark.parametrize("N,K,r,row", [(33, 48, 12, True), (300, 272, 36, True), (64, 256, 64, False), (70, 1040, 100, True),
+                                       (31, 80, 128, True), (65, 304, 132, True), (40, 512, 256, False)])
+def test_lora_merge_of_any_rank_on_the_matrix_cores_bit_exact(L, dev, N, K, r, row):
+    """Ranks between and beyond the powers of two (padded with zero products to the next one the kernel is built for) and
+    widths that are odd multiples of 16 (half of the last wave's columns do not exist)."""
+    w, ws = i8(N, K), torch.rand(N if row else 1, generator=G) * 0.002 + 0.0005
+    up, down = torch.randn(N, r, generator=G) * 0.05, torch.randn(r, K, generator=G) * 0.05
+    noise = torch.rand(N, K, generator=G)
+    want = O.lora_merge_sr(w.numpy(), ws.numpy(), noise.numpy(), up=up.numpy(), down=down.numpy(), lora_scale=0.7)
+    got = L.lora_merge_sr(w.to(dev), ws.to(dev) if row else float(ws[0]), noise.to(dev), up=up.to(dev), down=down.to(dev), lora_scale=0.7)
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("N,K,r", [(64, 256, 32), (96, 288, 16), (40, 100, 8)])
 def test_lora_merge_denormal_products_bit_exact(L, dev, N, K, r):
     """Rank-r products and partial sums in the binary32 denormal range (|up*down| ~ 1e-40), with a weight
