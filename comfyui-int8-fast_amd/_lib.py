@@ -8,12 +8,14 @@ library launches on torch's current HIP stream.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libi8f_gfx950.so")
+HOST_PATH = os.path.join(_HERE, "_i8f_host.so")
 
 BF16, F16, F32 = 0, 1, 2
 SCALE_TENSOR, SCALE_ROW = 0, 1
@@ -83,6 +85,25 @@ def lib() -> ctypes.CDLL:
         getattr(L, name).restype = i32
     _lib = L
     return L
+
+
+_host = None
+
+
+def host():
+    """The native host path (csrc/host/i8f_host.cpp), bound to the kernels' library; loaded once, raises like lib()."""
+    global _host
+    if _host is not None:
+        return _host
+    lib()
+    if not os.path.exists(HOST_PATH):
+        raise RuntimeError(f"{HOST_PATH} is missing: build it with `python {os.path.join(_HERE, 'build.py')}`")
+    spec = importlib.util.spec_from_file_location("_i8f_host", HOST_PATH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    mod.bind(LIB_PATH)
+    _host = mod
+    return mod
 
 
 EXPORTS = (
@@ -435,6 +456,7 @@ def _bias_arg(bias, N, device):
 
 _SPLITK_WORKSPACES = {}
 _SPLITK_COUNTER_BYTES = 4096
+SPLITK_MIN_K = 10240   # narrower layers never split their K range
 
 
 def _splitk_workspace(t: torch.Tensor, M: int, N: int, K: int):
@@ -447,7 +469,7 @@ def _splitk_workspace(t: torch.Tensor, M: int, N: int, K: int):
     overlap eager calls on this one): the call gets a workspace of its own from the graph's memory pool, with a
     fill kernel in front of it that clears the arrival words on every replay, and the memory goes back to the pool
     of the graph when the call returns (later nodes of the same graph run after this one)."""
-    if K < 10240 or M * N > 128 * 128 * 128:
+    if K < SPLITK_MIN_K or M * N > 128 * 128 * 128:
         return None
     nbytes = lib().i8f_linear_w8a8_workspace_bytes()
     if torch.cuda.is_current_stream_capturing():

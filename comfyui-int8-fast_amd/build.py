@@ -1,4 +1,4 @@
-"""Build libi8f_gfx950.so from csrc/*.hip with hipcc, in-tree.
+"""Build libi8f_gfx950.so from csrc/*.hip with hipcc and the host extension _i8f_host.so with g++, in-tree.
 
     python comfyui-int8-fast_amd/build.py [--force] [--keep-temps]
 
@@ -14,11 +14,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libi8f_gfx950.so")
+HOST_SRC = os.path.join(CSRC, "host", "i8f_host.cpp")
+HOST_LIB = os.path.join(HERE, "_i8f_host.so")
 
 # -ffp-contract=off and correctly rounded division are part of the numerical
 # contract (bit-exact quantiser, epilogue and merge); packed FP32 instructions
@@ -75,6 +78,19 @@ def _stale(target: str, deps: list[str]) -> bool:
     return any(os.path.getmtime(d) > t for d in deps)
 
 
+def host_command() -> list[str]:
+    """The compilation of the host extension (no device code: a CPython module against the installed torch)."""
+    import torch
+
+    t = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
+    include = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"), sysconfig.get_paths()["include"],
+               os.path.join(rocm, "include")]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            *(f for d in include for f in ("-isystem", d)), HOST_SRC, "-o", HOST_LIB, "-L" + os.path.join(t, "lib"),
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-Wl,-rpath," + os.path.join(t, "lib")]
+
+
 def build(force: bool = False, keep_temps: bool = False, verbose: bool = True) -> str:
     cc = hipcc()
     os.makedirs(OBJ, exist_ok=True)
@@ -90,6 +106,9 @@ def build(force: bool = False, keep_temps: bool = False, verbose: bool = True) -
                 cmd += ["-save-temps=obj"]
             jobs.append(cmd)
 
+    if force or _stale(HOST_LIB, [HOST_SRC] + headers):
+        jobs.append(host_command())
+
     def run(cmd):
         p = subprocess.run(cmd, capture_output=True, text=True)
         noise = "is not a recognized feature for this target"
@@ -101,8 +120,8 @@ def build(force: bool = False, keep_temps: bool = False, verbose: bool = True) -
             if verbose and err.strip():
                 print(err, file=sys.stderr)
             if rc != 0:
-                raise RuntimeError("hipcc failed: " + " ".join(cmd) + "\n" + err)
-    if force or jobs or _stale(LIB, objs):
+                raise RuntimeError("compilation failed: " + " ".join(cmd) + "\n" + err)
+    if force or _stale(LIB, objs):
         cmd = [cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs]
         p = subprocess.run(cmd, capture_output=True, text=True)
         if p.returncode != 0:

@@ -1,0 +1,355 @@
+// Host path of the quantised linear layers in eager mode: what Linear.forward does between the model's call and the
+// kernels -- argument checks, the memory of the result and of the int8 rows, the launches -- without the Python
+// interpreter.  A layer of a few hundred tokens runs for 5 to 20 microseconds on the GPU, less than the two dozen Python
+// calls and two ctypes calls of the general path take (77 x 3072 x 3072: 31 us a forward that way, 11 us this way).
+//
+//   bind(path)                  the kernels' library
+//   linear(...)                 one layer: Linear.forward with its optional prologue, gate and residual
+//   vector_fanout(...)          several small-batch layers that read the same rows, in one launch
+//
+// Every function takes the cases it can decide on cheaply and returns None for all others (tensors of other types,
+// devices or layouts, operands that need a cast or a copy, errors): the caller then goes the general way in Python, which
+// also words the errors.  Nothing is kept between calls.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <dlfcn.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../../include/i8f.h"
+
+namespace {
+
+// ---- the kernels' library -----------------------------------------------------------------
+#define I8F_ENTRY_POINTS(X)                                                                                              \
+    X(i8f_quant_rowwise) X(i8f_quant_rowwise_prologue) X(i8f_quant_rowwise_norm_modulate) X(i8f_quant_rowwise_rms_norm)  \
+    X(i8f_quant_rowwise_concat_gelu) X(i8f_rotate128) X(i8f_linear_w8a8_gated) X(i8f_linear_w8a16_small_m)               \
+    X(i8f_linear_w8a16_small_m_grouped)
+struct Library {
+#define X(name) decltype(&::name) name = nullptr;
+    I8F_ENTRY_POINTS(X)
+#undef X
+    bool bound = false;
+} lib;
+
+PyObject *bind(PyObject *, PyObject *arg) {
+    const char *path = PyUnicode_AsUTF8(arg);
+    if (!path) return nullptr;
+    void *h = dlopen(path, RTLD_NOW | RTLD_LOCAL);
+    if (!h) return PyErr_Format(PyExc_RuntimeError, "cannot load %s: %s", path, dlerror());
+#define X(name)                                                                                                    \
+    if (!(lib.name = (decltype(lib.name))dlsym(h, #name)))                                                         \
+        return PyErr_Format(PyExc_RuntimeError, "%s has no %s: build it again", path, #name);
+    I8F_ENTRY_POINTS(X)
+#undef X
+    lib.bound = true;
+    Py_RETURN_NONE;
+}
+
+// ---- arguments -----------------------------------------------------------------------------
+int code_of(at::ScalarType t) {
+    return t == at::kBFloat16 ? I8F_BF16 : t == at::kHalf ? I8F_F16 : t == at::kFloat ? I8F_F32 : -1;
+}
+
+// A plain torch.Tensor or Parameter (subclasses -- fake and wrapped tensors among them -- are the general path's).
+const at::Tensor *tensor(PyObject *o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+bool aligned16(const at::Tensor &t) { return (uintptr_t)t.const_data_ptr() % 16 == 0; }
+
+// The rows of t, all but its last dimension flattened, if they are a matrix of contiguous rows at one stride.
+bool rows_of(const at::Tensor &t, int64_t &M, int64_t &K, int64_t &ld) {
+    const int64_t d = t.dim();
+    if (d < 1) return false;
+    const auto sizes = t.sizes(), strides = t.strides();
+    K = sizes[d - 1], M = 1, ld = K;
+    if (K < 1 || (K > 1 && strides[d - 1] != 1)) return false;
+    int64_t expect = -1;  // stride that the next outer dimension has to have
+    for (int64_t i = d - 2; i >= 0; --i) {
+        if (sizes[i] == 1) continue;
+        if (sizes[i] == 0) return false;
+        if (expect < 0) ld = strides[i];
+        else if (strides[i] != expect) return false;
+        expect = strides[i] * sizes[i];
+        M *= sizes[i];
+    }
+    return ld >= K;
+}
+
+// A vector per leading index of x, shared by its tokens: [K], or [..., 1, K] with x's leading dimensions.
+// K: the last dimension of what it is applied to (x itself or the layer's output).
+bool broadcasts_over_tokens(const at::Tensor &x, int64_t K, const at::Tensor &v) {
+    if (v.scalar_type() != x.scalar_type() || v.device() != x.device() || !v.is_contiguous() || x.dim() < 2) return false;
+    if (v.dim() == 1) return v.size(0) == K;
+    if (v.dim() != x.dim() || v.size(-1) != K || v.size(-2) != 1) return false;
+    for (int64_t i = 0; i < x.dim() - 2; ++i)
+        if (v.size(i) != x.size(i)) return false;
+    return true;
+}
+
+// Weight, scale and bias of a layer as the kernels take them.
+struct Layer {
+    const int8_t *w = nullptr;
+    const float *ws = nullptr;
+    float ws_host = 0.0f;
+    int mode = I8F_SCALE_TENSOR, bias_code = I8F_BF16;
+    const void *bias = nullptr;
+    int64_t N = 0, K = 0;
+};
+
+bool layer_of(PyObject *weight, PyObject *scale, PyObject *bias, bool per_row, const at::Device &dev, Layer &l) {
+    const at::Tensor *w = tensor(weight);
+    if (!w || w->scalar_type() != at::kChar || w->dim() != 2 || w->device() != dev || !w->is_contiguous()) return false;
+    l.w = (const int8_t *)w->const_data_ptr(), l.N = w->size(0), l.K = w->size(1);
+    if (PyFloat_Check(scale)) {
+        if (per_row) return false;
+        l.ws_host = (float)PyFloat_AS_DOUBLE(scale);
+    } else {
+        const at::Tensor *s = tensor(scale);
+        if (!s || s->scalar_type() != at::kFloat || s->device() != dev || !s->is_contiguous() || s->numel() < 1) return false;
+        if (per_row && s->numel() != l.N) return false;
+        l.ws = (const float *)s->const_data_ptr();
+        l.mode = per_row && s->numel() != 1 ? I8F_SCALE_ROW : I8F_SCALE_TENSOR;  // (one scale: element 0 counts)
+    }
+    if (bias != Py_None) {
+        const at::Tensor *b = tensor(bias);
+        if (!b || b->device() != dev || !b->is_contiguous() || b->numel() != l.N || (l.bias_code = code_of(b->scalar_type())) < 0) return false;
+        l.bias = b->const_data_ptr();
+    }
+    return true;
+}
+
+at::Tensor empty(at::IntArrayRef size, at::ScalarType t, const at::Device &dev) {
+    return at::detail::empty_cuda(size, t, dev, std::nullopt);
+}
+
+// The output of a layer on x's tokens: x's leading dimensions and N columns.
+at::Tensor empty_output(const at::Tensor &x, int64_t N) {
+    c10::SmallVector<int64_t, 6> size(x.sizes().begin(), x.sizes().end());
+    size.back() = N;
+    return empty(size, x.scalar_type(), x.device());
+}
+
+struct Stream {
+    void *handle;
+    bool ok;
+    explicit Stream(const at::Device &dev) : handle(nullptr), ok(dev.is_cuda() && dev.index() == c10::hip::current_device()) {
+        if (ok) handle = (void *)c10::hip::getCurrentHIPStream(dev.index()).stream();
+    }
+};
+
+// ---- 16 rows or fewer: W8A16 ----------------------------------------------------------------
+PyObject *small_m(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, const Layer &l, bool rotate, void *stream) {
+    const int dt = code_of(x.scalar_type());
+    const void *xp = x.const_data_ptr();
+    at::Tensor rotated;
+    if (rotate) {
+        rotated = empty({M, K}, x.scalar_type(), x.device());
+        if (lib.i8f_rotate128(xp, dt, M, K, ld, rotated.data_ptr(), stream)) Py_RETURN_NONE;
+        xp = rotated.const_data_ptr(), ld = K;
+    }
+    at::Tensor y = empty_output(x, l.N);
+    if (lib.i8f_linear_w8a16_small_m(xp, dt, M, K, ld, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, y.data_ptr(), l.N, stream))
+        Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(y));
+}
+
+// linear(x, weight, scale, bias, per_row, rotate, small_rows, order, kind, mod_scale, mod_shift, eps, norm_weight, fused_add,
+//        gate, residual, workspace): kind, an i8f_prologue, names what is applied to x inside the quantiser
+PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 17) return PyErr_Format(PyExc_TypeError, "linear takes 17 arguments, got %zd", n);
+    const at::Tensor *xt = tensor(a[0]);
+    if (!lib.bound || !xt || !xt->is_cuda()) Py_RETURN_NONE;
+    const at::Tensor &x = *xt;
+    const int dt = code_of(x.scalar_type());
+    const bool per_row = a[4] == Py_True, rotate = a[5] == Py_True, fused_add = a[13] == Py_True;
+    int64_t M, K, ld;
+    Layer l;
+    if ((dt != I8F_BF16 && dt != I8F_F16) || !rows_of(x, M, K, ld) || !layer_of(a[1], a[2], a[3], per_row, x.device(), l)) Py_RETURN_NONE;
+    const int64_t small_rows = PyLong_AsLongLong(a[6]);
+    const int order = (int)PyLong_AsLong(a[7]), kind = (int)PyLong_AsLong(a[8]);
+    const bool gated = a[14] != Py_None, with_residual = a[15] != Py_None;
+    const Stream st(x.device());
+    if (!st.ok || (rotate && K % 128)) Py_RETURN_NONE;
+    if (M <= small_rows) {
+        if (kind != I8F_PRO_NONE || gated || with_residual || K != l.K) Py_RETURN_NONE;
+        return small_m(x, M, K, ld, l, rotate, st.handle);
+    }
+
+    // the operation in front of the layer and its operands
+    const at::Tensor *s = nullptr, *t = nullptr, *w = nullptr;
+    int64_t V = 1, Kall = K;
+    if (kind == I8F_PRO_MODULATE || kind == I8F_PRO_NORM_MODULATE || kind == I8F_PRO_RMS_NORM) {
+        s = a[9] == Py_None ? nullptr : tensor(a[9]), t = a[10] == Py_None ? nullptr : tensor(a[10]);
+        if ((a[9] != Py_None && !s) || (a[10] != Py_None && !t) || (kind != I8F_PRO_RMS_NORM && !(s && t))) Py_RETURN_NONE;
+        for (const at::Tensor *v : {s, t}) {
+            if (!v) continue;
+            if (!broadcasts_over_tokens(x, K, *v) || !aligned16(*v)) Py_RETURN_NONE;
+            V = v->numel() / K;
+        }
+        if (s && t && s->sizes() != t->sizes()) Py_RETURN_NONE;
+        if (V < 1 || M % V) Py_RETURN_NONE;
+        if (kind != I8F_PRO_MODULATE && (K > 16384 || K % 16 || (M > 1 && ld % 8) || !aligned16(x))) Py_RETURN_NONE;
+        if (kind == I8F_PRO_RMS_NORM && a[12] != Py_None) {
+            w = tensor(a[12]);
+            if (!w || w->scalar_type() != x.scalar_type() || w->dim() != 1 || w->size(0) != K || w->device() != x.device() || !w->is_contiguous() ||
+                !aligned16(*w))
+                Py_RETURN_NONE;
+        }
+    } else if (kind == I8F_PRO_CONCAT_GELU) {
+        s = tensor(a[9]);
+        int64_t Mb, Kb, ldb;
+        if (!s || s->scalar_type() != x.scalar_type() || s->device() != x.device() || s->dim() != x.dim() || !rows_of(*s, Mb, Kb, ldb)) Py_RETURN_NONE;
+        for (int64_t i = 0; i + 1 < x.dim(); ++i)
+            if (s->size(i) != x.size(i)) Py_RETURN_NONE;
+        Kall = K + Kb;
+        if (K % 16 || Kb % 16 || Kall > 16384 || (M > 1 && (ld % 8 || ldb % 8)) || !aligned16(x) || !aligned16(*s) || (rotate && Kb % 128)) Py_RETURN_NONE;
+    } else if (kind == I8F_PRO_SILU_GATE) {
+        s = tensor(a[9]);
+        if (!s || s->scalar_type() != x.scalar_type() || s->device() != x.device() || s->sizes() != x.sizes() || !s->is_contiguous()) Py_RETURN_NONE;
+    } else if (kind != I8F_PRO_NONE && kind != I8F_PRO_GELU_TANH && kind != I8F_PRO_GELU_ERF) {
+        Py_RETURN_NONE;
+    }
+    if (Kall != l.K) Py_RETURN_NONE;
+
+    // what follows the layer
+    const at::Tensor *gate = nullptr, *res = nullptr, *work = nullptr;
+    int64_t gate_rows = 1;
+    if (gated) {
+        gate = tensor(a[14]);
+        if (!gate || !broadcasts_over_tokens(x, l.N, *gate)) Py_RETURN_NONE;
+        const int64_t vecs = gate->numel() / l.N;
+        if (vecs < 1 || M % vecs) Py_RETURN_NONE;
+        gate_rows = M / vecs;
+    }
+    if (with_residual) {
+        res = tensor(a[15]);
+        if (!res || res->scalar_type() != x.scalar_type() || res->device() != x.device() || res->dim() != x.dim() || !res->is_contiguous() ||
+            res->numel() != M * l.N || res->size(-1) != l.N)
+            Py_RETURN_NONE;
+        for (int64_t i = 0; i + 1 < x.dim(); ++i)
+            if (res->size(i) != x.size(i)) Py_RETURN_NONE;
+    }
+    if (a[16] != Py_None) {
+        work = tensor(a[16]);
+        if (!work) Py_RETURN_NONE;
+    }
+
+    // one piece of memory for the int8 rows and, behind them, their scales; it goes back to the allocator when the call
+    // returns, for work behind these kernels on the same stream
+    const int64_t q_bytes = (M * Kall + 255) / 256 * 256;
+    at::Tensor scratch = empty({q_bytes + 4 * M}, at::kByte, x.device());
+    int8_t *q = (int8_t *)scratch.data_ptr();
+    float *qs = (float *)(q + q_bytes);
+    at::Tensor y = empty_output(x, l.N);
+    const void *xp = x.const_data_ptr(), *sp = s ? s->const_data_ptr() : nullptr, *tp = t ? t->const_data_ptr() : nullptr;
+    const int rb = rotate ? 128 : 0;
+    int rc;
+    switch (kind) {
+    case I8F_PRO_NONE: rc = lib.i8f_quant_rowwise(xp, dt, M, K, ld, rb, q, qs, st.handle); break;
+    case I8F_PRO_NORM_MODULATE:
+        rc = lib.i8f_quant_rowwise_norm_modulate(xp, dt, M, K, ld, (float)PyFloat_AsDouble(a[11]), sp, tp, M / V, fused_add, rb, q, qs, st.handle);
+        break;
+    case I8F_PRO_RMS_NORM:
+        rc = lib.i8f_quant_rowwise_rms_norm(xp, dt, M, K, ld, (float)PyFloat_AsDouble(a[11]), w ? w->const_data_ptr() : nullptr, sp, tp, M / V,
+                                            fused_add, rb, q, qs, st.handle);
+        break;
+    case I8F_PRO_CONCAT_GELU: {
+        int64_t Mb, Kb, ldb;
+        rows_of(*s, Mb, Kb, ldb);
+        rc = lib.i8f_quant_rowwise_concat_gelu(xp, dt, M, K, ld, sp, Kb, ldb, rb, q, qs, st.handle);
+        break;
+    }
+    case I8F_PRO_SILU_GATE: rc = lib.i8f_quant_rowwise_prologue(xp, dt, M, K, ld, kind, sp, nullptr, 1, rb, q, qs, st.handle); break;
+    default:
+        rc = lib.i8f_quant_rowwise_prologue(xp, dt, M, K, ld, kind == I8F_PRO_MODULATE && fused_add ? (int)I8F_PRO_MODULATE_FUSED : kind, sp, tp,
+                                            M / V, rb, q, qs, st.handle);
+    }
+    if (rc) Py_RETURN_NONE;
+    rc = lib.i8f_linear_w8a8_gated(q, qs, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, gate ? gate->const_data_ptr() : nullptr, gate_rows,
+                                   res ? res->const_data_ptr() : nullptr, y.data_ptr(), dt, M, l.N, l.K, order, work ? work->data_ptr() : nullptr,
+                                   work ? work->numel() : 0, st.handle);
+    if (rc) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(y));
+}
+
+// vector_fanout(x, weights, scales, biases, per_row, rotate): tuples with one entry per layer -> list of outputs
+PyObject *vector_fanout(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 6) return PyErr_Format(PyExc_TypeError, "vector_fanout takes 6 arguments, got %zd", n);
+    const at::Tensor *xt = tensor(a[0]);
+    if (!lib.bound || !xt || !xt->is_cuda()) Py_RETURN_NONE;
+    const at::Tensor &x = *xt;
+    const int dt = code_of(x.scalar_type());
+    int64_t M, K, ld;
+    const Stream st(x.device());
+    const Py_ssize_t count = PyTuple_Check(a[1]) ? PyTuple_GET_SIZE(a[1]) : 0;
+    const bool rotate = a[5] == Py_True;
+    if (!st.ok || (dt != I8F_BF16 && dt != I8F_F16) || !rows_of(x, M, K, ld) || M > 16 || count < 2 || count > I8F_MAX_LINEAR_GROUPS ||
+        (rotate && K % 128))
+        Py_RETURN_NONE;
+    for (int i = 2; i <= 4; ++i)
+        if (!PyTuple_Check(a[i]) || PyTuple_GET_SIZE(a[i]) != count) Py_RETURN_NONE;
+    Layer l[I8F_MAX_LINEAR_GROUPS];
+    int bias_code = -1;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        if (!layer_of(PyTuple_GET_ITEM(a[1], i), PyTuple_GET_ITEM(a[2], i), PyTuple_GET_ITEM(a[3], i), PyTuple_GET_ITEM(a[4], i) == Py_True,
+                      x.device(), l[i]) ||
+            l[i].K != K || l[i].mode != l[0].mode)
+            Py_RETURN_NONE;
+        if (l[i].bias) {
+            if (bias_code >= 0 && bias_code != l[i].bias_code) Py_RETURN_NONE;
+            bias_code = l[i].bias_code;
+        }
+    }
+    const void *xp = x.const_data_ptr();
+    at::Tensor rotated;
+    if (rotate) {
+        rotated = empty({M, K}, x.scalar_type(), x.device());
+        if (lib.i8f_rotate128(xp, dt, M, K, ld, rotated.data_ptr(), st.handle)) Py_RETURN_NONE;
+        xp = rotated.const_data_ptr(), ld = K;
+    }
+    i8f_small_m_group g[I8F_MAX_LINEAR_GROUPS];
+    at::Tensor y[I8F_MAX_LINEAR_GROUPS];
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        y[i] = empty_output(x, l[i].N);
+        g[i] = {xp, M, K, ld, l[i].w, l[i].ws, l[i].ws_host, l[i].bias, y[i].data_ptr(), l[i].N};
+    }
+    if (lib.i8f_linear_w8a16_small_m_grouped(g, (int)count, dt, l[0].mode, bias_code < 0 ? (int)I8F_BF16 : bias_code, st.handle)) Py_RETURN_NONE;
+    PyObject *out = PyList_New(count);
+    if (!out) return nullptr;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        PyObject *o = THPVariable_Wrap(std::move(y[i]));
+        if (!o) {
+            Py_DECREF(out);
+            return nullptr;
+        }
+        PyList_SET_ITEM(out, i, o);
+    }
+    return out;
+}
+
+// No C++ exception leaves an entry point: an allocator that has nothing left, say, becomes the general path's to report.
+template <PyObject *(*F)(PyObject *, PyObject *const *, Py_ssize_t)>
+PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t n) {
+    try {
+        PyObject *r = F(self, a, n);
+        if (r == Py_None) PyErr_Clear();  // (an operand that is no number: the general path words it)
+        return r;
+    } catch (const std::exception &) {
+        Py_RETURN_NONE;
+    }
+}
+
+PyMethodDef methods[] = {
+    {"bind", bind, METH_O, "bind(path): load the kernels' library"},
+    {"linear", (PyCFunction)(void (*)(void))guarded<linear>, METH_FASTCALL, "one quantised layer, or None"},
+    {"vector_fanout", (PyCFunction)(void (*)(void))guarded<vector_fanout>, METH_FASTCALL, "several small-batch layers, or None"},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_i8f_host", "Native host path of the INT8 linear layers.", -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__i8f_host(void) { return PyModule_Create(&module); }

@@ -162,6 +162,12 @@ def forward_fanout(layers, x, prologue: int = _lib.PRO_NONE, mod_scale=None, mod
                     and not (lin.comfy_cast_weights or len(lin.weight_function) > 0 or len(lin.bias_function) > 0)
                     and (lin.bias is None or lin.bias.device == x.device) and bool(getattr(lin, "_use_quarot", False)) == rot
                     and lin.weight.shape[1] == x.shape[-1] for lin in layers)):
+        if type(x) is Tensor:
+            scales = tuple(lin._get_weight_scale() for lin in layers)
+            outs = _lib.host().vector_fanout(x, tuple(lin.weight for lin in layers), scales, tuple(lin.bias for lin in layers),
+                                             tuple(lin._is_per_row for lin in layers), rot)
+            if outs is not None:
+                return outs
         x_2d = x.reshape(-1, x.shape[-1])
         x_in = _lib.rotate128(x_2d) if rot else x_2d
         problems = []
@@ -560,6 +566,23 @@ class Int8TensorwiseOps(manual_cast):
                 self.bias = nn.Parameter(out_bias, requires_grad=False)
 
         # -- forward ------------------------------------------------------------------------
+        def _forward_native(self, x, prologue, mod_scale, mod_shift, eps, gate, residual, norm_weight, fused_add):
+            """forward() without the interpreter's part of it, for a quantised layer whose tensors are all in place (no
+            managed casting, no dynamic LoRA, 16-bit contiguous rows on the current GPU); None for everything else."""
+            weight, scale = self._parameters.get("weight"), self._weight_scale_scalar
+            if scale is None:
+                scale = self._buffers.get("weight_scale")
+            if (not self._is_quantized or self.lora_A is not None or self.comfy_cast_weights or weight is None or scale is None
+                    or len(self.weight_function) > 0 or len(self.bias_function) > 0 or x.shape[-1] == 0):
+                return None
+            if prologue == _lib.PRO_MODULATE_FUSED:
+                prologue, fused_add = _lib.PRO_MODULATE, True
+            N, K = weight.shape
+            work = _lib._splitk_workspace(x, x.numel() // x.shape[-1], N, K) if K >= _lib.SPLITK_MIN_K else None
+            return _lib.host().linear(x, weight, scale, self._parameters.get("bias"), self._is_per_row, bool(self._use_quarot), SMALL_BATCH_ROWS,
+                                      int8_fused_kernel.DEFAULT_EPILOGUE, prologue, mod_scale, mod_shift, eps, norm_weight, bool(fused_add), gate,
+                                      residual, work)
+
         def forward(self, x: Tensor, prologue: int = _lib.PRO_NONE, mod_scale: Tensor | None = None,
                     mod_shift: Tensor | None = None, eps: float = 1e-6, gate: Tensor | None = None,
                     residual: Tensor | None = None, norm_weight: Tensor | None = None, fused_add: bool = False) -> Tensor:
@@ -577,6 +600,10 @@ class Int8TensorwiseOps(manual_cast):
             apply to the result: forward(h, gate=g, residual=x) returns x + g * linear(h), the gated residual of an
             adaLN-Zero block (g broadcast over the token dimension like the modulation vectors), formed inside the GEMM
             epilogue with the roundings of torch's two operations; gate or residual alone work the same way."""
+            if not torch.compiler.is_compiling() and type(x) is Tensor and x.is_cuda:
+                y = self._forward_native(x, prologue, mod_scale, mod_shift, eps, gate, residual, norm_weight, fused_add)
+                if y is not None:
+                    return y
             managed = self.comfy_cast_weights or len(self.weight_function) > 0 or len(self.bias_function) > 0
             fuse_epilogue = False
             if gate is not None or residual is not None:

@@ -434,3 +434,36 @@ def test_forward_fanout_equals_the_layers_own_forward(pkg, dev, quarot):
     per_token = (torch.randn(1, 50, 384, generator=g) * 0.3).bfloat16().to(dev)      # a scale torch would broadcast differently
     outs = pkg.forward_fanout([q, v], x, prologue=L.PRO_RMS_NORM, norm_weight=nw, mod_scale=per_token, eps=1e-5)
     assert all(torch.equal(o, lin(F.rms_norm(x, (384,), nw, 1e-5) * (1 + per_token))) for o, lin in zip(outs, (q, v)))
+
+
+@pytest.mark.parametrize("case", ["plain", "rotated", "one scale", "small batch", "small batch rotated", "strided rows", "modulate", "modulate fused",
+                                  "norm modulate", "rms norm", "gelu", "gelu erf", "silu gate", "concat gelu", "gate and residual", "long k"])
+def test_native_host_path_equals_the_general_path(pkg, dev, monkeypatch, case):
+    """Linear.forward through the native host path and with that path switched off: the same launches, so the same bits; the
+    native path has to have taken the case."""
+    L, ops = pkg._lib, pkg.Int8TensorwiseOps
+    B, T, K, N = 2, (5 if case.startswith("small") else 40), (10240 if case == "long k" else 384), 264
+    rotate = case.endswith("rotated")
+    q, s = L.quant_rowwise((torch.randn(N, K, generator=G) * 0.02).to(dev), rotate=rotate)
+    lin = load(ops.Linear(K, N, bias=True), {"l.weight": q, "l.weight_scale": s[:1].clone() if case == "one scale" else s,
+                                             "l.bias": torch.randn(N, generator=G).bfloat16().to(dev)})
+    lin._use_quarot = rotate
+    rand = lambda *shape: torch.randn(*shape, generator=G).bfloat16().to(dev)
+    x, vec = rand(B, T, K), lambda n: rand(B, 1, n)
+    kw = {"modulate": dict(prologue=L.PRO_MODULATE, mod_scale=vec(K), mod_shift=vec(K)),
+          "modulate fused": dict(prologue=L.PRO_MODULATE_FUSED, mod_scale=vec(K), mod_shift=vec(K)),
+          "norm modulate": dict(prologue=L.PRO_NORM_MODULATE, mod_scale=vec(K), mod_shift=vec(K), eps=1e-5),
+          "rms norm": dict(prologue=L.PRO_RMS_NORM, mod_scale=vec(K), norm_weight=rand(K)), "gelu": dict(prologue=L.PRO_GELU_TANH),
+          "gelu erf": dict(prologue=L.PRO_GELU_ERF), "silu gate": dict(prologue=L.PRO_SILU_GATE, mod_scale=rand(B, T, K)),
+          "concat gelu": dict(prologue=L.PRO_CONCAT_GELU, mod_scale=rand(B, T, 2 * 128)[..., 128:]),
+          "gate and residual": dict(gate=vec(N), residual=rand(B, T, N))}.get(case, {})
+    if case == "concat gelu":
+        x = rand(B, T, 512)[..., :256]
+    if case == "strided rows":
+        x = rand(B, T, K + 16)[..., :K]
+    native, taken = lin._forward_native, []
+    monkeypatch.setattr(lin, "_forward_native", lambda *a: taken.append(native(*a)) or taken[-1])
+    y = lin(x, **kw)
+    assert taken[0] is not None and y is taken[0] and y.shape == (B, T, N)
+    monkeypatch.setattr(lin, "_forward_native", lambda *a: None)
+    assert torch.equal(y, lin(x, **kw))
