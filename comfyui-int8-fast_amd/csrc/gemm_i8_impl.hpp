@@ -600,6 +600,15 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
                 __builtin_amdgcn_s_waitcnt(waitcnt_vm(YOUNGER) & 0xF0FF);
                 __builtin_amdgcn_s_barrier();
             }
+            // The waves of a SIMD leave the barrier together and the older one wins every issue slot: it ran a whole K-tile's
+            // MFMAs while the younger one had done a third of its own, then waited at the barrier with the matrix pipe half
+            // used.  With the two phases behind the barrier at a higher priority, a wave that is ahead yields to the one that is
+            // still in them: 2 250 cycles a K-tile of 256 x 256 instead of 2 380 (2 048 are its MFMAs).  In time 1 to 4 %: at
+            // the power limit the chip gives part of it back as a lower clock.
+            if constexpr (M16) {
+                if (last) __builtin_amdgcn_s_setprio(1);
+                if (ks == 1) __builtin_amdgcn_s_setprio(0);
+            }
             v4i(&xc)[XF] = (ks & 1) ? xb : xa;
             v4i(&xn)[XF] = (ks & 1) ? xa : xb;
             // (16x16x64: one set of column fragments, each replaced as soon as its last MFMA of a k-step has issued)
@@ -660,6 +669,7 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
         }
         ix = ix1, iw = iw1;
     }
+    if constexpr (M16) __builtin_amdgcn_s_setprio(0);
 
     // ---- epilogue ----------------------------------------------------------------------
     // The loads issued past the last tile move no data from memory but still zero-fill their LDS
@@ -1006,7 +1016,9 @@ namespace gemm {
 #ifndef I8F_WST
 #define I8F_WST 3
 #endif
-using CfgBig = Cfg<256, 256, 128, 2, 4, 2, 6, 0x4400, 16, I8F_WST>;  // 8 waves, 2 X and 3 W stages of 32 KB (all of the LDS), one workgroup per CU
+// 8 waves of 64 x 128, 2 X and 3 W stages of 32 KB (all of the LDS), one workgroup per CU.  (Waves of 128 x 64 read as much
+// from LDS but take 1 to 3 % longer: 8192^3 385 against 379 us, 4608 x 3072 x 12288 129.5 against 126 us.)
+using CfgBig = Cfg<256, 256, 128, 4, 2, 2, 6, 0x4400, 16, I8F_WST>;
 using CfgB192 = Cfg<256, 192, 128, 4, 2, 2, 6, 0x4300, 16, I8F_WST>;  // 8 waves of 64 x 96, 2 x 32 + 3 x 24 KB: fills 256 CUs where 256 x 256 leaves a partial round
 using CfgMid = Cfg<128, 128, 128, 2, 2, 2, 8>;   // 4 waves, 2 x 32 KB stages, two workgroups per CU (10 % slower with the 16x16x64 MFMA: 32x32x32)
 using CfgTall = Cfg<288, 256, 128, 3, 4, 2, 8, 0, 16>;  // 12 waves of 96 x 64, 2 x 72 KB stages
