@@ -21,6 +21,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../../include/i8f.h"
+#include "../w8a16_rotated.hpp"
 
 namespace {
 
@@ -28,7 +29,7 @@ namespace {
 #define I8F_ENTRY_POINTS(X)                                                                                              \
     X(i8f_quant_rowwise) X(i8f_quant_rowwise_prologue) X(i8f_quant_rowwise_norm_modulate) X(i8f_quant_rowwise_rms_norm)  \
     X(i8f_quant_rowwise_concat_gelu) X(i8f_rotate128) X(i8f_linear_w8a8_gated) X(i8f_linear_w8a16_small_m)               \
-    X(i8f_linear_w8a16_small_m_grouped)
+    X(i8f_linear_w8a16_small_m_grouped) X(i8f_internal_w8a16_rotated)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     I8F_ENTRY_POINTS(X)
@@ -145,13 +146,14 @@ struct Stream {
 PyObject *small_m(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, const Layer &l, bool rotate, void *stream) {
     const int dt = code_of(x.scalar_type());
     const void *xp = x.const_data_ptr();
-    at::Tensor rotated;
+    at::Tensor rotated, y = empty_output(x, l.N);
     if (rotate) {
+        if (!lib.i8f_internal_w8a16_rotated(xp, dt, M, K, ld, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, y.data_ptr(), l.N, stream))
+            return THPVariable_Wrap(std::move(y));
         rotated = empty({M, K}, x.scalar_type(), x.device());
         if (lib.i8f_rotate128(xp, dt, M, K, ld, rotated.data_ptr(), stream)) Py_RETURN_NONE;
         xp = rotated.const_data_ptr(), ld = K;
     }
-    at::Tensor y = empty_output(x, l.N);
     if (lib.i8f_linear_w8a16_small_m(xp, dt, M, K, ld, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, y.data_ptr(), l.N, stream))
         Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(y));

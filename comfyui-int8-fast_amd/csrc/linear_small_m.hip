@@ -15,6 +15,8 @@
 // differs between the two; the result is compared with a tolerance of one
 // rounding step of the output type.
 #include "i8f_common.hpp"
+#include "rotate_run.hpp"
+#include "w8a16_rotated.hpp"
 
 namespace i8f {
 namespace {
@@ -167,10 +169,16 @@ __device__ __forceinline__ v4f_t mma8(uint32_t wlo, uint32_t whi, v4u_t xk, floa
 // instruction touched.
 // (The body is shared by the kernel of one layer and the kernel of several layers in one launch: `block` is the
 // workgroup's number within its layer.)
-template <int DT, int NB, int WAVES>
+// ROT: x, 8 rows or fewer, is rotated on the way (the layer's weight is rotated; K % 128 == 0).  A step is one 128-block of
+// every row, so the wave rotates what it is about to multiply, 8 lanes of 16 elements to a row's block, and takes it through a
+// tile of its own into the operand layout.  Every workgroup rotates all of x again, mostly while its weights are on their
+// way; what it saves is the rotation's own launch (i8f_internal_w8a16_rotated has the figures).
+template <int DT, int NB, int WAVES, bool ROT>
 __device__ __forceinline__ void small_m_lds_body(const SmallMArgs &a, const int64_t block) {
     constexpr int COLS = NB * 16;
     constexpr int PITCH = 144;
+    constexpr int XPITCH = 256 + 16;
+    __shared__ __attribute__((aligned(16))) char xtiles[ROT ? WAVES : 1][ROT ? 8 * XPITCH : 16];
     __shared__ float red[WAVES][COLS][16];
     __shared__ __attribute__((aligned(16))) char tiles[WAVES][COLS * PITCH];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -182,6 +190,7 @@ __device__ __forceinline__ void small_m_lds_body(const SmallMArgs &a, const int6
     const bool xrow = r < (int)a.M;
     const char *xp = (const char *)a.x + (int64_t)(xrow ? r : 0) * a.ldx * 2;
     char *tile = tiles[wave];
+    [[maybe_unused]] char *xtile = xtiles[ROT ? wave : 0];
 
     const int8_t *frow[NB][2];
     float wsn[NB];
@@ -199,7 +208,10 @@ __device__ __forceinline__ void small_m_lds_body(const SmallMArgs &a, const int6
     }
 
     const v4u_t zero = {0u, 0u, 0u, 0u};
-    v4u_t wq[2][NB][2], xq[2][4];
+    v4u_t wq[2][NB][2], xq[2][ROT ? 2 : 4];
+    // the run of a row's 128-block that this lane rotates: lanes 4..7 of a group of 8 take runs 7..4 (rotate_run16)
+    [[maybe_unused]] const int run = (lane & 7) ^ (((lane >> 2) & 1) * 3);
+    [[maybe_unused]] const float s0 = (run & 1) ? -1.0f : 1.0f, s1 = (run & 2) ? -1.0f : 1.0f, s2 = (run & 4) ? -1.0f : 1.0f;
     auto fetch = [&](int t, int buf) __attribute__((always_inline)) {
         const int kw = t * 128;
         const bool wok = kw + lc * 16 + 16 <= K;
@@ -210,9 +222,16 @@ __device__ __forceinline__ void small_m_lds_body(const SmallMArgs &a, const int6
         // MFMA j takes k = kw + 32 j ... + 31, its lane group g the 8 values from 8 g on: the four groups of a row
         // read 64 contiguous bytes per instruction (with the groups 32 values apart every instruction touched twice
         // the cache lines, which is what M = 16 paid for: 21.7 -> 19.5 us at 18432 x 3072)
+        if constexpr (ROT) {
+            const bool in = lr < (int)a.M;
+            const char *src = (const char *)a.x + ((int64_t)(in ? lr : 0) * a.ldx + kw + run * 16) * 2;
+            xq[buf][0] = in ? *(const v4u_t *)src : zero;
+            xq[buf][1] = in ? *(const v4u_t *)(src + 16) : zero;
+            return;
+        }
         const int k = kw + g * 8;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < (ROT ? 0 : 4); ++j)
             xq[buf][j] = (xrow && k + 32 * j + 8 <= K) ? *(const v4u_t *)(xp + (int64_t)(k + 32 * j) * 2) : zero;
     };
     v4f_t acc[NB];
@@ -220,6 +239,20 @@ __device__ __forceinline__ void small_m_lds_body(const SmallMArgs &a, const int6
     for (int b = 0; b < NB; ++b) acc[b] = v4f_t{0.f, 0.f, 0.f, 0.f};
 
     auto compute = [&](int buf) __attribute__((always_inline)) {
+        if constexpr (ROT) {   // (in front of the weights' exchange: x comes from cache and is there first)
+            float v[16];
+            const v4u_t lo = xq[buf][0], hi = xq[buf][1];
+            expand16<DT>(make_uint4(lo.x, lo.y, lo.z, lo.w), make_uint4(hi.x, hi.y, hi.z, hi.w), v);
+            rotate_run16<DT>(v, s0, s1, s2);
+            uint32_t o[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e)   // (the values are of the dtype already)
+                o[e] = DT == I8F_BF16 ? (__float_as_uint(v[2 * e]) >> 16) | (__float_as_uint(v[2 * e + 1]) & 0xffff0000u)
+                                      : f32x2_to_f16x2_bits(v[2 * e], v[2 * e + 1]);
+            char *dst = xtile + lr * XPITCH + run * 32;
+            *(v4u_t *)dst = v4u_t{o[0], o[1], o[2], o[3]};
+            *(v4u_t *)(dst + 16) = v4u_t{o[4], o[5], o[6], o[7]};
+        }
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -229,6 +262,12 @@ __device__ __forceinline__ void small_m_lds_body(const SmallMArgs &a, const int6
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         v2u_t wa[NB][4];
+        v4u_t xk[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if constexpr (ROT) xk[j] = r < 8 ? *(const v4u_t *)(xtile + r % 8 * XPITCH + (32 * j + 8 * g) * 2) : zero;
+            else xk[j] = xq[buf][j];
+        }
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -237,7 +276,7 @@ __device__ __forceinline__ void small_m_lds_body(const SmallMArgs &a, const int6
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[b] = mma8<DT>(wa[b][j].x, wa[b][j].y, xq[buf][j], wsn[b], acc[b]);
+            for (int j = 0; j < 4; ++j) acc[b] = mma8<DT>(wa[b][j].x, wa[b][j].y, xk[j], wsn[b], acc[b]);
     };
 
     int t = wave;
@@ -275,9 +314,9 @@ __device__ __forceinline__ void small_m_lds_body(const SmallMArgs &a, const int6
     }
 }
 
-template <int DT, int NB, int WAVES>
+template <int DT, int NB, int WAVES, bool ROT>
 __global__ __launch_bounds__(WAVES * 64) void small_m_lds_kernel(const SmallMArgs a) {
-    small_m_lds_body<DT, NB, WAVES>(a, (int64_t)blockIdx.x);
+    small_m_lds_body<DT, NB, WAVES, ROT>(a, (int64_t)blockIdx.x);
 }
 
 // Several layers in one launch (the modulation projections of the image and of the text stream of a double-stream
@@ -290,7 +329,7 @@ struct SmallMGroups {
     int n;
 };
 
-template <int DT, int NB, int WAVES>
+template <int DT, int NB, int WAVES, bool ROT>
 __global__ __launch_bounds__(WAVES * 64) void small_m_lds_grouped_kernel(const SmallMGroups gg) {
     int grp = 0;
 #pragma unroll
@@ -301,13 +340,13 @@ __global__ __launch_bounds__(WAVES * 64) void small_m_lds_grouped_kernel(const S
 #pragma unroll
     for (int i = 1; i < MAX_SMALL_M_GROUPS; ++i)
         if (grp == i) a = gg.a[i];
-    small_m_lds_body<DT, NB, WAVES>(a, (int64_t)((int)blockIdx.x - gg.first_block[grp]));
+    small_m_lds_body<DT, NB, WAVES, ROT>(a, (int64_t)((int)blockIdx.x - gg.first_block[grp]));
 }
 
-template <int DT, int NB, int WAVES>
+template <int DT, int NB, int WAVES, bool ROT = false>
 int launch_lds(const SmallMArgs &a, hipStream_t st) {
     const int64_t cols = NB * 16;
-    hipLaunchKernelGGL((small_m_lds_kernel<DT, NB, WAVES>), dim3((unsigned)((a.N + cols - 1) / cols)), dim3(WAVES * 64), 0, st, a);
+    hipLaunchKernelGGL((small_m_lds_kernel<DT, NB, WAVES, ROT>), dim3((unsigned)((a.N + cols - 1) / cols)), dim3(WAVES * 64), 0, st, a);
     return check_launch();
 }
 
@@ -351,8 +390,8 @@ int launch_grouped(const SmallMArgs *as, int n, hipStream_t st) {
     }
     for (int i = n; i <= MAX_SMALL_M_GROUPS; ++i) gg.first_block[i] = (int)first;
     if (first > 0x7fffffff) return I8F_ERR_UNSUPPORTED;
-    if (two) hipLaunchKernelGGL((small_m_lds_grouped_kernel<DT, 2, 8>), dim3((unsigned)first), dim3(512), 0, st, gg);
-    else hipLaunchKernelGGL((small_m_lds_grouped_kernel<DT, 1, 8>), dim3((unsigned)first), dim3(512), 0, st, gg);
+    if (two) hipLaunchKernelGGL((small_m_lds_grouped_kernel<DT, 2, 8, false>), dim3((unsigned)first), dim3(512), 0, st, gg);
+    else hipLaunchKernelGGL((small_m_lds_grouped_kernel<DT, 1, 8, false>), dim3((unsigned)first), dim3(512), 0, st, gg);
     return check_launch();
 }
 
@@ -423,4 +462,23 @@ extern "C" int i8f_linear_w8a16_small_m(const void *x, int x_dtype, int64_t M, i
     case I8F_F16: return launch<I8F_F16>(a, st);
     default: return launch<I8F_F32>(a, st);
     }
+}
+
+// The layer of a rotated weight in one launch: up to 8 rows, while every workgroup finds a CU of its own and the rotation, which
+// is the same in every one of them, stays short beside the weight stream.  us per call, weights from HBM, against
+// i8f_rotate128 and the layer: 4 x 3072 -> 3072 7.6 and 8.0, 8 x 3072 -> 4096 7.4 and 8.3, 8 x 1536 -> 3072 4.8 and 6.6,
+// 4 x 256 -> 512 2.9 and 4.6; beyond the line 4 x 6144 -> 3072 12.8 and 11.0, 4 x 3072 -> 6144 11.3 and 10.4 (two passes of 8
+// rows: 9 x 3072 -> 3072 8.9 and 8.2).  From an eager layer the launch saved counts for more: 4 x 3072 -> 3072 6.7 and 10.3.
+extern "C" int i8f_internal_w8a16_rotated(const void *x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t *w, const float *w_scale,
+                                          float w_scale_host, int scale_mode, const void *bias, int bias_dtype, void *out, int64_t N, void *stream) {
+    using namespace i8f;
+    if (M < 1 || M > 8 || N < 1 || N > 4096 || K < 128 || K > 3072 || K % 128 || (x_dtype != I8F_BF16 && x_dtype != I8F_F16) ||
+        (bias && !valid_dtype(bias_dtype)) || !x || !w || !out || ldx < K || (scale_mode == I8F_SCALE_ROW && !w_scale))
+        return I8F_ERR_UNSUPPORTED;
+    if ((uintptr_t)w % 16 || (uintptr_t)x % 16 || ldx % 8) return I8F_ERR_UNSUPPORTED;
+    if (int rc = check_device()) return rc;
+    SmallMArgs a{};
+    a.x = x, a.M = M, a.K = K, a.ldx = ldx, a.N = N, a.w = w, a.ws = w_scale, a.ws_host = w_scale_host;
+    a.row_scale = scale_mode == I8F_SCALE_ROW, a.bias = bias, a.bias_dtype = bias_dtype, a.out = out;
+    return x_dtype == I8F_BF16 ? launch_lds<I8F_BF16, 1, 8, true>(a, (hipStream_t)stream) : launch_lds<I8F_F16, 1, 8, true>(a, (hipStream_t)stream);
 }

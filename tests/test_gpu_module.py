@@ -467,3 +467,21 @@ def test_native_host_path_equals_the_general_path(pkg, dev, monkeypatch, case):
     assert taken[0] is not None and y is taken[0] and y.shape == (B, T, N)
     monkeypatch.setattr(lin, "_forward_native", lambda *a: None)
     assert torch.equal(y, lin(x, **kw))
+
+
+@pytest.mark.parametrize("M,K,N,dt", [(1, 128, 9, torch.bfloat16), (8, 3072, 4096, torch.bfloat16), (4, 384, 3072, torch.float16), (7, 1280, 1001, torch.float16),
+                                      (9, 256, 64, torch.bfloat16), (3, 3200, 48, torch.bfloat16), (2, 256, 4104, torch.float16)])
+def test_small_batch_layer_of_a_rotated_weight_equals_rotation_and_layer(pkg, dev, M, K, N, dt):
+    """x rotated inside the small-batch kernel (8 rows, width 3072, 4096 outputs and less) or by a launch in front of it: the
+    same bits, rows at a stride and large, small and non-finite values included."""
+    L = pkg._lib
+    q, s = L.quant_rowwise((torch.randn(N, K, generator=G) * 0.02).to(dev), rotate=True)
+    lin = load(pkg.Int8TensorwiseOps.Linear(K, N, bias=True), {"l.weight": q, "l.weight_scale": s, "l.bias": torch.randn(N, generator=G).to(dt).to(dev)})
+    lin._use_quarot = True
+    x = (torch.randn(M, K + 24, generator=G) * torch.exp2(torch.randint(-12, 6, (M, K + 24), generator=G).float())).to(dt).to(dev)
+    x[-1, 0] = float("inf")
+    for rows in (x[:, :K].contiguous(), x[:, 8:K + 8]):
+        want = L.linear_w8a16_small_m(L.rotate128(rows), q, s, lin.bias)
+        got = lin(rows)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(), want.nan_to_num())
+        assert torch.isfinite(want[:-1]).all()
