@@ -44,63 +44,86 @@ __device__ __forceinline__ void finish_one(const GemmArgs &g, int acc, int m, in
 // last chunk, where K is no multiple of 16, is cut from the 16 bytes that end the row, so nothing outside the matrices is read.
 // LDS is double-buffered: one barrier per K-tile.  The accumulators go through LDS once more so that a wave stores whole
 // runs of a row, element by element: rows of N outputs start at any address.
-// What bounds it: the latency of the loads, a K-tile taking about as long as a round trip to L2 (333 x 1001 x 1160, 96
-// workgroups: 10.1 us for 0.8 GOP; 1536 us with one thread per output, the form this kernel replaces).
-template <int OUT, int BM, int BN>
-__global__ __launch_bounds__(256) void gemm_i8_ragged_kernel(const GemmArgs g) {
+// TINY: K < 16, where a row has no 16 bytes to end it.
+// What bounds it: 333 x 1001 x 1160 (96 workgroups) 9 us, 3 of them the launch, the first loads and the epilogue, then 0.4 us
+// a K-tile for the chain from LDS write to product and half as much again for chunks that straddle lines; 4096 x 3071 x 3083
+// 90 us, the loads of the two workgroups of a CU.  Two things made it that: the loads of a K-tile are issued without a branch
+// or a use near them (the compiler put a wait for all loads in flight at each join: 11.8 and 110 us before), and the
+// epilogue's operands come first instead of last.  Two waves to a SIMD is what the registers have to leave room for: with one
+// the larger shape takes 119 us.
+template <int OUT, int BM, int BN, bool TINY>
+__global__ __launch_bounds__(256, 2) void gemm_i8_ragged_kernel(const GemmArgs g) {
+    constexpr int AHEAD = 2;  // K-tiles in flight (4, 6 and 8 measured the same or slower)
     constexpr int BK = 128, MI = BM / 64, NJ = BN / 64;
     constexpr int XC = BM * 8 / 256, WC = BN * 8 / 256;  // 16-byte chunks per thread and K-tile
     constexpr int STAGE = (BM + BN) * BK;
     constexpr int PITCH = BN + 4;                         // ints per row of the output tile in LDS
     constexpr int SMEM = 2 * STAGE > BM * PITCH * 4 ? 2 * STAGE : BM * PITCH * 4;
-    static_assert(SMEM <= 160 * 1024 && 256 % BN == 0, "LDS; a thread keeps one column in the epilogue");
+    static_assert(SMEM + BM * 4 <= 160 * 1024 && 256 % BN == 0, "LDS; a thread keeps one column in the epilogue");
     __shared__ __attribute__((aligned(16))) char smem[SMEM];
+    __shared__ float s_xs[BM];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1, l32 = lane & 31, lhalf = lane >> 5;
     const int tiles_m = (g.M + BM - 1) / BM;
     const int m0 = (int)(blockIdx.x % (unsigned)tiles_m) * BM, n0 = (int)(blockIdx.x / (unsigned)tiles_m) * BN;
-    const int K = g.K, KT = (K + BK - 1) / BK;
+    const int K = g.K, KT = (int)(((int64_t)K + BK - 1) / BK);
 
-    const int8_t *src[XC + WC];   // this thread's chunks at K-tile 0; rows past the end repeat the last one (never stored)
+    // the epilogue's operands, requested in front of everything else: the thread's column, and (for all) the tile's rows
+    const int n = n0 + tid % BN;
+    float ws = 0.0f, b = 0.0f, xs = 0.0f;
+    if constexpr (OUT != OUT_I32) {
+        const int nc = min(n, g.N - 1);
+        ws = g.ws ? g.ws[g.row_scale ? nc : 0] : g.ws_host;
+        if (g.bias) {
+            if (g.bias_dtype == I8F_F32) b = ((const float *)g.bias)[nc];
+            else if (g.bias_dtype == I8F_BF16) b = bf16_bits_to_f32(((const uint16_t *)g.bias)[nc]);
+            else b = f16_bits_to_f32(((const uint16_t *)g.bias)[nc]);
+        }
+        if (tid < BM) xs = g.xs[min(m0 + tid, g.M - 1)];
+    }
+
+    const int8_t *src[XC + WC];   // the rows of this thread's chunks; rows past the end repeat the last one (never stored)
     int dst[XC + WC];
     const int c = tid & 7;
 #pragma unroll
     for (int t = 0; t < XC + WC; ++t) {
         const bool is_x = t < XC;
         const int row = (is_x ? t : t - XC) * 32 + (tid >> 3);
-        src[t] = (is_x ? g.x + (int64_t)min(m0 + row, g.M - 1) * K : g.w + (int64_t)min(n0 + row, g.N - 1) * K) + c * 16;
+        src[t] = is_x ? g.x + (int64_t)min(m0 + row, g.M - 1) * K : g.w + (int64_t)min(n0 + row, g.N - 1) * K;
         dst[t] = (is_x ? 0 : BM * BK) + row * BK + (c ^ swz<8>(row)) * 16;
     }
-    v4i reg[2][XC + WC];
+    v4i reg[AHEAD][XC + WC];
+    // A K-tile's loads and nothing else: no branch (past the last K-tile that one is fetched again) and no use of what they
+    // bring, or the compiler would wait for all of them here.
     auto fetch = [&](int kt, v4i (&r)[XC + WC]) __attribute__((always_inline)) {
-        const int kb = kt * BK;
-        if (kb + BK <= K) {
-#pragma unroll
-            for (int t = 0; t < XC + WC; ++t) __builtin_memcpy(&r[t], src[t] + kb, 16);
-        } else {
+        if constexpr (TINY) {  // K < 16: the only chunk with bytes in it is the first
 #pragma unroll
             for (int t = 0; t < XC + WC; ++t) {
-                const int left = K - kb - c * 16;  // bytes of the row from this chunk on
-                uint64_t lo = 0, hi = 0;
-                if (K >= 16) {  // the row's last 16 bytes, moved down by what precedes the chunk in them
-                    v4i v;
-                    __builtin_memcpy(&v, src[t] + kb + (left < 16 ? left - 16 : 0), 16);
-                    lo = (uint32_t)v.x | (uint64_t)(uint32_t)v.y << 32, hi = (uint32_t)v.z | (uint64_t)(uint32_t)v.w << 32;
-                    const int sh = left >= 16 ? 0 : (left > 0 ? (16 - left) * 8 : 128);
-                    if (sh >= 128) lo = hi = 0;
-                    else if (sh >= 64) lo = hi >> (sh - 64), hi = 0;
-                    else if (sh > 0) lo = lo >> sh | hi << (64 - sh), hi >>= sh;
-                } else {
-                    for (int e = 0; e < left; ++e) {
-                        const uint64_t b = (uint8_t)src[t][e];
-                        if (e < 8) lo |= b << (8 * e);
-                        else hi |= b << (8 * (e - 8));
-                    }
-                }
-                r[t] = v4i{(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
+                uint32_t b[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int e = 0; e < 15; ++e)
+                    if (c == 0 && e < K) b[e / 4] |= (uint32_t)(uint8_t)src[t][e] << (8 * (e % 4));
+                r[t] = v4i{(int)b[0], (int)b[1], (int)b[2], (int)b[3]};
             }
+        } else {
+            const uint32_t pos = min((uint32_t)min(kt, KT - 1) * BK + c * 16, (uint32_t)K - 16);
+#pragma unroll
+            for (int t = 0; t < XC + WC; ++t) __builtin_memcpy(&r[t], src[t] + pos, 16);
+        }
+    };
+    // of the last K-tile's chunks, which end with the row: what precedes the chunk in them is shifted out
+    const int left = K - (KT - 1) * BK - c * 16;
+    const int sh = TINY || left >= 16 ? 0 : (left > 0 ? (16 - left) * 8 : 128);
+    auto cut_tail = [&](v4i (&r)[XC + WC]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < XC + WC; ++t) {
+            uint64_t lo = (uint32_t)r[t].x | (uint64_t)(uint32_t)r[t].y << 32, hi = (uint32_t)r[t].z | (uint64_t)(uint32_t)r[t].w << 32;
+            if (sh >= 128) lo = hi = 0;
+            else if (sh >= 64) lo = hi >> (sh - 64), hi = 0;
+            else if (sh > 0) lo = lo >> sh | hi << (64 - sh), hi >>= sh;
+            r[t] = v4i{(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
         }
     };
 
@@ -114,34 +137,52 @@ __global__ __launch_bounds__(256) void gemm_i8_ragged_kernel(const GemmArgs g) {
 
     const int sw = swz<8>(l32);
     auto step = [&](int kt, v4i (&r)[XC + WC], char *st) __attribute__((always_inline)) {
+        if (kt == KT - 1) cut_tail(r);
 #pragma unroll
         for (int t = 0; t < XC + WC; ++t) *(v4i *)(st + dst[t]) = r[t];
-        if (kt + 2 < KT) fetch(kt + 2, r);
+        if constexpr (!TINY) fetch(kt + AHEAD, r);
         // (a bare barrier: __syncthreads() would also wait for the loads of the next K-tiles)
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        // (the small tile has one product per wave and k-step: all of its fragments first, one LDS latency instead of four)
+        constexpr int AT_ONCE = MI * NJ == 1 ? 4 : 1;
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const int ko = ((ks * 2 + lhalf) ^ sw) * 16;
-            v4i xf[MI], wf[NJ];
+        for (int k0 = 0; k0 < 4; k0 += AT_ONCE) {
+            v4i xf[AT_ONCE][MI], wf[AT_ONCE][NJ];
 #pragma unroll
-            for (int i = 0; i < MI; ++i) xf[i] = *(const v4i *)(st + (wm * (BM / 2) + i * 32 + l32) * BK + ko);
+            for (int u = 0; u < AT_ONCE; ++u) {
+                const int ko = (((k0 + u) * 2 + lhalf) ^ sw) * 16;
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) wf[j] = *(const v4i *)(st + BM * BK + (wn * (BN / 2) + j * 32 + l32) * BK + ko);
+                for (int i = 0; i < MI; ++i) xf[u][i] = *(const v4i *)(st + (wm * (BM / 2) + i * 32 + l32) * BK + ko);
 #pragma unroll
-            for (int i = 0; i < MI; ++i)
+                for (int j = 0; j < NJ; ++j) wf[u][j] = *(const v4i *)(st + BM * BK + (wn * (BN / 2) + j * 32 + l32) * BK + ko);
+            }
+            if constexpr (AT_ONCE > 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[j], xf[i], acc[i][j], 0, 0, 0);
+            for (int u = 0; u < AT_ONCE; ++u)
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[u][j], xf[u][i], acc[i][j], 0, 0, 0);
         }
     };
-    if (KT > 0) fetch(0, reg[0]);
-    if (KT > 1) fetch(1, reg[1]);
-    for (int kt = 0; kt < KT; kt += 2) {
-        step(kt, reg[0], smem);
-        if (kt + 1 < KT) step(kt + 1, reg[1], smem + STAGE);
+    if (KT > 0) {
+#pragma unroll
+        for (int u = 0; u < (TINY ? 1 : AHEAD); ++u) {
+            fetch(u, reg[u]);
+            __builtin_amdgcn_sched_barrier(0);  // (in the order in which they are waited for)
+        }
+    }
+    for (int kt = 0; kt < KT; kt += AHEAD) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            if (kt + u >= KT) break;
+            step(kt + u, reg[u], smem + (u & 1) * STAGE);
+        }
     }
 
     __syncthreads();
     int *const tile = (int *)smem;
+    if (tid < BM) s_xs[tid] = xs;
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -151,20 +192,10 @@ __global__ __launch_bounds__(256) void gemm_i8_ragged_kernel(const GemmArgs g) {
                 *(v4i *)(tile + (wm * (BM / 2) + i * 32 + l32) * PITCH + wn * (BN / 2) + j * 32 + qd * 8 + lhalf * 4) =
                     v4i{acc[i][j][4 * qd], acc[i][j][4 * qd + 1], acc[i][j][4 * qd + 2], acc[i][j][4 * qd + 3]};
     __syncthreads();
-    const int n = n0 + tid % BN;
     if (n >= g.N) return;
-    float ws = 0.0f, b = 0.0f;
-    if constexpr (OUT != OUT_I32) {
-        ws = g.ws ? g.ws[g.row_scale ? n : 0] : g.ws_host;
-        if (g.bias) {
-            if (g.bias_dtype == I8F_F32) b = ((const float *)g.bias)[n];
-            else if (g.bias_dtype == I8F_BF16) b = bf16_bits_to_f32(((const uint16_t *)g.bias)[n]);
-            else b = f16_bits_to_f32(((const uint16_t *)g.bias)[n]);
-        }
-    }
-#pragma unroll 4
+#pragma unroll 8
     for (int row = tid / BN; row < BM; row += 256 / BN) {
-        if (m0 + row < g.M) finish_one<OUT>(g, tile[row * PITCH + tid % BN], m0 + row, n, OUT == OUT_I32 ? 0.0f : g.xs[m0 + row], ws, b);
+        if (m0 + row < g.M) finish_one<OUT>(g, tile[row * PITCH + tid % BN], m0 + row, n, OUT == OUT_I32 ? 0.0f : s_xs[row], ws, b);
     }
 }
 
@@ -172,11 +203,12 @@ template <int OUT>
 int launch_ragged(const GemmArgs &g, hipStream_t st) {
     const int64_t t128 = (((int64_t)g.M + 127) / 128) * (((int64_t)g.N + 127) / 128);
     const int64_t t64 = (((int64_t)g.M + 63) / 64) * (((int64_t)g.N + 63) / 64);
-    // 128 x 128 tiles once they fill two workgroups on every CU: they fetch half the bytes per product, but a CU with one or two
-    // of them has too few loads in flight (2500 x 2501 x 1160, 400 tiles: 33.1 us against 29.0 with 64 x 64 tiles, four or
-    // five workgroups to a CU; 4096 x 3071 x 3083, 768 tiles: 102 us against 123)
-    if (t128 >= 512) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 128, 128>), dim3((unsigned)t128), dim3(256), 0, st, g);
-    else hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64>), dim3((unsigned)t64), dim3(256), 0, st, g);
+    // 128 x 128 tiles once there is one for every CU: half the bytes per product (1024 x 3001 x 3083, 192 tiles: 40.0 us
+    // against 41.4 with 64 x 64 tiles; 2500 x 2501 x 1160, 400 tiles: 26.7 both; 2100 x 3001 x 3083, 408 tiles: 62 against
+    // 83); below that they leave CUs idle (1500 x 1500 x 1500, 144 tiles: 21.9 against 16.2).
+    if (g.K < 16) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, true>), dim3((unsigned)t64), dim3(256), 0, st, g);
+    else if (t128 >= 256) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 128, 128, false>), dim3((unsigned)t128), dim3(256), 0, st, g);
+    else hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, false>), dim3((unsigned)t64), dim3(256), 0, st, g);
     return check_launch();
 }
 

@@ -521,7 +521,8 @@ def test_gemm_i32_misaligned_operands_use_the_generic_kernel(L, dev):
 
 @pytest.mark.parametrize("M,N,K", [
     (1, 1, 1), (3, 65, 15), (64, 64, 17), (65, 63, 127), (63, 129, 129), (70, 9, 263), (129, 1001, 1160),   # edges of tiles and of 16-byte chunks
-    (2050, 2047, 40), (2048, 2049, 143),                                                                    # 128 x 128 tiles
+    (2050, 2047, 40), (2048, 2049, 143), (2050, 2047, 390),                                                 # 128 x 128 tiles
+    (5, 30, 1), (66, 20, 16), (65, 33, 113), (64, 65, 255), (64, 65, 257), (30, 40, 500),                   # one to four K-tiles, every kind of tail
 ])
 def test_linear_w8a8_of_any_width_bit_exact(L, dev, M, N, K):
     """Widths and row counts that fit no tile (K % 16 != 0 or N % 8 != 0): integers, both epilogue orders and the gated
