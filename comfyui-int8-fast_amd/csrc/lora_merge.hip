@@ -231,7 +231,7 @@ __global__ __launch_bounds__(256) void lora_merge_band_kernel(const MergeArgs a,
 // D[k][n] = sum_j down[j][k] * up[n][j]: a lane then holds, for ONE weight row n, four groups of
 // four consecutive k, so the rounding step works on 16-byte noise and 4-byte weight pieces.
 //
-// A workgroup of 8 waves owns 256 columns (rank 64: 4 waves, 128 columns) and walks blocks of 32 rows (every bands-th one).  The noise of a
+// A workgroup of 8 waves owns 256 columns (ranks 48 and 64: 4 waves, 128 columns) and walks blocks of 32 rows (every bands-th one).  The noise of a
 // block goes from global memory straight into one of two LDS tiles (buffer_load ... lds: a wave
 // instruction moves 1 KB of one noise row, no registers involved) while the block before it is
 // worked on; weights and `up` travel through registers.  Every wave takes the 32 x 32 piece of its
@@ -254,7 +254,7 @@ typedef int v4i_t __attribute__((ext_vector_type(4)));
 
 template <int RANK>
 struct MfmaMergeLds {
-    static constexpr int WAVES = RANK == 64 ? 4 : 8, COLS = WAVES * 32;
+    static constexpr int WAVES = RANK == 48 || RANK == 64 ? 4 : 8, COLS = WAVES * 32;
     // One wave load moves 1 KB of noise: NZ_ROWS rows of the tile.  Pitch 260 words: the column reads of 16 rows hit 16
     // different bank groups; of two rows in one piece the second has its 16-byte chunks swapped in groups of four.
     static constexpr int NZ_ROWS = 1024 / (COLS * 4), NZ_PITCH = 1024 + 16;
@@ -291,9 +291,10 @@ __device__ __forceinline__ v4i_t buffer_resource(const void *p, uint32_t bytes) 
 
 // PAD: a.rank is a multiple of 4 below RANK, and the products beyond it are 0 * 0, which leave the sum as it is.
 template <int RANK, bool PAD>
-__global__ __launch_bounds__(MfmaMergeLds<RANK>::WAVES * 64, RANK <= 32 ? 4 : RANK == 64 ? 3 : 2) void lora_merge_mfma_kernel(const MergeArgs a, int bands) {
+__global__ __launch_bounds__(MfmaMergeLds<RANK>::WAVES * 64, RANK <= 32 ? 4 : RANK <= 64 ? 3 : 2) void lora_merge_mfma_kernel(const MergeArgs a, int bands) {
     using T = MfmaMergeLds<RANK>;
     constexpr int NT = T::WAVES * 64, P = RANK / 2;
+    static_assert(P % T::UPV == 0, "the products of a piece, UPV at a time");
     __shared__ __attribute__((aligned(16))) char lds[T::BYTES];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -438,7 +439,7 @@ __global__ __launch_bounds__(MfmaMergeLds<RANK>::WAVES * 64, RANK <= 32 ? 4 : RA
         if (__builtin_amdgcn_ballot_w64(!guard.fast(rs)) == 0) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                product(q * P / 4, (q + 1) * P / 4, acc_next);
+                product(q * P / (4 * UPV) * UPV, (q + 1) * P / (4 * UPV) * UPV, acc_next);
                 float r[4], nzv[4];
                 noise_quad(q, nzv);
 #pragma unroll
@@ -483,8 +484,8 @@ int launch_mfma(const MergeArgs &a, hipStream_t st) {
     // Two workgroups fit a CU (LDS), so 512 run at a time.  Bands are chosen for the fewest block steps on the busiest
     // CU: rounds of 512 workgroups times the blocks of a band, plus half a step for a workgroup's start (its first
     // product is not overlapped with anything); a tie goes to fewer rounds, then to more bands (more of the chip reading).
-    // (Rank 64 in workgroups of four waves, three to a CU; above it the slice of `down` leaves room for one of eight.)
-    constexpr int64_t SLOTS = RANK <= 32 ? 512 : RANK == 64 ? 768 : 256;
+    // (Ranks 48 and 64 in workgroups of four waves, three to a CU; above it the slice of `down` leaves room for one of eight.)
+    constexpr int64_t SLOTS = RANK <= 32 ? 512 : RANK <= 64 ? 768 : 256;
     int64_t max_bands = 4 * SLOTS / col_blocks + 1;
     if (max_bands > nblocks) max_bands = nblocks;
     if (max_bands > 65535) max_bands = 65535;
@@ -524,15 +525,23 @@ int run(MergeArgs &a, hipStream_t st) {
     if (fused && vec && a.w && a.N < (1ll << 31) && a.K % 16 == 0 && a.K < (1 << 24) && al(a.up, 16) && al(a.w, 16) && al(a.out, 16) &&
         a.rank % 4 == 0 && a.rank > 0) {
         // the next larger rank that is built, the rest zeros: a padded product costs no more than its share of RANK
-        // (3072 x 1552, an odd multiple of 16 columns, rank 32: 13.5 us against 22.3 us for the band form below)
+        // (3072 x 1552, an odd multiple of 16 columns, rank 32: 13.5 us against 22.3 us for the band form below).  Up to 32
+        // the noise stream hides the products and powers of two are enough; beyond, the products are the time, so every 16
+        // up to 128 and every 32 up to 256 is built: 9216 x 3072, us, padded to the next of 64, 96, 128, 192, 256 and as it
+        // is: rank 48 54.6 and 47.1, 80 78.2 and 70.2, 112 92.3 and 84.1, 160 144.5 and 126.9, 224 186.1 and 154.6.
         if (a.rank <= 4) return launch_mfma<4>(a, st);
         if (a.rank <= 8) return launch_mfma<8>(a, st);
         if (a.rank <= 16) return launch_mfma<16>(a, st);
         if (a.rank <= 32) return launch_mfma<32>(a, st);
+        if (a.rank <= 48) return launch_mfma<48>(a, st);
         if (a.rank <= 64) return launch_mfma<64>(a, st);
+        if (a.rank <= 80) return launch_mfma<80>(a, st);
         if (a.rank <= 96) return launch_mfma<96>(a, st);
+        if (a.rank <= 112) return launch_mfma<112>(a, st);
         if (a.rank <= 128) return launch_mfma<128>(a, st);
+        if (a.rank <= 160) return launch_mfma<160>(a, st);
         if (a.rank <= 192) return launch_mfma<192>(a, st);
+        if (a.rank <= 224) return launch_mfma<224>(a, st);
         if (a.rank <= 256) return launch_mfma<256>(a, st);
     }
     if (fused && vec && a.w && a.N < (1ll << 31)) {

@@ -1141,7 +1141,9 @@ def test_lora_merge_bit_exact(L, dev, N, K, r, row):
 
 
 @pytest.mark.parametrize("N,K,r,row", [(33, 48, 12, True), (300, 272, 36, True), (64, 256, 64, False), (70, 1040, 100, True),
-                                       (31, 80, 128, True), (65, 304, 132, True), (40, 512, 256, False)])
+                                       (31, 80, 128, True), (65, 304, 132, True), (40, 512, 256, False),
+                                       (70, 400, 48, True), (33, 272, 44, False), (65, 144, 80, False), (40, 528, 68, True),
+                                       (66, 304, 112, True), (32, 256, 160, False), (97, 80, 220, True), (64, 272, 224, True)])
 def test_lora_merge_of_any_rank_on_the_matrix_cores_bit_exact(L, dev, N, K, r, row):
     """Ranks between and beyond the powers of two (padded with zero products to the next one the kernel is built for) and
     widths that are odd multiples of 16 (half of the last wave's columns do not exist)."""
