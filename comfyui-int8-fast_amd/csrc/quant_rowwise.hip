@@ -860,6 +860,17 @@ int pick_nch(int per_thread, const void *x, int64_t M, int64_t K, int64_t ldx, i
     return launch_fast<DT, ROT, TPR, 8>(x, M, K, ldx, q, scale, st);
 }
 
+// Whether four waves share a row that one could hold (16-bit rows of nruns runs of 16 elements, at most 256).  With few rows a
+// SIMD has one wave or none, and the launch lasts as long as that wave's chain of vector instructions, 16 elements of it at a
+// time: four waves cut the chain to a run or less per lane, until the SIMDs have waves enough and the lanes that stay empty
+// (nruns of 256 work) cost more.  Without a rotation or a prologue the chain is short and both are the same.  us, one wave and
+// four: LayerNorm + modulation 512 x 3072 5.15 and 4.24, 256 x 4096 6.14 and 3.72, 2048 x 4096 9.71 and 8.80, 1024 x 2176 5.61 and
+// 5.10, 256 x 2048 4.01 and 3.62; rotation 77 x 3072 2.97 and 2.32.  Beyond the lines: 2048 x 2176 RMSNorm 6.82 and 7.56, 512 x 2048
+// GELU 2.63 and 2.75, 1024 x 1536 2.90 and 3.52.
+inline bool four_waves_to_a_row(int64_t nruns, int64_t M) {
+    return nruns > 192 ? M <= 2048 : nruns > 128 ? M <= 1024 : nruns > 64 && M <= 256;
+}
+
 template <int DT, bool ROT, int PRO = I8F_PRO_NONE>
 int dispatch(const void *x, int64_t M, int64_t K, int64_t ldx, int8_t *q, float *scale, hipStream_t st, const Prologue &pro = Prologue{}) {
     constexpr int EPC = Elem<DT>::EPC;
@@ -874,7 +885,8 @@ int dispatch(const void *x, int64_t M, int64_t K, int64_t ldx, int8_t *q, float 
     if constexpr (DT != I8F_F32) {
         const int64_t nruns = K / 16;
         if (aligned && K % 16 == 0 && (uintptr_t)q % 16 == 0 && nruns >= 1 && nruns <= 64 * 4 * 4) {
-            if (nruns <= 64 * 4) return pick_runs16<DT, ROT, 1, PRO>((int)((nruns + 63) / 64), x, M, K, ldx, q, scale, st, pro);
+            if (nruns <= 64 * 4 && !((ROT || PRO != I8F_PRO_NONE) && four_waves_to_a_row(nruns, M)))
+                return pick_runs16<DT, ROT, 1, PRO>((int)((nruns + 63) / 64), x, M, K, ldx, q, scale, st, pro);
             return pick_runs16<DT, ROT, 4, PRO>((int)((nruns + 255) / 256), x, M, K, ldx, q, scale, st, pro);
         }
     }

@@ -1302,3 +1302,18 @@ def test_linear_w8a16_small_m_grouped_equals_separate_calls(L, dev, dt, M, shape
         want = L.linear_w8a16_small_m(x, w, ws, b)
         assert y.shape == want.shape and y.dtype == want.dtype
         assert torch.equal(y.view(torch.int32) if dt == torch.float32 else y.view(torch.int16), want.view(torch.int32) if dt == torch.float32 else want.view(torch.int16))
+
+
+@pytest.mark.parametrize("K", [1024, 1040, 2048, 2064, 3072, 3088, 4096])
+def test_quantiser_with_four_waves_to_a_row_equals_one_wave(L, dev, K):
+    """Few rows are shared by four waves, many are held by one wave each: the same bits for every form whose result does not
+    depend on the order of a sum."""
+    x = (torch.randn(2056, K, generator=G) * torch.exp2(torch.randint(-8, 4, (2056, 1), generator=G).float())).bfloat16().to(dev)
+    x[3] = 0
+    gate = torch.randn(2056, K, generator=G).bfloat16().to(dev)
+    for kw in (dict(), dict(rotate=K % 128 == 0), dict(prologue=L.PRO_GELU_TANH), dict(prologue=L.PRO_SILU_GATE, mod_scale=gate)):
+        q, s = L.quant_rowwise(x, **kw)
+        for m in (1, 17, 256, 257, 1024, 1025, 2048):
+            part = {**kw, "mod_scale": gate[:m]} if "mod_scale" in kw else kw
+            qm, sm = L.quant_rowwise(x[:m], **part)
+            assert torch.equal(qm, q[:m]) and torch.equal(sm, s[:m]), (kw, m)
