@@ -338,7 +338,11 @@ template <PyObject *(*F)(PyObject *, PyObject *const *, Py_ssize_t)>
 PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t n) {
     try {
         PyObject *r = F(self, a, n);
-        if (r == Py_None) PyErr_Clear();  // (an operand that is no number: the general path words it)
+        if (PyErr_Occurred()) {  // an operand that is no number: the general path words it
+            PyErr_Clear();
+            Py_XDECREF(r);
+            Py_RETURN_NONE;
+        }
         return r;
     } catch (const std::exception &) {
         Py_RETURN_NONE;

@@ -485,3 +485,17 @@ def test_small_batch_layer_of_a_rotated_weight_equals_rotation_and_layer(pkg, de
         got = lin(rows)
         assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(), want.nan_to_num())
         assert torch.isfinite(want[:-1]).all()
+
+
+def test_an_operand_that_is_no_number_is_refused_as_by_the_general_path(pkg, dev, monkeypatch):
+    """eps as a text: the error of the general path, not one about a result with an exception set."""
+    L = pkg._lib
+    q, s = L.quant_rowwise((torch.randn(32, 128, generator=G) * 0.02).to(dev))
+    lin = load(pkg.Int8TensorwiseOps.Linear(128, 32, bias=False), {"l.weight": q, "l.weight_scale": s})
+    x, v = (torch.randn(n, 128, generator=G).bfloat16().to(dev) for n in (40, 1))
+    call = lambda: lin(x, prologue=L.PRO_NORM_MODULATE, mod_scale=v[0], mod_shift=v[0], eps="small")
+    with pytest.raises((ValueError, TypeError)):
+        call()
+    monkeypatch.setattr(lin, "_forward_native", lambda *a: None)
+    with pytest.raises((ValueError, TypeError)):
+        call()
