@@ -571,18 +571,21 @@ class Int8TensorwiseOps(manual_cast):
         # -- forward ------------------------------------------------------------------------
         def _forward_native(self, x, prologue, mod_scale, mod_shift, eps, gate, residual, norm_weight, fused_add):
             """forward() without the interpreter's part of it, for a quantised layer whose tensors are all in place (no
-            managed casting, no dynamic LoRA, 16-bit contiguous rows on the current GPU); None for everything else."""
-            weight, scale = self._parameters.get("weight"), self._weight_scale_scalar
+            managed casting, no dynamic LoRA, 16-bit contiguous rows on the current GPU); None for everything else.  A weight
+            or bias that is no parameter of the layer (pruned, parametrised, a buffer) is the general path's, too: it reads
+            the attributes, which are computed or kept elsewhere then."""
+            params, scale = self._parameters, self._weight_scale_scalar
+            weight = params.get("weight")
             if scale is None:
                 scale = self._buffers.get("weight_scale")
             if (not self._is_quantized or self.lora_A is not None or self.comfy_cast_weights or weight is None or scale is None
-                    or len(self.weight_function) > 0 or len(self.bias_function) > 0 or x.shape[-1] == 0):
+                    or "bias" not in params or len(self.weight_function) > 0 or len(self.bias_function) > 0 or x.shape[-1] == 0):
                 return None
             if prologue == _lib.PRO_MODULATE_FUSED:
                 prologue, fused_add = _lib.PRO_MODULATE, True
             N, K = weight.shape
             work = _lib._splitk_workspace(x, x.numel() // x.shape[-1], N, K) if K >= _lib.SPLITK_MIN_K else None
-            return _lib.host().linear(x, weight, scale, self._parameters.get("bias"), self._is_per_row, bool(self._use_quarot), SMALL_BATCH_ROWS,
+            return _lib.host().linear(x, weight, scale, params["bias"], self._is_per_row, bool(self._use_quarot), SMALL_BATCH_ROWS,
                                       int8_fused_kernel.DEFAULT_EPILOGUE, prologue, mod_scale, mod_shift, eps, norm_weight, bool(fused_add), gate,
                                       residual, work)
 

@@ -3,6 +3,8 @@ scale bookkeeping, ModelPatcher hooks, LoRA scale slicing, delta reconstruction,
 import numpy as np
 import pytest
 import torch
+import torch.nn.utils.parametrize
+import torch.nn.utils.prune
 
 
 @pytest.fixture(autouse=True)
@@ -174,3 +176,48 @@ def test_aliases_keep_the_reference_names(pkg):
     assert pkg.triton_int8_linear_per_row is pkg.hip_int8_linear_per_row
     with pytest.raises(ValueError):
         pkg.quantize_int8_axiswise(torch.zeros(4, 8), dim=0)
+
+
+class _Host:
+    """Stands in for the native host module: notes its arguments and leaves every call to the general path."""
+
+    def __init__(self):
+        self.calls = []
+
+    def linear(self, *args):
+        self.calls.append(args)
+
+
+@pytest.fixture
+def host(pkg, monkeypatch):
+    h = _Host()
+    monkeypatch.setattr(pkg._lib, "host", lambda: h)
+    return h
+
+
+def native(pkg, lin, x, **kw):
+    a = dict(prologue=pkg._lib.PRO_NONE, mod_scale=None, mod_shift=None, eps=1e-6, gate=None, residual=None, norm_weight=None, fused_add=False)
+    return lin._forward_native(x, **{**a, **kw})
+
+
+@pytest.mark.parametrize("kept_as", ["parameter", "none", "buffer", "attribute", "parametrised"])
+def test_native_host_path_never_drops_a_bias(pkg, host, kept_as):
+    """What the layer's bias attribute gives is what the native path is handed, or the call is left to the general path."""
+    lin = pkg.Int8TensorwiseOps.Linear(64, 32, bias=True)
+    load(lin, {"blk.0.lin.weight": torch.ones(32, 64, dtype=torch.int8), "blk.0.lin.weight_scale": torch.tensor(0.5),
+               "blk.0.lin.bias": torch.arange(32.0)})
+    if kept_as == "none":
+        lin.bias = None
+    elif kept_as == "buffer":
+        del lin.bias
+        lin.register_buffer("bias", torch.arange(32.0))
+    elif kept_as == "attribute":
+        torch.nn.utils.prune.identity(lin, "bias")
+    elif kept_as == "parametrised":
+        torch.nn.utils.parametrize.register_parametrization(lin, "bias", torch.nn.Identity())
+    assert (lin.bias is None) == (kept_as == "none")
+    assert native(pkg, lin, torch.zeros(20, 64, dtype=torch.bfloat16)) is None
+    if kept_as in ("parameter", "none"):
+        assert len(host.calls) == 1
+    for args in host.calls:
+        assert args[3] is lin.bias
