@@ -389,6 +389,7 @@ class INT8MergedLoRAPatchAdapter(LoRAAdapter):
         rows = delta_f if isinstance(delta_f, int) else delta_f.shape[0]
         return _slice_scale_mismatch_only(self.weight_scale, rows, offset)
 
+    @torch.no_grad()   # (factors may be parameters; products written into place have no backward)
     def _stacked_factors(self, weight, dev):
         """(up [N,R], down [R,K]) in float32 with up @ down the summed delta of the stack, or None where the patches are
         not all plain LoRAs of this weight or their ranks and widths are not those of the fused kernel's matrix-core form."""

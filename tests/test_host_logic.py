@@ -221,3 +221,20 @@ def test_native_host_path_never_drops_a_bias(pkg, host, kept_as):
         assert len(host.calls) == 1
     for args in host.calls:
         assert args[3] is lin.bias
+
+
+def stack(pkg, pairs, n=48, k=64):
+    """A stack adapter of (up, down) pairs with the strengths 1, 1/2, 1/4, ..., and an int8 weight for it."""
+    parts = [(pkg.INT8LoRAPatchAdapter({"k"}, (u, d, None, None, None, None), 0.01), 0.5**i) for i, (u, d) in enumerate(pairs)]
+    return pkg.INT8MergedLoRAPatchAdapter(parts, 0.01, seed=3), torch.zeros(n, k, dtype=torch.int8)
+
+
+def test_stacked_factors_of_loras_that_require_grad(pkg):
+    """LoRA factors that are parameters are stacked like any others."""
+    g = torch.Generator().manual_seed(5)
+    pairs = [(torch.nn.Parameter(torch.randn(48, r, generator=g)), torch.nn.Parameter(torch.randn(r, 64, generator=g))) for r in (4, 8)]
+    adapter, w = stack(pkg, pairs)
+    up, down = adapter._stacked_factors(w, torch.device("cpu"))
+    assert not up.requires_grad and not down.requires_grad
+    assert torch.equal(up, torch.cat([u.detach() for u, _ in pairs], 1))
+    assert torch.equal(down, torch.cat([d.detach() * 0.5**i for i, (_, d) in enumerate(pairs)]))
