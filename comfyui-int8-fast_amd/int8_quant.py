@@ -396,7 +396,8 @@ class INT8MergedLoRAPatchAdapter(LoRAAdapter):
         parts, rank = [], 0
         for adapter, strength in self.patches:
             plain = _plain_lora(adapter.weights)
-            if plain is None or weight.dim() != 2 or plain[0].shape[0] != weight.shape[0] or plain[1].shape[1] != weight.shape[1]:
+            if (plain is None or weight.dim() != 2 or plain[0].shape[0] != weight.shape[0] or plain[1].shape[1] != weight.shape[1]
+                    or plain[0].shape[1] != plain[1].shape[0]):
                 return None
             alpha, r = adapter.weights[2], plain[1].shape[0]
             parts.append((*plain, (alpha / r) * strength if alpha is not None else strength))

@@ -238,3 +238,12 @@ def test_stacked_factors_of_loras_that_require_grad(pkg):
     assert not up.requires_grad and not down.requires_grad
     assert torch.equal(up, torch.cat([u.detach() for u, _ in pairs], 1))
     assert torch.equal(down, torch.cat([d.detach() * 0.5**i for i, (_, d) in enumerate(pairs)]))
+
+
+def test_stacked_factors_refuses_a_lora_whose_factors_disagree_on_the_rank(pkg):
+    """Ranks that mismatch crosswise add up to the same total; such a stack is left to the general path, whose product
+    raises."""
+    adapter, w = stack(pkg, [(torch.ones(48, 16), torch.ones(32, 64)), (torch.ones(48, 32), torch.ones(16, 64))])
+    assert adapter._stacked_factors(w, torch.device("cpu")) is None
+    with pytest.raises(RuntimeError):
+        adapter.calculate_weight(torch.zeros(48, 64), "k", 1.0, 1.0, None, None)
