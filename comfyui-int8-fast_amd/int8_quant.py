@@ -402,7 +402,7 @@ class INT8MergedLoRAPatchAdapter(LoRAAdapter):
             alpha, r = adapter.weights[2], plain[1].shape[0]
             parts.append((*plain, (alpha / r) * strength if alpha is not None else strength))
             rank += r
-        if weight.shape[1] % 16 or rank % 4 or rank > 256:
+        if weight.shape[1] % 16 or rank % 4 or rank > 256 or rank == 0:
             return None
         up = torch.cat([u.to(dev, torch.float32) for u, _, _ in parts], dim=1)
         down, at = torch.empty((rank, weight.shape[1]), dtype=torch.float32, device=dev), 0

@@ -247,3 +247,11 @@ def test_stacked_factors_refuses_a_lora_whose_factors_disagree_on_the_rank(pkg):
     assert adapter._stacked_factors(w, torch.device("cpu")) is None
     with pytest.raises(RuntimeError):
         adapter.calculate_weight(torch.zeros(48, 64), "k", 1.0, 1.0, None, None)
+
+
+def test_stacked_factors_leaves_empty_loras_to_the_general_path(pkg):
+    """A stack of nothing but LoRAs of rank 0 has a delta of zeros, which the fused kernel has no form for."""
+    adapter, w = stack(pkg, [(torch.ones(48, 0), torch.ones(0, 64))] * 2)
+    assert adapter._stacked_factors(w, torch.device("cpu")) is None
+    adapter, w = stack(pkg, [(torch.ones(48, 0), torch.ones(0, 64)), (torch.ones(48, 4), torch.ones(4, 64))])
+    assert adapter._stacked_factors(w, torch.device("cpu"))[0].shape == (48, 4)
