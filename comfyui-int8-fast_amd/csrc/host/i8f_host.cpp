@@ -142,6 +142,11 @@ struct Stream {
     }
 };
 
+struct Owned {  // a new reference
+    PyObject *p = nullptr;
+    ~Owned() { Py_XDECREF(p); }
+};
+
 // ---- 16 rows or fewer: W8A16 ----------------------------------------------------------------
 PyObject *small_m(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, const Layer &l, bool rotate, void *stream) {
     const int dt = code_of(x.scalar_type());
@@ -160,7 +165,10 @@ PyObject *small_m(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, const L
 }
 
 // linear(x, weight, scale, bias, per_row, rotate, small_rows, order, kind, mod_scale, mod_shift, eps, norm_weight, fused_add,
-//        gate, residual, workspace): kind, an i8f_prologue, names what is applied to x inside the quantiser
+//        gate, residual, workspace): kind, an i8f_prologue, names what is applied to x inside the quantiser; workspace(x, M, N,
+// K) gives the memory of the K split or None.  It is called once a W8A8 call has passed every check, never for 16 rows or
+// fewer or for a call that goes the general way, which asks for its own: the memory stays with the stream, or with the graph
+// that is being captured, together with the kernel that clears it.
 PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 17) return PyErr_Format(PyExc_TypeError, "linear takes 17 arguments, got %zd", n);
     const at::Tensor *xt = tensor(a[0]);
@@ -235,9 +243,11 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
         for (int64_t i = 0; i + 1 < x.dim(); ++i)
             if (res->size(i) != x.size(i)) Py_RETURN_NONE;
     }
+    Owned work_object;
     if (a[16] != Py_None) {
-        work = tensor(a[16]);
-        if (!work) Py_RETURN_NONE;
+        work_object.p = PyObject_CallFunction(a[16], "OLLL", a[0], (long long)M, (long long)l.N, (long long)l.K);
+        if (!work_object.p) return nullptr;
+        if (work_object.p != Py_None && !(work = tensor(work_object.p))) Py_RETURN_NONE;
     }
 
     // one piece of memory for the int8 rows and, behind them, their scales; it goes back to the allocator when the call

@@ -585,8 +585,7 @@ class Int8TensorwiseOps(manual_cast):
                 return None
             if prologue == _lib.PRO_MODULATE_FUSED:
                 prologue, fused_add = _lib.PRO_MODULATE, True
-            N, K = weight.shape
-            work = _lib._splitk_workspace(x, x.numel() // x.shape[-1], N, K) if K >= _lib.SPLITK_MIN_K else None
+            work = _lib._splitk_workspace if weight.shape[-1] >= _lib.SPLITK_MIN_K else None   # (asked for by a call that can use it)
             return _lib.host().linear(x, weight, scale, params["bias"], self._is_per_row, bool(self._use_quarot), SMALL_BATCH_ROWS,
                                       int8_fused_kernel.DEFAULT_EPILOGUE, prologue, mod_scale, mod_shift, eps, norm_weight, bool(fused_add), gate,
                                       residual, work)

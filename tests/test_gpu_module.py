@@ -499,3 +499,34 @@ def test_an_operand_that_is_no_number_is_refused_as_by_the_general_path(pkg, dev
     monkeypatch.setattr(lin, "_forward_native", lambda *a: None)
     with pytest.raises((ValueError, TypeError)):
         call()
+
+
+@pytest.mark.parametrize("rows,declined", [(4, False), (40, False), (40, True)])
+def test_long_k_layer_asks_for_its_workspace_once_and_only_where_it_is_used(pkg, dev, monkeypatch, rows, declined):
+    """A layer with a K that is split, eager and in a graph: no memory for the split at 16 rows or fewer, one piece above,
+    also where the native path leaves the call to the general one; every replay gives the eager result."""
+    L, K, N = pkg._lib, 12288, 264
+    q, s = L.quant_rowwise((torch.randn(N, K, generator=G) * 0.02).to(dev))
+    lin = load(pkg.Int8TensorwiseOps.Linear(K, N, bias=False), {"l.weight": q, "l.weight_scale": s})
+    res = torch.randn(rows, 2 * N, generator=G).bfloat16().to(dev)[:, :N] if declined else None   # (rows at a stride)
+    x = torch.randn(rows, K, generator=G).bfloat16().to(dev)
+    give, asked = L._splitk_workspace, []
+    monkeypatch.setattr(L, "_splitk_workspace", lambda *a: asked.append(give(*a)) or asked[-1])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        lin(x, residual=res)
+    torch.cuda.current_stream().wait_stream(side)
+    uses = int(rows > 16)
+    assert len(asked) == uses and all(t is not None for t in asked)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = lin(x, residual=res)
+    assert len(asked) == 2 * uses
+    for i in range(3):
+        x.copy_(torch.randn(rows, K, generator=G))
+        want = lin(x, residual=res)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), f"replay {i}"

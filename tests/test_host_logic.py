@@ -255,3 +255,15 @@ def test_stacked_factors_leaves_empty_loras_to_the_general_path(pkg):
     assert adapter._stacked_factors(w, torch.device("cpu")) is None
     adapter, w = stack(pkg, [(torch.ones(48, 0), torch.ones(0, 64)), (torch.ones(48, 4), torch.ones(4, 64))])
     assert adapter._stacked_factors(w, torch.device("cpu"))[0].shape == (48, 4)
+
+
+@pytest.mark.parametrize("rows,k", [(4, 12288), (16, 10240), (17, 12288), (40, 12288), (40, 10224)])
+def test_native_host_path_takes_no_workspace_before_the_call_is_decided(pkg, host, monkeypatch, rows, k):
+    """The memory of the K split is asked for by the native function itself, behind its checks: a call that it does not take,
+    or one of 16 rows or fewer, costs none."""
+    asked = []
+    monkeypatch.setattr(pkg._lib, "_splitk_workspace", lambda *a: asked.append(a))
+    lin = pkg.Int8TensorwiseOps.Linear(k, 8, bias=False)
+    load(lin, {"blk.0.lin.weight": torch.ones(8, k, dtype=torch.int8), "blk.0.lin.weight_scale": torch.tensor(0.5)})
+    assert native(pkg, lin, torch.zeros(rows, k, dtype=torch.bfloat16)) is None
+    assert asked == [] and (host.calls[0][16] is None) == (k < pkg._lib.SPLITK_MIN_K)
