@@ -10,6 +10,10 @@
 // Every function takes the cases it can decide on cheaply and returns None for all others (tensors of other types,
 // devices or layouts, operands that need a cast or a copy, errors): the caller then goes the general way in Python, which
 // also words the errors.  Nothing is kept between calls.
+//
+// Everything that belongs to Python (arguments, the tensors' sizes and pointers) is read first; the allocations and the
+// launches then run without the interpreter's lock, as behind ctypes and torch's own operators: a full hardware queue or an
+// allocator that has to give memory back makes this thread wait, not the others.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -127,12 +131,20 @@ at::Tensor empty(at::IntArrayRef size, at::ScalarType t, const at::Device &dev) 
     return at::detail::empty_cuda(size, t, dev, std::nullopt);
 }
 
-// The output of a layer on x's tokens: x's leading dimensions and N columns.
-at::Tensor empty_output(const at::Tensor &x, int64_t N) {
-    c10::SmallVector<int64_t, 6> size(x.sizes().begin(), x.sizes().end());
+// The size of a layer's output on x's tokens: x's leading dimensions and N columns.
+using Size = c10::SmallVector<int64_t, 6>;
+Size output_size(const at::Tensor &x, int64_t N) {
+    Size size(x.sizes().begin(), x.sizes().end());
     size.back() = N;
-    return empty(size, x.scalar_type(), x.device());
+    return size;
 }
+
+// The interpreter's lock is released while one of these lives.  (Taking it again ends the thread where the interpreter has
+// been shut down meanwhile, by an unwinding that has to be let out of here.)
+struct WithoutGil {
+    PyThreadState *state = PyEval_SaveThread();
+    ~WithoutGil() noexcept(false) { PyEval_RestoreThread(state); }
+};
 
 struct Stream {
     void *handle;
@@ -149,18 +161,27 @@ struct Owned {  // a new reference
 
 // ---- 16 rows or fewer: W8A16 ----------------------------------------------------------------
 PyObject *small_m(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, const Layer &l, bool rotate, void *stream) {
-    const int dt = code_of(x.scalar_type());
+    const at::ScalarType type = x.scalar_type();
+    const at::Device dev = x.device();
+    const int dt = code_of(type);
     const void *xp = x.const_data_ptr();
-    at::Tensor rotated, y = empty_output(x, l.N);
-    if (rotate) {
-        if (!lib.i8f_internal_w8a16_rotated(xp, dt, M, K, ld, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, y.data_ptr(), l.N, stream))
-            return THPVariable_Wrap(std::move(y));
-        rotated = empty({M, K}, x.scalar_type(), x.device());
-        if (lib.i8f_rotate128(xp, dt, M, K, ld, rotated.data_ptr(), stream)) Py_RETURN_NONE;
-        xp = rotated.const_data_ptr(), ld = K;
+    const Size size = output_size(x, l.N);
+    at::Tensor rotated, y;
+    bool done = false;
+    {
+        const WithoutGil released;
+        y = empty(size, type, dev);
+        void *out = y.data_ptr();
+        done = rotate && !lib.i8f_internal_w8a16_rotated(xp, dt, M, K, ld, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, out, l.N, stream);
+        bool ready = true;
+        if (rotate && !done) {
+            rotated = empty({M, K}, type, dev);
+            ready = !lib.i8f_rotate128(xp, dt, M, K, ld, rotated.data_ptr(), stream);
+            xp = rotated.const_data_ptr(), ld = K;
+        }
+        if (ready && !done) done = !lib.i8f_linear_w8a16_small_m(xp, dt, M, K, ld, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, out, l.N, stream);
     }
-    if (lib.i8f_linear_w8a16_small_m(xp, dt, M, K, ld, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, y.data_ptr(), l.N, stream))
-        Py_RETURN_NONE;
+    if (!done) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(y));
 }
 
@@ -191,7 +212,12 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
 
     // the operation in front of the layer and its operands
     const at::Tensor *s = nullptr, *t = nullptr, *w = nullptr;
-    int64_t V = 1, Kall = K;
+    int64_t V = 1, Kall = K, Kb = 0, ldb = 0;
+    float eps = 0.0f;
+    if (kind == I8F_PRO_NORM_MODULATE || kind == I8F_PRO_RMS_NORM) {
+        eps = (float)PyFloat_AsDouble(a[11]);
+        if (PyErr_Occurred()) return nullptr;
+    }
     if (kind == I8F_PRO_MODULATE || kind == I8F_PRO_NORM_MODULATE || kind == I8F_PRO_RMS_NORM) {
         s = a[9] == Py_None ? nullptr : tensor(a[9]), t = a[10] == Py_None ? nullptr : tensor(a[10]);
         if ((a[9] != Py_None && !s) || (a[10] != Py_None && !t) || (kind != I8F_PRO_RMS_NORM && !(s && t))) Py_RETURN_NONE;
@@ -211,7 +237,7 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
         }
     } else if (kind == I8F_PRO_CONCAT_GELU) {
         s = tensor(a[9]);
-        int64_t Mb, Kb, ldb;
+        int64_t Mb;
         if (!s || s->scalar_type() != x.scalar_type() || s->device() != x.device() || s->dim() != x.dim() || !rows_of(*s, Mb, Kb, ldb)) Py_RETURN_NONE;
         for (int64_t i = 0; i + 1 < x.dim(); ++i)
             if (s->size(i) != x.size(i)) Py_RETURN_NONE;
@@ -250,40 +276,41 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
         if (work_object.p != Py_None && !(work = tensor(work_object.p))) Py_RETURN_NONE;
     }
 
-    // one piece of memory for the int8 rows and, behind them, their scales; it goes back to the allocator when the call
-    // returns, for work behind these kernels on the same stream
-    const int64_t q_bytes = (M * Kall + 255) / 256 * 256;
-    at::Tensor scratch = empty({q_bytes + 4 * M}, at::kByte, x.device());
-    int8_t *q = (int8_t *)scratch.data_ptr();
-    float *qs = (float *)(q + q_bytes);
-    at::Tensor y = empty_output(x, l.N);
-    const void *xp = x.const_data_ptr(), *sp = s ? s->const_data_ptr() : nullptr, *tp = t ? t->const_data_ptr() : nullptr;
-    const int rb = rotate ? 128 : 0;
+    const at::ScalarType type = x.scalar_type();
+    const at::Device dev = x.device();
+    const Size size = output_size(x, l.N);
+    const auto address = [](const at::Tensor *o) { return o ? o->const_data_ptr() : nullptr; };
+    const void *xp = x.const_data_ptr(), *sp = address(s), *tp = address(t), *wp = address(w), *gate_p = address(gate), *res_p = address(res);
+    void *work_p = work ? work->data_ptr() : nullptr;
+    const int64_t work_bytes = work ? work->numel() : 0;
+    at::Tensor scratch, y;
     int rc;
-    switch (kind) {
-    case I8F_PRO_NONE: rc = lib.i8f_quant_rowwise(xp, dt, M, K, ld, rb, q, qs, st.handle); break;
-    case I8F_PRO_NORM_MODULATE:
-        rc = lib.i8f_quant_rowwise_norm_modulate(xp, dt, M, K, ld, (float)PyFloat_AsDouble(a[11]), sp, tp, M / V, fused_add, rb, q, qs, st.handle);
-        break;
-    case I8F_PRO_RMS_NORM:
-        rc = lib.i8f_quant_rowwise_rms_norm(xp, dt, M, K, ld, (float)PyFloat_AsDouble(a[11]), w ? w->const_data_ptr() : nullptr, sp, tp, M / V,
-                                            fused_add, rb, q, qs, st.handle);
-        break;
-    case I8F_PRO_CONCAT_GELU: {
-        int64_t Mb, Kb, ldb;
-        rows_of(*s, Mb, Kb, ldb);
-        rc = lib.i8f_quant_rowwise_concat_gelu(xp, dt, M, K, ld, sp, Kb, ldb, rb, q, qs, st.handle);
-        break;
+    {
+        const WithoutGil released;
+        // one piece of memory for the int8 rows and, behind them, their scales; it goes back to the allocator when the call
+        // returns, for work behind these kernels on the same stream
+        const int64_t q_bytes = (M * Kall + 255) / 256 * 256;
+        scratch = empty({q_bytes + 4 * M}, at::kByte, dev);
+        int8_t *q = (int8_t *)scratch.data_ptr();
+        float *qs = (float *)(q + q_bytes);
+        y = empty(size, type, dev);
+        const int rb = rotate ? 128 : 0;
+        switch (kind) {
+        case I8F_PRO_NONE: rc = lib.i8f_quant_rowwise(xp, dt, M, K, ld, rb, q, qs, st.handle); break;
+        case I8F_PRO_NORM_MODULATE:
+            rc = lib.i8f_quant_rowwise_norm_modulate(xp, dt, M, K, ld, eps, sp, tp, M / V, fused_add, rb, q, qs, st.handle);
+            break;
+        case I8F_PRO_RMS_NORM: rc = lib.i8f_quant_rowwise_rms_norm(xp, dt, M, K, ld, eps, wp, sp, tp, M / V, fused_add, rb, q, qs, st.handle); break;
+        case I8F_PRO_CONCAT_GELU: rc = lib.i8f_quant_rowwise_concat_gelu(xp, dt, M, K, ld, sp, Kb, ldb, rb, q, qs, st.handle); break;
+        case I8F_PRO_SILU_GATE: rc = lib.i8f_quant_rowwise_prologue(xp, dt, M, K, ld, kind, sp, nullptr, 1, rb, q, qs, st.handle); break;
+        default:
+            rc = lib.i8f_quant_rowwise_prologue(xp, dt, M, K, ld, kind == I8F_PRO_MODULATE && fused_add ? (int)I8F_PRO_MODULATE_FUSED : kind, sp, tp,
+                                                M / V, rb, q, qs, st.handle);
+        }
+        if (!rc)
+            rc = lib.i8f_linear_w8a8_gated(q, qs, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, gate_p, gate_rows, res_p, y.data_ptr(), dt, M,
+                                           l.N, l.K, order, work_p, work_bytes, st.handle);
     }
-    case I8F_PRO_SILU_GATE: rc = lib.i8f_quant_rowwise_prologue(xp, dt, M, K, ld, kind, sp, nullptr, 1, rb, q, qs, st.handle); break;
-    default:
-        rc = lib.i8f_quant_rowwise_prologue(xp, dt, M, K, ld, kind == I8F_PRO_MODULATE && fused_add ? (int)I8F_PRO_MODULATE_FUSED : kind, sp, tp,
-                                            M / V, rb, q, qs, st.handle);
-    }
-    if (rc) Py_RETURN_NONE;
-    rc = lib.i8f_linear_w8a8_gated(q, qs, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, gate ? gate->const_data_ptr() : nullptr, gate_rows,
-                                   res ? res->const_data_ptr() : nullptr, y.data_ptr(), dt, M, l.N, l.K, order, work ? work->data_ptr() : nullptr,
-                                   work ? work->numel() : 0, st.handle);
     if (rc) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(y));
 }
@@ -316,20 +343,29 @@ PyObject *vector_fanout(PyObject *, PyObject *const *a, Py_ssize_t n) {
             bias_code = l[i].bias_code;
         }
     }
+    const at::ScalarType type = x.scalar_type();
+    const at::Device dev = x.device();
     const void *xp = x.const_data_ptr();
-    at::Tensor rotated;
-    if (rotate) {
-        rotated = empty({M, K}, x.scalar_type(), x.device());
-        if (lib.i8f_rotate128(xp, dt, M, K, ld, rotated.data_ptr(), st.handle)) Py_RETURN_NONE;
-        xp = rotated.const_data_ptr(), ld = K;
+    Size size[I8F_MAX_LINEAR_GROUPS];
+    for (Py_ssize_t i = 0; i < count; ++i) size[i] = output_size(x, l[i].N);
+    at::Tensor rotated, y[I8F_MAX_LINEAR_GROUPS];
+    bool done = true;
+    {
+        const WithoutGil released;
+        if (rotate) {
+            rotated = empty({M, K}, type, dev);
+            done = !lib.i8f_rotate128(xp, dt, M, K, ld, rotated.data_ptr(), st.handle);
+            xp = rotated.const_data_ptr(), ld = K;
+        }
+        i8f_small_m_group g[I8F_MAX_LINEAR_GROUPS];
+        for (Py_ssize_t i = 0; i < count; ++i) {
+            y[i] = empty(size[i], type, dev);
+            g[i] = {xp, M, K, ld, l[i].w, l[i].ws, l[i].ws_host, l[i].bias, y[i].data_ptr(), l[i].N};
+        }
+        if (done)
+            done = !lib.i8f_linear_w8a16_small_m_grouped(g, (int)count, dt, l[0].mode, bias_code < 0 ? (int)I8F_BF16 : bias_code, st.handle);
     }
-    i8f_small_m_group g[I8F_MAX_LINEAR_GROUPS];
-    at::Tensor y[I8F_MAX_LINEAR_GROUPS];
-    for (Py_ssize_t i = 0; i < count; ++i) {
-        y[i] = empty_output(x, l[i].N);
-        g[i] = {xp, M, K, ld, l[i].w, l[i].ws, l[i].ws_host, l[i].bias, y[i].data_ptr(), l[i].N};
-    }
-    if (lib.i8f_linear_w8a16_small_m_grouped(g, (int)count, dt, l[0].mode, bias_code < 0 ? (int)I8F_BF16 : bias_code, st.handle)) Py_RETURN_NONE;
+    if (!done) Py_RETURN_NONE;
     PyObject *out = PyList_New(count);
     if (!out) return nullptr;
     for (Py_ssize_t i = 0; i < count; ++i) {

@@ -1,5 +1,12 @@
 """The ComfyUI-facing layer on the GPU: Int8TensorwiseOps.Linear and the INT8 LoRA adapters
 produce what the oracle computes from the same inputs."""
+import ctypes
+import importlib.util
+import os
+import re
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 import torch
@@ -530,3 +537,35 @@ def test_long_k_layer_asks_for_its_workspace_once_and_only_where_it_is_used(pkg,
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want), f"replay {i}"
+
+
+def test_native_host_path_launches_without_the_interpreters_lock(pkg, dev, tmp_path):
+    """A copy of the host module, bound to a library that notes for each entry point whether its caller holds the lock: nobody
+    does, so other Python threads run while a launch or an allocation waits.  Nothing is launched here."""
+    L = pkg._lib
+    src = open(os.path.join(os.path.dirname(L.__file__), "csrc", "host", "i8f_host.cpp")).read()
+    names = re.findall(r"X\((i8f_\w+)\)", src)
+    assert len(names) >= 10
+    c, so, path = tmp_path / "stub.c", tmp_path / "stub.so", tmp_path / "_i8f_host.so"
+    c.write_text("extern int PyGILState_Check(void); int calls, held;\n"
+                 + "".join(f"int {n}() {{ ++calls, held += PyGILState_Check(); return {-2 if n == 'i8f_internal_w8a16_rotated' else 0}; }}\n" for n in names))
+    subprocess.run(["gcc", "-w", "-shared", "-fPIC", "-o", so, c], check=True)
+    shutil.copy(L.host().__file__, path)
+    spec = importlib.util.spec_from_file_location("_i8f_host", path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    mod.bind(str(so))
+    stub = ctypes.PyDLL(str(so))
+    calls, held = ctypes.c_int.in_dll(stub, "calls"), ctypes.c_int.in_dll(stub, "held")
+    assert stub.i8f_rotate128() == 0 and calls.value == 1 and held.value == 1      # the probe tells the two apart
+    calls.value = held.value = 0
+    w, x, v = torch.ones(32, 128, dtype=torch.int8, device=dev), torch.ones(40, 128, dtype=torch.bfloat16, device=dev), torch.ones(1, 128, dtype=torch.bfloat16, device=dev)
+
+    def linear(x, rotate, kind, s=None, t=None, k=128):
+        return mod.linear(x, w if k == 128 else w.repeat(1, k // 128), 0.5, None, False, rotate, 16, 0, kind, s, t, 1e-6, None, False, None, None, None)
+
+    outs = [linear(x[:4], False, L.PRO_NONE), linear(x[:4], True, L.PRO_NONE), linear(x, False, L.PRO_NONE), linear(x, True, L.PRO_GELU_TANH),
+            linear(x, False, L.PRO_MODULATE, v, v), linear(x, False, L.PRO_NORM_MODULATE, v, v), linear(x, False, L.PRO_RMS_NORM, v),
+            linear(x, False, L.PRO_SILU_GATE, x), linear(x, False, L.PRO_CONCAT_GELU, x, k=256), mod.vector_fanout(x[:4], (w, w), (0.5, 0.5), (None, None), (False, False), True)]
+    assert all(y is not None for y in outs)
+    assert calls.value == 1 + 3 + 7 * 2 + 2 and held.value == 0
