@@ -398,6 +398,10 @@ __device__ __forceinline__ void quant16_body(const char *__restrict__ x, int64_t
                                              int8_t *__restrict__ q, float *__restrict__ scale, const Prologue &pro,
                                              int64_t first_row) {
     static_assert(SEG == 1 || WPR == 1, "segments are for the one-wave-per-row form");
+    // A normalised row that one wave could hold (at most 256 runs): which form takes it depends on how many rows there are, and
+    // its sums must not.  Each of the four waves then takes the statistics of the whole row itself, from all of its runs and
+    // in the order of the one-wave form, and goes on with its own quarter of them.
+    constexpr bool WHOLE = WPR == 4 && RUNS == 1 && (PRO == I8F_PRO_NORM_MODULATE || PRO == I8F_PRO_RMS_NORM);
     constexpr int TPR = 64 * WPR;
     constexpr int ROWS = 256 / (TPR * SEG);  // rows per workgroup
     const int t = threadIdx.x % TPR;
@@ -411,9 +415,19 @@ __device__ __forceinline__ void quant16_body(const char *__restrict__ x, int64_t
     const float s0 = (p & 1) ? -1.0f : 1.0f, s1 = (p & 2) ? -1.0f : 1.0f, s2 = (p & 4) ? -1.0f : 1.0f;
 
     uint4 raw[RUNS][2];
+    [[maybe_unused]] uint4 whole[WHOLE ? 4 : 1][2];
     {
         const bool ok = FULL || m < M;
         const char *xrow = x + (ok ? m : 0) * ldx_bytes;
+        if constexpr (WHOLE) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int R = r * 64 + (p & 63);
+                const bool in = ok && R < nruns;
+                whole[r][0] = in ? *(const uint4 *)(xrow + R * 32) : make_uint4(0, 0, 0, 0);
+                whole[r][1] = in ? *(const uint4 *)(xrow + R * 32 + 16) : make_uint4(0, 0, 0, 0);
+            }
+        }
         [[maybe_unused]] const char *brow = nullptr;
         if constexpr (PRO == I8F_PRO_CONCAT_GELU) brow = (const char *)pro.b + (ok ? m : 0) * pro.ldb_bytes;
 #pragma unroll
@@ -435,13 +449,13 @@ __device__ __forceinline__ void quant16_body(const char *__restrict__ x, int64_t
     {
         float v[RUNS][16];
         float amax = 0.0f;
-        // A row's sum for the normalising prologues: over the wave, then (four waves to a row) over the waves' partial
-        // sums through LDS, always in the same order, so that launches agree bit for bit.  Two slots: the second sum
-        // of a LayerNorm may be written while a slower wave still reads the first.
+        // A row's sum for the normalising prologues: over the wave, then (four waves to a row, each with its own runs) over
+        // the waves' partial sums through LDS, always in the same order, so that launches agree bit for bit.  Two slots: the
+        // second sum of a LayerNorm may be written while a slower wave still reads the first.
         [[maybe_unused]] __shared__ float row_sums[2][ROWS][WPR];
         [[maybe_unused]] auto row_sum = [&](float part, int slot) {
             part = wave_sum_all(part);
-            if constexpr (WPR > 1) {
+            if constexpr (WPR > 1 && !WHOLE) {
                 if ((t & 63) == 0) row_sums[slot][rb][t / 64] = part;
                 __syncthreads();
                 part = row_sums[slot][rb][0];
@@ -458,14 +472,38 @@ __device__ __forceinline__ void quant16_body(const char *__restrict__ x, int64_t
             // differences (two passes over registers), y = (x - mean) / sqrt(var + eps) rounded to the dtype.
             static_assert(SEG == 1, "the row's statistics are taken by the waves that hold it whole");
             float sum = 0.0f;
+            [[maybe_unused]] float u[WHOLE ? 4 : 1][16];
+            if constexpr (WHOLE) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (r * 64 >= nruns) break;
+                    expand16<DT>(whole[r][0], whole[r][1], u[r]);
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) sum += u[r][j];
+                }
+            }
 #pragma unroll
             for (int r = 0; r < RUNS; ++r) {
                 expand16<DT>(raw[r][0], raw[r][1], v[r]);   // (runs beyond the row are zeros)
+                if constexpr (!WHOLE) {
 #pragma unroll
-                for (int j = 0; j < 16; ++j) sum += v[r][j];
+                    for (int j = 0; j < 16; ++j) sum += v[r][j];
+                }
             }
             const float mean = row_sum(sum, 0) / (float)K;
             float ss = 0.0f;
+            if constexpr (WHOLE) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (r * 64 + (p & 63) < nruns) {
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) {
+                            const float d = u[r][j] - mean;
+                            ss += d * d;
+                        }
+                    }
+                }
+            }
 #pragma unroll
             for (int r = 0; r < RUNS; ++r) {
                 const bool in = FULL || r * TPR + p < nruns;
@@ -473,7 +511,7 @@ __device__ __forceinline__ void quant16_body(const char *__restrict__ x, int64_t
                 for (int j = 0; j < 16; ++j) {
                     const float d = v[r][j] - mean;
                     v[r][j] = d;
-                    ss += in ? d * d : 0.0f;
+                    if constexpr (!WHOLE) ss += in ? d * d : 0.0f;
                 }
             }
             const float rstd = 1.0f / sqrtf(row_sum(ss, 1) / (float)K + pro.eps);
@@ -487,11 +525,23 @@ __device__ __forceinline__ void quant16_body(const char *__restrict__ x, int64_t
             // once to the dtype (torch's rms_norm); then the modulation's operations, each rounded, where s / t exist.
             static_assert(SEG == 1, "the row's statistics are taken by the waves that hold it whole");
             float ss = 0.0f;
+            if constexpr (WHOLE) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (r * 64 >= nruns) break;
+                    float u[16];
+                    expand16<DT>(whole[r][0], whole[r][1], u);
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) ss = __builtin_fmaf(u[j], u[j], ss);
+                }
+            }
 #pragma unroll
             for (int r = 0; r < RUNS; ++r) {
                 expand16<DT>(raw[r][0], raw[r][1], v[r]);   // (runs beyond the row are zeros)
+                if constexpr (!WHOLE) {
 #pragma unroll
-                for (int j = 0; j < 16; ++j) ss = __builtin_fmaf(v[r][j], v[r][j], ss);
+                    for (int j = 0; j < 16; ++j) ss = __builtin_fmaf(v[r][j], v[r][j], ss);
+                }
             }
             const float rstd = 1.0f / sqrtf(row_sum(ss, 0) / (float)K + pro.eps);
 #pragma unroll
@@ -864,11 +914,15 @@ int pick_nch(int per_thread, const void *x, int64_t M, int64_t K, int64_t ldx, i
 // SIMD has one wave or none, and the launch lasts as long as that wave's chain of vector instructions, 16 elements of it at a
 // time: four waves cut the chain to a run or less per lane, until the SIMDs have waves enough and the lanes that stay empty
 // (nruns of 256 work) cost more.  Without a rotation or a prologue the chain is short and both are the same.  us, one wave and
-// four: LayerNorm + modulation 512 x 3072 5.15 and 4.24, 256 x 4096 6.14 and 3.72, 2048 x 4096 9.71 and 8.80, 1024 x 2176 5.61 and
-// 5.10, 256 x 2048 4.01 and 3.62; rotation 77 x 3072 2.97 and 2.32.  Beyond the lines: 2048 x 2176 RMSNorm 6.82 and 7.56, 512 x 2048
-// GELU 2.63 and 2.75, 1024 x 1536 2.90 and 3.52.
-inline bool four_waves_to_a_row(int64_t nruns, int64_t M) {
-    return nruns > 192 ? M <= 2048 : nruns > 128 ? M <= 1024 : nruns > 64 && M <= 256;
+// four: rotation 77 x 3072 2.97 and 2.32; beyond the lines 512 x 2048 GELU 2.63 and 2.75.
+// The normalising forms cross over earlier, since each of the four waves takes the whole row's statistics (so that a row's bits
+// do not depend on this choice; with partial sums instead, in another order, it would be 0.1 to 0.7 us less).  LayerNorm and
+// modulation: 256 x 4096 6.13 and 4.16, 1024 x 4096 7.19 and 7.04, 512 x 3072 5.08 and 4.63, 256 x 2048 4.02 and 3.86; beyond the
+// lines 2048 x 4096 9.67 and 11.08, 1024 x 3072 5.90 and 6.09.  RMSNorm and rotation: 1024 x 4096 6.56 and 6.23, 512 x 3072 4.71
+// and 4.15; beyond 2048 x 4096 8.85 and 9.18, 1024 x 3072 5.41 and 5.61.
+inline bool four_waves_to_a_row(int64_t nruns, int64_t M, bool normalises) {
+    const int64_t many = normalises ? 512 : 1024;
+    return nruns > 192 ? M <= 2 * many : nruns > 128 ? M <= many : nruns > 64 && M <= 256;
 }
 
 template <int DT, bool ROT, int PRO = I8F_PRO_NONE>
@@ -885,7 +939,8 @@ int dispatch(const void *x, int64_t M, int64_t K, int64_t ldx, int8_t *q, float 
     if constexpr (DT != I8F_F32) {
         const int64_t nruns = K / 16;
         if (aligned && K % 16 == 0 && (uintptr_t)q % 16 == 0 && nruns >= 1 && nruns <= 64 * 4 * 4) {
-            if (nruns <= 64 * 4 && !((ROT || PRO != I8F_PRO_NONE) && four_waves_to_a_row(nruns, M)))
+            constexpr bool NORMALISES = PRO == I8F_PRO_NORM_MODULATE || PRO == I8F_PRO_RMS_NORM;
+            if (nruns <= 64 * 4 && !((ROT || PRO != I8F_PRO_NONE) && four_waves_to_a_row(nruns, M, NORMALISES)))
                 return pick_runs16<DT, ROT, 1, PRO>((int)((nruns + 63) / 64), x, M, K, ldx, q, scale, st, pro);
             return pick_runs16<DT, ROT, 4, PRO>((int)((nruns + 255) / 256), x, M, K, ldx, q, scale, st, pro);
         }
