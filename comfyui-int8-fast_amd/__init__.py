@@ -9,7 +9,7 @@ The package replaces the W8A8 linear hot path of ComfyUI-INT8-Fast:
     nodes               ComfyUI graph nodes (model loader, LoRA loaders); ComfyUI is imported when they run
     dynamic_lora        hook for un-merged LoRA side branches
     _lib                ctypes binding of libi8f_gfx950.so (include/i8f.h)
-    build               hipcc build of the library
+    build               build of the library (hipcc) and of the host extension (g++)
 
 The directory name is ComfyUI's convention for custom nodes and is not a Python
 identifier; ComfyUI imports such packages by path, and so do this repository's

@@ -13,9 +13,10 @@ import os
 
 import torch
 
+from .build import host_lib
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libi8f_gfx950.so")
-HOST_PATH = os.path.join(_HERE, "_i8f_host.so")
 
 BF16, F16, F32 = 0, 1, 2
 SCALE_TENSOR, SCALE_ROW = 0, 1
@@ -96,9 +97,10 @@ def host():
     if _host is not None:
         return _host
     lib()
-    if not os.path.exists(HOST_PATH):
-        raise RuntimeError(f"{HOST_PATH} is missing: build it with `python {os.path.join(_HERE, 'build.py')}`")
-    spec = importlib.util.spec_from_file_location("_i8f_host", HOST_PATH)
+    path = host_lib()
+    if not os.path.exists(path):
+        raise RuntimeError(f"{path} is missing (it belongs to this torch and this Python): build it with `python {os.path.join(_HERE, 'build.py')}`")
+    spec = importlib.util.spec_from_file_location("_i8f_host", path)
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)
     mod.bind(LIB_PATH)

@@ -1,4 +1,4 @@
-"""Build libi8f_gfx950.so from csrc/*.hip with hipcc and the host extension _i8f_host.so with g++, in-tree.
+"""Build libi8f_gfx950.so from csrc/*.hip with hipcc and the host extension (_i8f_host.*.so) with g++, in-tree.
 
     python comfyui-int8-fast_amd/build.py [--force] [--keep-temps]
 
@@ -21,7 +21,6 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libi8f_gfx950.so")
 HOST_SRC = os.path.join(CSRC, "host", "i8f_host.cpp")
-HOST_LIB = os.path.join(HERE, "_i8f_host.so")
 
 # -ffp-contract=off and correctly rounded division are part of the numerical
 # contract (bit-exact quantiser, epilogue and merge); packed FP32 instructions
@@ -78,6 +77,14 @@ def _stale(target: str, deps: list[str]) -> bool:
     return any(os.path.getmtime(d) > t for d in deps)
 
 
+def host_lib() -> str:
+    """The host extension's file.  It is compiled against the layout of one torch's tensors and one Python's objects, so both
+    are in its name: after an upgrade it is not found (and built again) instead of loaded."""
+    import torch
+
+    return os.path.join(HERE, f"_i8f_host.torch-{torch.__version__}.{sysconfig.get_config_var('SOABI')}.so")
+
+
 def host_command() -> list[str]:
     """The compilation of the host extension (no device code: a CPython module against the installed torch)."""
     import torch
@@ -87,7 +94,7 @@ def host_command() -> list[str]:
     include = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"), sysconfig.get_paths()["include"],
                os.path.join(rocm, "include")]
     return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-            *(f for d in include for f in ("-isystem", d)), HOST_SRC, "-o", HOST_LIB, "-L" + os.path.join(t, "lib"),
+            *(f for d in include for f in ("-isystem", d)), HOST_SRC, "-o", host_lib(), "-L" + os.path.join(t, "lib"),
             "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-Wl,-rpath," + os.path.join(t, "lib")]
 
 
@@ -106,7 +113,7 @@ def build(force: bool = False, keep_temps: bool = False, verbose: bool = True) -
                 cmd += ["-save-temps=obj"]
             jobs.append(cmd)
 
-    if force or _stale(HOST_LIB, [HOST_SRC] + headers):
+    if force or _stale(host_lib(), [HOST_SRC] + headers):
         jobs.append(host_command())
 
     def run(cmd):

@@ -1,5 +1,7 @@
 """Host-side behaviour of the ComfyUI-facing layer that needs no GPU: state-dict loading rules,
 scale bookkeeping, ModelPatcher hooks, LoRA scale slicing, delta reconstruction, Hadamard build."""
+import sysconfig
+
 import numpy as np
 import pytest
 import torch
@@ -267,3 +269,15 @@ def test_native_host_path_takes_no_workspace_before_the_call_is_decided(pkg, hos
     load(lin, {"blk.0.lin.weight": torch.ones(8, k, dtype=torch.int8), "blk.0.lin.weight_scale": torch.tensor(0.5)})
     assert native(pkg, lin, torch.zeros(rows, k, dtype=torch.bfloat16)) is None
     assert asked == [] and (host.calls[0][16] is None) == (k < pkg._lib.SPLITK_MIN_K)
+
+
+def test_host_extension_of_another_torch_or_python_is_not_loaded(pkg, monkeypatch):
+    """The extension is compiled against one torch and one Python: with others it is missing, and the error says what to do."""
+    L = pkg._lib
+    assert L.host() is L.host()
+    for place, name, value in ((torch, "__version__", "0.0.1+other"), (sysconfig, "get_config_var", lambda key: "cpython-00")):
+        with monkeypatch.context() as m:
+            m.setattr(L, "_host", None)
+            m.setattr(place, name, value)
+            with pytest.raises(RuntimeError, match="build.py"):
+                L.host()
