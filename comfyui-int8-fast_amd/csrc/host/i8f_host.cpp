@@ -109,6 +109,7 @@ bool layer_of(PyObject *weight, PyObject *scale, PyObject *bias, bool per_row, c
     const at::Tensor *w = tensor(weight);
     if (!w || w->scalar_type() != at::kChar || w->dim() != 2 || w->device() != dev || !w->is_contiguous()) return false;
     l.w = (const int8_t *)w->const_data_ptr(), l.N = w->size(0), l.K = w->size(1);
+    if (l.N < 1) return false;
     if (PyFloat_Check(scale)) {
         if (per_row) return false;
         l.ws_host = (float)PyFloat_AS_DOUBLE(scale);

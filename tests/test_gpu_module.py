@@ -569,3 +569,14 @@ def test_native_host_path_launches_without_the_interpreters_lock(pkg, dev, tmp_p
             linear(x, False, L.PRO_SILU_GATE, x), linear(x, False, L.PRO_CONCAT_GELU, x, k=256), mod.vector_fanout(x[:4], (w, w), (0.5, 0.5), (None, None), (False, False), True)]
     assert all(y is not None for y in outs)
     assert calls.value == 1 + 3 + 7 * 2 + 2 and held.value == 0
+
+
+def test_layer_without_outputs(pkg, dev):
+    """A layer of width 0: an empty result, and the general path's error for a gate of width 0 (no vectors to count)."""
+    lin = load(pkg.Int8TensorwiseOps.Linear(128, 0, bias=False), {"l.weight": torch.zeros(0, 128, dtype=torch.int8, device=dev), "l.weight_scale": torch.tensor(0.5)})
+    gate = torch.ones(0, dtype=torch.bfloat16, device=dev)
+    for rows in (4, 40):
+        x = torch.ones(rows, 128, dtype=torch.bfloat16, device=dev)
+        assert lin(x).shape == (rows, 0) and pkg.forward_fanout([lin, lin], x)[1].shape == (rows, 0)
+    with pytest.raises((RuntimeError, ValueError)):
+        lin(x, gate=gate)
