@@ -165,7 +165,7 @@ def forward_fanout(layers, x, prologue: int = _lib.PRO_NONE, mod_scale=None, mod
         if type(x) is Tensor:
             scales = tuple(lin._get_weight_scale() for lin in layers)
             outs = _lib.host().vector_fanout(x, tuple(lin.weight for lin in layers), scales, tuple(lin.bias for lin in layers),
-                                             tuple(lin._is_per_row for lin in layers), rot)
+                                             tuple(bool(lin._is_per_row) for lin in layers), rot)
             if outs is not None:
                 return outs
         x_2d = x.reshape(-1, x.shape[-1])
@@ -586,7 +586,7 @@ class Int8TensorwiseOps(manual_cast):
             if prologue == _lib.PRO_MODULATE_FUSED:
                 prologue, fused_add = _lib.PRO_MODULATE, True
             work = _lib._splitk_workspace if weight.shape[-1] >= _lib.SPLITK_MIN_K else None   # (asked for by a call that can use it)
-            return _lib.host().linear(x, weight, scale, params["bias"], self._is_per_row, bool(self._use_quarot), SMALL_BATCH_ROWS,
+            return _lib.host().linear(x, weight, scale, params["bias"], bool(self._is_per_row), bool(self._use_quarot), SMALL_BATCH_ROWS,
                                       int8_fused_kernel.DEFAULT_EPILOGUE, prologue, mod_scale, mod_shift, eps, norm_weight, bool(fused_add), gate,
                                       residual, work)
 

@@ -281,3 +281,13 @@ def test_host_extension_of_another_torch_or_python_is_not_loaded(pkg, monkeypatc
             m.setattr(place, name, value)
             with pytest.raises(RuntimeError, match="build.py"):
                 L.host()
+
+
+@pytest.mark.parametrize("flag", [True, 1, np.bool_(True), False, 0])
+def test_native_host_path_is_told_the_scale_mode_as_a_truth_value(pkg, host, flag):
+    """Per-row scales marked by anything true are per-row scales, as in the general path."""
+    lin = pkg.Int8TensorwiseOps.Linear(64, 32, bias=False)
+    load(lin, {"blk.0.lin.weight": torch.ones(32, 64, dtype=torch.int8), "blk.0.lin.weight_scale": torch.rand(32, 1)})
+    lin._is_per_row = flag
+    native(pkg, lin, torch.zeros(20, 64, dtype=torch.bfloat16))
+    assert host.calls[0][4] is bool(flag)
