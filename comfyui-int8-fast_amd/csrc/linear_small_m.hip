@@ -466,13 +466,15 @@ extern "C" int i8f_linear_w8a16_small_m(const void *x, int x_dtype, int64_t M, i
 
 // The layer of a rotated weight in one launch: up to 8 rows, while every workgroup finds a CU of its own and the rotation, which
 // is the same in every one of them, stays short beside the weight stream.  us per call, weights from HBM, against
-// i8f_rotate128 and the layer: 4 x 3072 -> 3072 7.6 and 8.0, 8 x 3072 -> 4096 7.4 and 8.3, 8 x 1536 -> 3072 4.8 and 6.6,
-// 4 x 256 -> 512 2.9 and 4.6; beyond the line 4 x 6144 -> 3072 12.8 and 11.0, 4 x 3072 -> 6144 11.3 and 10.4 (two passes of 8
-// rows: 9 x 3072 -> 3072 8.9 and 8.2).  From an eager layer the launch saved counts for more: 4 x 3072 -> 3072 6.7 and 10.3.
+// i8f_rotate128 and the layer, for 1, 4 and 8 rows: 1536 -> 3072 4.3, 4.4, 4.5 and 5.8, 6.0, 6.3; 3072 -> 3072 6.8, 6.9, 7.2 and
+// 7.0, 7.2, 7.7; 3840 -> 3072 8.2, 8.4, 8.6 and 8.1, 8.4, 8.8; 4096 -> 4096 9.4, 9.5, 9.5 and 10.1, 10.6, 10.8.  Beyond the lines
+// 5120 -> 3072 9.3, 9.5, 9.9 and 9.2, 9.5, 10.0; 6144 -> 3072 11.1, 11.3, 11.4 and 10.1, 10.4, 10.9; 4 x 3072 -> 6144 11.3 and 10.4;
+// two passes of 8 rows 9 x 3072 -> 3072 8.9 and 8.2.  From an eager layer the launch saved counts for more: 4 x 3072 -> 3072 6.7
+// and 10.3.
 extern "C" int i8f_internal_w8a16_rotated(const void *x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t *w, const float *w_scale,
                                           float w_scale_host, int scale_mode, const void *bias, int bias_dtype, void *out, int64_t N, void *stream) {
     using namespace i8f;
-    if (M < 1 || M > 8 || N < 1 || N > 4096 || K < 128 || K > 3072 || K % 128 || (x_dtype != I8F_BF16 && x_dtype != I8F_F16) ||
+    if (M < 1 || M > 8 || N < 1 || N > 4096 || K < 128 || K > 4096 || K % 128 || (x_dtype != I8F_BF16 && x_dtype != I8F_F16) ||
         (bias && !valid_dtype(bias_dtype)) || !x || !w || !out || ldx < K || (scale_mode == I8F_SCALE_ROW && !w_scale))
         return I8F_ERR_UNSUPPORTED;
     if ((uintptr_t)w % 16 || (uintptr_t)x % 16 || ldx % 8) return I8F_ERR_UNSUPPORTED;

@@ -477,9 +477,10 @@ def test_native_host_path_equals_the_general_path(pkg, dev, monkeypatch, case):
 
 
 @pytest.mark.parametrize("M,K,N,dt", [(1, 128, 9, torch.bfloat16), (8, 3072, 4096, torch.bfloat16), (4, 384, 3072, torch.float16), (7, 1280, 1001, torch.float16),
-                                      (9, 256, 64, torch.bfloat16), (3, 3200, 48, torch.bfloat16), (2, 256, 4104, torch.float16)])
+                                      (9, 256, 64, torch.bfloat16), (3, 3200, 48, torch.bfloat16), (2, 256, 4104, torch.float16),
+                                      (5, 4096, 4096, torch.float16), (2, 4224, 48, torch.bfloat16)])
 def test_small_batch_layer_of_a_rotated_weight_equals_rotation_and_layer(pkg, dev, M, K, N, dt):
-    """x rotated inside the small-batch kernel (8 rows, width 3072, 4096 outputs and less) or by a launch in front of it: the
+    """x rotated inside the small-batch kernel (8 rows, width 4096, 4096 outputs and less) or by a launch in front of it: the
     same bits, rows at a stride and large, small and non-finite values included."""
     L = pkg._lib
     q, s = L.quant_rowwise((torch.randn(N, K, generator=G) * 0.02).to(dev), rotate=True)
