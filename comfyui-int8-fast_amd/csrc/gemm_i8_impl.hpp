@@ -603,8 +603,11 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
             // The waves of a SIMD leave the barrier together and the older one wins every issue slot: it ran a whole K-tile's
             // MFMAs while the younger one had done a third of its own, then waited at the barrier with the matrix pipe half
             // used.  With the two phases behind the barrier at a higher priority, a wave that is ahead yields to the one that is
-            // still in them: 2 250 cycles a K-tile of 256 x 256 instead of 2 380 (2 048 are its MFMAs).  In time 1 to 4 %: at
-            // the power limit the chip gives part of it back as a lower clock.
+            // still in them.  Cycles of a K-tile without and with it (2 048 are the MFMAs of 256 x 256): 4608 x 3072 x 3072, 256 x
+            // 256, one set of operands 2 325 and 2 254, operands from HBM 2 355 and 2 292; at K = 12 288 2 297 and 2 226, 2 481 and
+            // 2 421; 288 x 256 and 256 x 288 2 861 and 2 662, 2 771 and 2 656; 256 x 192 1 867 and 1 811.  In time 0.5 to 2 %: at
+            // the power limit the chip gives most of it back as a lower clock (1.7 to 1.9 GHz).  The 256 x 96 tile is bound by its
+            // loads (1 257 and 1 260 cycles, 768 of them MFMAs) and is the same either way, within 1 % at eight shapes.
             if constexpr (M16) {
                 if (last) __builtin_amdgcn_s_setprio(1);
                 if (ks == 1) __builtin_amdgcn_s_setprio(0);
@@ -1118,7 +1121,8 @@ inline Tile choose_tile(int64_t M, int64_t N) {
     // dearer than 256 x 256 (more LDS and global->LDS traffic per MFMA) and the 288 x 256 tile of
     // twelve waves, or 256 x 288, about 2 % (they pay where they save a round: 4608 x 12288 takes 768
     // tiles of 288 x 256, three rounds, instead of 864 of 256 x 256, four; 4096 x 9216 takes 512 of
-    // 256 x 288, two rounds).  Outputs of fewer than 128
+    // 256 x 288, two rounds).  (By the cycles of a K-tile now 7 and 5 %: 1 811 and 2 660 against 2 254; with those prices the
+    // pick is the same on 118 of 122 shapes of up to 9729 x 21504.)  Outputs of fewer than 128
     // such tiles take 128 x 128 tiles with two stages if that gives at least one workgroup per CU,
     // else the four-stage configurations above.
     const int64_t CUS = 256;
@@ -1296,12 +1300,17 @@ int launch_cfg_grouped(const GemmArgs *gs, int n, hipStream_t st) {
 I8F_EXTERN_GROUPED(CfgBig) I8F_EXTERN_GROUPED(CfgB192) I8F_EXTERN_GROUPED(CfgTall) I8F_EXTERN_GROUPED(CfgWide)
 #undef I8F_EXTERN_GROUPED
 
-// Estimated shader cycles of one launch, for the choice between one launch for a group of problems and one launch per
-// problem; the constants are this kernel's measured figures.  A one-workgroup-per-CU tile costs its rounds over the 256
-// CUs times K-tiles times the time of a K-tile (2 970 cycles for 256 x 256, the others in proportion to their area and
-// their relative cost per operation, as choose_tile prices them); the few-tile configurations cost what their busiest
-// CU fetches at 33 bytes per cycle (with the K split: the model of choose_split); every launch 12 000 cycles of launch,
-// prologue and epilogue.
+// Prices of one launch, for the choice between one launch for a group of problems and one launch per problem.  A
+// one-workgroup-per-CU tile costs its rounds over the 256 CUs times K-tiles times the price of a K-tile (2 970 for 256 x 256,
+// the others in proportion to their area and their relative cost per operation, as choose_tile prices them); the few-tile
+// configurations cost what their busiest CU fetches, at 33 bytes to the unit (with the K split: the model of choose_split);
+// every launch 12 000 of launch, prologue and epilogue.  The unit was a shader cycle of an earlier form of the loop; the
+// present one takes 2 250 cycles a K-tile on one set of operands and 2 290 to 2 420 on operands from HBM.  What the prices are
+// held to is the choice: over 32 pairs (1024 ... 9216 and 77 ... 1024 rows, N and K 2048 ... 15360, operands from HBM) it is
+// 1.2 % from the faster of a group with any of the four tiles and separate launches, on average; in 28 pairs within 3.5 %.
+// With 2 300 for the K-tile (and 107, 105, 105 for the other tiles) it is 1.2 % as well: 4096 + 512 x 9216 x 3072 gains 2 %
+// and 2048 + 77 x 3072 x 3072 14 %, 1024 + 512 x 3072 x 3072 loses 5 % and 1024 + 512 x 12288 x 3072 10 %.  Neither sees that a
+// chip at its power limit gives a round that is not full a higher clock: 4096 + 256 x 12288 x 3072, one launch 151 us, two 139.
 constexpr int64_t LAUNCH_CYCLES = 12000;
 inline void tile_shape(Tile t, int *bm, int *bn) {
     int st = 0;
