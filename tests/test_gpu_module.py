@@ -6,6 +6,7 @@ import os
 import re
 import shutil
 import subprocess
+import threading
 
 import numpy as np
 import pytest
@@ -581,3 +582,62 @@ def test_layer_without_outputs(pkg, dev):
         assert lin(x).shape == (rows, 0) and pkg.forward_fanout([lin, lin], x)[1].shape == (rows, 0)
     with pytest.raises((RuntimeError, ValueError)):
         lin(x, gate=gate)
+
+
+@pytest.mark.parametrize("quarot", [False, True])
+@pytest.mark.parametrize("ranks,K,stacked", [((16, 32, 64), 256, True), ((4,), 256, True), ((3, 5), 272, True), ((3, 5, 6), 256, False), ((128, 128, 128), 256, False),
+                                             ((16, 32), 250, False), ((8, "loha"), 256, False), ((16, 32), 256, None)])
+def test_merged_adapter_stacked_and_summed(pkg, dev, quarot, ranks, K, stacked):
+    """A stack of LoRAs with its factors side by side: the oracle's fma chain over the stacked factors, each `down` times its
+    multiplier and then rotated; stacks that the fused kernel has no form for, and all with that form switched off (None):
+    the oracle fed with the sum of the reconstructed deltas.  A slice of a fused weight with the whole scale tensor too."""
+    pkg.Int8TensorwiseOps.enable_quarot = quarot
+    rotate, N = quarot and K % 128 == 0, 96
+    f = lambda *shape: torch.randn(*shape, generator=G) * 0.05
+    wq = torch.randint(-128, 128, (N, K), dtype=torch.int8, generator=G)
+    ws = torch.rand(3 * N, 1, generator=G) * 0.002 + 0.0005
+    weights = [(f(N, 4), f(4, K), 4.0, f(N, 4), f(4, K), None, None, None) if r == "loha" else (f(N, r), f(r, K), 2.0 * r if i else None, None, None, None)
+               for i, r in enumerate(ranks)]
+    strengths = [0.75 * (-0.5) ** i for i in range(len(ranks))]
+    merged = pkg.INT8MergedLoRAPatchAdapter([(pkg.INT8LoRAPatchAdapter({"k"}, w, ws), st) for w, st in zip(weights, strengths)], ws, seed=29)
+    merged.fuse_low_rank = stacked is not None
+    out = merged.calculate_weight(wq, "k", 1.0, 1.0, (0, N, N), None)
+    assert (merged._stacked_factors(wq, dev) is not None) == (stacked is not False)
+    noise = pkg.int8_quant._draw_noise((N, K), 29, dev).cpu().numpy()
+    if stacked:
+        down = torch.cat([w[1] * (st if w[2] is None else 2.0 * st) for w, st in zip(weights, strengths)]).numpy()
+        kw = dict(up=torch.cat([w[0] for w in weights], 1).numpy(), down=O.rotate(down, O.F32) if rotate else down)
+    else:
+        total = None
+        for w, st in zip(weights, strengths):
+            diff, mult = pkg.int8_quant.reconstruct_lora_diff(w, (N, K), dev, torch.float32, st)
+            total = diff * mult if total is None else total + diff * mult
+        kw = dict(delta=O.rotate(total.cpu().numpy(), O.F32) if rotate else total.cpu().numpy())
+    assert np.array_equal(out.numpy(), O.lora_merge_sr(wq.numpy(), ws[N:2 * N].numpy(), noise, **kw))
+
+
+def test_native_host_path_on_several_streams_and_threads(pkg, dev):
+    """Four threads, each with a stream of its own and layers of every route (a split K with its workspace of the stream, many
+    and few rows, rotated): the results of the same calls one after the other."""
+    L, jobs = pkg._lib, []
+    for rows, K, N, rotate in ((40, 12288, 264, False), (300, 384, 192, True), (4, 384, 192, True), (12, 12288, 64, False)):
+        q, s = L.quant_rowwise((torch.randn(N, K, generator=G) * 0.02).to(dev), rotate=rotate)
+        lin = load(pkg.Int8TensorwiseOps.Linear(K, N, bias=True), {"l.weight": q, "l.weight_scale": s, "l.bias": torch.randn(N, generator=G).bfloat16().to(dev)})
+        lin._use_quarot = rotate
+        jobs.append((lin, [torch.randn(rows, K, generator=G).bfloat16().to(dev) for _ in range(4)]))
+    want = [[lin(x) for x in xs] for lin, xs in jobs]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        stream = torch.cuda.Stream(dev)
+        with torch.no_grad(), torch.cuda.stream(stream):
+            got = [(j, lin(xs[i])) for _ in range(20) for j, (lin, xs) in enumerate(jobs)]
+            wrong.extend(j for j, y in got if not torch.equal(y, want[j][i]))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong

@@ -1336,3 +1336,31 @@ def test_normalised_rows_do_not_depend_on_how_many_there_are(L, dev, K, dt, rota
         for m in (1, 17, 256, 257, 512, 513, 1024, 1025, 2048):
             qm, sm = L.quant_rowwise(x[:m], rotate=rotate, **kw)
             assert torch.equal(qm, q[:m]) and torch.equal(sm, sc[:m]), (kw["prologue"], m)
+
+
+@pytest.mark.parametrize("M,K,dt,V", [(2056, 3840, torch.float16, 1), (1028, 3072, torch.bfloat16, 2), (1026, 2176, torch.bfloat16, 3), (260, 2048, torch.float16, 4)])
+def test_rotated_prologues_on_rows_held_by_one_wave(L, dev, M, K, dt, V):
+    """More rows than four waves to a row are taken for: every prologue together with the rotation in the one-wave form, two to
+    four runs to a lane, against the oracle and torch with the bars of the tests above."""
+    M -= M % V
+    if dt == torch.bfloat16:   # (binary16: torch's addcmul on this device rounds straight to binary16, this library and torch on the
+        test_quant_rowwise_modulate_prologue_bit_exact(L, dev, M, K, dt, True, V)   # CPU by way of binary32: 3 in a million differ)
+    test_quant_rowwise_gelu_prologue_within_tolerance(L, dev, M, K, dt, True, V)
+    test_quant_rowwise_gelu_erf_prologue_within_tolerance(L, dev, M, K, dt, True, V)
+    test_quant_rowwise_silu_gate_prologue_within_tolerance(L, dev, M, K, dt, True, V)
+    test_quant_rowwise_norm_modulate_prologue_within_tolerance(L, dev, M, K, dt, True, V, 1e-6)
+    test_quant_rowwise_rms_norm_prologue_within_tolerance(L, dev, M, K, dt, True, V, 1e-5, "wst")
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 70001, 30720), (70001, 9, 30701), (65552, 32776, 20)])
+def test_ragged_gemm_beyond_2_pow_31_elements(L, dev, M, N, K):
+    """A weight, activations or a result of more than 2^31 elements in the kernel for operands that fit no tile: every output
+    against the product in binary64, which holds these sums exactly."""
+    assert max(N * K, M * K, M * N) > 2**31
+    g = torch.Generator(device=dev).manual_seed(31)
+    a, w = (torch.randint(-127, 128, (n, K), dtype=torch.int8, generator=g, device=dev) for n in (M, N))
+    out = L.gemm_i32(a, w)
+    for m in range(0, M, 4096):
+        for n in range(0, N, 8192):
+            want = a[m:m + 4096].double() @ w[n:n + 8192].double().T
+            assert torch.equal(out[m:m + 4096, n:n + 8192].double(), want), (m, n)
