@@ -1055,8 +1055,8 @@ using CfgWide = Cfg<256, 288, 128, 4, 3, 2, 8, 0, 16>;  // 12 waves of 64 x 96, 
 // whole LDS -- were measured and are not kept: 39.8 us against 38.7 us at 4608 x 3072 x 3072, 130.3 against 125.2 us at
 // K = 12288.  The misses they take off the busy CUs do not pay for what their requests add to the XCD's L2 queues.)
 // (A 288 x 192 tile of twelve 96 x 48 waves, which covers 4608 x 3072 in exactly 256 workgroups, was measured and is not
-// kept: 42.9 us against 37.7 us for the 216 tiles of 256 x 256.  It moves 11 % more bytes per multiply-accumulate through a
-// load path that is already the bound, and with all 256 CUs multiplying the clock settles 8 % lower.)
+// kept: 42.9 us against 37.7 us for the 216 tiles of 256 x 256.  It moves 11 % more bytes per multiply-accumulate,
+// and with all 256 CUs multiplying the clock settles 8 % lower.)
 // Outputs of few tiles: about one workgroup per CU, so nothing hides the latency of the global->LDS
 // loads (the weight comes from HBM: a model's weights are far larger than the caches) but the loads in
 // flight; four stages instead of two, and the largest tile that still gives 192 workgroups.

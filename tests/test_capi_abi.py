@@ -197,5 +197,5 @@ def test_gemm_tile_reports_the_configuration_of_the_benchmark_shapes(L):
     assert L.gemm_tile(4608, 12288, 3072) == (288, 256, 2)
     assert L.gemm_tile(4608, 3072, 12288) == (256, 256, 2)
     assert L.gemm_tile(512, 12288, 3072) == (256, 96, 3)
-    assert L.gemm_tile(33, 64, 77) == (1, 1, 0)           # K % 16 != 0: the generic kernel
+    assert L.gemm_tile(33, 64, 77) == (1, 1, 0)           # K % 16 != 0: the ragged kernel
     assert L.lib().i8f_gemm_tile(0, 8, 16, None, None, None) == -1

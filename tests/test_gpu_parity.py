@@ -590,7 +590,7 @@ GATED_CASES = [
     (4600, 12288, 128, True, torch.float16, 1, True), (1000, 264, 384, False, torch.bfloat16, 4, True),      # 288 x 256; ragged
     (512, 3072, 12288, True, torch.bfloat16, 2, True),                                                       # few tiles, K split
     (300, 512, 256, True, torch.float32, 3, True), (130, 96, 128, True, torch.bfloat16, 1, False),           # binary32; gate alone
-    (257, 3076, 640, True, torch.float16, 1, True),                                                          # N % 8 != 0: the one-thread-per-output kernel
+    (257, 3076, 640, True, torch.float16, 1, True),                                                          # N % 8 != 0: the ragged kernel
 ]
 
 
@@ -1321,21 +1321,19 @@ def test_quantiser_with_four_waves_to_a_row_equals_one_wave(L, dev, K):
 
 @pytest.mark.parametrize("K,dt", [(1040, torch.bfloat16), (2048, torch.float16), (2064, torch.bfloat16), (3072, torch.bfloat16), (3840, torch.float16),
                                   (4096, torch.bfloat16), (4112, torch.bfloat16)])
-@pytest.mark.parametrize("rotate", [False, True])
-def test_normalised_rows_do_not_depend_on_how_many_there_are(L, dev, K, dt, rotate):
+def test_normalised_rows_do_not_depend_on_how_many_there_are(L, dev, K, dt):
     """LayerNorm and RMSNorm inside the quantiser: a row's int8 and its scale are the same bits alone, among few rows (four
     waves to a row) and among many (one wave), at row counts on both sides of every line."""
-    if rotate and K % 128:
-        pytest.skip("rotated widths are multiples of 128")
     x = (torch.randn(2056, K, generator=G) * torch.exp2(torch.randint(-4, 4, (2056, 1), generator=G).float()) + 0.25).to(dt)
     x[:, 5] *= 30
     x, (w, s, t) = x.to(dev), ((torch.randn(K, generator=G) * 0.2 + 1).to(dt).to(dev) for _ in range(3))
-    for kw in (dict(prologue=L.PRO_NORM_MODULATE, mod_scale=s, mod_shift=t, eps=1e-6),
-               dict(prologue=L.PRO_RMS_NORM, norm_weight=w, mod_scale=s, mod_shift=t, eps=1e-6, fused_add=True), dict(prologue=L.PRO_RMS_NORM, eps=1e-5)):
-        q, sc = L.quant_rowwise(x, rotate=rotate, **kw)
+    forms = (dict(prologue=L.PRO_NORM_MODULATE, mod_scale=s, mod_shift=t, eps=1e-6),
+             dict(prologue=L.PRO_RMS_NORM, norm_weight=w, mod_scale=s, mod_shift=t, eps=1e-6, fused_add=True), dict(prologue=L.PRO_RMS_NORM, eps=1e-5))
+    for kw in [{**f, "rotate": r} for f in forms for r in (False, True) if not r or K % 128 == 0]:
+        q, sc = L.quant_rowwise(x, **kw)
         for m in (1, 17, 256, 257, 512, 513, 1024, 1025, 2048):
-            qm, sm = L.quant_rowwise(x[:m], rotate=rotate, **kw)
-            assert torch.equal(qm, q[:m]) and torch.equal(sm, sc[:m]), (kw["prologue"], m)
+            qm, sm = L.quant_rowwise(x[:m], **kw)
+            assert torch.equal(qm, q[:m]) and torch.equal(sm, sc[:m]), (kw["prologue"], kw["rotate"], m)
 
 
 @pytest.mark.parametrize("M,K,dt,V", [(2056, 3840, torch.float16, 1), (1028, 3072, torch.bfloat16, 2), (1026, 2176, torch.bfloat16, 3), (260, 2048, torch.float16, 4)])
