@@ -81,8 +81,9 @@ def lib() -> ctypes.CDLL:
     L.i8f_linear_w8a16_small_m_grouped.argtypes = [vp, i32, i32, i32, i32, vp]
     L.i8f_sr_quant_delta.argtypes = [vp, vp, f32, i32, vp, i64, i64, vp, vp]
     L.i8f_lora_merge_sr.argtypes = [vp, vp, f32, i32, vp, vp, vp, i64, f32, vp, i64, i64, vp, vp]
+    L.i8f_lora_merge_sr_drawn.argtypes = [vp, vp, f32, i32, vp, vp, i64, f32, ctypes.c_uint64, i64, i64, i64, vp, vp, i64, vp]
     for name in ("i8f_quant_rowwise_concat_gelu", "i8f_quant_rowwise_rms_norm", "i8f_linear_w8a8_gated", "i8f_quant_rowwise", "i8f_quant_rowwise_grouped", "i8f_quant_rowwise_prologue", "i8f_quant_rowwise_norm_modulate", "i8f_quant_tensorwise", "i8f_quant_tensorwise_static", "i8f_rotate128", "i8f_gemm_i32", "i8f_linear_w8a8", "i8f_linear_w8a8_add", "i8f_linear_w8a8_splitk", "i8f_linear_w8a8_grouped", "i8f_linear_w8a8_lora",
-                 "i8f_linear_w8a16_small_m", "i8f_linear_w8a16_small_m_grouped", "i8f_sr_quant_delta", "i8f_lora_merge_sr"):
+                 "i8f_linear_w8a16_small_m", "i8f_linear_w8a16_small_m_grouped", "i8f_sr_quant_delta", "i8f_lora_merge_sr", "i8f_lora_merge_sr_drawn"):
         getattr(L, name).restype = i32
     _lib = L
     return L
@@ -791,6 +792,40 @@ def lora_merge_sr(w, w_scale, noise, delta=None, up=None, down=None, lora_scale=
     with _on(w.device):
         _check(lib().i8f_lora_merge_sr(_ptr(w), _ptr(ws), ws_host, mode, _ptr(delta), _ptr(up), _ptr(down), rank,
                                        float(lora_scale), _ptr(noise), N, K, _ptr(out), _stream(w)), "i8f_lora_merge_sr")
+    return out
+
+
+# The torch whose generator i8f_lora_merge_sr_drawn reproduces: which counter and which word an element of torch.rand takes is
+# not part of torch's interface.  Under any other version torch draws the noise.
+DRAWS_LIKE_TORCH = torch.__version__.split("+")[0].startswith("2.10.") and torch.version.hip is not None
+
+
+def lora_merge_sr_drawn(w, w_scale, generator, up, down, lora_scale=1.0):
+    """lora_merge_sr(w, w_scale, torch.rand(w.shape, generator=generator, device=w.device), up=up, down=down, ...) for a generator
+    that has just been seeded, without the noise tensor.  None where the kernel does not take the operands
+    (i8f_lora_merge_sr_drawn) or the installed torch may draw otherwise; the caller then draws the noise."""
+    if not DRAWS_LIKE_TORCH or not w.is_cuda or w.dim() != 2 or up.dim() != 2 or generator.device.type != "cuda":
+        return None
+    (N, K), rank = w.shape, up.shape[1]
+    if K % 16 or rank % 4 or not 0 < rank <= 256 or not 0 < N * K <= 1 << 29 or torch.cuda.is_current_stream_capturing():
+        return None
+    w = _i8_matrix(w, "w")
+    up = _f32_matrix(up, "up", w.device)
+    down = _f32_matrix(down, "down", w.device)
+    if up.shape[0] != N or down.shape != (rank, K):
+        raise ValueError(f"up must be [{N},r] and down [r,{K}]")
+    if (w.data_ptr() | up.data_ptr()) % 16:
+        return None
+    ws, ws_host, mode = _scale(w_scale, N, w.device)
+    out = torch.empty_like(w)
+    scratch = torch.empty(N * K, dtype=torch.int16, device=w.device)
+    # torch draws in blocks of 256 threads, as many as the GPU holds at most, each thread four elements at a time
+    props = torch.cuda.get_device_properties(w.device)
+    lanes = 256 * min(-(-N * K // 256), props.multi_processor_count * (props.max_threads_per_multi_processor // 256))
+    with _on(w.device):
+        _check(lib().i8f_lora_merge_sr_drawn(_ptr(w), _ptr(ws), ws_host, mode, _ptr(up), _ptr(down), rank, float(lora_scale),
+                                             generator.initial_seed() & 0xFFFFFFFFFFFFFFFF, lanes, N, K, _ptr(out), _ptr(scratch),
+                                             2 * N * K, _stream(w)), "i8f_lora_merge_sr_drawn")
     return out
 
 

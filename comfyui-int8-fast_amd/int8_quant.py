@@ -303,10 +303,22 @@ def _slice_scale_mismatch_only(ws, delta_rows: int, offset):
     return ws
 
 
-def _draw_noise(shape, seed: int, device) -> Tensor:
+def _seeded(seed: int, device) -> torch.Generator:
     gen = torch.Generator(device=device)
     gen.manual_seed(seed)
-    return torch.rand(shape, generator=gen, device=device, dtype=torch.float32)
+    return gen
+
+
+def _draw_noise(shape, seed: int, device) -> Tensor:
+    return torch.rand(shape, generator=_seeded(seed, device), device=device, dtype=torch.float32)
+
+
+def _merge_low_rank(w: Tensor, scale, seed: int, up: Tensor, down: Tensor, lora_scale=1.0) -> Tensor:
+    """The fused merge with the noise of _draw_noise, drawn inside the kernel where that is possible."""
+    merged = _lib.lora_merge_sr_drawn(w, scale, _seeded(seed, w.device), up, down, lora_scale)
+    if merged is None:
+        merged = _lib.lora_merge_sr(w, scale, _draw_noise(tuple(w.shape), seed, w.device), up=up, down=down, lora_scale=lora_scale)
+    return merged
 
 
 def _quarot_applies(weight: Tensor) -> bool:
@@ -350,7 +362,6 @@ class INT8LoRAPatchAdapter(LoRAAdapter):
         w_dev = weight.to(dev)
         rotate = _quarot_applies(weight)
         eff = self._get_effective_scale(weight.shape[0], offset)
-        noise = _draw_noise(tuple(weight.shape), self.seed, dev)
         plain = _plain_lora(self.weights) if self.fuse_low_rank else None
         if plain is not None and intermediate_dtype == torch.float32 and plain[1].shape[0] <= 256:
             up, down = (t.to(dev, torch.float32) for t in plain)
@@ -358,7 +369,7 @@ class INT8LoRAPatchAdapter(LoRAAdapter):
             mult = (alpha / down.shape[0]) * strength if alpha is not None else strength
             if rotate:  # rotating the rows of up @ down is rotating the rows of down
                 down = _lib.rotate128(down)
-            merged = _lib.lora_merge_sr(w_dev, eff, noise, up=up, down=down, lora_scale=mult)
+            merged = _merge_low_rank(w_dev, eff, self.seed, up, down, mult)
         else:
             diff, mult = reconstruct_lora_diff(self.weights, weight.shape, dev, intermediate_dtype, strength)
             if diff is None:
@@ -366,7 +377,7 @@ class INT8LoRAPatchAdapter(LoRAAdapter):
             delta = (diff * mult).float()
             if rotate:
                 delta = _lib.rotate128(delta, out=delta)
-            merged = _lib.lora_merge_sr(w_dev, eff, noise, delta=delta)
+            merged = _lib.lora_merge_sr(w_dev, eff, _draw_noise(tuple(weight.shape), self.seed, dev), delta=delta)
         return merged.to(home)
 
 
@@ -424,8 +435,7 @@ class INT8MergedLoRAPatchAdapter(LoRAAdapter):
                 if _quarot_applies(weight):   # rotating the rows of up @ down is rotating the rows of down
                     down = _lib.rotate128(down)
                 eff = self._get_effective_scale(weight.shape[0], offset)
-                noise = _draw_noise(tuple(weight.shape), self.seed, dev)
-                return _lib.lora_merge_sr(weight.to(dev), eff, noise, up=up, down=down).to(home)
+                return _merge_low_rank(weight.to(dev), eff, self.seed, up, down).to(home)
         total = None
         for adapter, lora_strength in self.patches:  # ComfyUI's own `strength` is ignored here, as in the reference
             diff, mult = reconstruct_lora_diff(adapter.weights, weight.shape, dev, intermediate_dtype, lora_strength)

@@ -1,0 +1,63 @@
+"""The LoRA merge that draws its noise itself, against the merge on torch's own noise: the same bits."""
+import ctypes
+
+import pytest
+import torch
+
+# Shapes: elements below, at and beyond the generator's 524288 threads and its calls of four times as many (a partial last
+# block, quarters that end inside a row); widths of one piece, of an odd number of 16, of several 256-column blocks and a rest;
+# rows that fill no block of 32; every kind of rank (padded, four-wave, eight-wave workgroups).
+CASES = [
+    # N, K, rank, seed, scale per row, std of the factors
+    (1, 16, 4, 27, True, 0.01), (17, 48, 12, -5, True, 0.01), (128, 4096, 16, 2**63 + 12345, True, 0.01), (513, 1040, 8, 1, False, 0.01),
+    (2049, 1024, 32, 2, True, 0.01), (682, 3088, 20, 3, True, 0.01), (7, 524288, 4, 4, True, 0.01), (700, 12288, 64, 5, True, 0.01),
+    (1000, 3072, 112, 6, True, 0.01), (333, 1552, 256, 7, True, 0.01), (4099, 2064, 48, 8, True, 0.01),
+    (400, 2064, 8, 9, True, 10.0),       # every quotient far outside int8
+    (400, 2064, 8, 10, True, 1e-20),     # products in the denormal range
+    (400, 2064, 16, 11, True, 0.25),     # quotients of some tens: many elements are redone
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,rank,seed,row,std", CASES)
+def test_drawn_merge_equals_the_merge_on_torchs_noise(pkg, L, dev, N, K, rank, seed, row, std):
+    if not L.DRAWS_LIKE_TORCH:
+        pytest.skip("this torch's generator is not the one that is reproduced")
+    g = torch.Generator(device=dev).manual_seed(N + K + rank)
+    w = torch.randint(-128, 128, (N, K), generator=g, device=dev, dtype=torch.int8)
+    ws = torch.rand(N if row else 1, generator=g, device=dev) * 0.002 + 0.0005
+    up, down = torch.randn(N, rank, generator=g, device=dev) * std, torch.randn(rank, K, generator=g, device=dev) * std
+    if N > 100:   # rows that have no quotient or leave the range of the approximate one
+        up[3], up[5], up[6] = float("nan"), float("inf"), 0.0
+        if row:
+            ws[7], ws[8] = 1e-39, 3e7
+    noise = pkg.int8_quant._draw_noise((N, K), seed, dev)
+    drawn = L.lora_merge_sr_drawn(w, ws, pkg.int8_quant._seeded(seed, dev), up, down, 0.75)
+    assert torch.equal(drawn, L.lora_merge_sr(w, ws, noise, up=up, down=down, lora_scale=0.75))
+
+
+@pytest.mark.gpu
+def test_adapters_draw_what_they_drew(pkg, L, dev, monkeypatch):
+    N, K = 640, 1040
+    w = torch.randint(-127, 128, (N, K), dtype=torch.int8, device=dev)
+    ws = torch.rand(N, 1, device=dev) * 0.002 + 0.0005
+    lora = lambda r: (torch.randn(N, r, device=dev) * 0.02, torch.randn(r, K, device=dev) * 0.02, float(r), None, None, None)
+    one = pkg.INT8LoRAPatchAdapter(set(), lora(16), ws, seed=7)
+    stack = pkg.INT8MergedLoRAPatchAdapter([(pkg.INT8LoRAPatchAdapter(set(), lora(r), ws), 0.5) for r in (3, 9, 8)], ws, seed=8)
+    now = [a.calculate_weight(w, "", 1.0, 1.0, None, None) for a in (one, stack)]
+    monkeypatch.setattr(L, "DRAWS_LIKE_TORCH", False)
+    for got, a in zip(now, (one, stack)):
+        assert torch.equal(got, a.calculate_weight(w, "", 1.0, 1.0, None, None))
+
+
+def test_drawn_merge_refuses_what_it_cannot_do(L):
+    one, null = ctypes.c_void_p(4096), None
+    call = lambda w=one, up=one, rank=8, lanes=256, N=4, K=16, ws=one, mode=0, nbytes=128: L.lib().i8f_lora_merge_sr_drawn(
+        w, ws, 1.0, mode, up, one, rank, 1.0, 0, lanes, N, K, one, one, nbytes, null)
+    INVALID, UNSUPPORTED = -1, -2
+    assert call(w=null) == INVALID and call(up=null) == INVALID and call(rank=0) == INVALID and call(lanes=0) == INVALID
+    assert call(ws=null, mode=1) == INVALID and call(mode=2) == INVALID and call(nbytes=127) == INVALID and call(N=-1) == INVALID
+    assert call(K=24) == UNSUPPORTED and call(rank=6) == UNSUPPORTED and call(rank=260) == UNSUPPORTED and call(lanes=100) == UNSUPPORTED
+    assert call(up=ctypes.c_void_p(4100)) == UNSUPPORTED and call(N=2**25 + 1) == UNSUPPORTED
+    assert call(N=2**24, nbytes=2**29) == UNSUPPORTED      # more calls of the generator than a launch has blocks
+    assert call(N=0) == 0 and call(K=0) == 0
