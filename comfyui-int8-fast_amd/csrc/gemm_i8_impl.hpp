@@ -948,21 +948,65 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
             constexpr int CPO = ROW_BYTES / 16;      // chunks per output row
             constexpr int EPCO = 16 / OB;            // output elements per chunk
             constexpr int PASSES = EPI_STRIPS * 32 * CPO / 64;
+            const int mw = m0 + wm * C::WTM + i0 * 32, nw = n0 + wn * C::WTN;   // first row and column of the staged strips
+            // Gate and addend of BATCH pieces are requested together, and those of the next batch before this one is used: a load
+            // behind each store, above which it may not be moved, is a trip to memory for every piece (35 to 54 K cycles of
+            // epilogue at 4608 x 3072, 9.6 K without gate and addend; 28 to 43 K in fours).  us, gate and addend, before and
+            // after: 4608 x 3072 x 3072 50.6 and 48.2, x 12288 156.7 and 153.3, 9729 x 3072 x 15360 370 and 361, 512 x 3072 x 12288 in
+            // 128 x 96 tiles and two slices 38.6 and 37.0.  Twelve waves
+            // have no registers for it (4096 x 9216 x 3072 in 256 x 288 tiles 136 and 141 us).
+            constexpr bool BATCHED = C::NT <= 512;
+            if ((!ggate && !gaddend) || !BATCHED) {
 #pragma unroll
-            for (int p = 0; p < PASSES; ++p) {
-                const int id = p * 64 + lane;
-                const int row = id / CPO, cc = id % CPO;
-                const uint4 val = *(const uint4 *)(ebuf + row * PITCH + cc * 16);
-                const int mm = m0 + wm * C::WTM + i0 * 32 + row;
-                const int nn = n0 + wn * C::WTN + cc * EPCO;
-                if (mm < gM && nn < gN)
-                {
-                    const int64_t off = ((int64_t)mm * gN + nn) * OB;
-                    uint4 v = val;
-                    if (ggate)
-                        v = mul_rounded<OUT>(v, *(const uint4 *)((const char *)ggate + ((int64_t)((uint32_t)mm / (uint32_t)ggate_rows) * gN + nn) * OB));
-                    if (gaddend) v = add_rounded<OUT>(v, *(const uint4 *)((const char *)gaddend + off));
-                    stream_store16((char *)gout + off, v);
+                for (int p = 0; p < PASSES; ++p) {
+                    const int id = p * 64 + lane;
+                    const int row = id / CPO, cc = id % CPO;
+                    const uint4 val = *(const uint4 *)(ebuf + row * PITCH + cc * 16);
+                    const int mm = mw + row, nn = nw + cc * EPCO;
+                    if (mm < gM && nn < gN) {
+                        const int64_t off = ((int64_t)mm * gN + nn) * OB;
+                        uint4 v = val;
+                        if constexpr (!BATCHED) {
+                            if (ggate)
+                                v = mul_rounded<OUT>(v, *(const uint4 *)((const char *)ggate + ((int64_t)((uint32_t)mm / (uint32_t)ggate_rows) * gN + nn) * OB));
+                            if (gaddend) v = add_rounded<OUT>(v, *(const uint4 *)((const char *)gaddend + off));
+                        }
+                        stream_store16((char *)gout + off, v);
+                    }
+                }
+            } else {
+                constexpr int BATCH = PASSES <= 8 ? PASSES : 4;
+                static_assert(PASSES % BATCH == 0, "whole batches");
+                uint4 gate_r[2][BATCH], add_r[2][BATCH];
+                const bool one_gate = !ggate || (uint32_t)mw / (uint32_t)ggate_rows == (uint32_t)min(mw + EPI_STRIPS * 32 - 1, gM - 1) / (uint32_t)ggate_rows;
+                const int first_gate = ggate ? (int)((uint32_t)mw / (uint32_t)ggate_rows) : 0;
+                auto fetch = [&](int p0, uint4 (&gr)[BATCH], uint4 (&ar)[BATCH]) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int u = 0; u < BATCH; ++u) {   // (rows and columns beyond the output repeat the last ones, unused)
+                        const int id = (p0 + u) * 64 + lane;
+                        const int mm = min(mw + id / CPO, gM - 1), nn = min(nw + id % CPO * EPCO, gN - EPCO);
+                        if (gaddend) ar[u] = *(const uint4 *)((const char *)gaddend + ((int64_t)mm * gN + nn) * OB);
+                        if (ggate) {
+                            const int gv = one_gate ? first_gate : (int)((uint32_t)mm / (uint32_t)ggate_rows);
+                            gr[u] = *(const uint4 *)((const char *)ggate + ((int64_t)gv * gN + nn) * OB);
+                        }
+                    }
+                };
+                fetch(0, gate_r[0], add_r[0]);
+#pragma unroll
+                for (int p0 = 0; p0 < PASSES; p0 += BATCH) {
+                    const int now = p0 / BATCH % 2;
+                    if (p0 + BATCH < PASSES) fetch(p0 + BATCH, gate_r[now ^ 1], add_r[now ^ 1]);
+#pragma unroll
+                    for (int u = 0; u < BATCH; ++u) {
+                        const int id = (p0 + u) * 64 + lane;
+                        const int row = id / CPO, cc = id % CPO;
+                        uint4 v = *(const uint4 *)(ebuf + row * PITCH + cc * 16);
+                        const int mm = mw + row, nn = nw + cc * EPCO;
+                        if (ggate) v = mul_rounded<OUT>(v, gate_r[now][u]);
+                        if (gaddend) v = add_rounded<OUT>(v, add_r[now][u]);
+                        if (mm < gM && nn < gN) stream_store16((char *)gout + ((int64_t)mm * gN + nn) * OB, v);
+                    }
                 }
             }
             __builtin_amdgcn_wave_barrier();
