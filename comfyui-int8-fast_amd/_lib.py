@@ -81,7 +81,9 @@ def lib() -> ctypes.CDLL:
     L.i8f_linear_w8a16_small_m_grouped.argtypes = [vp, i32, i32, i32, i32, vp]
     L.i8f_sr_quant_delta.argtypes = [vp, vp, f32, i32, vp, i64, i64, vp, vp]
     L.i8f_lora_merge_sr.argtypes = [vp, vp, f32, i32, vp, vp, vp, i64, f32, vp, i64, i64, vp, vp]
-    L.i8f_lora_merge_sr_drawn.argtypes = [vp, vp, f32, i32, vp, vp, i64, f32, ctypes.c_uint64, i64, i64, i64, vp, vp, i64, vp]
+    L.i8f_lora_merge_sr_drawn.argtypes = [vp, vp, f32, i32, vp, i32, f32, ctypes.c_uint64, i64, i64, i64, vp, vp, i64, vp]
+    L.i8f_lora_merge_sr_drawn_workspace_bytes.argtypes = [i64, i64, i64, i32]
+    L.i8f_lora_merge_sr_drawn_workspace_bytes.restype = i64
     for name in ("i8f_quant_rowwise_concat_gelu", "i8f_quant_rowwise_rms_norm", "i8f_linear_w8a8_gated", "i8f_quant_rowwise", "i8f_quant_rowwise_grouped", "i8f_quant_rowwise_prologue", "i8f_quant_rowwise_norm_modulate", "i8f_quant_tensorwise", "i8f_quant_tensorwise_static", "i8f_rotate128", "i8f_gemm_i32", "i8f_linear_w8a8", "i8f_linear_w8a8_add", "i8f_linear_w8a8_splitk", "i8f_linear_w8a8_grouped", "i8f_linear_w8a8_lora",
                  "i8f_linear_w8a16_small_m", "i8f_linear_w8a16_small_m_grouped", "i8f_sr_quant_delta", "i8f_lora_merge_sr", "i8f_lora_merge_sr_drawn"):
         getattr(L, name).restype = i32
@@ -800,32 +802,46 @@ def lora_merge_sr(w, w_scale, noise, delta=None, up=None, down=None, lora_scale=
 DRAWS_LIKE_TORCH = torch.__version__.split("+")[0].startswith("2.10.") and torch.version.hip is not None
 
 
-def lora_merge_sr_drawn(w, w_scale, generator, up, down, lora_scale=1.0):
+class _LoraFactors(ctypes.Structure):
+    _fields_ = [("up", ctypes.c_void_p), ("down", ctypes.c_void_p), ("rank", ctypes.c_int64), ("mult", ctypes.c_float)]
+
+
+def lora_merge_sr_drawn(w, w_scale, generator, factors, lora_scale=1.0):
     """lora_merge_sr(w, w_scale, torch.rand(w.shape, generator=generator, device=w.device), up=up, down=down, ...) for a generator
-    that has just been seeded, without the noise tensor.  None where the kernel does not take the operands
+    that has just been seeded, without the noise tensor.  factors: (up, down, mult) of one LoRA (mult is ignored) or of
+    several, whose factors are put side by side, each `down` times its mult.  None where the kernel does not take the operands
     (i8f_lora_merge_sr_drawn) or the installed torch may draw otherwise; the caller then draws the noise."""
-    if not DRAWS_LIKE_TORCH or not w.is_cuda or w.dim() != 2 or up.dim() != 2 or generator.device.type != "cuda":
+    if not DRAWS_LIKE_TORCH or not w.is_cuda or w.dim() != 2 or generator.device.type != "cuda" or not 0 < len(factors) <= 8:
         return None
-    (N, K), rank = w.shape, up.shape[1]
-    if K % 16 or rank % 4 or not 0 < rank <= 256 or not 0 < N * K <= 1 << 29 or torch.cuda.is_current_stream_capturing():
+    (N, K), rank = w.shape, 0
+    for up, down, mult in factors:
+        if up.dim() != 2 or down.dim() != 2 or up.shape[1] == 0 or not isinstance(mult, (int, float)):
+            return None
+        rank += up.shape[1]
+    if K % 16 or rank % 4 or rank > 256 or not 0 < N * K <= 1 << 29 or torch.cuda.is_current_stream_capturing():
         return None
     w = _i8_matrix(w, "w")
-    up = _f32_matrix(up, "up", w.device)
-    down = _f32_matrix(down, "down", w.device)
-    if up.shape[0] != N or down.shape != (rank, K):
-        raise ValueError(f"up must be [{N},r] and down [r,{K}]")
-    if (w.data_ptr() | up.data_ptr()) % 16:
+    kept = []   # (converted copies live until the launch)
+    arr = (_LoraFactors * len(factors))()
+    for slot, (up, down, mult) in zip(arr, factors):
+        up, down = _f32_matrix(up, "up", w.device), _f32_matrix(down, "down", w.device)
+        if up.shape[0] != N or down.shape != (up.shape[1], K):
+            raise ValueError(f"up must be [{N},r] and down [r,{K}]")
+        kept += [up, down]
+        slot.up, slot.down, slot.rank, slot.mult = up.data_ptr(), down.data_ptr(), up.shape[1], mult
+    if w.data_ptr() % 16 or (len(factors) == 1 and kept[0].data_ptr() % 16) or (len(factors) > 1 and (N + K) * rank >= 1 << 31):
         return None
     ws, ws_host, mode = _scale(w_scale, N, w.device)
+    L = lib()
     out = torch.empty_like(w)
-    scratch = torch.empty(N * K, dtype=torch.int16, device=w.device)
+    scratch = torch.empty(L.i8f_lora_merge_sr_drawn_workspace_bytes(N, K, rank, len(factors)), dtype=torch.uint8, device=w.device)
     # torch draws in blocks of 256 threads, as many as the GPU holds at most, each thread four elements at a time
     props = torch.cuda.get_device_properties(w.device)
     lanes = 256 * min(-(-N * K // 256), props.multi_processor_count * (props.max_threads_per_multi_processor // 256))
     with _on(w.device):
-        _check(lib().i8f_lora_merge_sr_drawn(_ptr(w), _ptr(ws), ws_host, mode, _ptr(up), _ptr(down), rank, float(lora_scale),
-                                             generator.initial_seed() & 0xFFFFFFFFFFFFFFFF, lanes, N, K, _ptr(out), _ptr(scratch),
-                                             2 * N * K, _stream(w)), "i8f_lora_merge_sr_drawn")
+        _check(L.i8f_lora_merge_sr_drawn(_ptr(w), _ptr(ws), ws_host, mode, arr, len(factors), float(lora_scale),
+                                         generator.initial_seed() & 0xFFFFFFFFFFFFFFFF, lanes, N, K, _ptr(out), _ptr(scratch),
+                                         scratch.numel(), _stream(w)), "i8f_lora_merge_sr_drawn")
     return out
 
 

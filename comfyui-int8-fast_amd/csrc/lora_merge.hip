@@ -156,13 +156,45 @@ __device__ __forceinline__ float uniform_of(uint32_t x) {
 // (The noise drawn inside the merge: a call gives four elements `lanes` apart, so a workgroup has to merge four far pieces of
 // the matrix together.  Bit for bit the same in 70 and 105 us, and slower than torch.rand and the merge below 20 M elements
 // or where K is no multiple of 64; not kept.)
-__global__ __launch_bounds__(256) void draw_words_kernel(uint32_t seed_lo, uint32_t seed_hi, uint32_t lanes, uint32_t numel, uint16_t *out) {
-    const uint32_t s0 = (blockIdx.x * 256 + threadIdx.x) * 8, at = 4 * blockIdx.y * lanes + s0;
+//
+// Several LoRAs: the first `extra` rows of workgroups write the factors side by side, up [N,R] and each `down` times its
+// multiplier (rounded) [R,K], while the others draw; torch does it in one launch for every LoRA and one more (9216 x 3072, ranks
+// 16, 32, 64: 11 us).
+constexpr int MAX_FACTORS = 8;
+struct Stack {
+    const float *up[MAX_FACTORS], *down[MAX_FACTORS];
+    float mult[MAX_FACTORS];
+    int first[MAX_FACTORS + 1];   // first rank of each; [n] = the sum R
+    int n;
+    uint32_t N, K;
+    float *up_out, *down_out;
+};
+
+__device__ __forceinline__ void stack_factors(const Stack &f, uint32_t at, uint32_t step) {
+    const uint32_t R = f.first[f.n], ups = f.N * R, all = ups + R * f.K;
+#pragma unroll 4
+    for (uint32_t i = at; i < all; i += step) {
+        const bool is_up = i < ups;
+        const uint32_t j = is_up ? i % R : (i - ups) / f.K;   // rank
+        int l = 0;
+#pragma unroll
+        for (int t = 1; t < MAX_FACTORS; ++t) l = t < f.n && (int)j >= f.first[t] ? t : l;
+        const uint32_t r = f.first[l + 1] - f.first[l], own = j - f.first[l];
+        if (is_up) f.up_out[i] = f.up[l][i / R * r + own];
+        else f.down_out[i - ups] = f.down[l][own * f.K + (i - ups) % f.K] * f.mult[l];
+    }
+}
+
+__global__ __launch_bounds__(256) void draw_words_kernel(uint32_t seed_lo, uint32_t seed_hi, uint32_t lanes, uint32_t numel, uint16_t *out, uint32_t extra,
+                                                         const Stack stack) {
+    if (blockIdx.y < extra) return stack_factors(stack, (blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x, extra * gridDim.x * 256);
+    const uint32_t chunk = blockIdx.y - extra;
+    const uint32_t s0 = (blockIdx.x * 256 + threadIdx.x) * 8, at = 4 * chunk * lanes + s0;
     if (s0 >= lanes || at >= numel) return;
     uint32_t x[8][4], top = 0;
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-        philox(blockIdx.y, s0 + t, seed_lo, seed_hi, x[t]);
+        philox(chunk, s0 + t, seed_lo, seed_hi, x[t]);
         top = max(max(top, max(x[t][0], x[t][1])), max(x[t][2], x[t][3]));
     }
     if (top >= ONE_WORDS) {
@@ -491,7 +523,7 @@ __global__ __launch_bounds__((MfmaMergeLds<RANK, DRAWN>::WAVES * 64), RANK <= 32
             // steps, and the definition's own product and quotient.  Together at most 1.08 * 2^-17 + 7 * 2^-24 * |z|; 1.125 * 2^-17
             // is asked for.  Of 256 elements with |z| of a few units one group in 200 is left open and redone.
             const float f = __builtin_amdgcn_rcpf(sc) * a.lora_scale;
-            const bool usual = (sc >= 0x1p-20f) & (sc <= 0x1p+20f) & (fabsf(f) >= 0x1p-100f) & (fabsf(f) <= 0x1p+100f);
+            const bool usual = sc >= 0x1p-20f && sc <= 0x1p+20f && fabsf(f) >= 0x1p-100f && fabsf(f) <= 0x1p+100f;
             float zmax[4] = {};
             uint32_t dmin[4], dmax[4];   // (bits, so that a NaN is the largest)
             __builtin_amdgcn_sched_barrier(0);
@@ -521,7 +553,7 @@ __global__ __launch_bounds__((MfmaMergeLds<RANK, DRAWN>::WAVES * 64), RANK <= 32
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const float eps = __builtin_fmaf(zmax[q], 7.0f * 0x1p-24f, 0x1.2p-17f);
-                const bool sure = usual & (zmax[q] <= 64.0f) & (dmin[q] >= __float_as_uint(eps)) & (dmax[q] <= __float_as_uint(1.0f - eps));
+                const bool sure = usual && zmax[q] <= 64.0f && dmin[q] >= __float_as_uint(eps) && dmax[q] <= __float_as_uint(1.0f - eps);
                 open |= __builtin_amdgcn_ballot_w64(!sure) != 0 ? 1u << q : 0u;
             }
             const uint32_t e0 = (uint32_t)(clampn(nb * 32 + l32) * a.K + k0) + wave * 32 + 4 * half;
@@ -751,30 +783,59 @@ extern "C" int i8f_lora_merge_sr(const int8_t *w, const float *w_scale, float w_
     return run(a, (hipStream_t)stream);
 }
 
+namespace {
+int64_t up256(int64_t bytes) { return (bytes + 255) / 256 * 256; }
+}  // namespace
+
+extern "C" int64_t i8f_lora_merge_sr_drawn_workspace_bytes(int64_t N, int64_t K, int64_t rank, int count) {
+    if (N < 0 || K < 0 || rank < 0 || N > (1 << 29) || K > (1 << 29) || rank > 256) return 0;
+    return up256(2 * N * K) + (count > 1 ? up256(4 * N * rank) + 4 * K * rank : 0);
+}
+
 extern "C" int i8f_lora_merge_sr_drawn(const int8_t *w, const float *w_scale, float w_scale_host, int scale_mode,
-                                       const float *up, const float *down, int64_t rank, float lora_scale,
+                                       const i8f_lora_factors *factors, int count, float lora_scale,
                                        uint64_t seed, int64_t lanes, int64_t N, int64_t K, int8_t *w_out,
                                        void *workspace, int64_t workspace_bytes, void *stream) {
     using namespace i8f;
     if (N < 0 || K < 0) return I8F_ERR_INVALID;
     if (scale_mode != I8F_SCALE_TENSOR && scale_mode != I8F_SCALE_ROW) return I8F_ERR_INVALID;
     if (N == 0 || K == 0) return I8F_OK;
-    if (!w || !w_out || !up || !down || !workspace || rank <= 0 || lanes <= 0) return I8F_ERR_INVALID;
+    if (!w || !w_out || !factors || count < 1 || !workspace || lanes <= 0) return I8F_ERR_INVALID;
     if (scale_mode == I8F_SCALE_ROW && !w_scale) return I8F_ERR_INVALID;
-    if (K % 16 || K >= (1 << 24) || N > (1 << 29) / K || rank % 4 || rank > 256 || lanes % 256 || lanes > (1 << 24)) return I8F_ERR_UNSUPPORTED;
-    if ((uintptr_t)w % 16 || (uintptr_t)w_out % 16 || (uintptr_t)up % 16 || (uintptr_t)workspace % 16) return I8F_ERR_UNSUPPORTED;
-    const int64_t chunks = (N * K + 4 * lanes - 1) / (4 * lanes);
-    if (chunks > 65535) return I8F_ERR_UNSUPPORTED;
-    if (workspace_bytes < 2 * N * K) return I8F_ERR_INVALID;
+    if (count > MAX_FACTORS) return I8F_ERR_UNSUPPORTED;
+    Stack stack{};
+    stack.n = count;
+    for (int i = 0; i < count; ++i) {
+        if (!factors[i].up || !factors[i].down || factors[i].rank <= 0) return I8F_ERR_INVALID;
+        if (factors[i].rank > 256 - stack.first[i]) return I8F_ERR_UNSUPPORTED;
+        stack.up[i] = factors[i].up, stack.down[i] = factors[i].down, stack.mult[i] = factors[i].mult;
+        stack.first[i + 1] = stack.first[i] + (int)factors[i].rank;
+    }
+    const int rank = stack.first[count];
+    if (K % 16 || K >= (1 << 24) || N > (1 << 29) / K || rank % 4 || lanes % 256 || lanes > (1 << 24)) return I8F_ERR_UNSUPPORTED;
+    if ((uintptr_t)w % 16 || (uintptr_t)w_out % 16 || (uintptr_t)workspace % 16 || (count == 1 && (uintptr_t)factors[0].up % 16)) return I8F_ERR_UNSUPPORTED;
+    if (count > 1 && (N + K) * rank >= (1ll << 31)) return I8F_ERR_UNSUPPORTED;   // (elements are counted in 32 bits)
+    const int64_t chunks = (N * K + 4 * lanes - 1) / (4 * lanes), columns = (lanes + 2047) / 2048;
+    // workgroups for the factors: 4 elements a thread, one round of the chip at most
+    int64_t extra = count > 1 ? ((N + K) * rank + 1023) / 1024 : 0;
+    extra = ((extra < 2048 ? extra : 2048) + columns - 1) / columns;
+    if (chunks + extra > 65535) return I8F_ERR_UNSUPPORTED;
+    if (workspace_bytes < i8f_lora_merge_sr_drawn_workspace_bytes(N, K, rank, count)) return I8F_ERR_INVALID;
     if (int rc = check_device()) return rc;
     hipStream_t st = (hipStream_t)stream;
     MergeArgs a{};
     a.w = w, a.ws = w_scale, a.ws_host = w_scale_host, a.row_scale = scale_mode == I8F_SCALE_ROW;
-    a.up = up, a.down = down, a.rank = (int)rank, a.lora_scale = lora_scale;
+    a.up = factors[0].up, a.down = factors[0].down, a.rank = rank, a.lora_scale = lora_scale;
     a.N = N, a.K = K, a.out = w_out;
     a.drawn = (const uint16_t *)workspace, a.seed_lo = (uint32_t)seed, a.seed_hi = (uint32_t)(seed >> 32), a.lanes = (uint32_t)lanes;
-    hipLaunchKernelGGL(draw_words_kernel, dim3((unsigned)((lanes + 2047) / 2048), (unsigned)chunks), dim3(256), 0, st, a.seed_lo, a.seed_hi, a.lanes,
-                       (uint32_t)(N * K), (uint16_t *)workspace);
+    if (count > 1) {
+        stack.N = (uint32_t)N, stack.K = (uint32_t)K;
+        stack.up_out = (float *)((char *)workspace + up256(2 * N * K));
+        stack.down_out = (float *)((char *)stack.up_out + up256(4 * N * rank));
+        a.up = stack.up_out, a.down = stack.down_out;
+    }
+    hipLaunchKernelGGL(draw_words_kernel, dim3((unsigned)columns, (unsigned)(chunks + extra)), dim3(256), 0, st, a.seed_lo, a.seed_hi, a.lanes,
+                       (uint32_t)(N * K), (uint16_t *)workspace, (uint32_t)extra, stack);
     if (int rc = check_launch()) return rc;
     return launch_rank<true>(a, st);
 }

@@ -315,7 +315,7 @@ def _draw_noise(shape, seed: int, device) -> Tensor:
 
 def _merge_low_rank(w: Tensor, scale, seed: int, up: Tensor, down: Tensor, lora_scale=1.0) -> Tensor:
     """The fused merge with the noise of _draw_noise, drawn inside the kernel where that is possible."""
-    merged = _lib.lora_merge_sr_drawn(w, scale, _seeded(seed, w.device), up, down, lora_scale)
+    merged = _lib.lora_merge_sr_drawn(w, scale, _seeded(seed, w.device), [(up, down, 1.0)], lora_scale)
     if merged is None:
         merged = _lib.lora_merge_sr(w, scale, _draw_noise(tuple(w.shape), seed, w.device), up=up, down=down, lora_scale=lora_scale)
     return merged
@@ -400,10 +400,9 @@ class INT8MergedLoRAPatchAdapter(LoRAAdapter):
         rows = delta_f if isinstance(delta_f, int) else delta_f.shape[0]
         return _slice_scale_mismatch_only(self.weight_scale, rows, offset)
 
-    @torch.no_grad()   # (factors may be parameters; products written into place have no backward)
-    def _stacked_factors(self, weight, dev):
-        """(up [N,R], down [R,K]) in float32 with up @ down the summed delta of the stack, or None where the patches are
-        not all plain LoRAs of this weight or their ranks and widths are not those of the fused kernel's matrix-core form."""
+    def _stack(self, weight):
+        """(up, down, multiplier) of each LoRA whose products summed are the delta, or None where the patches are not all
+        plain LoRAs of this weight or their ranks and widths are not those of the fused kernel's matrix-core form."""
         parts, rank = [], 0
         for adapter, strength in self.patches:
             plain = _plain_lora(adapter.weights)
@@ -415,8 +414,16 @@ class INT8MergedLoRAPatchAdapter(LoRAAdapter):
             rank += r
         if weight.shape[1] % 16 or rank % 4 or rank > 256 or rank == 0:
             return None
+        return parts
+
+    @torch.no_grad()   # (factors may be parameters; products written into place have no backward)
+    def _stacked_factors(self, weight, dev):
+        """(up [N,R], down [R,K]) in float32 with up @ down the summed delta of the stack, or None as _stack."""
+        parts = self._stack(weight)
+        if parts is None:
+            return None
         up = torch.cat([u.to(dev, torch.float32) for u, _, _ in parts], dim=1)
-        down, at = torch.empty((rank, weight.shape[1]), dtype=torch.float32, device=dev), 0
+        down, at = torch.empty((up.shape[1], weight.shape[1]), dtype=torch.float32, device=dev), 0
         for _, d, m in parts:   # (each product into its rows: no copy of all of them behind it, 5 us at 112 x 3072)
             torch.mul(d.to(dev, torch.float32), m, out=down[at:at + d.shape[0]])
             at += d.shape[0]
@@ -429,13 +436,19 @@ class INT8MergedLoRAPatchAdapter(LoRAAdapter):
         home = weight.device
         dev = compute_device() if weight.dtype == torch.int8 else home
         if weight.dtype == torch.int8 and intermediate_dtype == torch.float32 and self.fuse_low_rank:
-            stacked = self._stacked_factors(weight, dev)
-            if stacked is not None:
-                up, down = stacked
+            parts = self._stack(weight)
+            if parts is not None:
+                eff = self._get_effective_scale(weight.shape[0], offset)
+                w_dev = weight.to(dev)
+                several = [(u.to(dev, torch.float32), d.to(dev, torch.float32), m) for u, d, m in parts if d.shape[0]]
+                if len(several) > 1 and not _quarot_applies(weight):   # put side by side by the launch that draws the noise
+                    merged = _lib.lora_merge_sr_drawn(w_dev, eff, _seeded(self.seed, dev), several)
+                    if merged is not None:
+                        return merged.to(home)
+                up, down = self._stacked_factors(weight, dev)
                 if _quarot_applies(weight):   # rotating the rows of up @ down is rotating the rows of down
                     down = _lib.rotate128(down)
-                eff = self._get_effective_scale(weight.shape[0], offset)
-                return _merge_low_rank(weight.to(dev), eff, self.seed, up, down).to(home)
+                return _merge_low_rank(w_dev, eff, self.seed, up, down).to(home)
         total = None
         for adapter, lora_strength in self.patches:  # ComfyUI's own `strength` is ignored here, as in the reference
             diff, mult = reconstruct_lora_diff(adapter.weights, weight.shape, dev, intermediate_dtype, lora_strength)

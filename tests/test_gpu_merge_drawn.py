@@ -32,7 +32,7 @@ def test_drawn_merge_equals_the_merge_on_torchs_noise(pkg, L, dev, N, K, rank, s
         if row:
             ws[7], ws[8] = 1e-39, 3e7
     noise = pkg.int8_quant._draw_noise((N, K), seed, dev)
-    drawn = L.lora_merge_sr_drawn(w, ws, pkg.int8_quant._seeded(seed, dev), up, down, 0.75)
+    drawn = L.lora_merge_sr_drawn(w, ws, pkg.int8_quant._seeded(seed, dev), [(up, down, 1.0)], 0.75)
     assert torch.equal(drawn, L.lora_merge_sr(w, ws, noise, up=up, down=down, lora_scale=0.75))
 
 
@@ -44,20 +44,34 @@ def test_adapters_draw_what_they_drew(pkg, L, dev, monkeypatch):
     lora = lambda r: (torch.randn(N, r, device=dev) * 0.02, torch.randn(r, K, device=dev) * 0.02, float(r), None, None, None)
     one = pkg.INT8LoRAPatchAdapter(set(), lora(16), ws, seed=7)
     stack = pkg.INT8MergedLoRAPatchAdapter([(pkg.INT8LoRAPatchAdapter(set(), lora(r), ws), 0.5) for r in (3, 9, 8)], ws, seed=8)
-    now = [a.calculate_weight(w, "", 1.0, 1.0, None, None) for a in (one, stack)]
+    full = pkg.INT8MergedLoRAPatchAdapter([(pkg.INT8LoRAPatchAdapter(set(), lora(r), ws), 1.3) for r in (1, 2, 1, 40, 12, 64, 128, 8)], ws, seed=9)
+    nine = pkg.INT8MergedLoRAPatchAdapter([(pkg.INT8LoRAPatchAdapter(set(), lora(4), ws), 0.1 * i) for i in range(9)], ws, seed=10)
+    empty = pkg.INT8MergedLoRAPatchAdapter([(pkg.INT8LoRAPatchAdapter(set(), lora(4), ws), 0.7),
+                                            (pkg.INT8LoRAPatchAdapter(set(), (*lora(0)[:2], None, None, None, None), ws), 0.7)], ws, seed=11)
+    adapters = (one, stack, full, nine, empty)
+    now = [a.calculate_weight(w, "", 1.0, 1.0, None, None) for a in adapters]
     monkeypatch.setattr(L, "DRAWS_LIKE_TORCH", False)
-    for got, a in zip(now, (one, stack)):
+    for got, a in zip(now, adapters):
         assert torch.equal(got, a.calculate_weight(w, "", 1.0, 1.0, None, None))
 
 
 def test_drawn_merge_refuses_what_it_cannot_do(L):
     one, null = ctypes.c_void_p(4096), None
-    call = lambda w=one, up=one, rank=8, lanes=256, N=4, K=16, ws=one, mode=0, nbytes=128: L.lib().i8f_lora_merge_sr_drawn(
-        w, ws, 1.0, mode, up, one, rank, 1.0, 0, lanes, N, K, one, one, nbytes, null)
     INVALID, UNSUPPORTED = -1, -2
-    assert call(w=null) == INVALID and call(up=null) == INVALID and call(rank=0) == INVALID and call(lanes=0) == INVALID
-    assert call(ws=null, mode=1) == INVALID and call(mode=2) == INVALID and call(nbytes=127) == INVALID and call(N=-1) == INVALID
-    assert call(K=24) == UNSUPPORTED and call(rank=6) == UNSUPPORTED and call(rank=260) == UNSUPPORTED and call(lanes=100) == UNSUPPORTED
-    assert call(up=ctypes.c_void_p(4100)) == UNSUPPORTED and call(N=2**25 + 1) == UNSUPPORTED
-    assert call(N=2**24, nbytes=2**29) == UNSUPPORTED      # more calls of the generator than a launch has blocks
+
+    def call(w=one, factors=((4096, 4096, 8),), lanes=256, N=4, K=16, ws=one, mode=0, nbytes=None):
+        arr = (L._LoraFactors * max(1, len(factors)))(*((u, d, r, 1.0) for u, d, r in factors))
+        size = L.lib().i8f_lora_merge_sr_drawn_workspace_bytes(N, K, sum(r for _, _, r in factors), len(factors))
+        return L.lib().i8f_lora_merge_sr_drawn(w, ws, 1.0, mode, arr, len(factors), 1.0, 0, lanes, N, K, one, one,
+                                               size if nbytes is None else nbytes, null)
+
+    assert call(w=null) == INVALID and call(factors=((None, 4096, 8),)) == INVALID and call(factors=()) == INVALID and call(lanes=0) == INVALID
+    assert call(factors=((4096, 4096, 0),)) == INVALID and call(ws=null, mode=1) == INVALID and call(mode=2) == INVALID
+    assert call(nbytes=127) == INVALID and call(N=-1) == INVALID
+    assert call(factors=((4096, 4096, 4), (4096, 4096, 4)), nbytes=256) == INVALID          # the factors side by side need room
+    assert call(K=24) == UNSUPPORTED and call(factors=((4096, 4096, 6),)) == UNSUPPORTED and call(lanes=100) == UNSUPPORTED
+    assert call(factors=((4096, 4096, 260),)) == UNSUPPORTED and call(factors=((4096, 4096, 129), (4096, 4096, 128))) == UNSUPPORTED
+    assert call(factors=((4096, 4096, 4),) * 9) == UNSUPPORTED and call(factors=((4100, 4096, 8),)) == UNSUPPORTED
+    assert call(N=2**25 + 1) == UNSUPPORTED
+    assert call(N=2**24) == UNSUPPORTED      # more calls of the generator than a launch has blocks
     assert call(N=0) == 0 and call(K=0) == 0
