@@ -17,6 +17,7 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <ATen/autocast_mode.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
@@ -25,6 +26,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../../include/i8f.h"
+#include "../quant_lora_entry.hpp"
 #include "../w8a16_rotated.hpp"
 
 namespace {
@@ -33,7 +35,7 @@ namespace {
 #define I8F_ENTRY_POINTS(X)                                                                                              \
     X(i8f_quant_rowwise) X(i8f_quant_rowwise_prologue) X(i8f_quant_rowwise_norm_modulate) X(i8f_quant_rowwise_rms_norm)  \
     X(i8f_quant_rowwise_concat_gelu) X(i8f_rotate128) X(i8f_linear_w8a8_gated) X(i8f_linear_w8a16_small_m)               \
-    X(i8f_linear_w8a16_small_m_grouped) X(i8f_internal_w8a16_rotated)
+    X(i8f_linear_w8a16_small_m_grouped) X(i8f_internal_w8a16_rotated) X(i8f_linear_w8a8_lora) X(i8f_internal_quant_lora)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     I8F_ENTRY_POINTS(X)
@@ -186,13 +188,61 @@ PyObject *small_m(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, const L
     return THPVariable_Wrap(std::move(y));
 }
 
+// ---- a dynamic LoRA on the layer ---------------------------------------------------------------
+// Its first product by the launch that quantises x, the second inside the GEMM.  Two launches: with the BLAS library's call
+// between them and the interpreter's part of it all, the host took 63 us a layer and the GPU waited for it below 2000 rows.
+PyObject *linear_lora(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, const Layer &l, int order, PyObject *lora_a, PyObject *lora_b,
+                      PyObject *lora_alpha, const Stream &st) {
+    if (at::autocast::is_autocast_enabled(at::kCUDA)) Py_RETURN_NONE;  // (the product's type is then the context's)
+    const at::Tensor *A = tensor(lora_a), *B = tensor(lora_b);
+    for (const at::Tensor *f : {A, B})
+        if (!f || f->scalar_type() != x.scalar_type() || f->device() != x.device() || f->dim() != 2 || !f->is_contiguous() || !aligned16(*f)) Py_RETURN_NONE;
+    const int64_t R = A->size(0);
+    // (the GEMM's LoRA epilogue takes ranks in steps of 16 up to 64.  Every 16 rows read the factor once more: 16384 rows are as
+    // many as were measured, where the quantiser and the BLAS library's product still take longer at every rank)
+    if (A->size(1) != K || B->size(0) != l.N || B->size(1) != R || R % 16 || R < 16 || R > 64 || M > 16384) Py_RETURN_NONE;
+    if (K != l.K || K % 128 || K > (R > 32 ? 4096 : 6144) || l.N % 8 || ld % 8 || !aligned16(x) || (uintptr_t)l.w % 16 || (l.mode == I8F_SCALE_ROW && (uintptr_t)l.ws % 16) ||
+        (uintptr_t)l.bias % 16 || l.N * K >= (1ll << 31))
+        Py_RETURN_NONE;
+    float alpha = 0.0f;
+    const bool has_alpha = lora_alpha != Py_None;
+    if (has_alpha) {
+        if (!PyFloat_CheckExact(lora_alpha) && !PyLong_CheckExact(lora_alpha)) Py_RETURN_NONE;
+        alpha = (float)PyFloat_AsDouble(lora_alpha);
+        if (PyErr_Occurred()) return nullptr;
+    }
+    const at::ScalarType type = x.scalar_type();
+    const at::Device dev = x.device();
+    const Size size = output_size(x, l.N);
+    const int dt = code_of(type);
+    const void *xp = x.const_data_ptr(), *ap = A->const_data_ptr(), *bp = B->const_data_ptr();
+    at::Tensor scratch, y;
+    int rc;
+    {
+        const WithoutGil released;
+        const int64_t q_bytes = (M * K + 255) / 256 * 256, t_bytes = (2 * M * R + 255) / 256 * 256;
+        scratch = empty({q_bytes + t_bytes + 4 * M}, at::kByte, dev);
+        int8_t *q = (int8_t *)scratch.data_ptr();
+        void *t = q + q_bytes;
+        float *qs = (float *)(q + q_bytes + t_bytes);
+        y = empty(size, type, dev);
+        rc = lib.i8f_internal_quant_lora(xp, dt, M, K, ld, ap, R, q, qs, t, st.handle);
+        if (!rc)
+            rc = lib.i8f_linear_w8a8_lora(q, qs, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, t, bp, R, has_alpha, alpha, y.data_ptr(), dt, M,
+                                          l.N, K, order, st.handle);
+    }
+    if (rc) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(y));
+}
+
 // linear(x, weight, scale, bias, per_row, rotate, small_rows, order, kind, mod_scale, mod_shift, eps, norm_weight, fused_add,
-//        gate, residual, workspace): kind, an i8f_prologue, names what is applied to x inside the quantiser; workspace(x, M, N,
-// K) gives the memory of the K split or None.  It is called once a W8A8 call has passed every check, never for 16 rows or
-// fewer or for a call that goes the general way, which asks for its own: the memory stays with the stream, or with the graph
-// that is being captured, together with the kernel that clears it.
+//        gate, residual, workspace[, lora_A, lora_B, lora_alpha]): kind, an i8f_prologue, names what is applied to x inside the
+// quantiser; lora_A and lora_B are the factors of a dynamic LoRA that the layer has; workspace(x, M, N, K) gives the
+// memory of the K split or None.  It is called once a W8A8 call has passed every check, never for 16 rows or fewer, for a
+// layer with a LoRA or for a call that goes the general way, which asks for its own: the memory stays with the stream, or
+// with the graph that is being captured, together with the kernel that clears it.
 PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
-    if (n != 17) return PyErr_Format(PyExc_TypeError, "linear takes 17 arguments, got %zd", n);
+    if (n != 17 && n != 20) return PyErr_Format(PyExc_TypeError, "linear takes 17 or 20 arguments, got %zd", n);
     const at::Tensor *xt = tensor(a[0]);
     if (!lib.bound || !xt || !xt->is_cuda()) Py_RETURN_NONE;
     const at::Tensor &x = *xt;
@@ -206,6 +256,10 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const bool gated = a[14] != Py_None, with_residual = a[15] != Py_None;
     const Stream st(x.device());
     if (!st.ok || (rotate && K % 128)) Py_RETURN_NONE;
+    if (n == 20 && a[17] != Py_None) {
+        if (kind != I8F_PRO_NONE || gated || with_residual || rotate || M <= small_rows) Py_RETURN_NONE;
+        return linear_lora(x, M, K, ld, l, order, a[17], a[18], a[19], st);
+    }
     if (M <= small_rows) {
         if (kind != I8F_PRO_NONE || gated || with_residual || K != l.K) Py_RETURN_NONE;
         return small_m(x, M, K, ld, l, rotate, st.handle);

@@ -346,6 +346,8 @@ __device__ __forceinline__ float max3_abs(float m, float a, float b) {
 //     below the 1e-30 floor (every such value is checked on the host by the test suite);
 //   1 / scale = fma(e, y0, y0) with y0 the hardware reciprocal (1 ulp) and e = 1 - scale y0: correctly rounded unless
 //     the significand of scale is all ones (Markstein), which takes the division.
+// MIXED: the lanes hold scales of several rows (else one scale, tested as a scalar)
+template <bool MIXED = false>
 __device__ __forceinline__ void scale_and_inverse16(float amax, float &scale, float &inv) {
     const float y = 0x1.020408p-7f;  // RN(1 / 127)
     const float q = amax * y;
@@ -355,8 +357,10 @@ __device__ __forceinline__ void scale_and_inverse16(float amax, float &scale, fl
     const float y0 = __builtin_amdgcn_rcpf(s);
     const float e = __builtin_fmaf(-s, y0, 1.0f);
     float iv = __builtin_fmaf(e, y0, y0);
-    // (every lane holds the same scale: a scalar test and a branch that is practically never taken)
-    if (__builtin_expect((__builtin_amdgcn_readfirstlane(__float_as_uint(s)) & 0x7fffffu) == 0x7fffffu, 0)) iv = 1.0f / s;
+    // (a branch that is practically never taken)
+    const bool ones = MIXED ? __builtin_amdgcn_ballot_w64((__float_as_uint(s) & 0x7fffffu) == 0x7fffffu) != 0
+                            : (__builtin_amdgcn_readfirstlane(__float_as_uint(s)) & 0x7fffffu) == 0x7fffffu;
+    if (__builtin_expect(ones, 0)) iv = 1.0f / s;
     scale = s;
     inv = iv;
 }
@@ -366,10 +370,11 @@ __device__ __forceinline__ void scale_and_inverse16(float amax, float &scale, fl
 // select with the other bytes preserved), so nothing is left to shuffle: 32 instructions per run instead of 44.  An
 // instruction that writes part of a register must not be followed at once by a reader of that register: the four dwords
 // are worked on in turn, which puts three instructions between any two that touch the same one.
-__device__ __forceinline__ uint4 quant16_magic(const float (&v)[16], float inv) {
+// inv: the inverse scale of the first eight, inv2 that of the others.
+__device__ __forceinline__ uint4 quant16_magic(const float (&v)[16], float inv, float inv2) {
     float p[16];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) p[j] = v[j] * inv;
+    for (int j = 0; j < 16; ++j) p[j] = v[j] * (j < 8 ? inv : inv2);
     const float M = 12582912.0f;
     uint32_t o0, o1, o2, o3;
 #define I8F_SDWA_ADD(d, s, b) "v_add_f32_sdwa %" #d ", %" #s ", %20 dst_sel:BYTE_" #b " dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD\n\t"
@@ -384,6 +389,7 @@ __device__ __forceinline__ uint4 quant16_magic(const float (&v)[16], float inv) 
 #undef I8F_SDWA_ADD
     return make_uint4(o0, o1, o2, o3);
 }
+__device__ __forceinline__ uint4 quant16_magic(const float (&v)[16], float inv) { return quant16_magic(v, inv, inv); }
 
 // WPR waves share a row (1 or 4); each lane holds RUNS runs of 16 elements; one row per wave or group of
 // waves (walking several rows per wave with the next row's loads in flight measured slower at every size:
@@ -1178,3 +1184,5 @@ extern "C" int i8f_rotate128(const void *x, int dtype, int64_t M, int64_t K, int
     default: return launch_rotate<I8F_F32>(x, M, K, ldx, out, st);
     }
 }
+
+#include "quant_lora.hpp"

@@ -596,22 +596,27 @@ class Int8TensorwiseOps(manual_cast):
         # -- forward ------------------------------------------------------------------------
         def _forward_native(self, x, prologue, mod_scale, mod_shift, eps, gate, residual, norm_weight, fused_add):
             """forward() without the interpreter's part of it, for a quantised layer whose tensors are all in place (no
-            managed casting, no dynamic LoRA, 16-bit contiguous rows on the current GPU); None for everything else.  A weight
+            managed casting, 16-bit contiguous rows on the current GPU); None for everything else.  A weight
             or bias that is no parameter of the layer (pruned, parametrised, a buffer) is the general path's, too: it reads
             the attributes, which are computed or kept elsewhere then."""
             params, scale = self._parameters, self._weight_scale_scalar
             weight = params.get("weight")
             if scale is None:
                 scale = self._buffers.get("weight_scale")
-            if (not self._is_quantized or self.lora_A is not None or self.comfy_cast_weights or weight is None or scale is None
+            if (not self._is_quantized or self.comfy_cast_weights or weight is None or scale is None
                     or "bias" not in params or len(self.weight_function) > 0 or len(self.bias_function) > 0 or x.shape[-1] == 0):
                 return None
+            lora = ()
+            if self.lora_A is not None:
+                if self.lora_B is None or self._use_quarot or prologue != _lib.PRO_NONE or gate is not None or residual is not None:
+                    return None
+                lora = (self.lora_A, self.lora_B, self.lora_alpha)
             if prologue == _lib.PRO_MODULATE_FUSED:
                 prologue, fused_add = _lib.PRO_MODULATE, True
             work = _lib._splitk_workspace if weight.shape[-1] >= _lib.SPLITK_MIN_K else None   # (asked for by a call that can use it)
             return _lib.host().linear(x, weight, scale, params["bias"], bool(self._is_per_row), bool(self._use_quarot), SMALL_BATCH_ROWS,
                                       int8_fused_kernel.DEFAULT_EPILOGUE, prologue, mod_scale, mod_shift, eps, norm_weight, bool(fused_add), gate,
-                                      residual, work)
+                                      residual, work, *lora)
 
         def forward(self, x: Tensor, prologue: int = _lib.PRO_NONE, mod_scale: Tensor | None = None,
                     mod_shift: Tensor | None = None, eps: float = 1e-6, gate: Tensor | None = None,
@@ -758,8 +763,8 @@ class Int8TensorwiseOps(manual_cast):
                 if (rows > SMALL_BATCH_ROWS and lB.dtype == lA.dtype
                         and (self.lora_alpha is None or isinstance(self.lora_alpha, (int, float)))
                         and _lib.lora_side_fusable(rows, weight.shape[0], weight.shape[1], lA.shape[0], compute_dtype, lA.dtype)):
-                    # (the first product stays with torch: it is bound by the same per-CU load path whoever issues the
-                    # loads, and an own kernel for it measured no faster than the BLAS library's 9.5 us at 4608 x 3072)
+                    # (what _forward_native leaves: rotated activations, ranks that are no multiple of 16, factors that are
+                    # not in place, more than 16384 rows.  The first product is the BLAS library's here)
                     side_factors = (F.linear(x_side, lA), lB, self.lora_alpha)
                 else:
                     side = F.linear(F.linear(x_side, lA), lB)
