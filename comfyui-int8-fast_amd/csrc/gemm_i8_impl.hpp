@@ -567,6 +567,26 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
         }
     }
 
+    // The side branch's operands of the tile as 16-byte pieces (8 ranks): BM rows of side_t from m0 on, then BN rows of side_b
+    // from n0 on; rows beyond the matrix repeat its last row (their outputs are not stored), ranks beyond side_rank its last
+    // piece.  A thread's first SIDE_PER pieces, which are all of them up to rank 32, wait in registers like the other operands
+    // (twelve waves have none to spare: 4608 x 12288 x 3072 in 256 x 288 tiles 160 us as here, 165 with it).
+    constexpr bool SIDE_EARLY = SIDE && C::NT <= 512;
+    constexpr int SIDE_PER = ((BM + BN) * 4 + C::NT - 1) / C::NT;
+    [[maybe_unused]] const int side_shift = SIDE && g.side_rank > 32 ? 3 : 2;  // 4 or 8 pieces to a row
+    [[maybe_unused]] uint4 side_r[SIDE ? SIDE_PER : 1];
+    [[maybe_unused]] auto side_fetch = [&](int c0) {
+#pragma unroll
+        for (int u = 0; u < SIDE_PER; ++u) {
+            const int c = min(c0 + u * C::NT, ((BM + BN) << side_shift) - 1);
+            const int row = c >> side_shift, cc = min(c & ((1 << side_shift) - 1), (g.side_rank >> 3) - 1);
+            const char *src = row < BM ? (const char *)g.side_t : (const char *)g.side_b;
+            const int line = row < BM ? min(m0 + row, gM - 1) : min(n0 + row - BM, gN - 1);
+            side_r[u] = *(const uint4 *)(src + (int64_t)line * g.side_rank * 2 + cc * 16);
+        }
+    };
+    if constexpr (SIDE_EARLY) side_fetch(tid);
+
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(SPREAD_DMA ? (PRE - 1) * C::LOADS : (ASYM ? C::LOADS : cut(1))));  // younger tiles may be in flight
     __builtin_amdgcn_s_barrier();  // tile 0 is in LDS for everyone (no fence: nothing else has been written)
 
@@ -759,30 +779,17 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
         }
     }
     if constexpr (SIDE) {
-        // side_t rows m0 ... and side_b rows n0 ... of the tile in 16-byte pieces (8 ranks), each row filled up with zeros to
-        // 32 or 64 ranks; rows beyond the matrix repeat its last row (their outputs are not stored).  A thread's loads of 32
-        // ranks go out together, without a branch near them: one trip to memory instead of one for each piece.  What the
-        // side branch adds to the GEMM is this trip and its rounding steps, in an epilogue that nothing overlaps: with that
-        // and the fixed number of products below, us for rank 32 (64), before and after: 1357 x 9216 x 3072 47.8 -> 44.3
-        // (51.5 -> 46.6; 40 without a side branch), 4608 x 12288 x 3072 171.1 -> 165.4 (182.4 -> 173.0; 152).
-        const int cpr = g.side_rank >> 3;  // pieces per row
-        const int shift = g.side_rank > 32 ? 3 : 2;
-        constexpr int PER = ((BM + BN) * 4 + C::NT - 1) / C::NT;
-        for (int c0 = tid; c0 - tid < (BM + BN) << shift; c0 += PER * C::NT) {
-            uint4 piece[PER];
+        // Each row's pieces to LDS, filled up with zeros to 32 or 64 ranks.  What the side branch adds to the GEMM is its
+        // rounding steps, in an epilogue that nothing overlaps, and one trip to memory where the pieces have not been fetched.
+        // us at 1357 x 9216 x 3072, rank 32 (64), with the trip and a selection by alpha for every value 47.4 (48.6), now 45.9
+        // (47.5); 40 without a side branch.
+        for (int c0 = tid; c0 - tid < (BM + BN) << side_shift; c0 += SIDE_PER * C::NT) {
+            if (!SIDE_EARLY || c0 != tid) side_fetch(c0);
 #pragma unroll
-            for (int u = 0; u < PER; ++u) {
-                const int c = min(c0 + u * C::NT, ((BM + BN) << shift) - 1);
-                const int row = c >> shift, cc = min(c & ((1 << shift) - 1), cpr - 1);
-                const char *src = row < BM ? (const char *)g.side_t : (const char *)g.side_b;
-                const int line = row < BM ? min(m0 + row, gM - 1) : min(n0 + row - BM, gN - 1);
-                piece[u] = *(const uint4 *)(src + (int64_t)line * g.side_rank * 2 + cc * 16);
-            }
-#pragma unroll
-            for (int u = 0; u < PER; ++u) {  // (past the end the last piece again, by several threads alike)
-                const int c = min(c0 + u * C::NT, ((BM + BN) << shift) - 1);
-                const int row = c >> shift, cc = c & ((1 << shift) - 1);
-                *(uint4 *)(smem + SIDE_OFF + row * SIDE_PITCH + cc * 16) = cc < cpr ? piece[u] : make_uint4(0, 0, 0, 0);
+            for (int u = 0; u < SIDE_PER; ++u) {  // (past the end the last piece again, by several threads alike)
+                const int c = min(c0 + u * C::NT, ((BM + BN) << side_shift) - 1);
+                const int row = c >> side_shift, cc = c & ((1 << side_shift) - 1);
+                *(uint4 *)(smem + SIDE_OFF + row * SIDE_PITCH + cc * 16) = cc < g.side_rank >> 3 ? side_r[u] : make_uint4(0, 0, 0, 0);
             }
         }
     }
@@ -913,10 +920,7 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
                                 sacc = side_mfma<OUT>(bfr[ks], tfr, sacc);
                             }
 #pragma unroll
-                            for (int r = 0; r < 16; ++r) {
-                                const float v = round_to_dtype<SDT>(sacc[r]), scaled = round_to_dtype<SDT>(v * g.side_alpha);
-                                sd[r] = g.side_has_alpha ? scaled : v;
-                            }
+                            for (int r = 0; r < 16; ++r) sd[r] = round_to_dtype<SDT>(sacc[r]);
                         }
                         if constexpr (SIDE && M16) {
 #pragma unroll
@@ -925,10 +929,13 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
 #pragma unroll
                                 for (int ks = 0; ks < KS; ++ks) sacc = side_mfma16<OUT>(bfr16[ks], tfr16[u][ks], sacc);
 #pragma unroll
-                                for (int e = 0; e < 4; ++e) {
-                                    const float v = round_to_dtype<SDT>(sacc[e]), scaled = round_to_dtype<SDT>(v * g.side_alpha);
-                                    sd[4 * u + e] = g.side_has_alpha ? scaled : v;
-                                }
+                                for (int e = 0; e < 4; ++e) sd[4 * u + e] = round_to_dtype<SDT>(sacc[e]);
+                            }
+                        }
+                        if constexpr (SIDE) {
+                            if (g.side_has_alpha) {  // (a branch of the whole wave: as a selection it costs every value three instructions)
+#pragma unroll
+                                for (int e = 0; e < 4 * QPB; ++e) sd[e] = round_to_dtype<SDT>(sd[e] * g.side_alpha);
                             }
                         }
 #pragma unroll
