@@ -67,14 +67,20 @@ __device__ __forceinline__ void rotate_run16(float (&v)[16], float s0, float s1,
     dpp_fmac16<1>(v, s1);   // quad_perm [2,3,0,1]
     dpp_fmac16<2>(v, s2);   // row_half_mirror
     const float h = hadamard_entry<DT>() * (s0 * s1 * s2);
+    // bfloat16: the packed conversion with a zero in the low half leaves the rounded value in the high half, which IS its
+    // binary32 form: one instruction rounds and widens (two values per conversion would need two more instructions to pull
+    // them apart again).  binary16: two values to a conversion, one more each to widen them.
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const float a = v[j] * h;
-        // bfloat16: the packed conversion with a zero in the low half leaves the rounded value in the high half, which
-        // IS its binary32 form: one instruction rounds and widens (two values per conversion would need two more
-        // instructions to pull them apart again)
-        if constexpr (DT == I8F_BF16) v[j] = __uint_as_float(f32x2_to_bf16x2_bits(0.0f, a));
-        else v[j] = round_to_dtype<DT>(a);
+    for (int j = 0; j < 16; j += 2) {
+        if constexpr (DT == I8F_BF16) {
+            v[j] = __uint_as_float(f32x2_to_bf16x2_bits(0.0f, v[j] * h));
+            v[j + 1] = __uint_as_float(f32x2_to_bf16x2_bits(0.0f, v[j + 1] * h));
+        } else if constexpr (DT == I8F_F16) {
+            const half2v a = f32x2_to_half2(v[j] * h, v[j + 1] * h);
+            v[j] = (float)a.x, v[j + 1] = (float)a.y;
+        } else {
+            v[j] *= h, v[j + 1] *= h;
+        }
     }
 }
 
