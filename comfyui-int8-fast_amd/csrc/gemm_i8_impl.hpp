@@ -377,9 +377,11 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
     const int kt_first = slice * kt_per;
     const int KT = SPLITK ? max(min(kt_per, KT_all - kt_first), 0) : KT_all;
 
-    // `live` false (a tile index past the end, at the tail of the loop) turns every lane's offset
-    // out of range: the instruction is still issued, which keeps the loop body free of branches,
-    // but moves no data.
+    // `live` false (a tile index past the end, at the tail of the loop) makes the buffer empty, every
+    // lane out of range: the instruction is still issued, which keeps the loop body free of branches,
+    // but moves no data.  (One scalar selection for all loads of a tile, and vector offsets that never
+    // change: a selection per load took a vector instruction each and a register that the next one
+    // had to wait for.)
     // load r of tile kt: r < X_LOADS fetches a piece of the X tile, the others a piece of the W tile
     const uint32_t smem_base = (uint32_t)(uintptr_t)smem;
     // (sx, sw: the stage of the X and of the W tile that receives tile kt)
@@ -388,13 +390,15 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
         const int t = is_x ? r : r - C::X_LOADS;
         const uint32_t st = smem_base + (is_x ? sx * C::X_STRIDE : C::W_BASE + sw * C::W_STRIDE) + wave * 1024;
         const int kb = (kt_first + kt) * BK;
-        uint32_t vo = live ? (is_x ? xoff[t] : woff[t]) : OOB;
+        uint32_t vo = is_x ? xoff[t] : woff[t];
         int so = kb;
         if constexpr (KTAIL) {  // chunks past K are forced out of range per lane
             vo = (kb + (is_x ? xck[t] : wck[t]) < K && vo != OOB) ? vo + (uint32_t)kb : OOB;
             so = 0;
         }
-        dma16(is_x ? rx : rw, st + t * NW * 1024, vo, so);
+        v4i rsrc = is_x ? rx : rw;
+        rsrc.z = live ? rsrc.z : 0;
+        dma16(rsrc, st + t * NW * 1024, vo, so);
     };
     auto issue_one = [&](int kt, bool live, int r) { issue_to(kt, kt % S, kt % WS, live, r); };  // (prologue: kt is a constant)
     auto issue = [&](int kt, bool live) {
@@ -826,7 +830,8 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
     using F_ = std::false_type;
     using O0 = std::integral_constant<int, I8F_EPI_TORCH>;
     using O1 = std::integral_constant<int, I8F_EPI_FUSED>;
-    const int variant = (g.order == I8F_EPI_FUSED ? 4 : 0) | (row_scale ? 2 : 0) | (gbias ? 1 : 0);
+    constexpr bool BATCHED = C::NT <= 512 && !SIDE;  // gate and addend in batches, in epilogues of their own
+    const int variant = (BATCHED && (ggate || gaddend) ? 8 : 0) | (g.order == I8F_EPI_FUSED ? 4 : 0) | (row_scale ? 2 : 0) | (gbias ? 1 : 0);
 
     // The whole epilogue is instantiated once per variant and the variant is chosen ONCE, so that
     // the instructions a wave executes are contiguous in memory (the epilogue runs once per wave,
@@ -838,7 +843,7 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
     constexpr bool PRELOAD_ALL = C::NT <= 512 && !SIDE;
     // STEPS: 16-rank steps of the side product, known at compile time so that its operands' reads need no branches and
     // move ahead of their use (zero ranks add exact zeros: the sum starts at +0 and never becomes -0)
-    auto run_epilogue = [&](auto ORDER, auto ROW, auto BIAS, auto STEPS) __attribute__((always_inline)) {
+    auto run_epilogue = [&](auto ORDER, auto ROW, auto BIAS, auto STEPS, auto GATED) __attribute__((always_inline)) {
         [[maybe_unused]] constexpr int KS = decltype(STEPS)::value;
         constexpr int NPRE = PRELOAD_ALL ? NJ : 1;
         float4 wr[NPRE][NQ], br[NPRE][NQ];
@@ -960,10 +965,10 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
             // behind each store, above which it may not be moved, is a trip to memory for every piece (35 to 54 K cycles of
             // epilogue at 4608 x 3072, 9.6 K without gate and addend; 28 to 43 K in fours).  us, gate and addend, before and
             // after: 4608 x 3072 x 3072 50.6 and 48.2, x 12288 156.7 and 153.3, 9729 x 3072 x 15360 370 and 361, 512 x 3072 x 12288 in
-            // 128 x 96 tiles and two slices 38.6 and 37.0.  Twelve waves
-            // have no registers for it (4096 x 9216 x 3072 in 256 x 288 tiles 136 and 141 us).
-            constexpr bool BATCHED = C::NT <= 512;
-            if ((!ggate && !gaddend) || !BATCHED) {
+            // 128 x 96 tiles and two slices 38.6 and 37.0.  Twelve waves have no registers for it (4096 x 9216 x 3072 in 256 x 288
+            // tiles 136 and 141 us).  GATED is chosen with the variant, so that an epilogue without gate and addend stays
+            // contiguous: with a jump over their code the smallest outputs took 2 to 3 % longer (93 x 3200 x 3200 8.6 for 8.4 us).
+            if constexpr (!decltype(GATED)::value) {
 #pragma unroll
                 for (int p = 0; p < PASSES; ++p) {
                     const int id = p * 64 + lane;
@@ -973,7 +978,7 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
                     if (mm < gM && nn < gN) {
                         const int64_t off = ((int64_t)mm * gN + nn) * OB;
                         uint4 v = val;
-                        if constexpr (!BATCHED) {
+                        if constexpr (!BATCHED && !SIDE) {
                             if (ggate)
                                 v = mul_rounded<OUT>(v, *(const uint4 *)((const char *)ggate + ((int64_t)((uint32_t)mm / (uint32_t)ggate_rows) * gN + nn) * OB));
                             if (gaddend) v = add_rounded<OUT>(v, *(const uint4 *)((const char *)gaddend + off));
@@ -1021,20 +1026,31 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
     };
     auto choose = [&](auto STEPS) __attribute__((always_inline)) {
         switch (variant) {
-        case 0: run_epilogue(O0{}, F_{}, F_{}, STEPS); break;
-        case 1: run_epilogue(O0{}, F_{}, T_{}, STEPS); break;
-        case 2: run_epilogue(O0{}, T_{}, F_{}, STEPS); break;
-        case 3: run_epilogue(O0{}, T_{}, T_{}, STEPS); break;
-        case 4: run_epilogue(O1{}, F_{}, F_{}, STEPS); break;
-        case 5: run_epilogue(O1{}, F_{}, T_{}, STEPS); break;
-        case 6: run_epilogue(O1{}, T_{}, F_{}, STEPS); break;
-        default: run_epilogue(O1{}, T_{}, T_{}, STEPS); break;
+        case 0: run_epilogue(O0{}, F_{}, F_{}, STEPS, F_{}); break;
+        case 1: run_epilogue(O0{}, F_{}, T_{}, STEPS, F_{}); break;
+        case 2: run_epilogue(O0{}, T_{}, F_{}, STEPS, F_{}); break;
+        case 3: run_epilogue(O0{}, T_{}, T_{}, STEPS, F_{}); break;
+        case 4: run_epilogue(O1{}, F_{}, F_{}, STEPS, F_{}); break;
+        case 5: run_epilogue(O1{}, F_{}, T_{}, STEPS, F_{}); break;
+        case 6: run_epilogue(O1{}, T_{}, F_{}, STEPS, F_{}); break;
+        default: run_epilogue(O1{}, T_{}, T_{}, STEPS, F_{}); break;
+        case 8: if constexpr (BATCHED) run_epilogue(O0{}, F_{}, F_{}, STEPS, T_{}); break;
+        case 9: if constexpr (BATCHED) run_epilogue(O0{}, F_{}, T_{}, STEPS, T_{}); break;
+        case 10: if constexpr (BATCHED) run_epilogue(O0{}, T_{}, F_{}, STEPS, T_{}); break;
+        case 11: if constexpr (BATCHED) run_epilogue(O0{}, T_{}, T_{}, STEPS, T_{}); break;
+        case 12: if constexpr (BATCHED) run_epilogue(O1{}, F_{}, F_{}, STEPS, T_{}); break;
+        case 13: if constexpr (BATCHED) run_epilogue(O1{}, F_{}, T_{}, STEPS, T_{}); break;
+        case 14: if constexpr (BATCHED) run_epilogue(O1{}, T_{}, F_{}, STEPS, T_{}); break;
+        case 15: if constexpr (BATCHED) run_epilogue(O1{}, T_{}, T_{}, STEPS, T_{}); break;
         }
     };
     using S0 = std::integral_constant<int, 0>;
     if constexpr (OUT == OUT_I32) {
-        run_epilogue(O0{}, F_{}, F_{}, S0{});
-    } else if constexpr (SIDE) {
+        if constexpr (BATCHED) {
+            if (variant & 8) return run_epilogue(O0{}, F_{}, F_{}, S0{}, T_{});
+        }
+        run_epilogue(O0{}, F_{}, F_{}, S0{}, F_{});
+    } else if constexpr (SIDE) {  // (no gate and no addend beside a side branch)
         if (g.side_rank > 32) choose(std::integral_constant<int, 4>{});
         else choose(std::integral_constant<int, 2>{});
     } else {
