@@ -237,8 +237,8 @@ PyObject *linear_lora(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, con
 
 // linear(x, weight, scale, bias, per_row, rotate, small_rows, order, kind, mod_scale, mod_shift, eps, norm_weight, fused_add,
 //        gate, residual, workspace[, lora_A, lora_B, lora_alpha]): kind, an i8f_prologue, names what is applied to x inside the
-// quantiser; lora_A and lora_B are the factors of a dynamic LoRA that the layer has; workspace(x, M, N, K) gives the
-// memory of the K split or None.  It is called once a W8A8 call has passed every check, never for 16 rows or fewer, for a
+// quantiser; lora_A (or None) and lora_B are the factors of a dynamic LoRA; workspace(x, M, N, K) gives the memory of
+// the K split or None.  It is called once a W8A8 call has passed every check, never for 16 rows or fewer, for a
 // layer with a LoRA or for a call that goes the general way, which asks for its own: the memory stays with the stream, or
 // with the graph that is being captured, together with the kernel that clears it.
 PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {

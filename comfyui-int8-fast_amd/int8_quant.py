@@ -606,17 +606,18 @@ class Int8TensorwiseOps(manual_cast):
             if (not self._is_quantized or self.comfy_cast_weights or weight is None or scale is None
                     or "bias" not in params or len(self.weight_function) > 0 or len(self.bias_function) > 0 or x.shape[-1] == 0):
                 return None
-            lora = ()
             if self.lora_A is not None:
                 if self.lora_B is None or self._use_quarot or prologue != _lib.PRO_NONE or gate is not None or residual is not None:
                     return None
-                lora = (self.lora_A, self.lora_B, self.lora_alpha)
+                return _lib.host().linear(x, weight, scale, params["bias"], bool(self._is_per_row), False, SMALL_BATCH_ROWS,
+                                          int8_fused_kernel.DEFAULT_EPILOGUE, prologue, None, None, eps, None, False, None, None, None,
+                                          self.lora_A, self.lora_B, self.lora_alpha)
             if prologue == _lib.PRO_MODULATE_FUSED:
                 prologue, fused_add = _lib.PRO_MODULATE, True
             work = _lib._splitk_workspace if weight.shape[-1] >= _lib.SPLITK_MIN_K else None   # (asked for by a call that can use it)
             return _lib.host().linear(x, weight, scale, params["bias"], bool(self._is_per_row), bool(self._use_quarot), SMALL_BATCH_ROWS,
                                       int8_fused_kernel.DEFAULT_EPILOGUE, prologue, mod_scale, mod_shift, eps, norm_weight, bool(fused_add), gate,
-                                      residual, work, *lora)
+                                      residual, work)
 
         def forward(self, x: Tensor, prologue: int = _lib.PRO_NONE, mod_scale: Tensor | None = None,
                     mod_shift: Tensor | None = None, eps: float = 1e-6, gate: Tensor | None = None,
