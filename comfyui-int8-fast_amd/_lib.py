@@ -119,6 +119,9 @@ EXPORTS = (
 )
 
 
+ERR_UNSUPPORTED = -2   # I8F_ERR_UNSUPPORTED
+
+
 def _check(status: int, what: str) -> None:
     if status != 0:
         L = lib()
@@ -818,7 +821,7 @@ def lora_merge_sr_drawn(w, w_scale, generator, factors, lora_scale=1.0):
         if up.dim() != 2 or down.dim() != 2 or up.shape[1] == 0 or not isinstance(mult, (int, float)):
             return None
         rank += up.shape[1]
-    if K % 16 or rank % 4 or rank > 256 or not 0 < N * K <= 1 << 29 or torch.cuda.is_current_stream_capturing():
+    if K % 16 or K >= 1 << 24 or rank % 4 or rank > 256 or not 0 < N * K <= 1 << 29 or torch.cuda.is_current_stream_capturing():
         return None
     w = _i8_matrix(w, "w")
     kept = []   # (converted copies live until the launch)
@@ -839,9 +842,12 @@ def lora_merge_sr_drawn(w, w_scale, generator, factors, lora_scale=1.0):
     props = torch.cuda.get_device_properties(w.device)
     lanes = 256 * min(-(-N * K // 256), props.multi_processor_count * (props.max_threads_per_multi_processor // 256))
     with _on(w.device):
-        _check(L.i8f_lora_merge_sr_drawn(_ptr(w), _ptr(ws), ws_host, mode, arr, len(factors), float(lora_scale),
-                                         generator.initial_seed() & 0xFFFFFFFFFFFFFFFF, lanes, N, K, _ptr(out), _ptr(scratch),
-                                         scratch.numel(), _stream(w)), "i8f_lora_merge_sr_drawn")
+        status = L.i8f_lora_merge_sr_drawn(_ptr(w), _ptr(ws), ws_host, mode, arr, len(factors), float(lora_scale),
+                                           generator.initial_seed() & 0xFFFFFFFFFFFFFFFF, lanes, N, K, _ptr(out), _ptr(scratch),
+                                           scratch.numel(), _stream(w))
+    if status == ERR_UNSUPPORTED:   # (what the checks above let through and the kernels do not address)
+        return None
+    _check(status, "i8f_lora_merge_sr_drawn")
     return out
 
 

@@ -55,6 +55,25 @@ def test_adapters_draw_what_they_drew(pkg, L, dev, monkeypatch):
         assert torch.equal(got, a.calculate_weight(w, "", 1.0, 1.0, None, None))
 
 
+@pytest.mark.gpu
+def test_rows_too_long_for_the_drawn_merge_are_merged_on_torchs_noise(pkg, L, dev):
+    N, K, rank = 2, 1 << 24, 4
+    w = torch.randint(-127, 128, (N, K), dtype=torch.int8, device=dev)
+    up, down = torch.randn(N, rank, device=dev), torch.randn(rank, K, device=dev) * 0.01
+    assert L.lora_merge_sr_drawn(w, 0.004, pkg.int8_quant._seeded(5, dev), [(up, down, 1.0)]) is None
+    merged = pkg.INT8LoRAPatchAdapter(set(), (up, down, None, None, None, None), 0.004, seed=5).calculate_weight(w, "", 1.0, 1.0, None, None)
+    assert torch.equal(merged, L.lora_merge_sr(w, 0.004, pkg.int8_quant._draw_noise((N, K), 5, dev), up=up, down=down))
+
+
+@pytest.mark.gpu
+def test_what_the_entry_point_refuses_is_left_to_the_caller(pkg, L, dev, monkeypatch):
+    w = torch.randint(-127, 128, (32, 64), dtype=torch.int8, device=dev)
+    up, down = torch.randn(32, 4, device=dev), torch.randn(4, 64, device=dev)
+    assert L.lora_merge_sr_drawn(w, 0.004, pkg.int8_quant._seeded(5, dev), [(up, down, 1.0)]) is not None
+    monkeypatch.setattr(L.lib(), "i8f_lora_merge_sr_drawn", lambda *a: L.ERR_UNSUPPORTED)
+    assert L.lora_merge_sr_drawn(w, 0.004, pkg.int8_quant._seeded(5, dev), [(up, down, 1.0)]) is None
+
+
 def test_drawn_merge_refuses_what_it_cannot_do(L):
     one, null = ctypes.c_void_p(4096), None
     INVALID, UNSUPPORTED = -1, -2
@@ -72,6 +91,6 @@ def test_drawn_merge_refuses_what_it_cannot_do(L):
     assert call(K=24) == UNSUPPORTED and call(factors=((4096, 4096, 6),)) == UNSUPPORTED and call(lanes=100) == UNSUPPORTED
     assert call(factors=((4096, 4096, 260),)) == UNSUPPORTED and call(factors=((4096, 4096, 129), (4096, 4096, 128))) == UNSUPPORTED
     assert call(factors=((4096, 4096, 4),) * 9) == UNSUPPORTED and call(factors=((4100, 4096, 8),)) == UNSUPPORTED
-    assert call(N=2**25 + 1) == UNSUPPORTED
+    assert call(N=2**25 + 1) == UNSUPPORTED and call(N=1, K=2**24) == UNSUPPORTED and call(lanes=2**24 + 256) == UNSUPPORTED
     assert call(N=2**24) == UNSUPPORTED      # more calls of the generator than a launch has blocks
     assert call(N=0) == 0 and call(K=0) == 0
