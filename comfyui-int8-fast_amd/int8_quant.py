@@ -313,11 +313,13 @@ def _draw_noise(shape, seed: int, device) -> Tensor:
     return torch.rand(shape, generator=_seeded(seed, device), device=device, dtype=torch.float32)
 
 
-def _merge_low_rank(w: Tensor, scale, seed: int, up: Tensor, down: Tensor, lora_scale=1.0) -> Tensor:
-    """The fused merge with the noise of _draw_noise, drawn inside the kernel where that is possible."""
-    merged = _lib.lora_merge_sr_drawn(w, scale, _seeded(seed, w.device), [(up, down, 1.0)], lora_scale)
+def _merge_low_rank(w: Tensor, scale, generator: torch.Generator, up: Tensor, down: Tensor, lora_scale=1.0) -> Tensor:
+    """The fused merge with the noise of _draw_noise (generator: _seeded(...), not drawn from yet), drawn inside the kernel
+    where that is possible."""
+    merged = _lib.lora_merge_sr_drawn(w, scale, generator, [(up, down, 1.0)], lora_scale)
     if merged is None:
-        merged = _lib.lora_merge_sr(w, scale, _draw_noise(tuple(w.shape), seed, w.device), up=up, down=down, lora_scale=lora_scale)
+        noise = torch.rand(tuple(w.shape), generator=generator, device=w.device, dtype=torch.float32)
+        merged = _lib.lora_merge_sr(w, scale, noise, up=up, down=down, lora_scale=lora_scale)
     return merged
 
 
@@ -369,7 +371,7 @@ class INT8LoRAPatchAdapter(LoRAAdapter):
             mult = (alpha / down.shape[0]) * strength if alpha is not None else strength
             if rotate:  # rotating the rows of up @ down is rotating the rows of down
                 down = _lib.rotate128(down)
-            merged = _merge_low_rank(w_dev, eff, self.seed, up, down, mult)
+            merged = _merge_low_rank(w_dev, eff, _seeded(self.seed, w_dev.device), up, down, mult)
         else:
             diff, mult = reconstruct_lora_diff(self.weights, weight.shape, dev, intermediate_dtype, strength)
             if diff is None:
@@ -417,9 +419,11 @@ class INT8MergedLoRAPatchAdapter(LoRAAdapter):
         return parts
 
     @torch.no_grad()   # (factors may be parameters; products written into place have no backward)
-    def _stacked_factors(self, weight, dev):
-        """(up [N,R], down [R,K]) in float32 with up @ down the summed delta of the stack, or None as _stack."""
-        parts = self._stack(weight)
+    def _stacked_factors(self, weight, dev, parts=None):
+        """(up [N,R], down [R,K]) in float32 with up @ down the summed delta of the stack, or None as _stack, whose answer
+        `parts` is where the caller has it."""
+        if parts is None:
+            parts = self._stack(weight)
         if parts is None:
             return None
         up = torch.cat([u.to(dev, torch.float32) for u, _, _ in parts], dim=1)
@@ -439,16 +443,19 @@ class INT8MergedLoRAPatchAdapter(LoRAAdapter):
             parts = self._stack(weight)
             if parts is not None:
                 eff = self._get_effective_scale(weight.shape[0], offset)
-                w_dev = weight.to(dev)
-                several = [(u.to(dev, torch.float32), d.to(dev, torch.float32), m) for u, d, m in parts if d.shape[0]]
-                if len(several) > 1 and not _quarot_applies(weight):   # put side by side by the launch that draws the noise
-                    merged = _lib.lora_merge_sr_drawn(w_dev, eff, _seeded(self.seed, dev), several)
-                    if merged is not None:
-                        return merged.to(home)
-                up, down = self._stacked_factors(weight, dev)
-                if _quarot_applies(weight):   # rotating the rows of up @ down is rotating the rows of down
-                    down = _lib.rotate128(down)
-                return _merge_low_rank(w_dev, eff, self.seed, up, down).to(home)
+                w_dev, rotate = weight.to(dev), _quarot_applies(weight)
+                generator = _seeded(self.seed, w_dev.device)
+                # (moved and widened once, whichever route merges them: they often lie on the host in 16 bits)
+                parts = [(u.to(dev, torch.float32), d.to(dev, torch.float32), m) for u, d, m in parts if d.shape[0]]
+                merged = None
+                if len(parts) > 1 and not rotate:   # put side by side by the launch that draws the noise
+                    merged = _lib.lora_merge_sr_drawn(w_dev, eff, generator, parts)
+                if merged is None:
+                    up, down = self._stacked_factors(weight, dev, parts)
+                    if rotate:   # rotating the rows of up @ down is rotating the rows of down
+                        down = _lib.rotate128(down)
+                    merged = _merge_low_rank(w_dev, eff, generator, up, down)
+                return merged.to(home)
         total = None
         for adapter, lora_strength in self.patches:  # ComfyUI's own `strength` is ignored here, as in the reference
             diff, mult = reconstruct_lora_diff(adapter.weights, weight.shape, dev, intermediate_dtype, lora_strength)

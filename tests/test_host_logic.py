@@ -7,6 +7,7 @@ import pytest
 import torch
 import torch.nn.utils.parametrize
 import torch.nn.utils.prune
+from torch.utils._python_dispatch import TorchDispatchMode
 
 
 @pytest.fixture(autouse=True)
@@ -257,6 +258,41 @@ def test_stacked_factors_leaves_empty_loras_to_the_general_path(pkg):
     assert adapter._stacked_factors(w, torch.device("cpu")) is None
     adapter, w = stack(pkg, [(torch.ones(48, 0), torch.ones(0, 64)), (torch.ones(48, 4), torch.ones(4, 64))])
     assert adapter._stacked_factors(w, torch.device("cpu"))[0].shape == (48, 4)
+
+
+class Conversions(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.count = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.count += func is torch.ops.aten._to_copy.default
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("count,rotated", [(1, False), (1, True), (2, False), (2, True), (9, False), (9, True)])
+def test_a_merge_that_draws_no_noise_itself_prepares_its_operands_once(pkg, monkeypatch, count, rotated):
+    """Whichever route a stack takes in the end, every factor is moved and widened once and one generator is seeded; and so
+    for a single LoRA."""
+    monkeypatch.setattr(pkg.int8_quant, "compute_device", lambda: torch.device("cpu"))
+    monkeypatch.setattr(pkg.Int8TensorwiseOps, "enable_quarot", rotated)
+    monkeypatch.setattr(pkg._lib, "rotate128", lambda t: t)
+    monkeypatch.setattr(pkg._lib, "lora_merge_sr_drawn", lambda *a: None)
+    merges, seeds, seeded = [], [], pkg.int8_quant._seeded
+    monkeypatch.setattr(pkg.int8_quant, "_seeded", lambda *a: seeds.append(a) or seeded(*a))
+    monkeypatch.setattr(pkg._lib, "lora_merge_sr", lambda w, scale, noise, **k: merges.append((noise, k)) or w)
+    g = torch.Generator().manual_seed(6)
+    pairs = [(torch.randn(48, 4, generator=g).half(), torch.randn(4, 128, generator=g).half()) for _ in range(count)]
+    stacked, w = stack(pkg, pairs, k=128)
+    for adapter in (stacked, stacked.patches[0][0]):
+        loras, seed = len(getattr(adapter, "patches", [0])), adapter.seed
+        with Conversions() as conversions:
+            adapter.calculate_weight(w, "k", 1.0, 1.0, None, None)
+        assert conversions.count == 2 * loras and len(seeds) == 1
+        noise, operands = merges[0]
+        assert torch.equal(noise, torch.rand(48, 128, generator=torch.Generator().manual_seed(seed)))
+        assert torch.equal(operands["up"], torch.cat([u.float() for u, _ in pairs[:loras]], 1))
+        merges.clear(), seeds.clear()
 
 
 @pytest.mark.parametrize("rows,k", [(4, 12288), (16, 10240), (17, 12288), (40, 12288), (40, 10224)])
