@@ -37,6 +37,21 @@ def test_drawn_merge_equals_the_merge_on_torchs_noise(pkg, L, dev, N, K, rank, s
 
 
 @pytest.mark.gpu
+def test_drawn_merge_in_place(pkg, L, dev):
+    if not L.DRAWS_LIKE_TORCH:
+        pytest.skip("this torch's generator is not the one that is reproduced")
+    N, K, rank = 301, 1040, 16
+    w = torch.randint(-128, 128, (N, K), dtype=torch.int8, device=dev)
+    up, down = torch.randn(N, rank, device=dev) * 0.05, torch.randn(rank, K, device=dev) * 0.05
+    seeded = lambda: pkg.int8_quant._seeded(12, dev)
+    want = L.lora_merge_sr_drawn(w, 0.003, seeded(), [(up, down, 1.0)])
+    with pytest.MonkeyPatch.context() as m:
+        m.setattr(torch, "empty_like", lambda t: t)   # (the result is written over the weight)
+        got = L.lora_merge_sr_drawn(w, 0.003, seeded(), [(up, down, 1.0)])
+    assert got is w and torch.equal(w, want)
+
+
+@pytest.mark.gpu
 def test_adapters_draw_what_they_drew(pkg, L, dev, monkeypatch):
     N, K = 640, 1040
     w = torch.randint(-127, 128, (N, K), dtype=torch.int8, device=dev)
@@ -49,10 +64,48 @@ def test_adapters_draw_what_they_drew(pkg, L, dev, monkeypatch):
     empty = pkg.INT8MergedLoRAPatchAdapter([(pkg.INT8LoRAPatchAdapter(set(), lora(4), ws), 0.7),
                                             (pkg.INT8LoRAPatchAdapter(set(), (*lora(0)[:2], None, None, None, None), ws), 0.7)], ws, seed=11)
     adapters = (one, stack, full, nine, empty)
+    drawn, taken = L.lora_merge_sr_drawn, []
+
+    def watched(*a):
+        merged = drawn(*a)
+        taken.append(merged is not None)
+        return merged
+
+    monkeypatch.setattr(L, "lora_merge_sr_drawn", watched)
     now = [a.calculate_weight(w, "", 1.0, 1.0, None, None) for a in adapters]
+    if L.DRAWS_LIKE_TORCH:   # nine LoRAs are too many for the launch: put side by side by torch, they are one
+        assert taken == [True, True, True, False, True, True]
     monkeypatch.setattr(L, "DRAWS_LIKE_TORCH", False)
     for got, a in zip(now, adapters):
         assert torch.equal(got, a.calculate_weight(w, "", 1.0, 1.0, None, None))
+
+
+@pytest.mark.gpu
+def test_a_lora_of_strength_0_keeps_the_weight_and_the_fast_path(pkg, L, dev):
+    if not L.DRAWS_LIKE_TORCH:
+        pytest.skip("this torch's generator is not the one that is reproduced")
+    N, K, rank = 12288, 3072, 32
+    w = torch.randint(-128, 128, (N, K), dtype=torch.int8, device=dev)
+    up, down = torch.randn(N, rank, device=dev) * 0.01, torch.randn(rank, K, device=dev) * 0.01
+    generator = pkg.int8_quant._seeded(6, dev)
+    merge = lambda lora_scale: L.lora_merge_sr_drawn(w, 0.002, generator, [(up, down, 1.0)], lora_scale)
+    assert torch.equal(merge(0.0), w) and torch.equal(merge(-0.0), w)
+
+    def median_time(lora_scale):
+        times = []
+        for _ in range(15):
+            first, last = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            first.record()
+            merge(lora_scale)
+            last.record()
+            torch.cuda.synchronize()
+            times.append(first.elapsed_time(last))
+        return sorted(times)[7]
+
+    assert median_time(0.0) < 1.4 * median_time(1.0)   # (2.0 times where every element goes by the definition)
+    up[5, 3], down[2, 7] = float("inf"), float("nan")   # sums that are not finite stay so at strength 0
+    noise = pkg.int8_quant._draw_noise((N, K), 6, dev)
+    assert torch.equal(merge(0.0), L.lora_merge_sr(w, 0.002, noise, up=up, down=down, lora_scale=0.0))
 
 
 @pytest.mark.gpu
