@@ -611,7 +611,7 @@ class Int8TensorwiseOps(manual_cast):
             if scale is None:
                 scale = self._buffers.get("weight_scale")
             if (not self._is_quantized or self.comfy_cast_weights or weight is None or scale is None
-                    or "bias" not in params or len(self.weight_function) > 0 or len(self.bias_function) > 0 or x.shape[-1] == 0):
+                    or "bias" not in params or len(self.weight_function) > 0 or len(self.bias_function) > 0):
                 return None
             if self.lora_A is not None:
                 if self.lora_B is None or self._use_quarot or prologue != _lib.PRO_NONE or gate is not None or residual is not None:

@@ -641,3 +641,11 @@ def test_native_host_path_on_several_streams_and_threads(pkg, dev):
     for t in threads:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("rows", [4, 40])
+def test_a_layer_without_inputs_is_the_general_paths(pkg, dev, rows):
+    lin = load(pkg.Int8TensorwiseOps.Linear(0, 48, bias=False), {"l.weight": torch.zeros(48, 0, dtype=torch.int8, device=dev), "l.weight_scale": torch.tensor(0.5)})
+    x = torch.ones(rows, 0, dtype=torch.bfloat16, device=dev)
+    assert lin._forward_native(x, pkg._lib.PRO_NONE, None, None, 1e-6, None, None, None, False) is None
+    assert lin._forward_native(x, pkg._lib.PRO_GELU_TANH, None, None, 1e-6, torch.ones(48, dtype=torch.bfloat16, device=dev), None, None, False) is None
