@@ -191,27 +191,39 @@ PyObject *small_m(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, const L
 // ---- a dynamic LoRA on the layer ---------------------------------------------------------------
 // Its first product by the launch that quantises x, the second inside the GEMM.  Two launches: with the BLAS library's call
 // between them and the interpreter's part of it all, the host took 63 us a layer and the GPU waited for it below 2000 rows.
-PyObject *linear_lora(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, const Layer &l, int order, PyObject *lora_a, PyObject *lora_b,
-                      PyObject *lora_alpha, const Stream &st) {
-    if (at::autocast::is_autocast_enabled(at::kCUDA)) Py_RETURN_NONE;  // (the product's type is then the context's)
-    const at::Tensor *A = tensor(lora_a), *B = tensor(lora_b);
+// linear_lora(x, weight, scale, bias, per_row, order, lora_A, lora_B, lora_alpha): a layer of more than 16 rows with the factors
+// of a dynamic LoRA, no rotation, nothing in front and nothing behind.
+PyObject *linear_lora(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 9) return PyErr_Format(PyExc_TypeError, "linear_lora takes 9 arguments, got %zd", n);
+    const at::Tensor *xt = tensor(a[0]), *A = tensor(a[6]), *B = tensor(a[7]);
+    if (!lib.bound || !xt || !A || !B || A->dim() != 2 || !xt->is_cuda()) Py_RETURN_NONE;
+    const at::Tensor &x = *xt;
+    const int64_t R = A->size(0);  // (the GEMM's LoRA epilogue takes ranks in steps of 16 up to 64)
+    int64_t M, K, ld;
+    if (R % 16 || R < 16 || R > 64 || !rows_of(x, M, K, ld)) Py_RETURN_NONE;
+    // (every 16 rows read the factor once more: 16384 rows are as many as were measured, where the quantiser and the BLAS
+    // library's product still take longer at every rank)
+    if (M > 16384 || K % 128 || K > (R > 32 ? 4096 : 6144) || ld % 8) Py_RETURN_NONE;
+    Layer l;
+    const at::ScalarType type = x.scalar_type();
+    if ((type != at::kBFloat16 && type != at::kHalf) || !layer_of(a[1], a[2], a[3], a[4] == Py_True, x.device(), l)) Py_RETURN_NONE;
     for (const at::Tensor *f : {A, B})
-        if (!f || f->scalar_type() != x.scalar_type() || f->device() != x.device() || f->dim() != 2 || !f->is_contiguous() || !aligned16(*f)) Py_RETURN_NONE;
-    const int64_t R = A->size(0);
-    // (the GEMM's LoRA epilogue takes ranks in steps of 16 up to 64.  Every 16 rows read the factor once more: 16384 rows are as
-    // many as were measured, where the quantiser and the BLAS library's product still take longer at every rank)
-    if (A->size(1) != K || B->size(0) != l.N || B->size(1) != R || R % 16 || R < 16 || R > 64 || M > 16384) Py_RETURN_NONE;
-    if (K != l.K || K % 128 || K > (R > 32 ? 4096 : 6144) || l.N % 8 || ld % 8 || !aligned16(x) || (uintptr_t)l.w % 16 || (l.mode == I8F_SCALE_ROW && (uintptr_t)l.ws % 16) ||
-        (uintptr_t)l.bias % 16 || l.N * K >= (1ll << 31))
+        if (f->scalar_type() != type || f->device() != x.device() || f->dim() != 2 || !f->is_contiguous() || !aligned16(*f)) Py_RETURN_NONE;
+    if (A->size(1) != K || B->size(0) != l.N || B->size(1) != R) Py_RETURN_NONE;
+    if (K != l.K || l.N % 8 || !aligned16(x) || (uintptr_t)l.w % 16 || (l.mode == I8F_SCALE_ROW && (uintptr_t)l.ws % 16) || (uintptr_t)l.bias % 16 ||
+        l.N * K >= (1ll << 31))
         Py_RETURN_NONE;
+    if (at::autocast::is_autocast_enabled(at::kCUDA)) Py_RETURN_NONE;  // (the product's type is then the context's)
     float alpha = 0.0f;
-    const bool has_alpha = lora_alpha != Py_None;
+    const bool has_alpha = a[8] != Py_None;
     if (has_alpha) {
-        if (!PyFloat_CheckExact(lora_alpha) && !PyLong_CheckExact(lora_alpha)) Py_RETURN_NONE;
-        alpha = (float)PyFloat_AsDouble(lora_alpha);
+        if (!PyFloat_CheckExact(a[8]) && !PyLong_CheckExact(a[8])) Py_RETURN_NONE;
+        alpha = (float)PyFloat_AsDouble(a[8]);
         if (PyErr_Occurred()) return nullptr;
     }
-    const at::ScalarType type = x.scalar_type();
+    const Stream st(x.device());
+    if (!st.ok) Py_RETURN_NONE;
+    const int order = (int)PyLong_AsLong(a[5]);
     const at::Device dev = x.device();
     const Size size = output_size(x, l.N);
     const int dt = code_of(type);
@@ -236,13 +248,12 @@ PyObject *linear_lora(const at::Tensor &x, int64_t M, int64_t K, int64_t ld, con
 }
 
 // linear(x, weight, scale, bias, per_row, rotate, small_rows, order, kind, mod_scale, mod_shift, eps, norm_weight, fused_add,
-//        gate, residual, workspace[, lora_A, lora_B, lora_alpha]): kind, an i8f_prologue, names what is applied to x inside the
-// quantiser; lora_A (or None) and lora_B are the factors of a dynamic LoRA; workspace(x, M, N, K) gives the memory of
-// the K split or None.  It is called once a W8A8 call has passed every check, never for 16 rows or fewer, for a
-// layer with a LoRA or for a call that goes the general way, which asks for its own: the memory stays with the stream, or
-// with the graph that is being captured, together with the kernel that clears it.
+//        gate, residual, workspace): kind, an i8f_prologue, names what is applied to x inside the quantiser; workspace(x, M, N,
+// K) gives the memory of the K split or None.  It is called once a W8A8 call has passed every check, never for 16 rows or
+// fewer or for a call that goes the general way, which asks for its own: the memory stays with the stream, or with the graph
+// that is being captured, together with the kernel that clears it.
 PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
-    if (n != 17 && n != 20) return PyErr_Format(PyExc_TypeError, "linear takes 17 or 20 arguments, got %zd", n);
+    if (n != 17) return PyErr_Format(PyExc_TypeError, "linear takes 17 arguments, got %zd", n);
     const at::Tensor *xt = tensor(a[0]);
     if (!lib.bound || !xt || !xt->is_cuda()) Py_RETURN_NONE;
     const at::Tensor &x = *xt;
@@ -256,10 +267,6 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const bool gated = a[14] != Py_None, with_residual = a[15] != Py_None;
     const Stream st(x.device());
     if (!st.ok || (rotate && K % 128)) Py_RETURN_NONE;
-    if (n == 20 && a[17] != Py_None) {
-        if (kind != I8F_PRO_NONE || gated || with_residual || rotate || M <= small_rows) Py_RETURN_NONE;
-        return linear_lora(x, M, K, ld, l, order, a[17], a[18], a[19], st);
-    }
     if (M <= small_rows) {
         if (kind != I8F_PRO_NONE || gated || with_residual || K != l.K) Py_RETURN_NONE;
         return small_m(x, M, K, ld, l, rotate, st.handle);
@@ -453,6 +460,7 @@ PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"bind", bind, METH_O, "bind(path): load the kernels' library"},
     {"linear", (PyCFunction)(void (*)(void))guarded<linear>, METH_FASTCALL, "one quantised layer, or None"},
+    {"linear_lora", (PyCFunction)(void (*)(void))guarded<linear_lora>, METH_FASTCALL, "one quantised layer with a dynamic LoRA, or None"},
     {"vector_fanout", (PyCFunction)(void (*)(void))guarded<vector_fanout>, METH_FASTCALL, "several small-batch layers, or None"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_i8f_host", "Native host path of the INT8 linear layers.", -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -606,6 +606,12 @@ class Int8TensorwiseOps(manual_cast):
             managed casting, 16-bit contiguous rows on the current GPU); None for everything else.  A weight
             or bias that is no parameter of the layer (pruned, parametrised, a buffer) is the general path's, too: it reads
             the attributes, which are computed or kept elsewhere then."""
+            lora = self.lora_A
+            if lora is not None:   # (most of what has no native form is told by these: the general path comes behind them)
+                shape = lora.shape
+                if (self.lora_B is None or self._use_quarot or prologue != _lib.PRO_NONE or gate is not None or residual is not None
+                        or len(shape) != 2 or shape[0] % 16 or shape[1] > 6144 or x.numel() <= SMALL_BATCH_ROWS * shape[1]):
+                    return None
             params, scale = self._parameters, self._weight_scale_scalar
             weight = params.get("weight")
             if scale is None:
@@ -613,12 +619,9 @@ class Int8TensorwiseOps(manual_cast):
             if (not self._is_quantized or self.comfy_cast_weights or weight is None or scale is None
                     or "bias" not in params or len(self.weight_function) > 0 or len(self.bias_function) > 0):
                 return None
-            if self.lora_A is not None:
-                if self.lora_B is None or self._use_quarot or prologue != _lib.PRO_NONE or gate is not None or residual is not None:
-                    return None
-                return _lib.host().linear(x, weight, scale, params["bias"], bool(self._is_per_row), False, SMALL_BATCH_ROWS,
-                                          int8_fused_kernel.DEFAULT_EPILOGUE, prologue, None, None, eps, None, False, None, None, None,
-                                          self.lora_A, self.lora_B, self.lora_alpha)
+            if lora is not None:
+                return _lib.host().linear_lora(x, weight, scale, params["bias"], bool(self._is_per_row), int8_fused_kernel.DEFAULT_EPILOGUE,
+                                               lora, self.lora_B, self.lora_alpha)
             if prologue == _lib.PRO_MODULATE_FUSED:
                 prologue, fused_add = _lib.PRO_MODULATE, True
             work = _lib._splitk_workspace if weight.shape[-1] >= _lib.SPLITK_MIN_K else None   # (asked for by a call that can use it)

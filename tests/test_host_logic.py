@@ -1,6 +1,7 @@
 """Host-side behaviour of the ComfyUI-facing layer that needs no GPU: state-dict loading rules,
 scale bookkeeping, ModelPatcher hooks, LoRA scale slicing, delta reconstruction, Hadamard build."""
 import sysconfig
+import types
 
 import numpy as np
 import pytest
@@ -327,3 +328,26 @@ def test_native_host_path_is_told_the_scale_mode_as_a_truth_value(pkg, host, fla
     lin._is_per_row = flag
     native(pkg, lin, torch.zeros(20, 64, dtype=torch.bfloat16))
     assert host.calls[0][4] is bool(flag)
+
+
+def test_a_lora_without_a_native_form_does_not_ask_for_one(pkg, monkeypatch):
+    """Rank, rows and width tell it before anything is prepared for the native path; what they let through reaches it."""
+    lin = pkg.Int8TensorwiseOps.Linear(64, 48, bias=False, dtype=torch.bfloat16)
+    lin.weight = torch.nn.Parameter(torch.zeros(48, 64, dtype=torch.int8), requires_grad=False)
+    lin._is_quantized, lin._weight_scale_scalar = True, 0.01
+    asked = []
+    monkeypatch.setattr(pkg._lib, "host", lambda: types.SimpleNamespace(linear_lora=lambda *a: asked.append(a)))
+
+    def call(rank, rows, lora_b=True, rotated=False, width=64, **other):
+        lin.lora_A = torch.zeros(rank, width, dtype=torch.bfloat16)
+        lin.lora_B = torch.zeros(48, rank, dtype=torch.bfloat16) if lora_b else None
+        lin._use_quarot = rotated
+        del asked[:]
+        args = dict(prologue=pkg._lib.PRO_NONE, mod_scale=None, mod_shift=None, eps=1e-6, gate=None, residual=None, norm_weight=None, fused_add=False)
+        assert lin._forward_native(torch.zeros(rows, width, dtype=torch.bfloat16), **{**args, **other}) is None
+        return len(asked)
+
+    assert call(16, 17) == 1 and call(64, 17) == 1
+    assert call(8, 40) == 0 and call(16, 16) == 0 and call(16, 40, lora_b=False) == 0 and call(16, 40, rotated=True) == 0
+    assert call(16, 40, width=6272) == 0 and call(16, 40, gate=torch.zeros(48)) == 0 and call(16, 40, residual=torch.zeros(40, 48)) == 0
+    assert call(16, 40, prologue=pkg._lib.PRO_GELU_TANH) == 0
