@@ -548,7 +548,8 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
     // is done.  Nothing looks at the results before the epilogue: indices are clamped instead of
     // predicated and the conversion happens after the loop, so no instruction in between waits for
     // them (the wait for tile 0 below counts them among the younger loads it may leave in flight, and
-    // so waits for up to three loads of tile 1 more than it has to).
+    // so waits for as many loads of tile 1 more than it has to: up to three, and where a side branch's rows are requested
+    // here too, SIDE_PER of those, four in 256 x 256 tiles).
     constexpr int XS_PER = (BM + C::NT - 1) / C::NT, WS_PER = (BN + C::NT - 1) / C::NT;
     float xs_r[XS_PER], ws_r[WS_PER];
     uint32_t bias_r[WS_PER];
