@@ -831,7 +831,7 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
     using F_ = std::false_type;
     using O0 = std::integral_constant<int, I8F_EPI_TORCH>;
     using O1 = std::integral_constant<int, I8F_EPI_FUSED>;
-    constexpr bool BATCHED = C::NT <= 512 && !SIDE;  // gate and addend in batches, in epilogues of their own
+    constexpr bool BATCHED = C::NT <= 512 && !SIDE && OUT != OUT_I32;  // gate and addend in batches, in epilogues of their own
     const int variant = (BATCHED && (ggate || gaddend) ? 8 : 0) | (g.order == I8F_EPI_FUSED ? 4 : 0) | (row_scale ? 2 : 0) | (gbias ? 1 : 0);
 
     // The whole epilogue is instantiated once per variant and the variant is chosen ONCE, so that
@@ -979,7 +979,7 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
                     if (mm < gM && nn < gN) {
                         const int64_t off = ((int64_t)mm * gN + nn) * OB;
                         uint4 v = val;
-                        if constexpr (!BATCHED && !SIDE) {
+                        if constexpr (!BATCHED && !SIDE && OUT != OUT_I32) {
                             if (ggate)
                                 v = mul_rounded<OUT>(v, *(const uint4 *)((const char *)ggate + ((int64_t)((uint32_t)mm / (uint32_t)ggate_rows) * gN + nn) * OB));
                             if (gaddend) v = add_rounded<OUT>(v, *(const uint4 *)((const char *)gaddend + off));
@@ -1047,10 +1047,7 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
     };
     using S0 = std::integral_constant<int, 0>;
     if constexpr (OUT == OUT_I32) {
-        if constexpr (BATCHED) {
-            if (variant & 8) return run_epilogue(O0{}, F_{}, F_{}, S0{}, T_{});
-        }
-        run_epilogue(O0{}, F_{}, F_{}, S0{}, F_{});
+        run_epilogue(O0{}, F_{}, F_{}, S0{}, F_{});  // (the raw product: no gate and no addend)
     } else if constexpr (SIDE) {  // (no gate and no addend beside a side branch)
         if (g.side_rank > 32) choose(std::integral_constant<int, 4>{});
         else choose(std::integral_constant<int, 2>{});
