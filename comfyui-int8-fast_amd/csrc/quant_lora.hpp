@@ -19,9 +19,10 @@ __device__ __forceinline__ v4f lora_mfma(v4u a, v4u b, v4f c) {
 // rounding); x is read once for both.  Eight waves share the rows: wave w takes blocks w, w + 8, ... of 64 columns of all
 // sixteen.  Eight neighbouring lanes load the 128 bytes of a row, of x and of A alike, and the tiles change to the matrix
 // unit's layout in LDS of the wave's own.  Loading that layout directly, with neighbouring lanes in different rows, moves 16
-// bytes a cycle and CU, and took 11.4 us at 1357 x 3072, rank 32, where this takes 7.7 and the quantiser and the BLAS
-// library's product 4.2 + 8.8 us; at 4608 rows 15.2 against 7.1 + 9.5, at 9729 24 against 28, at 16384 and rank 64 47 against
-// 49.  Bound by a CU's loads: 16 rows of x and the whole of A, 290 KB of them, for each workgroup; with more rows to share A
+// bytes a cycle and CU, and took 11.4 us at 1357 x 3072, rank 32.  us of a launch in a replayed graph, against the quantiser's
+// and that of the BLAS library's product, on one x and on twelve in turn (from HBM): 1357 x 3072, rank 32 7.3 against 2.9 +
+// 6.5 and 7.8 against 3.7 + 7.7 (a profiler shows 8.5); 4608 rows 13.9, 4.7 + 8.2 and 18.1, 8.9 + 11.9; 9729 rows 24.0, 13.9 + 13.0
+// and 27.6, 16.7 + 16.6; 16384 rows, rank 64 44.4, 22.0 + 18.7 and 48.5, 26.6 + 23.3.  Bound by a CU's loads: 16 rows of x and the whole of A, 290 KB of them, for each workgroup; with more rows to share A
 // the chip would stand idle at the sizes where it matters, and registers for two workgroups a CU (128) spill: 15.2 -> 17.9.
 // BLOCKS: 64-column blocks to a wave at most; FEWEST: that every wave has.
 template <int DT, int RT, int BLOCKS, int FEWEST>
