@@ -20,8 +20,8 @@ extern "C" {
  * (rounded); of one LoRA mult is not looked at.  The result is that of i8f_lora_merge_sr on these factors and this noise, bit
  * for bit (INT8LoRAPatchAdapter / INT8MergedLoRAPatchAdapter.calculate_weight, int8_quant.py:293-318, 382-404).
  * up [N,rank] and down [rank,K] of each are float.  At most 8 LoRAs, K % 16 == 0, K < 2^24, the sum of the ranks a
- * multiple of 4 and <= 256, N K <= 2^29, lanes % 256 == 0, lanes <= 2^24, N K / (4 lanes) (and, of a stack, some blocks for
- * its factors) within the 65535 blocks of a launch, a stack's (N + K) rank < 2^31, w, w_out, workspace and the `up` of a
+ * multiple of 4 and <= 256, N K <= 2^29, lanes % 256 == 0, lanes <= 2^24, N K / (4 lanes) within the 65535 blocks of a
+ * launch, a stack's (N + K) rank < 2^31, w, w_out, workspace and the `up` of a
  * single LoRA 16-byte aligned; else I8F_ERR_UNSUPPORTED.  workspace: any contents.  w_out may equal w.
  */
 typedef struct {

@@ -15,7 +15,31 @@ CASES = [
     (400, 2064, 8, 9, True, 10.0),       # every quotient far outside int8
     (400, 2064, 8, 10, True, 1e-20),     # products in the denormal range
     (400, 2064, 16, 11, True, 0.25),     # quotients of some tens: many elements are redone
+    # every number of 16-rank steps that is built, on rows and columns around a tile's 32 and 128
+    (31, 128, 16, 12, True, 0.01), (32, 144, 32, 13, True, 0.01), (33, 112, 48, 14, True, 0.01), (64, 272, 64, 15, False, 0.01),
+    (65, 256, 80, 16, True, 0.01), (95, 368, 96, 17, True, 0.02), (97, 384, 112, 18, True, 0.02), (130, 400, 128, 19, True, 0.02),
+    (161, 496, 160, 20, False, 0.02), (200, 528, 192, 21, True, 0.02), (223, 640, 224, 22, True, 0.02), (300, 784, 256, 23, True, 0.05),
+    (3000, 272, 32, 24, True, 0.1),      # quotients that have to be saturated before they are added
+    (640, 272, 256, 25, True, 0.5),      # an error bound that leaves a good part of the elements to the definition
 ]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [0.0, 1e-30, 1e-36, float("nan"), float("inf"), -0.001])
+def test_drawn_merge_of_rows_without_a_usual_scale(pkg, L, dev, scale):
+    """Single rows, which go to the list of open elements, and whole blocks of them, which are passed over and redone."""
+    if not L.DRAWS_LIKE_TORCH:
+        pytest.skip("this torch's generator is not the one that is reproduced")
+    N, K, rank = 200, 400, 12
+    g = torch.Generator(device=dev).manual_seed(5)
+    w = torch.randint(-128, 128, (N, K), generator=g, device=dev, dtype=torch.int8)
+    ws = torch.rand(N, generator=g, device=dev) * 0.002 + 0.0005
+    ws[5] = scale
+    ws[64:160] = scale
+    up, down = torch.randn(N, rank, generator=g, device=dev) * 0.02, torch.randn(rank, K, generator=g, device=dev) * 0.02
+    noise = pkg.int8_quant._draw_noise((N, K), 9, dev)
+    drawn = L.lora_merge_sr_drawn(w, ws, pkg.int8_quant._seeded(9, dev), [(up, down, 1.0)], 0.75)
+    assert torch.equal(drawn, L.lora_merge_sr(w, ws, noise, up=up, down=down, lora_scale=0.75))
 
 
 @pytest.mark.gpu
