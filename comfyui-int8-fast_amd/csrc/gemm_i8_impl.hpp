@@ -32,6 +32,7 @@
 #include "splitk_protocol.h"
 #include <algorithm>
 #include <atomic>
+#include <numeric>
 
 namespace i8f {
 namespace gemm {
@@ -964,9 +965,8 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
             const int mw = m0 + wm * C::WTM + i0 * 32, nw = n0 + wn * C::WTN;   // first row and column of the staged strips
             // Gate and addend of BATCH pieces are requested together, and those of the next batch before this one is used: a load
             // behind each store, above which it may not be moved, is a trip to memory for every piece (35 to 54 K cycles of
-            // epilogue at 4608 x 3072, 9.6 K without gate and addend; 28 to 43 K in fours).  us, gate and addend, before and
-            // after: 4608 x 3072 x 3072 50.6 and 48.2, x 12288 156.7 and 153.3, 9729 x 3072 x 15360 370 and 361, 512 x 3072 x 12288 in
-            // 128 x 96 tiles and two slices 38.6 and 37.0.  Twelve waves have no registers for it (4096 x 9216 x 3072 in 256 x 288
+            // epilogue at 4608 x 3072, 9.6 K without gate and addend; 512 x 3072 x 12288 in 128 x 96 tiles and two slices 38.6 us,
+            // 37.0 in fours).  Twelve waves have no registers for it (4096 x 9216 x 3072 in 256 x 288
             // tiles 136 and 141 us).  GATED is chosen with the variant, so that an epilogue without gate and addend stays
             // contiguous: with a jump over their code the smallest outputs took 2 to 3 % longer (93 x 3200 x 3200 8.6 for 8.4 us).
             if constexpr (!decltype(GATED)::value) {
@@ -988,39 +988,54 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
                     }
                 }
             } else {
-                constexpr int BATCH = PASSES <= 8 ? PASSES : 4;
-                static_assert(PASSES % BATCH == 0, "whole batches");
-                uint4 gate_r[2][BATCH], add_r[2][BATCH];
+                // After PERIOD passes a lane's pieces lie in the same columns again: where one gate serves all rows of the wave, its
+                // pieces are these few, fetched once.  (Fetched beside every addend's they were half of the requests, of which a CU
+                // has 64 in flight.  us, operands from HBM, gate and addend: 4608 x 3072 x 3072 50.5 and 44.0, x 12288 147 and 139.4,
+                // 9729 x 3072 x 15360 352 and 341; without gate and addend 39, 136, 336.)
+                constexpr int PERIOD = CPO / std::gcd(64, CPO);
                 const bool one_gate = !ggate || (uint32_t)mw / (uint32_t)ggate_rows == (uint32_t)min(mw + EPI_STRIPS * 32 - 1, gM - 1) / (uint32_t)ggate_rows;
                 const int first_gate = ggate ? (int)((uint32_t)mw / (uint32_t)ggate_rows) : 0;
-                auto fetch = [&](int p0, uint4 (&gr)[BATCH], uint4 (&ar)[BATCH]) __attribute__((always_inline)) {
+                auto passes = [&](auto ONE_GATE) __attribute__((always_inline)) {
+                    constexpr bool ONCE = decltype(ONE_GATE)::value && PERIOD < PASSES;
+                    constexpr int BATCH = PASSES <= 8 ? PASSES : ONCE && PASSES % 8 == 0 ? 8 : 4;
+                    static_assert(PASSES % BATCH == 0, "whole batches");
+                    uint4 gate_r[ONCE ? 1 : 2][ONCE ? PERIOD : BATCH], add_r[2][BATCH];
+                    auto gate_piece = [&](int gv, int nn) { return *(const uint4 *)((const char *)ggate + ((int64_t)gv * gN + nn) * OB); };
+                    auto fetch = [&](int p0, int at) __attribute__((always_inline)) {
 #pragma unroll
-                    for (int u = 0; u < BATCH; ++u) {   // (rows and columns beyond the output repeat the last ones, unused)
-                        const int id = (p0 + u) * 64 + lane;
-                        const int mm = min(mw + id / CPO, gM - 1), nn = min(nw + id % CPO * EPCO, gN - EPCO);
-                        if (gaddend) ar[u] = *(const uint4 *)((const char *)gaddend + ((int64_t)mm * gN + nn) * OB);
-                        if (ggate) {
-                            const int gv = one_gate ? first_gate : (int)((uint32_t)mm / (uint32_t)ggate_rows);
-                            gr[u] = *(const uint4 *)((const char *)ggate + ((int64_t)gv * gN + nn) * OB);
+                        for (int u = 0; u < BATCH; ++u) {   // (rows and columns beyond the output repeat the last ones, unused)
+                            const int id = (p0 + u) * 64 + lane;
+                            const int mm = min(mw + id / CPO, gM - 1), nn = min(nw + id % CPO * EPCO, gN - EPCO);
+                            if (gaddend) add_r[at][u] = *(const uint4 *)((const char *)gaddend + ((int64_t)mm * gN + nn) * OB);
+                            if constexpr (!ONCE) {
+                                if (ggate) gate_r[at][u] = gate_piece(decltype(ONE_GATE)::value ? first_gate : (int)((uint32_t)mm / (uint32_t)ggate_rows), nn);
+                            }
+                        }
+                    };
+                    if constexpr (ONCE) {
+#pragma unroll
+                        for (int u = 0; u < PERIOD; ++u)
+                            if (ggate) gate_r[0][u] = gate_piece(first_gate, min(nw + (u * 64 + lane) % CPO * EPCO, gN - EPCO));
+                    }
+                    fetch(0, 0);
+#pragma unroll
+                    for (int p0 = 0; p0 < PASSES; p0 += BATCH) {
+                        const int now = p0 / BATCH % 2;
+                        if (p0 + BATCH < PASSES) fetch(p0 + BATCH, now ^ 1);
+#pragma unroll
+                        for (int u = 0; u < BATCH; ++u) {
+                            const int id = (p0 + u) * 64 + lane;
+                            const int row = id / CPO, cc = id % CPO;
+                            uint4 v = *(const uint4 *)(ebuf + row * PITCH + cc * 16);
+                            const int mm = mw + row, nn = nw + cc * EPCO;
+                            if (ggate) v = mul_rounded<OUT>(v, ONCE ? gate_r[0][(p0 + u) % PERIOD] : gate_r[now][ONCE ? 0 : u]);
+                            if (gaddend) v = add_rounded<OUT>(v, add_r[now][u]);
+                            if (mm < gM && nn < gN) stream_store16((char *)gout + ((int64_t)mm * gN + nn) * OB, v);
                         }
                     }
                 };
-                fetch(0, gate_r[0], add_r[0]);
-#pragma unroll
-                for (int p0 = 0; p0 < PASSES; p0 += BATCH) {
-                    const int now = p0 / BATCH % 2;
-                    if (p0 + BATCH < PASSES) fetch(p0 + BATCH, gate_r[now ^ 1], add_r[now ^ 1]);
-#pragma unroll
-                    for (int u = 0; u < BATCH; ++u) {
-                        const int id = (p0 + u) * 64 + lane;
-                        const int row = id / CPO, cc = id % CPO;
-                        uint4 v = *(const uint4 *)(ebuf + row * PITCH + cc * 16);
-                        const int mm = mw + row, nn = nw + cc * EPCO;
-                        if (ggate) v = mul_rounded<OUT>(v, gate_r[now][u]);
-                        if (gaddend) v = add_rounded<OUT>(v, add_r[now][u]);
-                        if (mm < gM && nn < gN) stream_store16((char *)gout + ((int64_t)mm * gN + nn) * OB, v);
-                    }
-                }
+                if (one_gate) passes(T_{});
+                else passes(F_{});
             }
             __builtin_amdgcn_wave_barrier();
         }

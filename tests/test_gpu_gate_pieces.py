@@ -1,0 +1,22 @@
+"""The gated residual where the pieces of a gate are shared by the passes of a wave and where they are not: rows per gate that
+end inside a wave's tile, tiles whose passes repeat their columns every time (128 columns) or every third time (96), ragged edges."""
+import pytest
+import torch
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,rows_per_gate,dtype", [
+    (4032, 3072, 128, 4032, torch.bfloat16), (4032, 3072, 128, 96, torch.bfloat16), (4000, 3064, 256, 40, torch.float16),  # 256 x 192
+    (4608, 3072, 128, 4608, torch.bfloat16), (4608, 3072, 128, 288, torch.float16), (4600, 3064, 128, 8, torch.bfloat16),  # 256 x 256
+    (512, 3072, 12288, 512, torch.bfloat16), (510, 3064, 12288, 85, torch.bfloat16),                                       # 128 x 96, K split
+    (500, 9208, 256, 50, torch.float16), (100, 1000, 128, 25, torch.float32), (650, 6144, 128, 130, torch.bfloat16),
+])
+def test_gated_residual_equals_the_tensor_operations(L, dev, M, N, K, rows_per_gate, dtype):
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    x, scale = L.quant_rowwise(torch.randn(M, K, generator=g, device=dev))
+    w, ws = L.quant_rowwise(torch.randn(N, K, generator=g, device=dev) * 0.02)
+    gate = torch.randn(M // rows_per_gate, N, generator=g, device=dev).to(dtype)
+    residual = torch.randn(M, N, generator=g, device=dev).to(dtype)
+    plain = L.linear_w8a8(x, scale, w, ws, None, dtype, L.EPI_TORCH)
+    got = L.linear_w8a8(x, scale, w, ws, None, dtype, L.EPI_TORCH, addend=residual, gate=gate)
+    assert torch.equal(got, residual + gate.repeat_interleave(rows_per_gate, 0) * plain)
