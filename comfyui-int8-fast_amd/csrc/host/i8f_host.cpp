@@ -5,6 +5,7 @@
 //
 //   bind(path)                  the kernels' library
 //   linear(...)                 one layer: Linear.forward with its optional prologue, gate and residual
+//   fanout(...)                 several layers that read the same tokens, quantised once
 //   vector_fanout(...)          several small-batch layers that read the same rows, in one launch
 //
 // Every function takes the cases it can decide on cheaply and returns None for all others (tensors of other types,
@@ -34,7 +35,7 @@ namespace {
 // ---- the kernels' library -----------------------------------------------------------------
 #define I8F_ENTRY_POINTS(X)                                                                                              \
     X(i8f_quant_rowwise) X(i8f_quant_rowwise_prologue) X(i8f_quant_rowwise_norm_modulate) X(i8f_quant_rowwise_rms_norm)  \
-    X(i8f_quant_rowwise_concat_gelu) X(i8f_rotate128) X(i8f_linear_w8a8_gated) X(i8f_linear_w8a16_small_m)               \
+    X(i8f_quant_rowwise_concat_gelu) X(i8f_rotate128) X(i8f_linear_w8a8_gated) X(i8f_linear_w8a8_grouped) X(i8f_linear_w8a16_small_m) \
     X(i8f_linear_w8a16_small_m_grouped) X(i8f_internal_w8a16_rotated) X(i8f_linear_w8a8_lora) X(i8f_internal_quant_lora)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -248,30 +249,27 @@ PyObject *linear_lora(PyObject *, PyObject *const *a, Py_ssize_t n) {
     return THPVariable_Wrap(std::move(y));
 }
 
-// linear(x, weight, scale, bias, per_row, rotate, small_rows, order, kind, mod_scale, mod_shift, eps, norm_weight, fused_add,
-//        gate, residual, workspace): kind, an i8f_prologue, names what is applied to x inside the quantiser; workspace(x, M, N,
-// K) gives the memory of the K split or None.  It is called once a W8A8 call has passed every check, never for 16 rows or
-// fewer or for a call that goes the general way, which asks for its own: the memory stays with the stream, or with the graph
-// that is being captured, together with the kernel that clears it.
-PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
-    if (n != 17) return PyErr_Format(PyExc_TypeError, "linear takes 17 arguments, got %zd", n);
-    const at::Tensor *xt = tensor(a[0]);
-    if (!lib.bound || !xt || !xt->is_cuda()) Py_RETURN_NONE;
-    const at::Tensor &x = *xt;
-    const int dt = code_of(x.scalar_type());
-    const bool per_row = a[4] == Py_True, rotate = a[5] == Py_True, fused_add = a[13] == Py_True;
-    int64_t M, K, ld;
-    Layer l;
-    if ((dt != I8F_BF16 && dt != I8F_F16) || !rows_of(x, M, K, ld) || !layer_of(a[1], a[2], a[3], per_row, x.device(), l)) Py_RETURN_NONE;
-    const int64_t small_rows = PyLong_AsLongLong(a[6]);
-    const int order = (int)PyLong_AsLong(a[7]), kind = (int)PyLong_AsLong(a[8]);
-    const bool gated = a[14] != Py_None, with_residual = a[15] != Py_None;
-    const Stream st(x.device());
-    if (!st.ok || (rotate && K % 128)) Py_RETURN_NONE;
-    if (M <= small_rows) {
-        if (kind != I8F_PRO_NONE || gated || with_residual || K != l.K) Py_RETURN_NONE;
-        return small_m(x, M, K, ld, l, rotate, st.handle);
+constexpr int MAX_FANOUT = 8;
+
+PyObject *list_of(at::Tensor *y, Py_ssize_t count) {
+    PyObject *out = PyList_New(count);
+    if (!out) return nullptr;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        PyObject *o = THPVariable_Wrap(std::move(y[i]));
+        if (!o) {
+            Py_DECREF(out);
+            return nullptr;
+        }
+        PyList_SET_ITEM(out, i, o);
     }
+    return out;
+}
+
+// The W8A8 form of linear and fanout, whose arguments these are; a gate or a residual for one layer only.
+PyObject *w8a8(PyObject *const *a, const at::Tensor &x, int64_t M, int64_t K, int64_t ld, const Layer *l, int count, const Stream &st) {
+    const int dt = code_of(x.scalar_type()), order = (int)PyLong_AsLong(a[7]), kind = (int)PyLong_AsLong(a[8]);
+    const bool rotate = a[5] == Py_True, fused_add = a[13] == Py_True, gated = a[14] != Py_None, with_residual = a[15] != Py_None;
+    if (count != 1 && (gated || with_residual)) Py_RETURN_NONE;
 
     // the operation in front of the layer and its operands
     const at::Tensor *s = nullptr, *t = nullptr, *w = nullptr;
@@ -312,41 +310,43 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     } else if (kind != I8F_PRO_NONE && kind != I8F_PRO_GELU_TANH && kind != I8F_PRO_GELU_ERF) {
         Py_RETURN_NONE;
     }
-    if (Kall != l.K) Py_RETURN_NONE;
+    for (int i = 0; i < count; ++i)
+        if (l[i].K != Kall) Py_RETURN_NONE;
 
     // what follows the layer
     const at::Tensor *gate = nullptr, *res = nullptr, *work = nullptr;
     int64_t gate_rows = 1;
     if (gated) {
         gate = tensor(a[14]);
-        if (!gate || !broadcasts_over_tokens(x, l.N, *gate)) Py_RETURN_NONE;
-        const int64_t vecs = gate->numel() / l.N;
+        if (!gate || !broadcasts_over_tokens(x, l[0].N, *gate)) Py_RETURN_NONE;
+        const int64_t vecs = gate->numel() / l[0].N;
         if (vecs < 1 || M % vecs) Py_RETURN_NONE;
         gate_rows = M / vecs;
     }
     if (with_residual) {
         res = tensor(a[15]);
         if (!res || res->scalar_type() != x.scalar_type() || res->device() != x.device() || res->dim() != x.dim() || !res->is_contiguous() ||
-            res->numel() != M * l.N || res->size(-1) != l.N)
+            res->numel() != M * l[0].N || res->size(-1) != l[0].N)
             Py_RETURN_NONE;
         for (int64_t i = 0; i + 1 < x.dim(); ++i)
             if (res->size(i) != x.size(i)) Py_RETURN_NONE;
     }
     Owned work_object;
     if (a[16] != Py_None) {
-        work_object.p = PyObject_CallFunction(a[16], "OLLL", a[0], (long long)M, (long long)l.N, (long long)l.K);
+        work_object.p = PyObject_CallFunction(a[16], "OLLL", a[0], (long long)M, (long long)l[0].N, (long long)Kall);
         if (!work_object.p) return nullptr;
         if (work_object.p != Py_None && !(work = tensor(work_object.p))) Py_RETURN_NONE;
     }
 
     const at::ScalarType type = x.scalar_type();
     const at::Device dev = x.device();
-    const Size size = output_size(x, l.N);
+    Size size[MAX_FANOUT];
+    for (int i = 0; i < count; ++i) size[i] = output_size(x, l[i].N);
     const auto address = [](const at::Tensor *o) { return o ? o->const_data_ptr() : nullptr; };
     const void *xp = x.const_data_ptr(), *sp = address(s), *tp = address(t), *wp = address(w), *gate_p = address(gate), *res_p = address(res);
     void *work_p = work ? work->data_ptr() : nullptr;
     const int64_t work_bytes = work ? work->numel() : 0;
-    at::Tensor scratch, y;
+    at::Tensor scratch, y[MAX_FANOUT];
     int rc;
     {
         const WithoutGil released;
@@ -356,7 +356,7 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
         scratch = empty({q_bytes + 4 * M}, at::kByte, dev);
         int8_t *q = (int8_t *)scratch.data_ptr();
         float *qs = (float *)(q + q_bytes);
-        y = empty(size, type, dev);
+        for (int i = 0; i < count; ++i) y[i] = empty(size[i], type, dev);
         const int rb = rotate ? 128 : 0;
         switch (kind) {
         case I8F_PRO_NONE: rc = lib.i8f_quant_rowwise(xp, dt, M, K, ld, rb, q, qs, st.handle); break;
@@ -370,12 +370,72 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
             rc = lib.i8f_quant_rowwise_prologue(xp, dt, M, K, ld, kind == I8F_PRO_MODULATE && fused_add ? (int)I8F_PRO_MODULATE_FUSED : kind, sp, tp,
                                                 M / V, rb, q, qs, st.handle);
         }
-        if (!rc)
-            rc = lib.i8f_linear_w8a8_gated(q, qs, l.w, l.ws, l.ws_host, l.mode, l.bias, l.bias_code, gate_p, gate_rows, res_p, y.data_ptr(), dt, M,
-                                           l.N, l.K, order, work_p, work_bytes, st.handle);
+        if (!rc && count == 1)
+            rc = lib.i8f_linear_w8a8_gated(q, qs, l[0].w, l[0].ws, l[0].ws_host, l[0].mode, l[0].bias, l[0].bias_code, gate_p, gate_rows, res_p,
+                                           y[0].data_ptr(), dt, M, l[0].N, l[0].K, order, work_p, work_bytes, st.handle);
+        for (int first = 0, next; count > 1 && !rc && first < count; first = next) {  // layers of one form, a launch for as many as the library puts together
+            i8f_linear_group g[I8F_MAX_LINEAR_GROUPS] = {};
+            int bias_code = -1;
+            for (next = first; next < count && next - first < I8F_MAX_LINEAR_GROUPS; ++next) {
+                const Layer &o = l[next];
+                if (o.N != l[first].N || o.mode != l[first].mode || (o.bias && bias_code >= 0 && o.bias_code != bias_code)) break;
+                if (o.bias) bias_code = o.bias_code;
+                i8f_linear_group &e = g[next - first];
+                e.a = q, e.a_scale = qs, e.w = o.w, e.w_scale = o.ws, e.w_scale_host = o.ws_host, e.bias = o.bias, e.out = y[next].data_ptr(), e.M = M;
+                e.rows_per_gate = 1;
+            }
+            rc = lib.i8f_linear_w8a8_grouped(g, next - first, l[first].mode, bias_code < 0 ? (int)I8F_BF16 : bias_code, dt, l[first].N, Kall, order, work_p,
+                                             work_bytes, st.handle);
+        }
     }
     if (rc) Py_RETURN_NONE;
-    return THPVariable_Wrap(std::move(y));
+    return count == 1 ? THPVariable_Wrap(std::move(y[0])) : list_of(y, count);
+}
+
+// linear(x, weight, scale, bias, per_row, rotate, small_rows, order, kind, mod_scale, mod_shift, eps, norm_weight, fused_add,
+//        gate, residual, workspace): kind, an i8f_prologue, names what is applied to x inside the quantiser; workspace(x, M, N,
+// K) gives the memory of the K split or None.  It is called once a W8A8 call has passed every check, never for 16 rows or
+// fewer or for a call that goes the general way, which asks for its own: the memory stays with the stream, or with the graph
+// that is being captured, together with the kernel that clears it.
+PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 17) return PyErr_Format(PyExc_TypeError, "linear takes 17 arguments, got %zd", n);
+    const at::Tensor *xt = tensor(a[0]);
+    if (!lib.bound || !xt || !xt->is_cuda()) Py_RETURN_NONE;
+    const at::Tensor &x = *xt;
+    const int dt = code_of(x.scalar_type());
+    const bool per_row = a[4] == Py_True, rotate = a[5] == Py_True;
+    int64_t M, K, ld;
+    Layer l;
+    if ((dt != I8F_BF16 && dt != I8F_F16) || !rows_of(x, M, K, ld) || !layer_of(a[1], a[2], a[3], per_row, x.device(), l)) Py_RETURN_NONE;
+    const Stream st(x.device());
+    if (!st.ok || (rotate && K % 128)) Py_RETURN_NONE;
+    if (M <= PyLong_AsLongLong(a[6])) {
+        if (PyLong_AsLong(a[8]) != I8F_PRO_NONE || a[14] != Py_None || a[15] != Py_None || K != l.K) Py_RETURN_NONE;
+        return small_m(x, M, K, ld, l, rotate, st.handle);
+    }
+    return w8a8(a, x, M, K, ld, &l, 1, st);
+}
+
+// fanout(the arguments of linear): weight, scale, bias and per_row are tuples with an entry for each layer; a list of outputs.
+// Not for 16 rows or fewer.
+PyObject *fanout(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    if (n != 17) return PyErr_Format(PyExc_TypeError, "fanout takes 17 arguments, got %zd", n);
+    const at::Tensor *xt = tensor(a[0]);
+    if (!lib.bound || !xt || !xt->is_cuda()) Py_RETURN_NONE;
+    const at::Tensor &x = *xt;
+    const int dt = code_of(x.scalar_type());
+    const Py_ssize_t count = PyTuple_Check(a[1]) ? PyTuple_GET_SIZE(a[1]) : 0;
+    int64_t M, K, ld;
+    if ((dt != I8F_BF16 && dt != I8F_F16) || count < 2 || count > MAX_FANOUT || x.dim() < 2 || !rows_of(x, M, K, ld)) Py_RETURN_NONE;
+    for (int i = 2; i <= 4; ++i)
+        if (!PyTuple_Check(a[i]) || PyTuple_GET_SIZE(a[i]) != count) Py_RETURN_NONE;
+    Layer l[MAX_FANOUT];
+    for (Py_ssize_t i = 0; i < count; ++i)
+        if (!layer_of(PyTuple_GET_ITEM(a[1], i), PyTuple_GET_ITEM(a[2], i), PyTuple_GET_ITEM(a[3], i), PyTuple_GET_ITEM(a[4], i) == Py_True, x.device(), l[i]))
+            Py_RETURN_NONE;
+    const Stream st(x.device());
+    if (!st.ok || (a[5] == Py_True && K % 128) || M <= PyLong_AsLongLong(a[6])) Py_RETURN_NONE;
+    return w8a8(a, x, M, K, ld, l, (int)count, st);
 }
 
 // vector_fanout(x, weights, scales, biases, per_row, rotate): tuples with one entry per layer -> list of outputs
@@ -429,17 +489,7 @@ PyObject *vector_fanout(PyObject *, PyObject *const *a, Py_ssize_t n) {
             done = !lib.i8f_linear_w8a16_small_m_grouped(g, (int)count, dt, l[0].mode, bias_code < 0 ? (int)I8F_BF16 : bias_code, st.handle);
     }
     if (!done) Py_RETURN_NONE;
-    PyObject *out = PyList_New(count);
-    if (!out) return nullptr;
-    for (Py_ssize_t i = 0; i < count; ++i) {
-        PyObject *o = THPVariable_Wrap(std::move(y[i]));
-        if (!o) {
-            Py_DECREF(out);
-            return nullptr;
-        }
-        PyList_SET_ITEM(out, i, o);
-    }
-    return out;
+    return list_of(y, count);
 }
 
 // No C++ exception leaves an entry point: an allocator that has nothing left, say, becomes the general path's to report.
@@ -461,6 +511,7 @@ PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"bind", bind, METH_O, "bind(path): load the kernels' library"},
     {"linear", (PyCFunction)(void (*)(void))guarded<linear>, METH_FASTCALL, "one quantised layer, or None"},
+    {"fanout", (PyCFunction)(void (*)(void))guarded<fanout>, METH_FASTCALL, "several quantised layers of the same tokens, or None"},
     {"linear_lora", (PyCFunction)(void (*)(void))guarded<linear_lora>, METH_FASTCALL, "one quantised layer with a dynamic LoRA, or None"},
     {"vector_fanout", (PyCFunction)(void (*)(void))guarded<vector_fanout>, METH_FASTCALL, "several small-batch layers, or None"},
     {nullptr, nullptr, 0, nullptr}};

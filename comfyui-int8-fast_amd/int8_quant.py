@@ -141,6 +141,26 @@ def forward_pair(layers, xs, gates=None, residuals=None):
                                                   xs[0].dtype, rotate=rot, gates=gates, residuals=residuals)
 
 
+def _fanout_native(layers, x, rotate, prologue, mod_scale, mod_shift, eps, norm_weight, fused_add):
+    """forward_fanout() without the interpreter's part of it, as Linear._forward_native; None for everything else.  (Three layers of
+    1536 columns on 300 tokens: 75 us a call on the general path, 23 here.)"""
+    weights, scales, biases = [], [], []
+    for lin in layers:
+        params, scale = lin._parameters, getattr(lin, "_weight_scale_scalar", None)
+        weight = params.get("weight")
+        if scale is None:
+            scale = lin._buffers.get("weight_scale")
+        if (not getattr(lin, "_is_quantized", False) or lin.comfy_cast_weights or lin.lora_A is not None or weight is None or scale is None or "bias" not in params
+                or len(lin.weight_function) > 0 or len(lin.bias_function) > 0 or bool(getattr(lin, "_use_quarot", False)) != rotate):
+            return None
+        weights.append(weight)
+        scales.append(scale)
+        biases.append(params["bias"])
+    work = _lib._splitk_workspace if weights[0].shape[-1] >= _lib.SPLITK_MIN_K else None
+    return _lib.host().fanout(x, tuple(weights), tuple(scales), tuple(biases), tuple(bool(lin._is_per_row) for lin in layers), rotate, SMALL_BATCH_ROWS,
+                              int8_fused_kernel.DEFAULT_EPILOGUE, prologue, mod_scale, mod_shift, eps, norm_weight, bool(fused_add), None, None, work)
+
+
 def forward_fanout(layers, x, prologue: int = _lib.PRO_NONE, mod_scale=None, mod_shift=None, eps: float = 1e-6, norm_weight=None,
                    fused_add: bool = False):
     """[layer(x) for layer in layers] for quantised layers that read the same activations (separate q, k and v projections,
@@ -180,6 +200,10 @@ def forward_fanout(layers, x, prologue: int = _lib.PRO_NONE, mod_scale=None, mod
                     ws = ws.reshape(-1)[:1]
             problems.append((x_in, lin.weight, ws, lin.bias))
         return [y.reshape(*x.shape[:-1], y.shape[-1]) for y in _lib.linear_w8a16_small_m_grouped(problems)]
+    if len(layers) >= 2 and not torch.compiler.is_compiling() and type(x) is Tensor and x.is_cuda and x.dim() >= 2:
+        outs = _fanout_native(layers, x, rot, prologue, mod_scale, mod_shift, eps, norm_weight, fused_add)
+        if outs is not None:
+            return outs
     ok = len(layers) >= 2 and not torch.compiler.is_compiling() and x.is_cuda and x.dim() >= 2 \
         and x.numel() // max(1, x.shape[-1]) > SMALL_BATCH_ROWS and x.dtype in (torch.float16, torch.bfloat16)
     for lin in layers:
@@ -213,7 +237,7 @@ def forward_fanout(layers, x, prologue: int = _lib.PRO_NONE, mod_scale=None, mod
     lead = x.shape[:-1]
     q, s = _lib.quant_rowwise(x.reshape(-1, x.shape[-1]), rotate=rot, prologue=prologue, mod_scale=mod_scale, mod_shift=mod_shift,
                               eps=eps, norm_weight=norm_weight, fused_add=fused_add)
-    outs = []
+    problems = []
     for lin in layers:
         ws = lin._get_weight_scale()
         if isinstance(ws, Tensor):
@@ -221,9 +245,10 @@ def forward_fanout(layers, x, prologue: int = _lib.PRO_NONE, mod_scale=None, mod
                 ws = ws.to(x.device, non_blocking=True)
             if not lin._is_per_row and ws.numel() != 1:
                 ws = ws.reshape(-1)[:1]
-        y = _lib.linear_w8a8(q, s, lin.weight, ws, lin.bias, x.dtype, int8_fused_kernel.DEFAULT_EPILOGUE)
-        outs.append(y.reshape(*lead, lin.weight.shape[0]))
-    return outs
+        problems.append((q, s, lin.weight, ws, lin.bias))
+    # Layers of one shape go out in one launch where the library finds that cheaper (8000 x 5120 into three of 5120 columns: 8 rounds of
+    # tiles for 9; 576 and 541 us, 3000 x 3584 into three 121 and 106 us).
+    return [y.reshape(*lead, y.shape[-1]) for y in _lib.linear_w8a8_grouped(problems, x.dtype, int8_fused_kernel.DEFAULT_EPILOGUE)]
 
 
 # --------------------------------------------------------------------------- LoRA delta reconstruction
