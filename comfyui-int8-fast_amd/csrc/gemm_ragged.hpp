@@ -45,25 +45,29 @@ __device__ __forceinline__ void finish_one(const GemmArgs &g, int acc, int m, in
 // LDS is double-buffered: one barrier per K-tile.  The accumulators go through LDS once more so that a wave stores whole
 // runs of a row, element by element: rows of N outputs start at any address.
 // TINY: K < 16, where a row has no 16 bytes to end it.
-// What bounds it: 333 x 1001 x 1160 (96 workgroups) 9 us, 3 of them the launch, the first loads and the epilogue, then 0.4 us
-// a K-tile for the chain from LDS write to product and half as much again for chunks that straddle lines; 4096 x 3071 x 3083
+// GROUPS of four waves take every GROUPS-th K-tile each, with stages of their own, and their sums meet in LDS in the epilogue:
+// integers, so that the order changes nothing.
+// What bounds it: 333 x 1001 x 1160 (96 workgroups) 7.5 us, 3 of them the launch, the first loads and the epilogue, then 0.9 us
+// a pair of K-tiles: the chain from LDS write to product, and half as much again for chunks that straddle lines.  One group, and
+// so ten links instead of five, takes 9.1 us, four groups 8.3 (17 x 1500 x 1500 7.9, 6.4 and 6.9; 500 x 1400 x 1400 9.8, 8.1 and 9.0); 4096 x 3071 x 3083
 // 90 us, the loads of the two workgroups of a CU.  Two things made it that: the loads of a K-tile are issued without a branch
 // or a use near them (the compiler put a wait for all loads in flight at each join: 11.8 and 110 us before), and the
 // epilogue's operands come first instead of last.  Two waves to a SIMD is what the registers have to leave room for: with one
 // the larger shape takes 119 us.
-template <int OUT, int BM, int BN, bool TINY>
-__global__ __launch_bounds__(256, 2) void gemm_i8_ragged_kernel(const GemmArgs g) {
+template <int OUT, int BM, int BN, bool TINY, int GROUPS = 1>
+__global__ __launch_bounds__((256 * GROUPS), (GROUPS < 2 ? 2 : GROUPS)) void gemm_i8_ragged_kernel(const GemmArgs g) {
     constexpr int AHEAD = 2;  // K-tiles in flight (4, 6 and 8 measured the same or slower)
     constexpr int BK = 128, MI = BM / 64, NJ = BN / 64;
     constexpr int XC = BM * 8 / 256, WC = BN * 8 / 256;  // 16-byte chunks per thread and K-tile
     constexpr int STAGE = (BM + BN) * BK;
     constexpr int PITCH = BN + 4;                         // ints per row of the output tile in LDS
-    constexpr int SMEM = 2 * STAGE > BM * PITCH * 4 ? 2 * STAGE : BM * PITCH * 4;
+    constexpr int SMEM_GROUP = 2 * STAGE > BM * PITCH * 4 ? 2 * STAGE : BM * PITCH * 4, SMEM = GROUPS * SMEM_GROUP;
     static_assert(SMEM + BM * 4 <= 160 * 1024 && 256 % BN == 0, "LDS; a thread keeps one column in the epilogue");
     __shared__ __attribute__((aligned(16))) char smem[SMEM];
     __shared__ float s_xs[BM];
 
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int tid = threadIdx.x & 255, lane = tid & 63;   // within the group of four waves
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1, l32 = lane & 31, lhalf = lane >> 5;
     const int tiles_m = (g.M + BM - 1) / BM;
@@ -81,7 +85,7 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_ragged_kernel(const GemmArgs g
             else if (g.bias_dtype == I8F_BF16) b = bf16_bits_to_f32(((const uint16_t *)g.bias)[nc]);
             else b = f16_bits_to_f32(((const uint16_t *)g.bias)[nc]);
         }
-        if (tid < BM) xs = g.xs[min(m0 + tid, g.M - 1)];
+        if ((int)threadIdx.x < BM) xs = g.xs[min(m0 + tid, g.M - 1)];
     }
 
     const int8_t *src[XC + WC];   // the rows of this thread's chunks; rows past the end repeat the last one (never stored)
@@ -140,9 +144,10 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_ragged_kernel(const GemmArgs g
         if (kt == KT - 1) cut_tail(r);
 #pragma unroll
         for (int t = 0; t < XC + WC; ++t) *(v4i *)(st + dst[t]) = r[t];
-        if constexpr (!TINY) fetch(kt + AHEAD, r);
+        if constexpr (!TINY) fetch(kt + AHEAD * GROUPS, r);
         // (a bare barrier: __syncthreads() would also wait for the loads of the next K-tiles)
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (GROUPS > 1 && kt >= KT) return;   // (the other groups' last K-tiles)
         // (the small tile has one product per wave and k-step: all of its fragments first, one LDS latency instead of four)
         constexpr int AT_ONCE = MI * NJ == 1 ? 4 : 1;
 #pragma unroll
@@ -168,21 +173,21 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_ragged_kernel(const GemmArgs g
     if (KT > 0) {
 #pragma unroll
         for (int u = 0; u < (TINY ? 1 : AHEAD); ++u) {
-            fetch(u, reg[u]);
+            fetch(u * GROUPS + group, reg[u]);
             __builtin_amdgcn_sched_barrier(0);  // (in the order in which they are waited for)
         }
     }
-    for (int kt = 0; kt < KT; kt += AHEAD) {
+    for (int kt = 0; kt < KT; kt += AHEAD * GROUPS) {
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) {
-            if (kt + u >= KT) break;
-            step(kt + u, reg[u], smem + (u & 1) * STAGE);
+            if (kt + u * GROUPS >= KT) break;
+            step(kt + u * GROUPS + group, reg[u], smem + group * SMEM_GROUP + (u & 1) * STAGE);
         }
     }
 
     __syncthreads();
-    int *const tile = (int *)smem;
-    if (tid < BM) s_xs[tid] = xs;
+    int *const tile = (int *)(smem + group * SMEM_GROUP);
+    if ((int)threadIdx.x < BM) s_xs[tid] = xs;
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -194,8 +199,13 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_ragged_kernel(const GemmArgs g
     __syncthreads();
     if (n >= g.N) return;
 #pragma unroll 8
-    for (int row = tid / BN; row < BM; row += 256 / BN) {
-        if (m0 + row < g.M) finish_one<OUT>(g, tile[row * PITCH + tid % BN], m0 + row, n, OUT == OUT_I32 ? 0.0f : s_xs[row], ws, b);
+    for (int row = (int)threadIdx.x / BN; row < BM; row += 256 * GROUPS / BN) {
+        if (m0 + row < g.M) {
+            int sum = 0;
+#pragma unroll
+            for (int o = 0; o < GROUPS; ++o) sum += ((const int *)(smem + o * SMEM_GROUP))[row * PITCH + tid % BN];
+            finish_one<OUT>(g, sum, m0 + row, n, OUT == OUT_I32 ? 0.0f : s_xs[row], ws, b);
+        }
     }
 }
 
@@ -208,6 +218,7 @@ int launch_ragged(const GemmArgs &g, hipStream_t st) {
     // 83); below that they leave CUs idle (1500 x 1500 x 1500, 144 tiles: 21.9 against 16.2).
     if (g.K < 16) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, true>), dim3((unsigned)t64), dim3(256), 0, st, g);
     else if (t128 >= 256) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 128, 128, false>), dim3((unsigned)t128), dim3(256), 0, st, g);
+    else if (t64 <= 256) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, false, 2>), dim3((unsigned)t64), dim3(512), 0, st, g);
     else hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, false>), dim3((unsigned)t64), dim3(256), 0, st, g);
     return check_launch();
 }
