@@ -730,7 +730,8 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (tid == 0) {
-            unsigned word = __hip_atomic_load(g.arrivals + tile, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), next;
+            // (what it finds if it is the last, for whom the way to memory and back counts; any other finds out what is there)
+            unsigned word = g.splitk_tag << 8 | (unsigned)(g.splits - 1), next;
             uint32_t before;
             do {
                 next = splitk_arrive(word, g.splitk_tag, (uint32_t)g.splits, &before);
@@ -740,22 +741,28 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
         }
         __syncthreads();
         if (s_arrived + 1 != (unsigned)g.splits) return;
-        for (int o = 0; o < g.splits; ++o) {
-            if (o == slice) continue;
-            const int *theirs = g.partials + ((int64_t)o * T + tile) * (BM * BN);
+        // (the others two at a time, so that eight loads are on their way together)
+        const int others = g.splits - 1;
+        auto other = [&](int i) { return g.partials + ((int64_t)(i + (i >= slice)) * T + tile) * (BM * BN); };
 #pragma unroll
-            for (int q0 = 0; q0 < QUADS; q0 += 4) {
-                v4i v[4];
-                const int *p0 = theirs + ((int64_t)q0 * C::NT + tid) * 4;
-                asm volatile("global_load_dwordx4 %0, %4, off sc1\n\tglobal_load_dwordx4 %1, %5, off sc1\n\t"
-                             "global_load_dwordx4 %2, %6, off sc1\n\tglobal_load_dwordx4 %3, %7, off sc1\n\ts_waitcnt vmcnt(0)"
-                             : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
-                             : "v"(p0), "v"(p0 + C::NT * 4), "v"(p0 + 2 * C::NT * 4), "v"(p0 + 3 * C::NT * 4)
+        for (int q0 = 0; q0 < QUADS; q0 += 4) {
+            const int at = (q0 * C::NT + tid) * 4;
+            for (int o = 0; o < others; o += 2) {
+                const bool two = o + 1 < others;
+                v4i v[8];
+                const int *p0 = other(o) + at, *p1 = other(two ? o + 1 : o) + at;
+                asm volatile("global_load_dwordx4 %0, %8, off sc1\n\tglobal_load_dwordx4 %1, %9, off sc1\n\t"
+                             "global_load_dwordx4 %2, %10, off sc1\n\tglobal_load_dwordx4 %3, %11, off sc1\n\t"
+                             "global_load_dwordx4 %4, %12, off sc1\n\tglobal_load_dwordx4 %5, %13, off sc1\n\t"
+                             "global_load_dwordx4 %6, %14, off sc1\n\tglobal_load_dwordx4 %7, %15, off sc1\n\ts_waitcnt vmcnt(0)"
+                             : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7])
+                             : "v"(p0), "v"(p0 + C::NT * 4), "v"(p0 + 2 * C::NT * 4), "v"(p0 + 3 * C::NT * 4),
+                               "v"(p1), "v"(p1 + C::NT * 4), "v"(p1 + 2 * C::NT * 4), "v"(p1 + 3 * C::NT * 4)
                              : "memory");
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                     const int qd = q0 + u, i = qd / (NJ * QPB), j = qd / QPB % NJ;
-                    quad_add(i, j, qd % QPB, v[u]);
+                    quad_add(i, j, qd % QPB, two ? v[u] + v[4 + u] : v[u]);
                 }
             }
         }
@@ -1256,13 +1263,16 @@ constexpr int64_t SPLITK_COUNTER_BYTES = 4096, SPLITK_WORKSPACE_BYTES = SPLITK_C
 
 // Few tiles and a long K: the tile's K range is dealt over `splits` workgroups, which exchange their sums through
 // memory (integer sums, so the result is the same).  It pays where it fills idle CUs and a slice still has a long
-// loop: measured with weights from HBM, 512 x 3072 x 12288 42 -> 34 us, 256 x 3072 x 12288 33 -> 26 us,
-// 64 x 3072 x 12288 33 -> 15 us, nothing at K = 6144.  A candidate costs what its busiest CU fetches,
-// (K / splits) (BM + BN), plus 7 splits BM BN for the exchange (fitted to those measurements); one round of
-// workgroups at most, slices of at least 2048.
+// loop: with weights from HBM 512 x 3072 x 12288 42 -> 35 us, 64 x 3072 x 12288 33 -> 16 us.  A candidate costs what its
+// busiest CU fetches, (K / splits) (BM + BN), plus 7 splits BM BN for the exchange (fitted to K >= 10240); one round of
+// workgroups at most, slices of at least 2048.  Below K = 10240 the price has to fall to 0.7 of the unsplit one: what it
+// promises less for gains nothing (ratio 0.73: 256 x 3072 x 9216 25.0 and 25.8 us; 0.97: 512 x 2048 x 4096 11.6 and 15.2), what
+// it promises more for does (0.68: 512 x 3072 x 9216 32.8 and 29.8; 0.36: 33 x 1024 x 8192 13.9 and 10.9).  From K = 6144 on a
+// whole linear pass is faster for it (128 x 1536 x 6144 15.3 -> 14.0 us, 33 x 1024 x 8192 16.3 -> 13.6); at 4096 and 5120 the
+// kernel gains 1.5 us and the host has as much more to do for the workspace (64 x 3072 x 4608 12.5 and 12.7).
 inline void choose_split(int64_t M, int64_t N, int64_t K, Tile &t, int &splits) {
     splits = 1;
-    if (K < 10240) return;
+    if (K < 6144) return;
     if (t != TILE_MID_DEEP && t != TILE_M96_DEEP && t != TILE_S64_DEEP && t != TILE_T64_DEEP) return;
     const int64_t CUS = 256;
     struct Cand { Tile tile; int bm, bn; };
@@ -1275,6 +1285,7 @@ inline void choose_split(int64_t M, int64_t N, int64_t K, Tile &t, int &splits) 
             if (best < 0 || cost < best) best = cost, splits = 1;  // (t stays)
         }
     }
+    if (K < 10240) best = best * 7 / 10;
     Tile keep = t;
     for (const Cand &c : cands) {
         const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);

@@ -325,7 +325,7 @@ int i8f_linear_w8a8_add(const int8_t *a, const float *a_scale, const int8_t *w, 
                         int order, void *stream);
 
 /*
- * i8f_linear_w8a8_add with a workspace, which lets outputs of few tiles and a long K (K >= 10240: a text
+ * i8f_linear_w8a8_add with a workspace, which lets outputs of few tiles and a long K (K >= 6144: a text
  * stream's down-projection, a decode-sized batch) deal the K range of a tile over several workgroups that
  * exchange their integer sums through the workspace.  Same arguments, same results bit for bit (integer
  * sums do not depend on their order); the same Triton launches as i8f_linear_w8a8 (int8_fused_kernel.py:216,
