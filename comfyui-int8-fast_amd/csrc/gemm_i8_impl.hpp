@@ -321,14 +321,23 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
     const int l32 = lane & 31, lhalf = lane >> 5;
 
     // ---- workgroup id -> output tile -------------------------------------------------
+    // (With a K split the range that is walked is the tiles of the first slice, then those of the second: an XCD has one slice or
+    // two and fetches those parts of X alone, which every XCD otherwise fetches whole.  us with operands from HBM, every slice of
+    // a tile on one XCD and this: 512 x 3072 x 12288 35.5 and 34.9, 256 x 28.0 and 27.4, 512 x 1024 x 8192 15.9 and 15.7.)
     int tile_m, tile_n;
+    [[maybe_unused]] int slice = 0, tile_no = 0;
     {
-        const int T = tiles_m * tiles_n;
-        const int bid = SPLITK ? __builtin_amdgcn_readfirstlane(wg_id % T) : wg_id;  // the K slices of a tile are T workgroup ids apart
+        const int T = SPLITK ? tiles_m * tiles_n * g.splits : tiles_m * tiles_n;
         const int per = (T + 7) / 8;
         const int tall = (T % 8 == 0) ? 8 : (T % 8);
-        const int xcd = bid % 8, loc = bid / 8;
-        const int L = xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
+        const int xcd = wg_id % 8, loc = wg_id / 8;
+        int L = xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
+        if constexpr (SPLITK) {
+            // (integer division runs on the vector ALUs: readfirstlane brings the quotients back to scalar registers, where the
+            // K offset of the loads has to be)
+            slice = __builtin_amdgcn_readfirstlane(L / (tiles_m * tiles_n));
+            tile_no = L = __builtin_amdgcn_readfirstlane(L % (tiles_m * tiles_n));
+        }
         const int in_group = C::GROUP_M * tiles_n;
         const int grp = L / in_group;
         const int first_m = grp * C::GROUP_M;
@@ -371,9 +380,6 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
 
     // SPLITK: this workgroup multiplies k-tiles [kt_first, kt_first + KT) of its output tile only
     const int KT_all = (K + BK - 1) / BK;
-    // (integer division runs on the vector ALUs: readfirstlane brings the quotients back to scalar registers, where the
-    // K offset of the loads has to be)
-    [[maybe_unused]] const int slice = SPLITK ? __builtin_amdgcn_readfirstlane(wg_id / (tiles_m * tiles_n)) : 0;
     const int kt_per = SPLITK ? __builtin_amdgcn_readfirstlane((KT_all + g.splits - 1) / g.splits) : KT_all;
     const int kt_first = slice * kt_per;
     const int KT = SPLITK ? max(min(kt_per, KT_all - kt_first), 0) : KT_all;
@@ -714,7 +720,7 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
         // agree, and the count is taken once this workgroup's stores are acknowledged: no cache-wide write-back or
         // invalidate, which a release/acquire fence pair at agent scope would cost every workgroup on the XCD.
         __shared__ unsigned s_arrived;
-        const int T = tiles_m * tiles_n, tile = __builtin_amdgcn_readfirstlane(wg_id % T);
+        const int T = tiles_m * tiles_n, tile = tile_no;
         constexpr int QUADS = MI * NJ * QPB;
         static_assert(QUADS % 4 == 0, "the partial sums are read back four quads at a time");
         int *mine = g.partials + ((int64_t)slice * T + tile) * (BM * BN);
