@@ -168,6 +168,21 @@ __device__ __forceinline__ v4i make_rsrc(const void *p, uint32_t bytes) {
     return r;
 }
 
+// `bytes` of a tensor from byte `at` on as a buffer, empty without a tensor.  Pieces of an [M,N] tensor past its last row load zeros
+// and are not stored, so a lane's offset is a 32-bit number that its column fixes (OUT_OF_ROW past the last one; at most 16 rows of
+// less than 2^28 bytes below it), and the rows move on in the descriptor, by scalar instructions.
+constexpr uint32_t OUT_OF_ROW = 0xfffffff0u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_at(const void *p, int64_t at, int64_t bytes) {
+    const uint32_t records = !p || bytes <= 0 ? 0u : bytes < 0xffffff00ll ? (uint32_t)bytes : 0xffffff00u;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>((const char *)p + at), 0, records, 0x00020000);
+}
+__device__ __forceinline__ uint4 buffer_load16(__amdgpu_buffer_rsrc_t r, uint32_t at) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, 0, 0));
+}
+__device__ __forceinline__ void buffer_store16(uint4 v, __amdgpu_buffer_rsrc_t r, uint32_t at) {   // (non-temporal)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u_t, v), r, (int)at, 0, 2);
+}
+
 template <int OUT>
 struct OutElem {
     static constexpr int BYTES = (OUT == OUT_BF16 || OUT == OUT_F16) ? 2 : 4;
@@ -876,8 +891,64 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
 #pragma unroll
             for (int j = 0; j < NJ; ++j) fetch_cols(j, wr[j], br[j]);
         }
+        // A pass of the wave stores 64 pieces of 16 bytes of the staged strips; after PERIOD passes (GROUP_ROWS rows) a lane's pieces
+        // lie in the same columns again.
+        constexpr int CPO = ROW_BYTES / 16;      // pieces per output row
+        constexpr int EPCO = 16 / OB;            // output elements per piece
+        constexpr int PASSES = EPI_STRIPS * 32 * CPO / 64;
+        constexpr int PERIOD = CPO / std::gcd(64, CPO), GROUP_ROWS = 64 * PERIOD / CPO;
+        static_assert(PASSES % PERIOD == 0, "whole groups of rows");
+        const int64_t row_bytes = (int64_t)gN * OB;
+        const int nw = n0 + wn * C::WTN;         // the wave's first column
+        uint32_t at[PERIOD];                     // of a piece from the group's first row on, in the output and in what is staged
+        int st_at[PERIOD];
+#pragma unroll
+        for (int q = 0; q < PERIOD; ++q) {
+            const int id = q * 64 + lane, row = id / CPO, cc = id % CPO;
+            at[q] = nw + cc * EPCO < gN ? (uint32_t)row * (uint32_t)row_bytes + (uint32_t)(cc * 16) : OUT_OF_ROW;
+            st_at[q] = row * PITCH + cc * 16;
+        }
 #pragma unroll
         for (int i0 = 0; i0 < MI; i0 += EPI_STRIPS) {
+            const int mw = m0 + wm * C::WTM + i0 * 32;   // first row of the strips staged together
+            const int64_t strip_at = mw * row_bytes + nw * OB, strip_bytes = (gM - mw) * row_bytes - nw * OB;
+            auto rows_of = [&](const void *p, int pass) {
+                const int64_t down = pass / PERIOD * GROUP_ROWS * row_bytes;
+                return buffer_at(p, strip_at + down, strip_bytes - down);
+            };
+            auto staged = [&](int pass) { return *(const uint4 *)(ebuf + st_at[pass % PERIOD] + pass / PERIOD * GROUP_ROWS * PITCH); };
+            // Gate and addend: BATCH pieces of the addend are requested in front of the conversion, whose 700 instructions they arrive
+            // under, and the next batch before one is used (a load behind each store, above which it may not be moved, would be a
+            // trip to memory for every piece; twelve waves have no registers for it: 4096 x 9216 x 3072 in 256 x 288 tiles 136 and 141
+            // us).  Where one gate serves all rows of the wave its pieces are PERIOD, fetched once.  An absent one is 1 or -0, which change
+            // nothing, so that no branch stands between a request and its use: with branches the first piece waited for every
+            // request, and a piece took 68 vector instructions where it takes 50.  us, operands from HBM, gate and addend, with
+            // branches, 64-bit addresses and requests behind the conversion and as it is here: 4608 x 3072 x 3072 48.5 and 46.7,
+            // 8192 x 4096 x 4096 121.8 and 117.0, 4096 x 3840 x 3840 58.0 and 56.0, 512 x 3072 x 12288 36.7 and 35.5.
+            // GATED is chosen with the variant, so that an epilogue without gate and addend stays contiguous: with a jump over their
+            // code the smallest outputs took 2 to 3 % longer (93 x 3200 x 3200 8.6 for 8.4 us).  That one keeps its guarded stores: by
+            // way of buffers 4096 x 9216 x 3072 took 100.3 for 98.6 us, and nothing was faster.
+            constexpr int BATCH = PASSES <= 8 ? PASSES : PASSES % 8 == 0 ? 8 : 4;
+            static_assert(PASSES % BATCH == 0, "whole batches");
+            constexpr uint32_t ONE = OUT == OUT_F32 ? 0x3f800000u : OUT == OUT_BF16 ? 0x3f803f80u : 0x3c003c00u;
+            constexpr uint32_t MINUS_ZERO = OUT == OUT_F32 ? 0x80000000u : 0x80008000u;
+            [[maybe_unused]] const uint32_t no_gate = ggate ? 0u : ONE, no_addend = gaddend ? 0u : MINUS_ZERO;
+            auto or4 = [](uint4 v, uint32_t bits) { return make_uint4(v.x | bits, v.y | bits, v.z | bits, v.w | bits); };
+            [[maybe_unused]] uint4 gate_r[PERIOD], add_r[2][BATCH];
+            [[maybe_unused]] auto fetch_addend = [&](int p0, int to) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < BATCH; ++u) add_r[to][u] = buffer_load16(rows_of(gaddend, p0 + u), at[(p0 + u) % PERIOD]);
+            };
+            [[maybe_unused]] bool one_gate = true;
+            if constexpr (decltype(GATED)::value) {
+                const int first_gate = ggate ? (int)((uint32_t)min(mw, gM - 1) / (uint32_t)ggate_rows) : 0;
+                one_gate = !ggate || first_gate == (int)((uint32_t)min(mw + EPI_STRIPS * 32 - 1, gM - 1) / (uint32_t)ggate_rows);
+                const auto gate = buffer_at(ggate, first_gate * row_bytes + nw * OB, row_bytes - nw * OB);
+#pragma unroll
+                for (int q = 0; q < PERIOD; ++q)
+                    gate_r[q] = buffer_load16(gate, (uint32_t)((q * 64 + lane) % CPO * 16));
+                fetch_addend(0, 0);
+            }
 #pragma unroll
             for (int is = 0; is < EPI_STRIPS; ++is) {
                 const int i = i0 + is;
@@ -972,16 +1043,6 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
             }
             __builtin_amdgcn_wave_barrier();
             // read the staged rows back row-contiguously and store 16 bytes per lane
-            constexpr int CPO = ROW_BYTES / 16;      // chunks per output row
-            constexpr int EPCO = 16 / OB;            // output elements per chunk
-            constexpr int PASSES = EPI_STRIPS * 32 * CPO / 64;
-            const int mw = m0 + wm * C::WTM + i0 * 32, nw = n0 + wn * C::WTN;   // first row and column of the staged strips
-            // Gate and addend of BATCH pieces are requested together, and those of the next batch before this one is used: a load
-            // behind each store, above which it may not be moved, is a trip to memory for every piece (35 to 54 K cycles of
-            // epilogue at 4608 x 3072, 9.6 K without gate and addend; 512 x 3072 x 12288 in 128 x 96 tiles and two slices 38.6 us,
-            // 37.0 in fours).  Twelve waves have no registers for it (4096 x 9216 x 3072 in 256 x 288
-            // tiles 136 and 141 us).  GATED is chosen with the variant, so that an epilogue without gate and addend stays
-            // contiguous: with a jump over their code the smallest outputs took 2 to 3 % longer (93 x 3200 x 3200 8.6 for 8.4 us).
             if constexpr (!decltype(GATED)::value) {
 #pragma unroll
                 for (int p = 0; p < PASSES; ++p) {
@@ -1001,49 +1062,25 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
                     }
                 }
             } else {
-                // After PERIOD passes a lane's pieces lie in the same columns again: where one gate serves all rows of the wave, its
-                // pieces are these few, fetched once.  (Fetched beside every addend's they were half of the requests, of which a CU
-                // has 64 in flight.  us, operands from HBM, gate and addend: 4608 x 3072 x 3072 50.5 and 44.0, x 12288 147 and 139.4,
-                // 9729 x 3072 x 15360 352 and 341; without gate and addend 39, 136, 336.)
-                constexpr int PERIOD = CPO / std::gcd(64, CPO);
-                const bool one_gate = !ggate || (uint32_t)mw / (uint32_t)ggate_rows == (uint32_t)min(mw + EPI_STRIPS * 32 - 1, gM - 1) / (uint32_t)ggate_rows;
-                const int first_gate = ggate ? (int)((uint32_t)mw / (uint32_t)ggate_rows) : 0;
                 auto passes = [&](auto ONE_GATE) __attribute__((always_inline)) {
-                    constexpr bool ONCE = decltype(ONE_GATE)::value && PERIOD < PASSES;
-                    constexpr int BATCH = PASSES <= 8 ? PASSES : ONCE && PASSES % 8 == 0 ? 8 : 4;
-                    static_assert(PASSES % BATCH == 0, "whole batches");
-                    uint4 gate_r[ONCE ? 1 : 2][ONCE ? PERIOD : BATCH], add_r[2][BATCH];
-                    auto gate_piece = [&](int gv, int nn) { return *(const uint4 *)((const char *)ggate + ((int64_t)gv * gN + nn) * OB); };
-                    auto fetch = [&](int p0, int at) __attribute__((always_inline)) {
-#pragma unroll
-                        for (int u = 0; u < BATCH; ++u) {   // (rows and columns beyond the output repeat the last ones, unused)
-                            const int id = (p0 + u) * 64 + lane;
-                            const int mm = min(mw + id / CPO, gM - 1), nn = min(nw + id % CPO * EPCO, gN - EPCO);
-                            if (gaddend) add_r[at][u] = *(const uint4 *)((const char *)gaddend + ((int64_t)mm * gN + nn) * OB);
-                            if constexpr (!ONCE) {
-                                if (ggate) gate_r[at][u] = gate_piece(decltype(ONE_GATE)::value ? first_gate : (int)((uint32_t)mm / (uint32_t)ggate_rows), nn);
-                            }
-                        }
-                    };
-                    if constexpr (ONCE) {
-#pragma unroll
-                        for (int u = 0; u < PERIOD; ++u)
-                            if (ggate) gate_r[0][u] = gate_piece(first_gate, min(nw + (u * 64 + lane) % CPO * EPCO, gN - EPCO));
-                    }
-                    fetch(0, 0);
 #pragma unroll
                     for (int p0 = 0; p0 < PASSES; p0 += BATCH) {
                         const int now = p0 / BATCH % 2;
-                        if (p0 + BATCH < PASSES) fetch(p0 + BATCH, now ^ 1);
+                        if (p0 + BATCH < PASSES) fetch_addend(p0 + BATCH, now ^ 1);
+                        [[maybe_unused]] uint4 own[decltype(ONE_GATE)::value ? 1 : BATCH];
+                        if constexpr (!decltype(ONE_GATE)::value) {
+#pragma unroll
+                            for (int u = 0; u < BATCH; ++u) {   // (rows and columns beyond the output repeat the last ones, unused)
+                                const int id = (p0 + u) * 64 + lane, mm = min(mw + id / CPO, gM - 1), nn = min(nw + id % CPO * EPCO, gN - EPCO);
+                                own[u] = *(const uint4 *)((const char *)ggate + ((int64_t)((uint32_t)mm / (uint32_t)ggate_rows) * gN + nn) * OB);
+                            }
+                        }
 #pragma unroll
                         for (int u = 0; u < BATCH; ++u) {
-                            const int id = (p0 + u) * 64 + lane;
-                            const int row = id / CPO, cc = id % CPO;
-                            uint4 v = *(const uint4 *)(ebuf + row * PITCH + cc * 16);
-                            const int mm = mw + row, nn = nw + cc * EPCO;
-                            if (ggate) v = mul_rounded<OUT>(v, ONCE ? gate_r[0][(p0 + u) % PERIOD] : gate_r[now][ONCE ? 0 : u]);
-                            if (gaddend) v = add_rounded<OUT>(v, add_r[now][u]);
-                            if (mm < gM && nn < gN) stream_store16((char *)gout + ((int64_t)mm * gN + nn) * OB, v);
+                            const int p = p0 + u;
+                            uint4 v = mul_rounded<OUT>(staged(p), or4(decltype(ONE_GATE)::value ? gate_r[p % PERIOD] : own[u], no_gate));
+                            v = add_rounded<OUT>(v, or4(add_r[now][u], no_addend));
+                            buffer_store16(v, rows_of(gout, p), at[p % PERIOD]);
                         }
                     }
                 };

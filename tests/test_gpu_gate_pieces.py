@@ -20,3 +20,38 @@ def test_gated_residual_equals_the_tensor_operations(L, dev, M, N, K, rows_per_g
     plain = L.linear_w8a8(x, scale, w, ws, None, dtype, L.EPI_TORCH)
     got = L.linear_w8a8(x, scale, w, ws, None, dtype, L.EPI_TORCH, addend=residual, gate=gate)
     assert torch.equal(got, residual + gate.repeat_interleave(rows_per_gate, 0) * plain)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,rows_per_gate,dtype", [
+    (4600, 3064, 128, 4600, torch.bfloat16), (4600, 3064, 128, 46, torch.float16),   # 256 x 256
+    (4000, 3064, 256, 4000, torch.float16), (600, 1000, 128, 200, torch.float32), (17, 40, 128, 1, torch.bfloat16),
+    (510, 3064, 12288, 85, torch.bfloat16),                                          # 128 x 96, K split
+])
+@pytest.mark.parametrize("absent", ["gate", "residual", "neither"])
+def test_absent_operands_signed_zeros_infinities_and_the_residual_as_output(L, dev, M, N, K, rows_per_gate, dtype, absent):
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x, scale = L.quant_rowwise(torch.randn(M, K, generator=g, device=dev))
+    w, ws = L.quant_rowwise(torch.randn(N, K, generator=g, device=dev) * 0.02)
+    x[::5] = 0                                       # rows of zeros, negative ones where the weight's scale is negative
+    ws[::3] *= -1
+    scale[1::16] = float("inf")
+    gate = torch.randn(M // rows_per_gate, N, generator=g, device=dev).to(dtype)
+    residual = torch.randn(M, N, generator=g, device=dev).to(dtype)
+    residual[::2, ::7], gate[:, ::11] = -0.0, 0.0
+    plain = L.linear_w8a8(x, scale, w, ws, None, dtype, L.EPI_TORCH)
+    want, rows = plain, gate.repeat_interleave(rows_per_gate, 0)
+    if absent != "gate":
+        want = rows * want
+    if absent != "residual":
+        want = residual + want
+    guard = torch.full((M + 64, N), 7.0, dtype=dtype, device=dev)
+    out = guard[:M]
+    out.copy_(residual)
+    L.linear_w8a8(x, scale, w, ws, None, dtype, L.EPI_TORCH, addend=None if absent == "residual" else out,
+                  gate=None if absent == "gate" else gate, out=out)
+    whole = torch.int32 if dtype == torch.float32 else torch.int16
+    nan = want.isnan()
+    assert torch.equal(out.isnan(), nan)
+    assert torch.equal(out.view(whole)[~nan], want.view(whole)[~nan])
+    assert bool((guard[M:] == 7.0).all())
