@@ -540,8 +540,9 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
     // Two ways to keep the stages full.  With two stages a stage is refilled right after the barrier
     // that frees it (tile kt+S from the last phase of iteration kt on), in one burst or, by the SPLIT
     // of the configuration, over that phase and the following ones of iteration kt+1.  With three
-    // or more the refill of the stage freed by the PREVIOUS iteration is dealt out over the whole of
-    // iteration kt (tile kt+S-1): a wave that issues many loads at once blocks on the load queue, and
+    // or more the refill of the stage freed by the PREVIOUS iteration is dealt out over
+    // iteration kt (tile kt+S-1) up to its barrier (over the whole of it, the last loads had less time to land: us with
+    // operands from HBM 512 x 12288 x 3072 26.7 and 26.0, 400 x 9216 x 3072 24.3 and 23.8, 300 x 3072 x 3072 9.1 and 8.8): a wave that issues many loads at once blocks on the load queue, and
     // while it is blocked it issues no MFMAs either.  Loads past the last tile are issued all the
     // same (they move nothing), so the number of loads in flight at any point is a constant.
     constexpr bool SPREAD_DMA = S >= 3;
@@ -641,9 +642,9 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
             const bool last = ks == KS - 1;
             if (last) {
                 // my part of tile kt+1 has landed and my LDS reads of tile kt have returned; what may
-                // still be in flight are the younger tiles (and, spread, the part of the newest one
-                // that the earlier phases of this iteration have issued)
-                constexpr int YOUNGER = SPREAD_DMA ? (S - 3) * C::LOADS + (KS - 1) * C::LOADS / KS : (ASYM ? C::W_LOADS : 0);
+                // still be in flight are the younger tiles (the newest of which, where loads are dealt
+                // out, the earlier phases of this iteration have issued)
+                constexpr int YOUNGER = SPREAD_DMA ? (S - 2) * C::LOADS : (ASYM ? C::W_LOADS : 0);
                 __builtin_amdgcn_s_waitcnt(waitcnt_vm(YOUNGER) & 0xF0FF);
                 __builtin_amdgcn_s_barrier();
             }
@@ -680,8 +681,8 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
             const int ftx = kt + S - (behind ? 0 : 1), ftw = kt + WS - (behind ? 0 : 1);
             const int fsx = behind ? ix : ixp, fsw = behind ? iw : iwp;
             // this phase's share of its loads
-            const int la = SPREAD_DMA ? ks * C::LOADS / KS : (last ? 0 : cut(ks + 1));
-            const int lb = SPREAD_DMA ? (ks + 1) * C::LOADS / KS : (last ? cut(1) : cut(ks + 2));
+            const int la = SPREAD_DMA ? (last ? C::LOADS : ks * C::LOADS / (KS - 1)) : (last ? 0 : cut(ks + 1));
+            const int lb = SPREAD_DMA ? (last ? C::LOADS : (ks + 1) * C::LOADS / (KS - 1)) : (last ? cut(1) : cut(ks + 2));
             [[maybe_unused]] int frag = 0;  // row fragments of the next phase requested so far
 #pragma unroll
             for (int r = 0; r < MN; ++r) {
