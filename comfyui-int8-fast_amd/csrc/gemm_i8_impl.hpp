@@ -250,9 +250,7 @@ __device__ __forceinline__ uint4 add_rounded(uint4 y, uint4 s) {
                 const float hi = bf16_bits_to_f32(yv[e] >> 16) + bf16_bits_to_f32(sv[e] >> 16);
                 o[e] = f32x2_to_bf16x2_bits(lo, hi);
             } else {
-                const float lo = f16_bits_to_f32(yv[e] & 0xffffu) + f16_bits_to_f32(sv[e] & 0xffffu);
-                const float hi = f16_bits_to_f32(yv[e] >> 16) + f16_bits_to_f32(sv[e] >> 16);
-                o[e] = f32x2_to_f16x2_bits(lo, hi);
+                o[e] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, yv[e]) + __builtin_bit_cast(half2v, sv[e]));
             }
         }
         return make_uint4(o[0], o[1], o[2], o[3]);
@@ -280,9 +278,7 @@ __device__ __forceinline__ uint4 mul_rounded(uint4 y, uint4 s) {
                 const float hi = bf16_bits_to_f32(yv[e] >> 16) * bf16_bits_to_f32(sv[e] >> 16);
                 o[e] = f32x2_to_bf16x2_bits(lo, hi);
             } else {
-                const float lo = f16_bits_to_f32(yv[e] & 0xffffu) * f16_bits_to_f32(sv[e] & 0xffffu);
-                const float hi = f16_bits_to_f32(yv[e] >> 16) * f16_bits_to_f32(sv[e] >> 16);
-                o[e] = f32x2_to_f16x2_bits(lo, hi);
+                o[e] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, yv[e]) * __builtin_bit_cast(half2v, sv[e]));
             }
         }
         return make_uint4(o[0], o[1], o[2], o[3]);

@@ -75,10 +75,6 @@ __device__ __forceinline__ uint32_t f32_to_f16_bits(float v) {
     asm("" : "+v"(v));
     return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v);
 }
-__device__ __forceinline__ uint32_t f32x2_to_f16x2_bits(float lo, float hi) {
-    return f32_to_f16_bits(lo) | (f32_to_f16_bits(hi) << 16);
-}
-
 // two values of one binary16 dword: arithmetic on them is packed, each result rounded once, as the same operation in binary32
 // rounded afterwards is (a product of two is exact there, a sum's second rounding does not show: 24 >= 2 * 11 + 2 bits)
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
@@ -86,6 +82,10 @@ __device__ __forceinline__ half2v f32x2_to_half2(float lo, float hi) {
     typedef float f2 __attribute__((ext_vector_type(2)));
     asm("" : "+v"(lo), "+v"(hi));  // (as in f32_to_f16_bits)
     return __builtin_convertvector((f2){lo, hi}, half2v);
+}
+// (one conversion of two values: two conversions, a shift and an or are four instructions)
+__device__ __forceinline__ uint32_t f32x2_to_f16x2_bits(float lo, float hi) {
+    return __builtin_bit_cast(uint32_t, f32x2_to_half2(lo, hi));
 }
 
 // value rounded to the storage dtype and widened again

@@ -145,7 +145,7 @@ __device__ __forceinline__ uint32_t dequant_pair(uint32_t word, int e, float ws)
     const float a = (float)(int)(int8_t)(word >> (8 * e)) * ws;
     const float b = (float)(int)(int8_t)(word >> (8 * e + 8)) * ws;
     if constexpr (DT == I8F_BF16) return f32x2_to_bf16x2_bits(a, b);
-    else return f32_to_f16_bits(a) | (f32_to_f16_bits(b) << 16);
+    else return f32x2_to_f16x2_bits(a, b);
 }
 
 template <int DT>

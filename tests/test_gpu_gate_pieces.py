@@ -39,6 +39,9 @@ def test_absent_operands_signed_zeros_infinities_and_the_residual_as_output(L, d
     gate = torch.randn(M // rows_per_gate, N, generator=g, device=dev).to(dtype)
     residual = torch.randn(M, N, generator=g, device=dev).to(dtype)
     residual[::2, ::7], gate[:, ::11] = -0.0, 0.0
+    gate[:, 1::13] *= 1e-4                            # products below binary16's normal numbers, with a residual that keeps them
+    residual[1::2, 1::13] = 0.0
+    scale[2::4] *= 1e-2
     plain = L.linear_w8a8(x, scale, w, ws, None, dtype, L.EPI_TORCH)
     want, rows = plain, gate.repeat_interleave(rows_per_gate, 0)
     if absent != "gate":
