@@ -194,6 +194,8 @@ template <int OUT, int ORDER, bool ROW, bool BIAS, bool SIDE = false>
 __device__ __forceinline__ void epilogue_quad(const int (&a4)[4], float xs, const float4 w4, const float4 b4,
                                               char *dst, const float *side4 = nullptr) {
     constexpr int DT = OUT == OUT_BF16 ? I8F_BF16 : (OUT == OUT_F16 ? I8F_F16 : I8F_F32);
+    // binary16: what is added to the rounded product is added in packed operations, which round as the widened ones do
+    constexpr bool HALF = OUT == OUT_F16 && ORDER == I8F_EPI_TORCH;
     const float wsv[4] = {w4.x, w4.y, w4.z, w4.w};
     const float bv[4] = {b4.x, b4.y, b4.z, b4.w};
     float y[4];
@@ -209,16 +211,28 @@ __device__ __forceinline__ void epilogue_quad(const int (&a4)[4], float xs, cons
                 const float sc = wsv[e] * xs;
                 t = a * sc;
             }
-            t = round_to_dtype<DT>(t);
-            if constexpr (BIAS) t = t + round_to_dtype<DT>(bv[e]);
+            if constexpr (!HALF) {
+                t = round_to_dtype<DT>(t);
+                if constexpr (BIAS) t = t + round_to_dtype<DT>(bv[e]);
+            }
         } else {
             const float sc = xs * wsv[e];
             t = a * sc;
             if constexpr (BIAS) t = t + bv[e];
         }
         // the side branch is added to the ROUNDED result, as a tensor addition would (y + side.to(y.dtype))
-        if constexpr (SIDE) t = round_to_dtype<DT>(t) + side4[e];
+        if constexpr (SIDE && !HALF) t = round_to_dtype<DT>(t) + side4[e];
         y[e] = t;
+    }
+    if constexpr (HALF) {
+        half2v o[2] = {f32x2_to_half2(y[0], y[1]), f32x2_to_half2(y[2], y[3])};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if constexpr (BIAS) o[h] = o[h] + f32x2_to_half2(bv[2 * h], bv[2 * h + 1]);
+            if constexpr (SIDE) o[h] = o[h] + f32x2_to_half2(side4[2 * h], side4[2 * h + 1]);   // (values of binary16)
+        }
+        *(uint2 *)dst = make_uint2(__builtin_bit_cast(uint32_t, o[0]), __builtin_bit_cast(uint32_t, o[1]));
+        return;
     }
     if constexpr (OUT == OUT_BF16) {
         *(uint2 *)dst = make_uint2(f32x2_to_bf16x2_bits(y[0], y[1]), f32x2_to_bf16x2_bits(y[2], y[3]));
