@@ -350,18 +350,24 @@ int launch_lds(const SmallMArgs &a, hipStream_t st) {
     return check_launch();
 }
 
-// 16-column blocks of a workgroup.  What counts is the blocks of the busiest CU and then how often it fetches the activations,
-// once for each of its workgroups: one block while every CU gets one at most, then two or three while that is one workgroup to a
-// CU, and two again beyond (three keep 146 registers, so that no second workgroup fits beside them: 18432 x 3072, one row, 15.1 us
-// in twos, 17.4 in threes).  A short K leaves a wave one or two steps, and then several workgroups to a CU hide each other's ends: the
-// larger form needs a K, or rows whose fetches weigh more.  us with weights from HBM, 1 and 16 rows: 6144 x 3072 ones 7.5 and 10.5, twos
-// 7.2 and 8.8; 8192 x 1536 5.5 and 7.1, 5.9 and 7.0; 8192 x 5120 11.2 and 16.9, 11.1 and 13.6; 9216 x 3072 twos 10.8 and 14.4, threes
-// 9.7 and 11.6; 12288 x 1536 7.3 and 9.3, 7.8 and 9.0; 12288 x 3072 11.3 and 14.7, 10.7 and 12.6; 12288 x 5120 16.6 and 22.6, 15.1 and
-// 17.6.  The sums are the same in every form.
-int blocks_to_workgroup(int64_t blocks, int64_t M, int64_t K) {
-    if (blocks <= 256) return 1;
-    if (blocks <= 512) return K >= 2560 || M > 6 ? 2 : 1;
-    return blocks <= 768 && (K >= 2304 || M > 8) ? 3 : 2;
+// 16-column blocks of a workgroup, for the layers of one launch.  What counts is the blocks of the busiest CU and then how often it
+// fetches the activations, once for each of its workgroups: one block while every CU gets one at most, then two or three while that is
+// one workgroup to a CU, and two again beyond (three keep 146 registers, so that no second workgroup fits beside them: 18432 x 3072,
+// one row, 15.1 us in twos, 17.4 in threes; three layers of 4096 columns, whose threes are 258 workgroups, 11.7 and 17.0).  A short K
+// leaves a wave one or two steps, and then several workgroups to a CU hide each other's ends: the larger form needs a K, or rows whose
+// fetches weigh more.  us with weights from HBM, 1 and 16 rows: 6144 x 3072 ones 7.5 and 10.5, twos 7.2 and 8.8; 8192 x 1536 5.5 and
+// 7.1, 5.9 and 7.0; 8192 x 5120 11.2 and 16.9, 11.1 and 13.6; 9216 x 3072 twos 10.8 and 14.4, threes 9.7 and 11.6; 12288 x 1536 7.3 and
+// 9.3, 7.8 and 9.0; 12288 x 3072 11.3 and 14.7, 10.7 and 12.6; 12288 x 5120 16.6 and 22.6, 15.1 and 17.6.  8 rows: twice 3952 x 1664
+// ones 6.9, twos 7.2; 6144 x 2048 6.8 and 6.4.  The sums are the same in every form.
+int blocks_to_workgroup(const SmallMArgs *as, int n) {
+    int64_t workgroups[4] = {}, M = 0, K = as[0].K;
+    for (int i = 0; i < n; ++i) {
+        for (int form = 1; form <= 3; ++form) workgroups[form] += (as[i].N + 16 * form - 1) / (16 * form);
+        M = as[i].M > M ? as[i].M : M, K = as[i].K < K ? as[i].K : K;
+    }
+    if (workgroups[1] <= 256) return 1;
+    if (workgroups[2] <= 256) return K >= 2560 || M * K >= 7 * 2048 ? 2 : 1;
+    return workgroups[3] <= 256 && (K >= 2304 || M > 8) ? 3 : 2;
 }
 
 template <int DT>
@@ -372,7 +378,7 @@ int launch(const SmallMArgs &a, hipStream_t st) {
         if (vec && a.K < (1ll << 30)) {
             // (Workgroups of 4 waves, which are all resident at once where 8-wave ones spill into a thin second round --
             // 18432 columns are 576 workgroups on 512 places -- measured no faster: 13.9 against 13.5 us.)
-            switch (blocks_to_workgroup((a.N + 15) / 16, a.M, a.K)) {
+            switch (blocks_to_workgroup(&a, 1)) {
             case 1: return launch_lds<DT, 1, 8>(a, st);
             case 2: return launch_lds<DT, 2, 8>(a, st);
             default: return launch_lds<DT, 3, 8>(a, st);
@@ -390,9 +396,7 @@ template <int DT>
 int launch_grouped(const SmallMArgs *as, int n, hipStream_t st) {
     SmallMGroups gg{};
     gg.n = n;
-    int64_t blocks = 0, rows = 0, narrowest = as[0].K;
-    for (int i = 0; i < n; ++i) blocks += (as[i].N + 15) / 16, rows = as[i].M > rows ? as[i].M : rows, narrowest = as[i].K < narrowest ? as[i].K : narrowest;
-    const int together = blocks_to_workgroup(blocks, rows, narrowest);   // as for one layer
+    const int together = blocks_to_workgroup(as, n);
     const int64_t cols = 16 * together;
     int64_t first = 0;
     for (int i = 0; i < n; ++i) {

@@ -29,7 +29,8 @@ def test_columns_do_not_depend_on_how_many_share_a_workgroup(L, dev, M, N, K, dt
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,Ns,K", [(1, (4096, 16), 2560), (7, (4104, 4088), 144), (1, (6152, 2048), 2304), (16, (40, 8200, 2000), 144)])
+@pytest.mark.parametrize("M,Ns,K", [(1, (4096, 16), 2560), (7, (4104, 4088), 144), (1, (6152, 2048), 2304), (16, (40, 8200, 2000), 144),
+                                    (1, (4096, 4096, 4096), 2304), (2, (4097, 3, 4000, 4188), 2560)])
 def test_layers_in_one_launch_take_the_same_forms(L, dev, M, Ns, K):
     layers = [_layer(L, dev, M, N, K, torch.bfloat16) for N in Ns]
     for layer, got in zip(layers, L.linear_w8a16_small_m_grouped(layers)):
