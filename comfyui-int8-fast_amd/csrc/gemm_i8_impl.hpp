@@ -169,9 +169,12 @@ __device__ __forceinline__ v4i make_rsrc(const void *p, uint32_t bytes) {
 }
 
 // `bytes` of a tensor from byte `at` on as a buffer, empty without a tensor.  Pieces of an [M,N] tensor past its last row load zeros
-// and are not stored, so a lane's offset is a 32-bit number that its column fixes (OUT_OF_ROW past the last one; at most 16 rows of
-// less than 2^28 bytes below it), and the rows move on in the descriptor, by scalar instructions.
+// and are not stored, so a lane's offset is a 32-bit number that its column fixes (OUT_OF_ROW past the last one), and the rows move
+// on in the descriptor, by scalar instructions.  Below it are at most 16 rows of 16-bit values or 8 of 32-bit ones (GROUP_ROWS), which
+// stay within 32 bits up to GATED_MAX_N columns.
 constexpr uint32_t OUT_OF_ROW = 0xfffffff0u;
+constexpr int GATED_MAX_N = (1 << 27) - 8;
+inline bool gate_addressable(const GemmArgs &g) { return (!g.gate && !g.addend) || g.N <= GATED_MAX_N; }   // (a wider one: K = 0 only)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_at(const void *p, int64_t at, int64_t bytes) {
     const uint32_t records = !p || bytes <= 0 ? 0u : bytes < 0xffffff00ll ? (uint32_t)bytes : 0xffffff00u;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>((const char *)p + at), 0, records, 0x00020000);
@@ -909,6 +912,7 @@ __device__ __forceinline__ void gemm_i8_body(const int8_t *gx, const int8_t *gw,
         constexpr int PASSES = EPI_STRIPS * 32 * CPO / 64;
         constexpr int PERIOD = CPO / std::gcd(64, CPO), GROUP_ROWS = 64 * PERIOD / CPO;
         static_assert(PASSES % PERIOD == 0, "whole groups of rows");
+        static_assert((int64_t)GROUP_ROWS * OB <= 32, "a group of GATED_MAX_N columns stays within 32 bits");
         const int64_t row_bytes = (int64_t)gN * OB;
         const int nw = n0 + wn * C::WTN;         // the wave's first column
         uint32_t at[PERIOD];                     // of a piece from the group's first row on, in the output and in what is staged
@@ -1382,7 +1386,7 @@ int launch(GemmArgs &g, hipStream_t st) {
                          ((uintptr_t)g.out % 16 == 0) && ((int64_t)g.N * g.K < (1ll << 31)) &&
                          (!g.ws || !g.row_scale || (uintptr_t)g.ws % 16 == 0) &&
                          (!g.bias || (uintptr_t)g.bias % 16 == 0) && (!g.addend || (uintptr_t)g.addend % 16 == 0) &&
-                         (!g.gate || (uintptr_t)g.gate % 16 == 0);
+                         (!g.gate || (uintptr_t)g.gate % 16 == 0) && gate_addressable(g);
     // The buffer descriptors address 2^31 bytes: more activations than that go in row blocks.
     if (aligned && (int64_t)g.M * g.K >= (1ll << 31) && (int64_t)256 * g.K < (1ll << 31)) {
         const int rows_per = (int)((((1ll << 31) - 1) / g.K) / 256 * 256);
@@ -1504,7 +1508,7 @@ int launch_group(GemmArgs *gs, int n, hipStream_t st) {
         together = (g.K % 128 == 0) && (g.N % 8 == 0) && ((uintptr_t)g.x % 16 == 0) && ((uintptr_t)g.w % 16 == 0) &&
                    ((uintptr_t)g.out % 16 == 0) && ((int64_t)g.N * g.K < (1ll << 31)) && ((int64_t)g.M * g.K < (1ll << 31)) &&
                    (!g.ws || !g.row_scale || (uintptr_t)g.ws % 16 == 0) && (!g.bias || (uintptr_t)g.bias % 16 == 0) &&
-                   (!g.addend || (uintptr_t)g.addend % 16 == 0) && (!g.gate || (uintptr_t)g.gate % 16 == 0) && !g.side_t;
+                   (!g.addend || (uintptr_t)g.addend % 16 == 0) && (!g.gate || (uintptr_t)g.gate % 16 == 0) && gate_addressable(g) && !g.side_t;
     }
     Tile t = TILE_BIG;
     if (together) {

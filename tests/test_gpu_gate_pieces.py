@@ -58,3 +58,20 @@ def test_absent_operands_signed_zeros_infinities_and_the_residual_as_output(L, d
     assert torch.equal(out.isnan(), nan)
     assert torch.equal(out.view(whole)[~nan], want.view(whole)[~nan])
     assert bool((guard[M:] == 7.0).all())
+
+
+@pytest.mark.gpu
+def test_rows_wider_than_the_pieces_offsets(L, dev):
+    """Columns beyond 2^27, which only a product over no columns at all has: sixteen rows of them exceed 32 bits."""
+    M, N = 17, 2**28 + 8
+    g = torch.Generator(device=dev).manual_seed(3)
+    a, w = (torch.empty(n, 0, dtype=torch.int8, device=dev) for n in (M, N))
+    draw = lambda *size: torch.empty(size, dtype=torch.bfloat16, device=dev).normal_(generator=g)
+    bias, gate, residual = draw(N), draw(1, N), draw(M, N)
+    call = lambda **kw: L.linear_w8a8(a, torch.ones(M, device=dev), w, 0.5, bias, torch.bfloat16, L.EPI_TORCH, addend=residual, gate=gate, **kw)
+    want = [r + gate[0] * bias for r in residual]
+    out = call()
+    assert all(torch.equal(o, v) for o, v in zip(out, want))
+    out.zero_()
+    L.linear_w8a8_grouped([(a, torch.ones(M, device=dev), w, 0.5, bias, residual, gate)] * 2, torch.bfloat16, L.EPI_TORCH, outs=[out, out])
+    assert all(torch.equal(o, v) for o, v in zip(out, want))
