@@ -332,8 +332,10 @@ PyObject *w8a8(PyObject *const *a, const at::Tensor &x, int64_t M, int64_t K, in
             if (res->size(i) != x.size(i)) Py_RETURN_NONE;
     }
     Owned work_object;
-    if (a[16] != Py_None) {
-        work_object.p = PyObject_CallFunction(a[16], "OLLL", a[0], (long long)M, (long long)l[0].N, (long long)Kall);
+    if (a[16] != Py_None) {   // (the narrowest layer has the fewest tiles: what it cannot use, none can)
+        int64_t narrowest = l[0].N;
+        for (int i = 1; i < count; ++i) narrowest = l[i].N < narrowest ? l[i].N : narrowest;
+        work_object.p = PyObject_CallFunction(a[16], "OLLL", a[0], (long long)M, (long long)narrowest, (long long)Kall);
         if (!work_object.p) return nullptr;
         if (work_object.p != Py_None && !(work = tensor(work_object.p))) Py_RETURN_NONE;
     }
@@ -394,9 +396,9 @@ PyObject *w8a8(PyObject *const *a, const at::Tensor &x, int64_t M, int64_t K, in
 
 // linear(x, weight, scale, bias, per_row, rotate, small_rows, order, kind, mod_scale, mod_shift, eps, norm_weight, fused_add,
 //        gate, residual, workspace): kind, an i8f_prologue, names what is applied to x inside the quantiser; workspace(x, M, N,
-// K) gives the memory of the K split or None.  It is called once a W8A8 call has passed every check, never for 16 rows or
-// fewer or for a call that goes the general way, which asks for its own: the memory stays with the stream, or with the graph
-// that is being captured, together with the kernel that clears it.
+// K) gives the memory of the K split, which the layers of one call share, or None.  It is called once a W8A8 call has passed
+// every check, never for 16 rows or fewer or for a call that goes the general way, which asks for its own: the memory stays
+// with the stream, or with the graph that is being captured, together with the kernel that clears it.
 PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 17) return PyErr_Format(PyExc_TypeError, "linear takes 17 arguments, got %zd", n);
     const at::Tensor *xt = tensor(a[0]);

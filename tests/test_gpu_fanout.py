@@ -63,3 +63,46 @@ def test_calls_that_the_native_fanout_leaves_to_the_general_path(pkg, L, dev):
     assert native(lins, x) is None
     lins[1]._use_quarot, lins[1].lora_A = False, torch.randn(16, 256, device=dev).bfloat16()
     assert native(lins, x) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("widths", [(3456, 256, 256), (256, 3456), (256, 256)])
+def test_narrow_layers_keep_their_k_split_beside_wide_ones(pkg, L, dev, widths, monkeypatch):
+    """Eager, on a stream of its own and captured: the partial sums show that the layers of 256 columns were split (135 tiles of
+    128 x 128, those of 3456, are more than a split takes)."""
+    rows, K = 520, 10240
+    lins = layers_of(pkg, dev, widths, K, torch.bfloat16)
+    x = torch.randn(rows, K, device=dev).bfloat16()
+    want = [lin(x) for lin in lins]
+    handed, ask = [], L._splitk_workspace
+    monkeypatch.setattr(L, "_splitk_workspace", lambda *a: handed.append(ask(*a)) or handed[-1])
+    untouched = 0x5a5a5a5a   # (no sum of 10240 products)
+
+    def partials(work):
+        return work[L._SPLITK_COUNTER_BYTES:].view(torch.int32)
+
+    def check(outs):
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, v) for o, v in zip(outs, want))
+        written = int((partials(handed[-1]) != untouched).sum())
+        assert written >= 520 * 256 and int(handed[-1][:L._SPLITK_COUNTER_BYTES].sum()) == 0
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    for stream in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(stream):
+            partials(ask(x, rows, 256, K)).fill_(untouched)
+            check(pkg.forward_fanout(lins, x))
+    assert len(handed) == 2 and handed[0].data_ptr() != handed[1].data_ptr()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = pkg.forward_fanout(lins, x)
+    assert len(handed) == 3 and all(handed[2].data_ptr() != h.data_ptr() for h in handed[:2])
+    for _ in range(3):
+        partials(handed[2]).fill_(untouched)
+        for o in outs:
+            o.zero_()
+        graph.replay()
+        check(outs)
+        assert all(torch.equal(o, v) for o, v in zip(pkg.forward_fanout(lins, x), want))   # an eager call in between
+        handed.pop()
