@@ -31,6 +31,9 @@ struct MergeArgs {
     const float *noise;
     int64_t N, K;
     int8_t *out;
+    // instead of noise: the upper halves of the generator's words (draw_words_kernel), and what gives the words themselves
+    const uint16_t *drawn;
+    uint32_t seed_lo, seed_hi, lanes;
 };
 
 // A weight row's scale with what the fast quotient below needs.
@@ -96,6 +99,65 @@ __device__ __forceinline__ void sr_row(const float (&delta)[NE], const float (&n
     }
 #pragma unroll
     for (int e = 0; e < NE; ++e) r[e] = sr_round(xs[e], noise[e]);
+}
+
+// ---- noise drawn here, for few elements --------------------------------------------------------------------------
+// The upper 16 bits of every element's word (0 for those that give 0), and the merge below reading them instead of the numbers; only
+// the elements whose rounding the other 16 bits decide draw their word again.  A thread calls the generator for eight
+// neighbouring lanes, 32 elements.  These two launches wait for less than those of lora_merge_drawn.hip, which splits the factors first
+// and lists what is open: where there are few elements or products that is what counts (takes_few_form, with both sides measured).
+//
+// Several LoRAs: the first `extra` rows of workgroups write the factors side by side, up [N,R] and each `down` times its
+// multiplier (rounded) [R,K], while the others draw.
+struct Stack {
+    const float *up[MAX_FACTORS], *down[MAX_FACTORS];
+    float mult[MAX_FACTORS];
+    int first[MAX_FACTORS + 1];   // first rank of each; [n] = the sum R
+    int n;
+    uint32_t N, K;
+    float *up_out, *down_out;
+};
+
+__device__ __forceinline__ void stack_factors(const Stack &f, uint32_t at, uint32_t step) {
+    const uint32_t R = f.first[f.n], ups = f.N * R, all = ups + R * f.K;
+#pragma unroll 4
+    for (uint32_t i = at; i < all; i += step) {
+        const bool is_up = i < ups;
+        const uint32_t j = is_up ? i % R : (i - ups) / f.K;   // rank
+        int l = 0;
+#pragma unroll
+        for (int t = 1; t < MAX_FACTORS; ++t) l = t < f.n && (int)j >= f.first[t] ? t : l;
+        const uint32_t r = f.first[l + 1] - f.first[l], own = j - f.first[l];
+        if (is_up) f.up_out[i] = f.up[l][i / R * r + own];
+        else f.down_out[i - ups] = f.down[l][own * f.K + (i - ups) % f.K] * f.mult[l];
+    }
+}
+
+__global__ __launch_bounds__(256) void draw_words_kernel(uint32_t seed_lo, uint32_t seed_hi, uint32_t lanes, uint32_t numel, uint16_t *out, uint32_t extra,
+                                                         const Stack stack) {
+    if (blockIdx.y < extra) return stack_factors(stack, (blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x, extra * gridDim.x * 256);
+    const uint32_t chunk = blockIdx.y - extra;
+    const uint32_t s0 = (blockIdx.x * 256 + threadIdx.x) * 8, at = 4 * chunk * lanes + s0;
+    if (s0 >= lanes || at >= numel) return;
+    uint32_t x[8][4], top = 0;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        philox(chunk, s0 + t, seed_lo, seed_hi, x[t]);
+        top = max(max(top, max(x[t][0], x[t][1])), max(x[t][2], x[t][3]));
+    }
+    if (top >= ONE_WORDS) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x[t][q] = x[t][q] >= ONE_WORDS ? 0u : x[t][q];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        uint32_t o[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_perm(x[2 * t + 1][q], x[2 * t][q], 0x07060302u);  // two upper halves
+        if (at + q * lanes < numel) stream_store16(out + at + q * lanes, make_uint4(o[0], o[1], o[2], o[3]));
+    }
 }
 
 // VEC: 4 elements per thread with 16-byte loads when K % 4 == 0 and pointers are aligned, else 1
@@ -230,12 +292,13 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i_t __attribute__((ext_vector_type(4)));
 
-template <int RANK>
+template <int RANK, bool DRAWN>
 struct MfmaMergeLds {
     static constexpr int WAVES = RANK == 48 || RANK == 64 ? 4 : 8, COLS = WAVES * 32;
     // One wave load moves 1 KB of noise: NZ_ROWS rows of the tile.  Pitch 260 words: the column reads of 16 rows hit 16
     // different bank groups; of two rows in one piece the second has its 16-byte chunks swapped in groups of four.
-    static constexpr int NZ_ROWS = 256 / COLS, NZ_PITCH = 1024 + 16;
+    static constexpr int NZ_SIZE = DRAWN ? 2 : 4;   // bytes of noise to an element
+    static constexpr int NZ_ROWS = 1024 / (COLS * NZ_SIZE), NZ_PITCH = 1024 + 16;
     static constexpr int UPV = RANK <= 32 ? 1 : 4;   // products whose `up` operands one LDS read brings
     static constexpr int UP_PITCH = RANK * 4 + 4 * UPV;
     static constexpr int WB_PITCH = COLS + 16;
@@ -268,9 +331,9 @@ __device__ __forceinline__ v4i_t buffer_resource(const void *p, uint32_t bytes) 
 }
 
 // PAD: a.rank is a multiple of 4 below RANK, and the products beyond it are 0 * 0, which leave the sum as it is.
-template <int RANK, bool PAD>
-__global__ __launch_bounds__((MfmaMergeLds<RANK>::WAVES * 64), RANK <= 32 ? 4 : RANK <= 64 ? 3 : 2) void lora_merge_mfma_kernel(const MergeArgs a, int bands) {
-    using T = MfmaMergeLds<RANK>;
+template <int RANK, bool PAD, bool DRAWN>
+__global__ __launch_bounds__((MfmaMergeLds<RANK, DRAWN>::WAVES * 64), RANK <= 32 ? 4 : RANK <= 64 ? 3 : 2) void lora_merge_mfma_kernel(const MergeArgs a, int bands) {
+    using T = MfmaMergeLds<RANK, DRAWN>;
     constexpr int NT = T::WAVES * 64, P = RANK / 2;
     static_assert(P % T::UPV == 0, "the products of a piece, UPV at a time");
     __shared__ __attribute__((aligned(16))) char lds[T::BYTES];
@@ -299,13 +362,15 @@ __global__ __launch_bounds__((MfmaMergeLds<RANK>::WAVES * 64), RANK <= 32 ? 4 : 
     // Noise: wave w moves 1 KB pieces w, w + WAVES, ... of a block (NZ_ROWS rows each), a lane 16 bytes.  The buffer
     // starts at the block's first row and the workgroup's first column and ends with the array, so rows past N
     // read as zeros (their results are not stored).
-    const uint32_t row_bytes = (uint32_t)a.K * 4u;
+    const uint32_t row_bytes = (uint32_t)a.K * T::NZ_SIZE;
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
-    const uint32_t nz_lane = T::NZ_ROWS == 1 ? (uint32_t)lane * 16u : (uint32_t)half * row_bytes + (uint32_t)(l32 ^ (4 * half)) * 16u;
+    constexpr int NZ_LANES = 64 / T::NZ_ROWS;   // of a wave load, to a row
+    const uint32_t nz_lane = DRAWN ? (uint32_t)(lane / NZ_LANES) * row_bytes + (uint32_t)(lane % NZ_LANES) * 16u
+                             : T::NZ_ROWS == 1 ? (uint32_t)lane * 16u : (uint32_t)half * row_bytes + (uint32_t)(l32 ^ (4 * half)) * 16u;
     auto fetch_noise = [&](int64_t nb, int buf) __attribute__((always_inline)) {
         const int64_t first = nb * 32 * a.K + k0;
-        const int64_t left = (a.N * a.K - first) * 4;
-        const v4i_t rsrc = buffer_resource(a.noise + first, left < 0xffffffffll ? (uint32_t)left : 0xffffffffu);
+        const int64_t left = (a.N * a.K - first) * T::NZ_SIZE;
+        const v4i_t rsrc = buffer_resource(DRAWN ? (const char *)(a.drawn + first) : (const char *)(a.noise + first), left < 0xffffffffll ? (uint32_t)left : 0xffffffffu);
 #pragma unroll
         for (int i = 0; i < 32 / (T::NZ_ROWS * T::WAVES); ++i)
             buffer_to_lds16(rsrc, lds_base + T::NZ + buf * T::NZ_BYTES + (wave + T::WAVES * i) * T::NZ_PITCH, nz_lane,
@@ -398,47 +463,109 @@ __global__ __launch_bounds__((MfmaMergeLds<RANK>::WAVES * 64), RANK <= 32 ? 4 : 
         };
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc_next[i] = 0.0f;
-        const RowScale rs = row_scale(sc);
-        float d[16];
-        SrGuard guard;
-        auto noise_quad = [&](int q, float (&nzv)[4]) __attribute__((always_inline)) {
-            const int chunk = wave * 8 + 2 * q + half;
-            const v4f nz = *(const v4f *)(T::NZ_ROWS == 1 ? nz_tile + l32 * T::NZ_PITCH + chunk * 16
-                                                          : nz_tile + (l32 >> 1) * T::NZ_PITCH + (l32 & 1) * 512 + (chunk ^ (4 * (l32 & 1))) * 16);
-            nzv[0] = nz.x, nzv[1] = nz.y, nzv[2] = nz.z, nzv[3] = nz.w;
-        };
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {  // the noise is read again where it is used: sixteen registers fewer across the block
-            float nzv[4], dq[4];
-            noise_quad(q, nzv);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) dq[e] = d[4 * q + e] = acc_cur[4 * q + e] * a.lora_scale;
-            guard.add(dq, nzv);
-        }
-        if (__builtin_amdgcn_ballot_w64(!guard.fast(rs)) == 0) {
+        if constexpr (DRAWN) {
+            // floor(xs) + (noise < frac) is the whole number above z = xs - noise, unless z is so close to one that the other
+            // halves of the words, or the roundings on the way, leave it open.  How far z may be from the definition's: 2^-17, a
+            // word's upper half taken at the middle of its range; 2^-24 * 2.1, the roundings of noise and fraction; and 7 * 2^-24
+            // * |xs|, |xs| <= |z| + 1: two units for the reciprocal and one each for its product with lora_scale, the two fma
+            // steps, and the definition's own product and quotient.  Together at most 1.08 * 2^-17 + 7 * 2^-24 * |z|; 1.125 * 2^-17
+            // is asked for.  Of 256 elements with |z| of a few units one group in 200 is left open and redone.
+            const float f = __builtin_amdgcn_rcpf(sc) * a.lora_scale;
+            // (lora_scale 0, a LoRA switched off by its strength: xs is 0, or NaN with a sum that is not finite, and so is z plus the
+            // noise.  Left to the definition every element drew its word again: 12288 x 3072, rank 32, 133 us with the noise for 66.)
+            const bool usual = sc >= 0x1p-20f && sc <= 0x1p+20f && (fabsf(f) >= 0x1p-100f || a.lora_scale == 0.0f) && fabsf(f) <= 0x1p+100f;
+            float zmax[4] = {};
+            uint32_t dmin[4], dmax[4];   // (bits, so that a NaN is the largest)
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 product(q * P / (4 * UPV) * UPV, (q + 1) * P / (4 * UPV) * UPV, acc_next);
-                float r[4], nzv[4];
-                noise_quad(q, nzv);
+                const uint2 n4 = *(const uint2 *)(nz_tile + (l32 / T::NZ_ROWS) * T::NZ_PITCH + (l32 % T::NZ_ROWS) * (T::COLS * 2) + (wave * 32 + 8 * q + 4 * half) * 2);
+                const uint32_t n[4] = {n4.x & 0xffffu, n4.x >> 16, n4.y & 0xffffu, n4.y >> 16};
+                float r[4];
+                dmin[q] = 0xffffffffu, dmax[q] = 0u;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) r[e] = sr_round(fast_quotient(d[4 * q + e], rs), nzv[e]);
+                for (int e = 0; e < 4; ++e) {
+                    const float z = __builtin_fmaf((float)n[e], -0x1p-16f, __builtin_fmaf(acc_cur[4 * q + e], f, -0x1p-17f));
+                    r[e] = ceilf(z);
+                    const uint32_t d = __float_as_uint(r[e] - z);
+                    zmax[q] = fmaxf(zmax[q], fabsf(z)), dmin[q] = min(dmin[q], d), dmax[q] = max(dmax[q], d);
+                }
                 o[q] = add_sat8_pack(weight_quad(q), r);
             }
 #pragma unroll
             for (int i = 0; i < P; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);        // one matrix instruction
-                __builtin_amdgcn_sched_group_barrier(0x002, P <= 112 ? 224 / P : 2, 0);  // its share of the vector work
+                __builtin_amdgcn_sched_group_barrier(0x002, P <= 96 ? 192 / P : 2, 0);  // its share of the vector work
             }
-        } else {  // some lane needs the division: every lane takes it
-            product(0, P, acc_next);
+            __builtin_amdgcn_sched_barrier(0);
+            uint32_t open = 0;   // groups of four that have a lane without an answer
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                float r[4], nzv[4];
+                const float eps = __builtin_fmaf(zmax[q], 7.0f * 0x1p-24f, 0x1.2p-17f);
+                const bool sure = usual && zmax[q] <= 64.0f && dmin[q] >= __float_as_uint(eps) && dmax[q] <= __float_as_uint(1.0f - eps);
+                open |= __builtin_amdgcn_ballot_w64(!sure) != 0 ? 1u << q : 0u;
+            }
+            const uint32_t e0 = (uint32_t)(clampn(nb * 32 + l32) * a.K + k0) + wave * 32 + 4 * half;
+            while (__builtin_expect(open != 0, 0)) {  // by the definition, from the whole words
+                const int q = __builtin_ctz(open);
+                open &= open - 1;
+                const uint32_t e = e0 + 8 * q, i = e / a.lanes, lane_of = e - i * a.lanes;
+                float r[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    uint32_t x[4];
+                    philox(i / 4, lane_of + t, a.seed_lo, a.seed_hi, x);
+                    const uint32_t lo = i & 1 ? x[1] : x[0], hi = i & 1 ? x[3] : x[2];
+                    const float acc = q == 0 ? acc_cur[t] : q == 1 ? acc_cur[4 + t] : q == 2 ? acc_cur[8 + t] : acc_cur[12 + t];
+                    r[t] = sr_round(acc * a.lora_scale / sc, uniform_of(i & 2 ? hi : lo));
+                }
+                const uint32_t v = add_sat8_pack(weight_quad(q), r);
+                o[0] = q == 0 ? v : o[0], o[1] = q == 1 ? v : o[1], o[2] = q == 2 ? v : o[2], o[3] = q == 3 ? v : o[3];
+            }
+        } else {
+            const RowScale rs = row_scale(sc);
+            float d[16];
+            SrGuard guard;
+            auto noise_quad = [&](int q, float (&nzv)[4]) __attribute__((always_inline)) {
+                const int chunk = wave * 8 + 2 * q + half;
+                const v4f nz = *(const v4f *)(T::NZ_ROWS == 1 ? nz_tile + l32 * T::NZ_PITCH + chunk * 16
+                                                              : nz_tile + (l32 >> 1) * T::NZ_PITCH + (l32 & 1) * 512 + (chunk ^ (4 * (l32 & 1))) * 16);
+                nzv[0] = nz.x, nzv[1] = nz.y, nzv[2] = nz.z, nzv[3] = nz.w;
+            };
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {  // the noise is read again where it is used: sixteen registers fewer across the block
+                float nzv[4], dq[4];
                 noise_quad(q, nzv);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) r[e] = sr_round(d[4 * q + e] / rs.sc, nzv[e]);
-                o[q] = add_sat8_pack(weight_quad(q), r);
+                for (int e = 0; e < 4; ++e) dq[e] = d[4 * q + e] = acc_cur[4 * q + e] * a.lora_scale;
+                guard.add(dq, nzv);
+            }
+            if (__builtin_amdgcn_ballot_w64(!guard.fast(rs)) == 0) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    product(q * P / (4 * UPV) * UPV, (q + 1) * P / (4 * UPV) * UPV, acc_next);
+                    float r[4], nzv[4];
+                    noise_quad(q, nzv);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) r[e] = sr_round(fast_quotient(d[4 * q + e], rs), nzv[e]);
+                    o[q] = add_sat8_pack(weight_quad(q), r);
+                }
+#pragma unroll
+                for (int i = 0; i < P; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);        // one matrix instruction
+                    __builtin_amdgcn_sched_group_barrier(0x002, P <= 112 ? 224 / P : 2, 0);  // its share of the vector work
+                }
+            } else {  // some lane needs the division: every lane takes it
+                product(0, P, acc_next);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    float r[4], nzv[4];
+                    noise_quad(q, nzv);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) r[e] = sr_round(d[4 * q + e] / rs.sc, nzv[e]);
+                    o[q] = add_sat8_pack(weight_quad(q), r);
+                }
             }
         }
         acc_cur = acc_next;
@@ -455,9 +582,9 @@ __global__ __launch_bounds__((MfmaMergeLds<RANK>::WAVES * 64), RANK <= 32 ? 4 : 
     }
 }
 
-template <int RANK>
+template <int RANK, bool DRAWN>
 int launch_mfma(const MergeArgs &a, hipStream_t st) {
-    using T = MfmaMergeLds<RANK>;
+    using T = MfmaMergeLds<RANK, DRAWN>;
     const int64_t col_blocks = (a.K + T::COLS - 1) / T::COLS, nblocks = (a.N + 31) / 32;
     if (col_blocks > 0x7fffffffll) return I8F_ERR_UNSUPPORTED;
     // Two workgroups fit a CU (LDS), so 512 run at a time.  Bands are chosen for the fewest block steps on the busiest
@@ -475,34 +602,38 @@ int launch_mfma(const MergeArgs &a, hipStream_t st) {
             best = rounds * steps2, best_rounds = rounds, bands = b;
     }
     const dim3 grid((unsigned)col_blocks, (unsigned)bands);
-    if (a.rank == RANK) {
-        hipLaunchKernelGGL((lora_merge_mfma_kernel<RANK, false>), grid, dim3(T::WAVES * 64), 0, st, a, (int)bands);
-        return check_launch();
+    if constexpr (!DRAWN) {
+        if (a.rank == RANK) {
+            hipLaunchKernelGGL((lora_merge_mfma_kernel<RANK, false, false>), grid, dim3(T::WAVES * 64), 0, st, a, (int)bands);
+            return check_launch();
+        }
     }
-    hipLaunchKernelGGL((lora_merge_mfma_kernel<RANK, true>), grid, dim3(T::WAVES * 64), 0, st, a, (int)bands);
+    hipLaunchKernelGGL((lora_merge_mfma_kernel<RANK, true, DRAWN>), grid, dim3(T::WAVES * 64), 0, st, a, (int)bands);
     return check_launch();
 }
 
+template <bool DRAWN>
 int launch_rank(const MergeArgs &a, hipStream_t st) {
     // the next larger rank that is built, the rest zeros: a padded product costs no more than its share of RANK
     // (3072 x 1552, an odd multiple of 16 columns, rank 32: 13.5 us against 22.3 us for the band form below).  Up to 32
     // the noise stream hides the products and powers of two are enough; beyond, the products are the time, so every 16
     // up to 128 and every 32 up to 256 is built: 9216 x 3072, us, padded to the next of 64, 96, 128, 192, 256 and as it
     // is: rank 48 54.6 and 47.1, 80 78.2 and 70.2, 112 92.3 and 84.1, 160 144.5 and 126.9, 224 186.1 and 154.6.
-    if (a.rank <= 4) return launch_mfma<4>(a, st);
-    if (a.rank <= 8) return launch_mfma<8>(a, st);
-    if (a.rank <= 16) return launch_mfma<16>(a, st);
-    if (a.rank <= 32) return launch_mfma<32>(a, st);
-    if (a.rank <= 48) return launch_mfma<48>(a, st);
-    if (a.rank <= 64) return launch_mfma<64>(a, st);
-    if (a.rank <= 80) return launch_mfma<80>(a, st);
-    if (a.rank <= 96) return launch_mfma<96>(a, st);
-    if (a.rank <= 112) return launch_mfma<112>(a, st);
-    if (a.rank <= 128) return launch_mfma<128>(a, st);
-    if (a.rank <= 160) return launch_mfma<160>(a, st);
-    if (a.rank <= 192) return launch_mfma<192>(a, st);
-    if (a.rank <= 224) return launch_mfma<224>(a, st);
-    return launch_mfma<256>(a, st);
+    if (a.rank <= 4) return launch_mfma<4, DRAWN>(a, st);
+    if (a.rank <= 8) return launch_mfma<8, DRAWN>(a, st);
+    if (a.rank <= 16) return launch_mfma<16, DRAWN>(a, st);
+    if (a.rank <= 32) return launch_mfma<32, DRAWN>(a, st);
+    if (a.rank <= 48) return launch_mfma<48, DRAWN>(a, st);
+    if (a.rank <= 64) return launch_mfma<64, DRAWN>(a, st);
+    if (a.rank <= 80) return launch_mfma<80, DRAWN>(a, st);
+    if (a.rank <= 96) return launch_mfma<96, DRAWN>(a, st);
+    if (a.rank <= 112) return launch_mfma<112, DRAWN>(a, st);
+    if (a.rank <= 128) return launch_mfma<128, DRAWN>(a, st);
+    if (a.rank <= 160) return launch_mfma<160, DRAWN>(a, st);
+    if (a.rank <= 192) return launch_mfma<192, DRAWN>(a, st);
+    if (a.rank <= 224) return launch_mfma<224, DRAWN>(a, st);
+    if constexpr (DRAWN) return I8F_ERR_UNSUPPORTED;   // (FEW_MAX_RANK)
+    else return launch_mfma<256, DRAWN>(a, st);
 }
 
 template <int RANK>
@@ -528,7 +659,7 @@ int run(MergeArgs &a, hipStream_t st) {
     // (K < 2^24: the 32 rows of a block are addressed with 32-bit byte offsets from the block's first element)
     if (fused && vec && a.w && a.N < (1ll << 31) && a.K % 16 == 0 && a.K < (1 << 24) && al(a.up, 16) && al(a.w, 16) && al(a.out, 16) &&
         a.rank % 4 == 0 && a.rank > 0 && a.rank <= 256)
-        return launch_rank(a, st);
+        return launch_rank<false>(a, st);
     if (fused && vec && a.w && a.N < (1ll << 31)) {
         switch (a.rank) {
         case 4: return launch_band<4>(a, st);
@@ -602,3 +733,40 @@ extern "C" int i8f_lora_merge_sr(const int8_t *w, const float *w_scale, float w_
     a.noise = noise, a.N = N, a.K = K, a.out = w_out;
     return run(a, (hipStream_t)stream);
 }
+
+namespace i8f {
+
+int64_t merge_few_workspace_bytes(int64_t N, int64_t K, int64_t rank, int count) {
+    return up256(2 * N * K) + (count > 1 ? up256(4 * N * rank) + 4 * K * rank : 0);
+}
+
+int merge_few(const DrawnCall &c, hipStream_t st) {
+    const int64_t N = c.N, K = c.K, columns = (c.lanes + 2047) / 2048, chunks = (N * K + 4 * c.lanes - 1) / (4 * c.lanes);
+    // workgroups for the factors: 4 elements a thread, one round of the chip at most
+    int64_t extra = c.count > 1 ? ((N + K) * c.rank + 1023) / 1024 : 0;
+    extra = ((extra < 2048 ? extra : 2048) + columns - 1) / columns;
+    if (chunks + extra > 65535) return I8F_ERR_UNSUPPORTED;
+    MergeArgs a{};
+    a.w = c.w, a.ws = c.ws, a.ws_host = c.ws_host, a.row_scale = c.row_scale;
+    a.up = c.factors[0].up, a.down = c.factors[0].down, a.rank = c.rank, a.lora_scale = c.lora_scale;
+    a.N = N, a.K = K, a.out = c.out;
+    a.drawn = (const uint16_t *)c.workspace, a.seed_lo = (uint32_t)c.seed, a.seed_hi = (uint32_t)(c.seed >> 32), a.lanes = (uint32_t)c.lanes;
+    Stack stack{};
+    stack.n = c.count;
+    for (int i = 0; i < c.count; ++i) {
+        stack.up[i] = c.factors[i].up, stack.down[i] = c.factors[i].down, stack.mult[i] = c.factors[i].mult;
+        stack.first[i + 1] = stack.first[i] + (int)c.factors[i].rank;
+    }
+    if (c.count > 1) {
+        stack.N = (uint32_t)N, stack.K = (uint32_t)K;
+        stack.up_out = (float *)((char *)c.workspace + up256(2 * N * K));
+        stack.down_out = (float *)((char *)stack.up_out + up256(4 * N * c.rank));
+        a.up = stack.up_out, a.down = stack.down_out;
+    }
+    hipLaunchKernelGGL(draw_words_kernel, dim3((unsigned)columns, (unsigned)(chunks + extra)), dim3(256), 0, st, a.seed_lo, a.seed_hi, a.lanes,
+                       (uint32_t)(N * K), (uint16_t *)c.workspace, (uint32_t)extra, stack);
+    if (int rc = check_launch()) return rc;
+    return launch_rank<true>(a, st);
+}
+
+}  // namespace i8f

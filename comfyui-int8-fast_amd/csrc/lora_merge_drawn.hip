@@ -1,5 +1,5 @@
 // The low-rank merge that draws its noise: two launches whose result is, bit for bit, that of the merge on torch's own noise
-// (lora_merge.hip).
+// (lora_merge.hip, where the form for few elements is, too).
 //
 //   draw_bytes_kernel    the upper byte of every element's random word, and the factors in the form the merge multiplies
 //   merge_drawn_kernel   an approximate quotient from 16-bit matrix products, rounded against those bytes; the few
@@ -7,12 +7,11 @@
 //
 // Both approximations only ever say "certain" or "open", so neither can change a result.
 //
-// us, 12288 x 3072 rank 32, 9216 x 3072 ranks 16 + 32 + 64, 3072 x 12288 rank 128, 12288 x 12288 rank 8, 1024 x 1024 rank 16: both launches
-// 53, 57, 87, 173, 12.4 (the first 17, 15, 18, 57, 5.5).  With 16-bit halves of the words and binary32 products, whose 64 cycles a pair of
-// ranks share the SIMD with the vector instructions, 66, 97, 140, 174, 9.0; with torch.rand and the merge on its tensor 86, 121 for
-// the first two.
+// us, 12288 x 3072 rank 32, 9216 x 3072 ranks 16 + 32 + 64, 3072 x 12288 rank 128, 12288 x 12288 rank 8: both launches
+// 53, 57, 87, 173 (the first 17, 15, 18, 57).  With 16-bit halves of the words and binary32 products, whose 64 cycles a pair of
+// ranks share the SIMD with the vector instructions (the form for few elements), 66, 97, 140, 174; with torch.rand and the merge on
+// its tensor 86, 121 for the first two.
 #include "merge_round.hpp"
-#include "../../include/i8f_drawn.h"
 
 namespace i8f {
 namespace {
@@ -20,7 +19,6 @@ namespace {
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
-constexpr int MAX_FACTORS = 8;
 constexpr int PIECE = 8;   // ranks in a 16-byte piece of binary16
 
 // The factors of the LoRAs that are merged together, and what the first launch makes of them: of several, `up` side by side
@@ -592,54 +590,36 @@ int launch_merge(const DrawnArgs &a, hipStream_t st) {
     }
 }
 
-int64_t up256(int64_t bytes) { return (bytes + 255) / 256 * 256; }
+// Few elements, or few products: which form is the faster one.  us, both launches, the form of lora_merge.hip and this one: 1024 x 1024 rank 16
+// 9.0 and 12.4, rank 128 18.4 and 19.3, 2048 x 1024 rank 32 11.1 and 14.5, rank 64 14.0 and 16.6, 2048 x 2048 rank 16 13.2 and 14.2, rank 64 18.7 and
+// 17.7, 3072 x 3072 rank 8 17.3 and 19.5, rank 16 18.5 and 19.7, rank 32 22.1 and 21.6, 3840 x 3840 rank 16 25.2 and 25.8, 5120 x 4096
+// rank 16 31.6 and 29.4; of ranks up to 4, 3840 x 3840 22.8 and 25.4, 10408 x 2672 40.1 and 41.6, 12288 x 3072 45.9 and 44.2.
+bool takes_few_form(int64_t N, int64_t K, int64_t rank) {
+    const int64_t weight = rank <= 4 ? 8 : rank <= 16 ? 16 : rank;
+    return rank <= FEW_MAX_RANK && N * K * weight < (1ll << 28);
+}
 
-}  // namespace
-}  // namespace i8f
-
-extern "C" int64_t i8f_lora_merge_sr_drawn_workspace_bytes(int64_t N, int64_t K, int64_t rank, int count) {
-    using namespace i8f;
-    if (N < 0 || K < 0 || rank < 0 || N > (1 << 29) || K > (1 << 29) || rank > 256) return 0;
+int64_t many_workspace_bytes(int64_t N, int64_t K, int64_t rank, int count) {
     const int64_t steps = steps_of(rank), column_blocks = column_blocks_of(K);
     const int64_t split = up256(N * steps * 64) + up256(N * 8) + up256(column_blocks * steps * 2048) + up256(column_blocks * 8);
     return up256(N * K) + split + up256(4 * K * rank) + (count > 1 ? 4 * N * rank : 0);
 }
 
-extern "C" int i8f_lora_merge_sr_drawn(const int8_t *w, const float *w_scale, float w_scale_host, int scale_mode,
-                                       const i8f_lora_factors *factors, int count, float lora_scale,
-                                       uint64_t seed, int64_t lanes, int64_t N, int64_t K, int8_t *w_out,
-                                       void *workspace, int64_t workspace_bytes, void *stream) {
-    using namespace i8f;
-    if (N < 0 || K < 0) return I8F_ERR_INVALID;
-    if (scale_mode != I8F_SCALE_TENSOR && scale_mode != I8F_SCALE_ROW) return I8F_ERR_INVALID;
-    if (N == 0 || K == 0) return I8F_OK;
-    if (!w || !w_out || !factors || count < 1 || !workspace || lanes <= 0) return I8F_ERR_INVALID;
-    if (scale_mode == I8F_SCALE_ROW && !w_scale) return I8F_ERR_INVALID;
-    if (count > MAX_FACTORS) return I8F_ERR_UNSUPPORTED;
+int merge_many(const DrawnCall &c, hipStream_t st) {
+    const int64_t N = c.N, K = c.K, lanes = c.lanes, chunks = (N * K + 4 * lanes - 1) / (4 * lanes);
     Factors f{};
-    f.n = count;
-    for (int i = 0; i < count; ++i) {
-        if (!factors[i].up || !factors[i].down || factors[i].rank <= 0) return I8F_ERR_INVALID;
-        if (factors[i].rank > 256 - f.first[i]) return I8F_ERR_UNSUPPORTED;
-        f.up[i] = factors[i].up, f.down[i] = factors[i].down, f.mult[i] = factors[i].mult;
-        f.first[i + 1] = f.first[i] + (int)factors[i].rank;
+    f.n = c.count;
+    for (int i = 0; i < c.count; ++i) {
+        f.up[i] = c.factors[i].up, f.down[i] = c.factors[i].down, f.mult[i] = c.factors[i].mult;
+        f.first[i + 1] = f.first[i] + (int)c.factors[i].rank;
     }
-    const int rank = f.first[count];
-    if (K % 16 || K >= (1 << 24) || N > (1 << 29) / K || rank % 4 || lanes % 256 || lanes > (1 << 24)) return I8F_ERR_UNSUPPORTED;
-    if ((uintptr_t)w % 16 || (uintptr_t)w_out % 16 || (uintptr_t)workspace % 16 || (count == 1 && (uintptr_t)factors[0].up % 16)) return I8F_ERR_UNSUPPORTED;
-    if (count > 1 && (N + K) * rank >= (1ll << 31)) return I8F_ERR_UNSUPPORTED;   // (elements are counted in 32 bits)
-    const int64_t chunks = (N * K + 4 * lanes - 1) / (4 * lanes);
-    if (chunks > 65535) return I8F_ERR_UNSUPPORTED;
-    if (workspace_bytes < i8f_lora_merge_sr_drawn_workspace_bytes(N, K, rank, count)) return I8F_ERR_INVALID;
-    if (int rc = check_device()) return rc;
-    hipStream_t st = (hipStream_t)stream;
-    char *at = (char *)workspace;
+    char *at = (char *)c.workspace;
     DrawnArgs a{};
-    a.w = w, a.ws = w_scale, a.ws_host = w_scale_host, a.row_scale = scale_mode == I8F_SCALE_ROW;
-    a.up = factors[0].up, a.rank = rank, a.lora_scale = lora_scale;
-    a.N = (uint32_t)N, a.K = (uint32_t)K, a.out = w_out;
-    a.seed_lo = (uint32_t)seed, a.seed_hi = (uint32_t)(seed >> 32), a.lanes = (uint32_t)lanes;
-    f.N = a.N, f.K = a.K, f.pieces = 2 * steps_of(rank);
+    a.w = c.w, a.ws = c.ws, a.ws_host = c.ws_host, a.row_scale = c.row_scale;
+    a.up = c.factors[0].up, a.rank = c.rank, a.lora_scale = c.lora_scale;
+    a.N = (uint32_t)N, a.K = (uint32_t)K, a.out = c.out;
+    a.seed_lo = (uint32_t)c.seed, a.seed_hi = (uint32_t)(c.seed >> 32), a.lanes = (uint32_t)lanes;
+    f.N = a.N, f.K = a.K, f.pieces = 2 * steps_of(c.rank);
     const int64_t column_blocks = column_blocks_of(K);
     uint4 *const noise = (uint4 *)at;
     a.noise = noise, at += up256(N * K);
@@ -647,8 +627,8 @@ extern "C" int i8f_lora_merge_sr_drawn(const int8_t *w, const float *w_scale, fl
     a.rows = f.rows = (float2 *)at, at += up256(N * 8);
     a.split_down = f.split_down = (uint4 *)at, at += up256(column_blocks * f.pieces * 1024);
     a.columns = f.columns = (float2 *)at, at += up256(column_blocks * 8);
-    a.down = f.down_out = (float *)at, at += up256(4 * K * rank);
-    if (count > 1) a.up = f.up_out = (float *)at;
+    a.down = f.down_out = (float *)at, at += up256(4 * K * c.rank);
+    if (c.count > 1) a.up = f.up_out = (float *)at;
     // rows of K that the generator's threads cover, of which a thread takes 16 elements; blocks of `up`: 32 rows, half a round of the
     // chip at most
     const int64_t rows = (lanes + K - 1) / K, columns = (rows * (K / 16) + 255) / 256, row_blocks = (N + 31) / 32 < 1024 ? (N + 31) / 32 : 1024;
@@ -665,4 +645,55 @@ extern "C" int i8f_lora_merge_sr_drawn(const int8_t *w, const float *w_scale, fl
     if (!once)
         if (int rc = draw(first_chunk, first_chunk + chunks)) return rc;
     return launch_merge(a, st);
+}
+
+}  // namespace
+}  // namespace i8f
+
+// form: 0 the one for few elements, 1 the other, -1 the faster one
+extern "C" int64_t i8f_internal_merge_drawn_workspace_bytes(int form, int64_t N, int64_t K, int64_t rank, int count) {
+    using namespace i8f;
+    if (N < 0 || K < 0 || rank < 0 || N > (1 << 29) || K > (1 << 29) || rank > 256) return 0;
+    return (form < 0 ? takes_few_form(N, K, rank) : form == 0) ? merge_few_workspace_bytes(N, K, rank, count) : many_workspace_bytes(N, K, rank, count);
+}
+
+extern "C" int i8f_internal_merge_drawn(int form, const int8_t *w, const float *w_scale, float w_scale_host, int scale_mode,
+                                        const i8f_lora_factors *factors, int count, float lora_scale,
+                                        uint64_t seed, int64_t lanes, int64_t N, int64_t K, int8_t *w_out,
+                                        void *workspace, int64_t workspace_bytes, void *stream) {
+    using namespace i8f;
+    if (N < 0 || K < 0) return I8F_ERR_INVALID;
+    if (scale_mode != I8F_SCALE_TENSOR && scale_mode != I8F_SCALE_ROW) return I8F_ERR_INVALID;
+    if (N == 0 || K == 0) return I8F_OK;
+    if (!w || !w_out || !factors || count < 1 || !workspace || lanes <= 0) return I8F_ERR_INVALID;
+    if (scale_mode == I8F_SCALE_ROW && !w_scale) return I8F_ERR_INVALID;
+    if (count > MAX_FACTORS) return I8F_ERR_UNSUPPORTED;
+    int rank = 0;
+    for (int i = 0; i < count; ++i) {
+        if (!factors[i].up || !factors[i].down || factors[i].rank <= 0) return I8F_ERR_INVALID;
+        if (factors[i].rank > 256 - rank) return I8F_ERR_UNSUPPORTED;
+        rank += (int)factors[i].rank;
+    }
+    if (K % 16 || K >= (1 << 24) || N > (1 << 29) / K || rank % 4 || lanes % 256 || lanes > (1 << 24)) return I8F_ERR_UNSUPPORTED;
+    if ((uintptr_t)w % 16 || (uintptr_t)w_out % 16 || (uintptr_t)workspace % 16 || (count == 1 && (uintptr_t)factors[0].up % 16)) return I8F_ERR_UNSUPPORTED;
+    if (count > 1 && (N + K) * rank >= (1ll << 31)) return I8F_ERR_UNSUPPORTED;   // (elements are counted in 32 bits)
+    if ((N * K + 4 * lanes - 1) / (4 * lanes) > 65535) return I8F_ERR_UNSUPPORTED;
+    const bool few = form < 0 ? takes_few_form(N, K, rank) : form == 0;
+    if (few && rank > FEW_MAX_RANK) return I8F_ERR_UNSUPPORTED;
+    if (workspace_bytes < i8f_internal_merge_drawn_workspace_bytes(form, N, K, rank, count)) return I8F_ERR_INVALID;
+    if (int rc = check_device()) return rc;
+    const DrawnCall call{w, w_scale, w_scale_host, scale_mode == I8F_SCALE_ROW, factors, count, rank, lora_scale, seed, lanes, N, K, w_out, workspace};
+    return few ? merge_few(call, (hipStream_t)stream) : merge_many(call, (hipStream_t)stream);
+}
+
+extern "C" int64_t i8f_lora_merge_sr_drawn_workspace_bytes(int64_t N, int64_t K, int64_t rank, int count) {
+    return i8f_internal_merge_drawn_workspace_bytes(-1, N, K, rank, count);
+}
+
+extern "C" int i8f_lora_merge_sr_drawn(const int8_t *w, const float *w_scale, float w_scale_host, int scale_mode,
+                                       const i8f_lora_factors *factors, int count, float lora_scale,
+                                       uint64_t seed, int64_t lanes, int64_t N, int64_t K, int8_t *w_out,
+                                       void *workspace, int64_t workspace_bytes, void *stream) {
+    return i8f_internal_merge_drawn(-1, w, w_scale, w_scale_host, scale_mode, factors, count, lora_scale, seed, lanes, N, K, w_out, workspace,
+                                    workspace_bytes, stream);
 }

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "i8f_common.hpp"
+#include "../../include/i8f_drawn.h"
 
 namespace i8f {
 namespace {
@@ -52,5 +53,27 @@ __device__ __forceinline__ float uniform_of(uint32_t x) {
     return x >= ONE_WORDS ? 0.0f : __builtin_fmaf((float)x, 0x1p-32f, 0x1p-32f);
 }
 
+constexpr int MAX_FACTORS = 8;
+int64_t up256(int64_t bytes) { return (bytes + 255) / 256 * 256; }
+
 }  // namespace
+
+// A checked call of i8f_lora_merge_sr_drawn, and its form for few elements (lora_merge.hip), of ranks up to FEW_MAX_RANK.
+struct DrawnCall {
+    const int8_t *w;
+    const float *ws;
+    float ws_host;
+    bool row_scale;
+    const i8f_lora_factors *factors;
+    int count, rank;   // rank: the sum
+    float lora_scale;
+    uint64_t seed;
+    int64_t lanes, N, K;
+    int8_t *out;
+    void *workspace;
+};
+constexpr int64_t FEW_MAX_RANK = 224;
+int64_t merge_few_workspace_bytes(int64_t N, int64_t K, int64_t rank, int count);
+int merge_few(const DrawnCall &c, hipStream_t st);
+
 }  // namespace i8f

@@ -171,3 +171,58 @@ def test_drawn_merge_refuses_what_it_cannot_do(L):
     assert call(N=2**25 + 1) == UNSUPPORTED and call(N=1, K=2**24) == UNSUPPORTED and call(lanes=2**24 + 256) == UNSUPPORTED
     assert call(N=2**24) == UNSUPPORTED      # more calls of the generator than a launch has blocks
     assert call(N=0) == 0 and call(K=0) == 0
+
+
+def force(L, monkeypatch, form):
+    """From here on the drawn merge takes form 0 (few elements) or 1."""
+    lib = L.lib()
+    run, size = lib.i8f_internal_merge_drawn, lib.i8f_internal_merge_drawn_workspace_bytes
+    run.argtypes = [ctypes.c_int, *lib.i8f_lora_merge_sr_drawn.argtypes]
+    size.argtypes, size.restype = [ctypes.c_int, *lib.i8f_lora_merge_sr_drawn_workspace_bytes.argtypes], ctypes.c_int64
+    monkeypatch.setattr(lib, "i8f_lora_merge_sr_drawn", lambda *a: run(form, *a))
+    monkeypatch.setattr(lib, "i8f_lora_merge_sr_drawn_workspace_bytes", lambda *a: size(form, *a))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,rank,seed,row,std", CASES)
+@pytest.mark.parametrize("form", [0, 1])
+def test_both_forms_of_the_drawn_merge(pkg, L, dev, monkeypatch, form, N, K, rank, seed, row, std):
+    force(L, monkeypatch, form)
+    if form == 0 and rank > 224:
+        assert L.lora_merge_sr_drawn(torch.zeros(N, K, dtype=torch.int8, device=dev), 0.5, pkg.int8_quant._seeded(seed, dev),
+                                     [(torch.zeros(N, rank, device=dev), torch.zeros(rank, K, device=dev), 1.0)]) is None
+    else:
+        test_drawn_merge_equals_the_merge_on_torchs_noise(pkg, L, dev, N, K, rank, seed, row, std)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("scale", [0.0, 1e-30, float("nan"), -0.001])
+def test_both_forms_of_rows_without_a_usual_scale(pkg, L, dev, monkeypatch, form, scale):
+    force(L, monkeypatch, form)
+    test_drawn_merge_of_rows_without_a_usual_scale(pkg, L, dev, scale)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("N,K,ranks", [(33, 48, (3, 9, 8)), (640, 1040, (16, 32, 64)), (1025, 2064, (4, 4)), (40, 272, (1, 2, 1, 40, 12, 64, 72, 8))])
+def test_both_forms_of_a_stack(pkg, L, dev, monkeypatch, form, N, K, ranks):
+    if not L.DRAWS_LIKE_TORCH:
+        pytest.skip("this torch's generator is not the one that is reproduced")
+    force(L, monkeypatch, form)
+    g = torch.Generator(device=dev).manual_seed(N)
+    w = torch.randint(-128, 128, (N, K), generator=g, device=dev, dtype=torch.int8)
+    parts = [(torch.randn(N, r, generator=g, device=dev) * 0.02, torch.randn(r, K, generator=g, device=dev) * 0.02, 0.3 * i - 0.5) for i, r in enumerate(ranks)]
+    got = L.lora_merge_sr_drawn(w, 0.002, pkg.int8_quant._seeded(3, dev), parts)
+    up, down = torch.cat([u for u, _, _ in parts], 1), torch.cat([d * m for _, d, m in parts])
+    assert torch.equal(got, L.lora_merge_sr(w, 0.002, pkg.int8_quant._draw_noise((N, K), 3, dev), up=up, down=down))
+
+
+def test_which_form_the_drawn_merge_takes(L):
+    """By the memory that it asks for: few elements, or few products, take the form with two bytes of noise to an element."""
+    size = L.lib().i8f_lora_merge_sr_drawn_workspace_bytes
+    few = lambda N, K, rank, count=1: size(N, K, rank, count) == 2 * N * K + (4 * (N + K) * rank if count > 1 else 0)
+    assert few(16, 3072, 16) and few(1024, 1024, 16) and few(1024, 1024, 224) and few(3072, 3072, 16) and few(2048, 1024, 32)
+    assert few(3840, 3840, 16) and few(10408, 2672, 4) and few(1280, 1280, 32, 2)
+    assert not few(1024, 1024, 256) and not few(2048, 2048, 64) and not few(4096, 4096, 16) and not few(3072, 3072, 32)
+    assert not few(12288, 3072, 4) and not few(12288, 3072, 32) and not few(9216, 3072, 112, 3)
