@@ -565,7 +565,7 @@ int launch_steps(const DrawnArgs &a, hipStream_t st) {
 }
 
 // the steps that are built: every one up to 8, then 10, 12 and 16 (14 have a tile's rows of `up` in registers that spill: 9216 x 3072, rank
-// 224, 178 us, in 16 steps FIGURE14)
+// 224, 178 us, in 16 steps 145)
 int steps_of(int64_t rank) {
     const int s = (int)((rank + 15) / 16);
     return s <= 1 ? 1 : s <= 8 ? s : s <= 12 ? (s + 1) / 2 * 2 : 16;
@@ -590,12 +590,14 @@ int launch_merge(const DrawnArgs &a, hipStream_t st) {
     }
 }
 
-// Few elements, or few products: which form is the faster one.  us, both launches, the form of lora_merge.hip and this one: 1024 x 1024 rank 16
-// 9.0 and 12.4, rank 128 18.4 and 19.3, 2048 x 1024 rank 32 11.1 and 14.5, rank 64 14.0 and 16.6, 2048 x 2048 rank 16 13.2 and 14.2, rank 64 18.7 and
-// 17.7, 3072 x 3072 rank 8 17.3 and 19.5, rank 16 18.5 and 19.7, rank 32 22.1 and 21.6, 3840 x 3840 rank 16 25.2 and 25.8, 5120 x 4096
-// rank 16 31.6 and 29.4; of ranks up to 4, 3840 x 3840 22.8 and 25.4, 10408 x 2672 40.1 and 41.6, 12288 x 3072 45.9 and 44.2.
+// Few elements, or few products: which form is the faster one.  us, both launches, operands from HBM, the form of lora_merge.hip and this one:
+// rank 16 1024 x 1024 8.9 and 12.6, 3072 x 3072 18.5 and 19.7, 3840 x 3840 25.1 and 26.3, 5120 x 4096 31.4 and 29.7; rank 32 2048 x 1024 10.5
+// and 14.4, 2048 x 2048 14.6 and 15.5, 12288 x 1024 25.7 and 24.5; rank 64 2048 x 1024 14.0 and 16.6, 2048 x 2048 18.7 and 17.7; rank 128 1024 x 1024
+// 18.4 and 19.3.  Of ranks up to 8 the products are nothing and the noise's other byte is all that this form saves: rank 8 12288 x 3072 46.4 and 49.9,
+// 6144 x 4608 37.5 and 37.1, 18432 x 3072 66.3 and 68.4, 8192 x 8192 77.7 and 70.3, 6144 x 12288 89.4 and 85.6; rank 4 45.3 and 49.6, 36.3 and
+// 36.9, 63.9 and 68.1, 75.4 and 69.5, 86.0 and 85.3.
 bool takes_few_form(int64_t N, int64_t K, int64_t rank) {
-    const int64_t weight = rank <= 4 ? 8 : rank <= 16 ? 16 : rank;
+    const int64_t weight = rank <= 8 ? 4 : rank <= 16 ? 16 : rank;
     return rank <= FEW_MAX_RANK && N * K * weight < (1ll << 28);
 }
 
