@@ -309,23 +309,23 @@ __device__ __forceinline__ int8_t add_sat8(uint32_t w, float r) { return (int8_t
 // CU where they fit the registers (twelve: 35 us, eight: 38.5); beyond rank 64 a tile's rows of `up` leave room for eight (rank 112 42 us,
 // twelve with spills 66).  All products of a tile first, for four chains instead of one, or those of the next block beside the
 // rounding of this one: no faster.  Answers for the whole of a wave at its end, by byte stores over what is stored: 37 for 35 us.
-// STEPS: 16-rank steps of the padded product.
-template <int STEPS>
+// STEPS: 16-rank steps of the padded product.  PER_CU: workgroups that share the waves of a CU.
+template <int STEPS, int PER_CU>
 struct DrawnShape {
     static constexpr int BLOCKS = STEPS <= 12 ? 4 : 2, COLS = 32 * BLOCKS;         // 32-column blocks of a workgroup
-    static constexpr int WAVES = STEPS <= 2 ? 16 : STEPS <= 4 ? 12 : 8, PER_SIMD = WAVES / 4;
+    static constexpr int PER_SIMD = STEPS <= 2 ? 4 : STEPS <= 4 ? 3 : 2, WAVES = 4 * PER_SIMD / PER_CU;
     static constexpr int PANEL = BLOCKS * STEPS * 2048;                           // `down`, two parts of 1 KB to a block and step
     static constexpr int PITCH = COLS + 16, TILE = 32 * PITCH;                    // a wave's weights
     static constexpr int MOST_OPEN = 48, LIST = BLOCKS * MOST_OPEN;               // open elements of a block, of a tile
     static constexpr int LATER = 32;                                              // elements left to the definition after which it is turned to
     static constexpr int WAVE = TILE + LIST * 8 + (LATER + LIST) * 5;
     static constexpr int BYTES = PANEL + WAVES * ((WAVE + 15) / 16 * 16);
-    static_assert(BYTES + 64 <= 160 * 1024, "LDS");
+    static_assert((BYTES + 64) * PER_CU <= 160 * 1024, "LDS");
 };
 
-template <int STEPS>
-__global__ __launch_bounds__((DrawnShape<STEPS>::WAVES * 64), DrawnShape<STEPS>::PER_SIMD) void merge_drawn_kernel(const DrawnArgs a) {
-    using T = DrawnShape<STEPS>;
+template <int STEPS, int PER_CU>
+__global__ __launch_bounds__((DrawnShape<STEPS, PER_CU>::WAVES * 64), (DrawnShape<STEPS, PER_CU>::PER_SIMD)) void merge_drawn_kernel(const DrawnArgs a) {
+    using T = DrawnShape<STEPS, PER_CU>;
     constexpr int NT = T::WAVES * 64, BLOCKS = T::BLOCKS, COLS = T::COLS;
     __shared__ __attribute__((aligned(16))) char lds[T::BYTES];
     __shared__ float back[BLOCKS];
@@ -554,14 +554,38 @@ __global__ __launch_bounds__((DrawnShape<STEPS>::WAVES * 64), DrawnShape<STEPS>:
     }
 }
 
+// Workgroups of a column panel, as many as the CUs hold, and the tiles that the busiest CU gets.
+struct Bands {
+    int64_t columns, bands, busiest;
+    Bands(const DrawnArgs &a, int cols, int64_t per_cu) {
+        const int64_t nblocks = ((int64_t)a.N + 31) / 32, slots = 256 * per_cu;
+        columns = ((int64_t)a.K + cols - 1) / cols;
+        bands = slots / columns;
+        bands = bands < 1 ? 1 : bands > nblocks ? nblocks : bands;
+        busiest = (columns * bands + slots - 1) / slots * per_cu * ((nblocks + bands - 1) / bands);
+    }
+};
+
+template <int STEPS, int PER_CU>
+int launch_shape(const DrawnArgs &a, const Bands &b, hipStream_t st) {
+    hipLaunchKernelGGL((merge_drawn_kernel<STEPS, PER_CU>), dim3((unsigned)b.columns, (unsigned)b.bands), dim3(DrawnShape<STEPS, PER_CU>::WAVES * 64), 0, st, a);
+    return check_launch();
+}
+
+// Whole panels to a workgroup and whole workgroups to a CU leave CUs idle where the panels divide 256 badly (18432 columns are 144 panels).
+// Two workgroups of eight waves to a CU are dealt out more evenly but put every panel into LDS twice as often.  us, one and two, with
+// the busiest CU's tiles: 2048 x 18432 rank 16 59.2 and 53.9 (64 and 44), 12288 x 12288 rank 8 172 and 159 (192 and 154), 3072 x 12288
+// rank 16 53.9 and 51.4, rank 32 56.3 and 53.8 (48 and 40), 4096 x 11008 rank 16 61.0 and 57.5 (64 and 52), 2048 x 11008 rank 16 36.9 and 35.7
+// (32 and 26); 4096 x 8320 rank 32 48.3 and 49.3 (43 and 38), 12288 x 3072 rank 32 46.7 and 48.3 (39 and 38).  Six waves, of ranks above 32, do
+// not fill the four SIMDs evenly: 4096 x 11008 rank 48 68 and 82.
 template <int STEPS>
 int launch_steps(const DrawnArgs &a, hipStream_t st) {
-    using T = DrawnShape<STEPS>;
-    const int64_t columns = (a.K + T::COLS - 1) / T::COLS, nblocks = (a.N + 31) / 32, slots = 256;
-    int64_t bands = slots / columns, most = nblocks;
-    bands = bands < 1 ? 1 : bands > most ? most : bands;
-    hipLaunchKernelGGL((merge_drawn_kernel<STEPS>), dim3((unsigned)columns, (unsigned)bands), dim3(T::WAVES * 64), 0, st, a);
-    return check_launch();
+    const Bands one(a, DrawnShape<STEPS, 1>::COLS, 1);
+    if constexpr (STEPS <= 2) {
+        const Bands two(a, DrawnShape<STEPS, 2>::COLS, 2);
+        if (two.busiest * 20 <= one.busiest * 17) return launch_shape<STEPS, 2>(a, two, st);
+    }
+    return launch_shape<STEPS, 1>(a, one, st);
 }
 
 // the steps that are built: every one up to 8, then 10, 12 and 16 (14 have a tile's rows of `up` in registers that spill: 9216 x 3072, rank

@@ -226,3 +226,11 @@ def test_which_form_the_drawn_merge_takes(L):
     assert few(3840, 3840, 16) and few(10408, 2672, 4) and few(12288, 3072, 8) and few(18432, 3072, 4) and few(1280, 1280, 32, 2)
     assert not few(1024, 1024, 256) and not few(2048, 2048, 64) and not few(4096, 4096, 16) and not few(3072, 3072, 32)
     assert not few(8192, 8192, 4) and not few(12288, 3072, 12) and not few(12288, 3072, 32) and not few(9216, 3072, 112, 3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,rank", [(640, 18432, 16), (333, 18448, 28), (1000, 11008, 8), (5, 20480, 4)])
+def test_two_workgroups_to_a_cu(pkg, L, dev, monkeypatch, N, K, rank):
+    """Widths whose panels leave a good part of the CUs without one, full and with a rest (5 rows: not enough for it)."""
+    force(L, monkeypatch, 1)
+    test_drawn_merge_equals_the_merge_on_torchs_noise(pkg, L, dev, N, K, rank, 4, True, 0.01)
