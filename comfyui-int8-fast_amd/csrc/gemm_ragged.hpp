@@ -99,8 +99,10 @@ __global__ __launch_bounds__((256 * GROUPS), (GROUPS < 2 ? 2 : GROUPS)) void gem
         dst[t] = (is_x ? 0 : BM * BK) + row * BK + (c ^ swz<8>(row)) * 16;
     }
     v4i reg[AHEAD][XC + WC];
-    // A K-tile's loads and nothing else: no branch (past the last K-tile that one is fetched again) and no use of what they
-    // bring, or the compiler would wait for all of them here.
+    // A K-tile's loads and nothing else: no branch and no use of what they bring, or the compiler would wait for all of them here.
+    // Past the last K-tile every lane fetches the same 16 bytes: K-tiles that nobody needs are as many as needed ones where K is
+    // short, and with K odd their chunks cost as much as any (us, one group, two that fetch the last K-tile again, two as here: 30 x 301 x 17 5.0, 5.5
+    // and 4.4, 35 x 967 x 257 5.8, 6.4 and 5.7, 512 x 2041 x 121 6.2, 6.5 and 5.5; with K = 640, where a chunk is one line's, 5.8, 5.0 and 5.1).
     auto fetch = [&](int kt, v4i (&r)[XC + WC]) __attribute__((always_inline)) {
         if constexpr (TINY) {  // K < 16: the only chunk with bytes in it is the first
 #pragma unroll
@@ -112,9 +114,10 @@ __global__ __launch_bounds__((256 * GROUPS), (GROUPS < 2 ? 2 : GROUPS)) void gem
                 r[t] = v4i{(int)b[0], (int)b[1], (int)b[2], (int)b[3]};
             }
         } else {
-            const uint32_t pos = min((uint32_t)min(kt, KT - 1) * BK + c * 16, (uint32_t)K - 16);
+            const bool there = kt < KT;
+            const uint32_t pos = min((uint32_t)kt * BK + c * 16, (uint32_t)K - 16);
 #pragma unroll
-            for (int t = 0; t < XC + WC; ++t) __builtin_memcpy(&r[t], src[t] + pos, 16);
+            for (int t = 0; t < XC + WC; ++t) __builtin_memcpy(&r[t], there ? src[t] + pos : g.w, 16);
         }
     };
     // of the last K-tile's chunks, which end with the row: what precedes the chunk in them is shifted out
