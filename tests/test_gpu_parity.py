@@ -698,13 +698,13 @@ SPLITK_CASES = [
     (250, 3064, 12304, torch.float16),    # ragged everywhere, K not a multiple of the 128-byte K-tile
     (64, 3072, 12288, torch.bfloat16),    # 64 x 64 tiles, five slices of unequal length
     (100, 1000, 16400, torch.float32),
-    (16, 12288, 10240, torch.bfloat16),   # the shortest K that is split
+    (16, 12288, 10240, torch.bfloat16),   # from this K on the price alone decides, and captured calls are split
 ]
 
 
 @pytest.mark.parametrize("M,N,K,odt", SPLITK_CASES)
 def test_linear_w8a8_k_split_bit_exact(L, dev, M, N, K, odt):
-    """Outputs of few tiles with K >= 10240 take the K split when a workspace is given (the Python layer keeps one
+    """Outputs of few tiles with K >= 6144 take the K split when a workspace is given (the Python layer keeps one
     per stream): bit-equal to the oracle and to the same call without a workspace, the arrival counters are zero
     again afterwards, and a second call on the same workspace gives the same result."""
     x = acts(M, K)
