@@ -106,3 +106,33 @@ def test_narrow_layers_keep_their_k_split_beside_wide_ones(pkg, L, dev, widths, 
         check(outs)
         assert all(torch.equal(o, v) for o, v in zip(pkg.forward_fanout(lins, x), want))   # an eager call in between
         handed.pop()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,K,widths,dtype,opts,reason", [
+    (300, 512, (1536, 1536, 1536), torch.bfloat16, {}, "patched"), (4096, 256, (3840, 3840, 3840), torch.float16, {"rotate": True}, "patched"),
+    (40, 256, (64,) * 9, torch.bfloat16, {}, "count"), (33, 384, (64, 64, 192, 8, 8, 8, 8, 192, 100), torch.float16, {}, "count"),
+    (100, 384, (96, 192, 192, 8), torch.bfloat16, {"per_row": (False, True, True, True), "bias": (True, False, True, True)}, "patched"),
+    (70, 256, (128, 128, 128), torch.float16, {"per_row": (False, True, False)}, "patched"), (520, 10240, (3456, 256, 256), torch.bfloat16, {}, "patched"),
+    (50, 200, (100, 100), torch.bfloat16, {}, "patched"), (64, 256, (128, 128), torch.bfloat16, {}, "bias"),
+])
+def test_the_general_path_of_the_fanout_is_the_layers_own_forward(pkg, L, dev, rows, K, widths, dtype, opts, reason, monkeypatch):
+    """What the native call leaves: more layers than it takes, a bias of another type behind one launch's, and, to have every
+    form here, calls that it would take."""
+    lins = layers_of(pkg, dev, widths, K, dtype, **opts)
+    if reason == "bias":
+        lins[1].bias = torch.nn.Parameter(lins[1].bias.float(), requires_grad=False)
+    if reason in ("patched", "bias"):
+        monkeypatch.setattr(pkg.int8_quant, "_fanout_native", lambda *a: None)
+    grouped, reached = L.linear_w8a8_grouped, []
+    monkeypatch.setattr(L, "linear_w8a8_grouped", lambda *a: reached.append(len(a[0])) or grouped(*a))
+    x = torch.randn(1, rows, K, device=dev).to(dtype)
+    scale, shift, weight = (torch.randn(K, device=dev).to(dtype) * 0.2 for _ in range(3))
+    calls = [{}, {"prologue": L.PRO_MODULATE, "mod_scale": scale, "mod_shift": shift}]
+    if K % 16 == 0:
+        calls += [{"prologue": L.PRO_RMS_NORM, "norm_weight": weight, "mod_scale": scale, "eps": 1e-5}]
+    for t in (x, x[0]):
+        for kw in calls:
+            outs = pkg.forward_fanout(lins, t, **kw)
+            assert all(torch.equal(o, lin(t, **kw)) for o, lin in zip(outs, lins)) and len(outs) == len(lins)
+    assert reached == [len(lins)] * (2 * len(calls))
