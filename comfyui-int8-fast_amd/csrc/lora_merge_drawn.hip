@@ -395,9 +395,11 @@ __global__ __launch_bounds__((DrawnShape<STEPS, PER_CU>::WAVES * 64), (DrawnShap
     // and column (which bound the sum of the products' magnitudes): 2^-24 for each of the definition's additions, twice that for
     // each of the matrix unit's (whatever its inner order is; the cross products go first, and what their additions lose is below
     // 2^-9 of that), 3 * 2^-22 for the two splits and the product of the low parts, 2^-22 for parts below binary16's normal
-    // range, 7 * 2^-24 for the reciprocal, the products with lora_scale and f, and the definition's own product and quotient.
+    // range, 7 * 2^-24 for the reciprocal, the products with lora_scale and f, and the definition's own product and quotient, 2^-24 for
+    // the difference of quotient and noise, whose rounding grows with the quotient (2^-16 at 300, beyond which it is not asked for).
+    // That is 3 rank + 24 times 2^-24; 32 leaves something for the norms' and this bound's own roundings.
     const float coefficient = (float)(3 * a.rank + 32) * 0x1p-24f;
-    constexpr float ROUNDINGS = 0x1p-22f;   // of noise, difference and fraction, which are at most 1 and are rounded a few times
+    constexpr float ROUNDINGS = 0x1p-22f;   // of the same difference where the quotient is below 1, and of the distances, which are
     // the products of 32 columns with the block's rows
     auto product = [&](int b, v16f &acc) __attribute__((always_inline)) {
 #pragma unroll

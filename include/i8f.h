@@ -329,7 +329,8 @@ int i8f_linear_w8a8_add(const int8_t *a, const float *a_scale, const int8_t *w, 
  * stream's down-projection, a decode-sized batch) deal the K range of a tile over several workgroups that
  * exchange their integer sums through the workspace.  Same arguments, same results bit for bit (integer
  * sums do not depend on their order); the same Triton launches as i8f_linear_w8a8 (int8_fused_kernel.py:216,
- * 357), whose grids cover the output only.  512 x 3072 x 12288 with weights from HBM: 42 -> 34 us.
+ * 357), whose grids cover the output only.  512 x 3072 x 12288 with weights from HBM: 42 -> 35 us.  (A caller that clears the
+ * arrival words by a kernel in front of every call, as in a captured graph, gains nothing below K = 10240.)
  *   workspace        device memory of i8f_linear_w8a8_workspace_bytes() bytes (16 MB + 4 KB), 16-byte aligned,
  *                    whose first 4096 bytes (one arrival word per output tile) are ZERO before the first call;
  *                    every call that completes leaves them zero again.  Each launch stamps its arrival words
