@@ -200,7 +200,7 @@ def forward_fanout(layers, x, prologue: int = _lib.PRO_NONE, mod_scale=None, mod
                     ws = ws.reshape(-1)[:1]
             problems.append((x_in, lin.weight, ws, lin.bias))
         return [y.reshape(*x.shape[:-1], y.shape[-1]) for y in _lib.linear_w8a16_small_m_grouped(problems)]
-    if len(layers) >= 2 and not torch.compiler.is_compiling() and type(x) is Tensor and x.is_cuda and x.dim() >= 2:
+    if 2 <= len(layers) <= 8 and not torch.compiler.is_compiling() and type(x) is Tensor and x.is_cuda and x.dim() >= 2:   # (as many as it takes)
         outs = _fanout_native(layers, x, rot, prologue, mod_scale, mod_shift, eps, norm_weight, fused_add)
         if outs is not None:
             return outs
@@ -246,9 +246,24 @@ def forward_fanout(layers, x, prologue: int = _lib.PRO_NONE, mod_scale=None, mod
             if not lin._is_per_row and ws.numel() != 1:
                 ws = ws.reshape(-1)[:1]
         problems.append((q, s, lin.weight, ws, lin.bias))
-    # Layers of one shape go out in one launch where the library finds that cheaper (8000 x 5120 into three of 5120 columns: 8 rounds of
-    # tiles for 9; 576 and 541 us, 3000 x 3584 into three 121 and 106 us).
-    return [y.reshape(*lead, y.shape[-1]) for y in _lib.linear_w8a8_grouped(problems, x.dtype, int8_fused_kernel.DEFAULT_EPILOGUE)]
+    # Layers of one form go out in one launch where the library finds that cheaper (8000 x 5120 into three of 5120 columns: 8 rounds of
+    # tiles for 9; 576 and 541 us, 3000 x 3584 into three 121 and 106 us).  Runs of them: a grouped call of several forms, or of more
+    # layers than a launch takes, looks at every operand twice (nine layers of 1536 columns on 300 x 512: 227 us a call, 173 one by one).
+    runs, last = [], None
+    for lin, p in zip(layers, problems):
+        form = (p[2].numel(), lin._is_per_row)   # (one width: as many elements, as many columns)
+        if form == last and len(runs[-1]) < _lib.MAX_LINEAR_GROUPS and len({r[4].dtype for r in (*runs[-1], p) if r[4] is not None}) < 2:
+            runs[-1].append(p)
+        else:
+            runs.append([p])
+            last = form
+    outs = []
+    for run in runs:
+        if len(run) == 1:
+            outs.append(_lib.linear_w8a8(*run[0], x.dtype, int8_fused_kernel.DEFAULT_EPILOGUE))
+        else:
+            outs += _lib.linear_w8a8_grouped(run, x.dtype, int8_fused_kernel.DEFAULT_EPILOGUE)
+    return [y.reshape(*lead, y.shape[-1]) for y in outs]
 
 
 # --------------------------------------------------------------------------- LoRA delta reconstruction

@@ -124,8 +124,8 @@ def test_the_general_path_of_the_fanout_is_the_layers_own_forward(pkg, L, dev, r
         lins[1].bias = torch.nn.Parameter(lins[1].bias.float(), requires_grad=False)
     if reason in ("patched", "bias"):
         monkeypatch.setattr(pkg.int8_quant, "_fanout_native", lambda *a: None)
-    grouped, reached = L.linear_w8a8_grouped, []
-    monkeypatch.setattr(L, "linear_w8a8_grouped", lambda *a: reached.append(len(a[0])) or grouped(*a))
+    look, looked = L._i8_matrix, []
+    monkeypatch.setattr(L, "_i8_matrix", lambda *a: looked.append(a[1]) or look(*a))
     x = torch.randn(1, rows, K, device=dev).to(dtype)
     scale, shift, weight = (torch.randn(K, device=dev).to(dtype) * 0.2 for _ in range(3))
     calls = [{}, {"prologue": L.PRO_MODULATE, "mod_scale": scale, "mod_shift": shift}]
@@ -133,6 +133,7 @@ def test_the_general_path_of_the_fanout_is_the_layers_own_forward(pkg, L, dev, r
         calls += [{"prologue": L.PRO_RMS_NORM, "norm_weight": weight, "mod_scale": scale, "eps": 1e-5}]
     for t in (x, x[0]):
         for kw in calls:
+            looked.clear()
             outs = pkg.forward_fanout(lins, t, **kw)
+            assert looked == ["a", "w"] * len(lins)   # (every layer's operands once)
             assert all(torch.equal(o, lin(t, **kw)) for o, lin in zip(outs, lins)) and len(outs) == len(lins)
-    assert reached == [len(lins)] * (2 * len(calls))
