@@ -234,3 +234,10 @@ def test_two_workgroups_to_a_cu(pkg, L, dev, monkeypatch, N, K, rank):
     """Widths whose panels leave a good part of the CUs without one, full and with a rest (5 rows: not enough for it)."""
     force(L, monkeypatch, 1)
     test_drawn_merge_equals_the_merge_on_torchs_noise(pkg, L, dev, N, K, rank, 4, True, 0.01)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [0, 1])
+def test_both_forms_in_place(pkg, L, dev, monkeypatch, form):
+    force(L, monkeypatch, form)
+    test_drawn_merge_in_place(pkg, L, dev)
