@@ -745,7 +745,6 @@ int merge_few(const DrawnCall &c, hipStream_t st) {
     // workgroups for the factors: 4 elements a thread, one round of the chip at most
     int64_t extra = c.count > 1 ? ((N + K) * c.rank + 1023) / 1024 : 0;
     extra = ((extra < 2048 ? extra : 2048) + columns - 1) / columns;
-    if (chunks + extra > 65535) return I8F_ERR_UNSUPPORTED;
     MergeArgs a{};
     a.w = c.w, a.ws = c.ws, a.ws_host = c.ws_host, a.row_scale = c.row_scale;
     a.up = c.factors[0].up, a.down = c.factors[0].down, a.rank = c.rank, a.lora_scale = c.lora_scale;
@@ -763,9 +762,15 @@ int merge_few(const DrawnCall &c, hipStream_t st) {
         stack.down_out = (float *)((char *)stack.up_out + up256(4 * N * c.rank));
         a.up = stack.up_out, a.down = stack.down_out;
     }
-    hipLaunchKernelGGL(draw_words_kernel, dim3((unsigned)columns, (unsigned)(chunks + extra)), dim3(256), 0, st, a.seed_lo, a.seed_hi, a.lanes,
-                       (uint32_t)(N * K), (uint16_t *)c.workspace, (uint32_t)extra, stack);
-    if (int rc = check_launch()) return rc;
+    auto draw = [&](int64_t blocks, int64_t factor_blocks) {   // rows of blocks
+        hipLaunchKernelGGL(draw_words_kernel, dim3((unsigned)columns, (unsigned)blocks), dim3(256), 0, st, a.seed_lo, a.seed_hi, a.lanes,
+                           (uint32_t)(N * K), (uint16_t *)c.workspace, (uint32_t)factor_blocks, stack);
+        return check_launch();
+    };
+    const bool once = chunks + extra <= 65535;
+    if (int rc = draw(once ? chunks + extra : extra, extra)) return rc;
+    if (!once)
+        if (int rc = draw(chunks, 0)) return rc;
     return launch_rank<true>(a, st);
 }
 

@@ -559,9 +559,9 @@ __global__ __launch_bounds__((DrawnShape<STEPS, PER_CU>::WAVES * 64), (DrawnShap
 // Workgroups of a column panel, as many as the CUs hold, and the tiles that the busiest CU gets.
 struct Bands {
     int64_t columns, bands, busiest;
-    Bands(const DrawnArgs &a, int cols, int64_t per_cu) {
-        const int64_t nblocks = ((int64_t)a.N + 31) / 32, slots = 256 * per_cu;
-        columns = ((int64_t)a.K + cols - 1) / cols;
+    Bands(int64_t N, int64_t K, int cols, int64_t per_cu) {
+        const int64_t nblocks = (N + 31) / 32, slots = 256 * per_cu;
+        columns = (K + cols - 1) / cols;
         bands = slots / columns;
         bands = bands < 1 ? 1 : bands > nblocks ? nblocks : bands;
         busiest = (columns * bands + slots - 1) / slots * per_cu * ((nblocks + bands - 1) / bands);
@@ -580,12 +580,15 @@ int launch_shape(const DrawnArgs &a, const Bands &b, hipStream_t st) {
 // rank 16 53.9 and 51.4, rank 32 56.3 and 53.8 (48 and 40), 4096 x 11008 rank 16 61.0 and 57.5 (64 and 52), 2048 x 11008 rank 16 36.9 and 35.7
 // (32 and 26); 4096 x 8320 rank 32 48.3 and 49.3 (43 and 38), 12288 x 3072 rank 32 46.7 and 48.3 (39 and 38).  Six waves, of ranks above 32, do
 // not fill the four SIMDs evenly: 4096 x 11008 rank 48 68 and 82.
+constexpr int MAX_SHARED_STEPS = 2;
+inline bool two_to_a_cu(const Bands &one, const Bands &two) { return two.busiest * 20 <= one.busiest * 17; }
+
 template <int STEPS>
 int launch_steps(const DrawnArgs &a, hipStream_t st) {
-    const Bands one(a, DrawnShape<STEPS, 1>::COLS, 1);
-    if constexpr (STEPS <= 2) {
-        const Bands two(a, DrawnShape<STEPS, 2>::COLS, 2);
-        if (two.busiest * 20 <= one.busiest * 17) return launch_shape<STEPS, 2>(a, two, st);
+    const Bands one(a.N, a.K, DrawnShape<STEPS, 1>::COLS, 1);
+    if constexpr (STEPS <= MAX_SHARED_STEPS) {
+        const Bands two(a.N, a.K, DrawnShape<STEPS, 2>::COLS, 2);
+        if (two_to_a_cu(one, two)) return launch_shape<STEPS, 2>(a, two, st);
     }
     return launch_shape<STEPS, 1>(a, one, st);
 }
@@ -616,15 +619,37 @@ int launch_merge(const DrawnArgs &a, hipStream_t st) {
     }
 }
 
-// Few elements, or few products: which form is the faster one.  us, both launches, operands from HBM, the form of lora_merge.hip and this one:
-// rank 16 1024 x 1024 8.9 and 12.6, 3072 x 3072 18.5 and 19.7, 3840 x 3840 25.1 and 26.3, 5120 x 4096 31.4 and 29.7; rank 32 2048 x 1024 10.5
-// and 14.4, 2048 x 2048 14.6 and 15.5, 12288 x 1024 25.7 and 24.5; rank 64 2048 x 1024 14.0 and 16.6, 2048 x 2048 18.7 and 17.7; rank 128 1024 x 1024
-// 18.4 and 19.3.  Of ranks up to 8 the products are nothing and the noise's other byte is all that this form saves: rank 8 12288 x 3072 46.4 and 49.9,
-// 6144 x 4608 37.5 and 37.1, 18432 x 3072 66.3 and 68.4, 8192 x 8192 77.7 and 70.3, 6144 x 12288 89.4 and 85.6; rank 4 45.3 and 49.6, 36.3 and
-// 36.9, 63.9 and 68.1, 75.4 and 69.5, 86.0 and 85.3.
-bool takes_few_form(int64_t N, int64_t K, int64_t rank) {
-    const int64_t weight = rank <= 8 ? 4 : rank <= 16 ? 16 : rank;
-    return rank <= FEW_MAX_RANK && N * K * weight < (1ll << 28);
+// Which form is the faster one, by an estimate of both in us (a sum of what they do, fitted to 1279 shapes of 64 to 18432 rows, 128 to 14000
+// columns and ranks 4 to 192, alone and in stacks, operands from HBM).  It is off by 6 and 5 % (standard deviation), and what it picks is
+// 0.5 % slower than the better one on average, over 10 % in 11 of them; a line at N K rank = 2^28 is 0.9 % slower where K % 128 == 0, 3 % elsewhere.
+// Few elements are the case for the form of lora_merge.hip: 1024 x 1024 rank 16 8.9 and 12.6 us, 3072 x 3072 rank 16 18.5 and 19.7, 2048 x 1024
+// rank 32 10.5 and 14.4, rank 64 14.0 and 16.6, and of ranks up to 8, whose products are nothing, more: 12288 x 3072 rank 8 46.4 and 49.9, 18432 x 3072
+// rank 4 63.9 and 68.1.  Against it: 2048 x 2048 rank 64 18.7 and 17.7, 5120 x 4096 rank 16 31.4 and 29.7, 8192 x 8192 rank 4 75.4 and 69.5; columns
+// that are no whole lines (1168 x 1632 ranks 4 + 64 + 4 24.6 and 18.7, 392 x 10016 ranks 4 + 64 30.2 and 21.6).
+bool takes_few_form(int64_t N, int64_t K, int64_t rank, int count) {
+    if (rank > FEW_MAX_RANK || N < 1 || K < 1 || N * K >= (1ll << 26)) return false;   // (8192 x 8192 is the first beyond what was fitted)
+    const double elements = (double)N * K * 0x1p-20, factors = (double)(N + K) * rank * 0x1p-20, stack = count > 1;
+    // the form for few elements: wave steps of a SIMD (launch_mfma, roughly), of which each is products of the padded rank
+    const int64_t padded = rank <= 8 ? (rank + 3) / 4 * 4 : rank <= 32 ? (rank <= 16 ? 16 : 32) : rank <= 128 ? (rank + 15) / 16 * 16 : (rank + 31) / 32 * 32;
+    const int64_t waves = padded == 48 || padded == 64 ? 4 : 8, slots = padded <= 32 ? 512 : padded <= 64 ? 768 : 256;
+    const int64_t columns = (K + 32 * waves - 1) / (32 * waves), nblocks = (N + 31) / 32;
+    const int64_t fit = slots / columns, bands = fit < 1 ? 1 : fit < nblocks ? fit : nblocks;
+    const double few_steps = (double)((columns * bands + 255) / 256 * ((nblocks + bands - 1) / bands) * waves / 4);
+    // the other: tiles of the busiest CU and of a wave
+    const int64_t steps = steps_of(rank), waves_of_cu = steps <= 2 ? 16 : steps <= 4 ? 12 : 8;
+    const int cols = steps <= 12 ? 128 : 64;
+    const Bands one(N, K, cols, 1), two(N, K, cols, 2);
+    const double busiest = (double)(steps <= MAX_SHARED_STEPS && two_to_a_cu(one, two) ? two : one).busiest;
+    const double tiles = (double)(int64_t)((busiest + waves_of_cu - 1) / waves_of_cu);
+    double few, many;
+    if (K % 128 == 0) {
+        few = 7.37 + 0.688 * elements + 0.0451 * padded + few_steps * (0.225 + 0.0168 * padded) + stack * (0.43 + 5.17 * factors);
+        many = 9.35 + 0.368 * elements + 0.577 * steps + 0.527 * busiest + tiles * (1.007 + 0.416 * steps) + 3.14 * factors + 0.77 * stack;
+    } else {
+        few = 9.10 + 0.575 * elements + 0.0528 * padded + few_steps * (0.402 + 0.0159 * padded) + stack * (0.88 + 4.42 * factors);
+        many = 10.57 + 0.769 * elements + 0.467 * steps + busiest * (0.275 + 0.0044 * steps) + tiles * (0.156 + 0.464 * steps) + 3.27 * factors + 0.89 * stack;
+    }
+    return few < many;
 }
 
 int64_t many_workspace_bytes(int64_t N, int64_t K, int64_t rank, int count) {
@@ -682,7 +707,7 @@ int merge_many(const DrawnCall &c, hipStream_t st) {
 extern "C" int64_t i8f_internal_merge_drawn_workspace_bytes(int form, int64_t N, int64_t K, int64_t rank, int count) {
     using namespace i8f;
     if (N < 0 || K < 0 || rank < 0 || N > (1 << 29) || K > (1 << 29) || rank > 256) return 0;
-    return (form < 0 ? takes_few_form(N, K, rank) : form == 0) ? merge_few_workspace_bytes(N, K, rank, count) : many_workspace_bytes(N, K, rank, count);
+    return (form < 0 ? takes_few_form(N, K, rank, count) : form == 0) ? merge_few_workspace_bytes(N, K, rank, count) : many_workspace_bytes(N, K, rank, count);
 }
 
 extern "C" int i8f_internal_merge_drawn(int form, const int8_t *w, const float *w_scale, float w_scale_host, int scale_mode,
@@ -706,7 +731,7 @@ extern "C" int i8f_internal_merge_drawn(int form, const int8_t *w, const float *
     if ((uintptr_t)w % 16 || (uintptr_t)w_out % 16 || (uintptr_t)workspace % 16 || (count == 1 && (uintptr_t)factors[0].up % 16)) return I8F_ERR_UNSUPPORTED;
     if (count > 1 && (N + K) * rank >= (1ll << 31)) return I8F_ERR_UNSUPPORTED;   // (elements are counted in 32 bits)
     if ((N * K + 4 * lanes - 1) / (4 * lanes) > 65535) return I8F_ERR_UNSUPPORTED;
-    const bool few = form < 0 ? takes_few_form(N, K, rank) : form == 0;
+    const bool few = form < 0 ? takes_few_form(N, K, rank, count) : form == 0;
     if (few && rank > FEW_MAX_RANK) return I8F_ERR_UNSUPPORTED;
     if (workspace_bytes < i8f_internal_merge_drawn_workspace_bytes(form, N, K, rank, count)) return I8F_ERR_INVALID;
     if (int rc = check_device()) return rc;
