@@ -242,3 +242,23 @@ def test_two_workgroups_to_a_cu(pkg, L, dev, monkeypatch, N, K, rank):
 def test_both_forms_in_place(pkg, L, dev, monkeypatch, form):
     force(L, monkeypatch, form)
     test_drawn_merge_in_place(pkg, L, dev)
+
+
+@pytest.mark.gpu
+def test_a_generator_of_few_threads_takes_a_launch_for_the_factors_of_its_own(L, dev):
+    """256 threads: the calls of the generator and the blocks for a stack's factors are more rows of blocks than a launch has."""
+    N, K, ranks, lib = 4096, 16368, (4, 4), L.lib()
+    run, size = lib.i8f_internal_merge_drawn, lib.i8f_internal_merge_drawn_workspace_bytes
+    run.argtypes = [ctypes.c_int, *lib.i8f_lora_merge_sr_drawn.argtypes]
+    size.argtypes, size.restype = [ctypes.c_int, *lib.i8f_lora_merge_sr_drawn_workspace_bytes.argtypes], ctypes.c_int64
+    g = torch.Generator(device=dev).manual_seed(8)
+    w = torch.randint(-128, 128, (N, K), generator=g, device=dev, dtype=torch.int8)
+    parts = [(torch.randn(N, r, generator=g, device=dev) * 0.02, torch.randn(r, K, generator=g, device=dev) * 0.02) for r in ranks]
+    arr = (L._LoraFactors * 2)(*((u.data_ptr(), d.data_ptr(), u.shape[1], 0.5) for u, d in parts))
+    outs = []
+    for form in (0, 1):
+        out, scratch = torch.empty_like(w), torch.empty(size(form, N, K, sum(ranks), 2), dtype=torch.uint8, device=dev)
+        assert run(form, w.data_ptr(), None, 0.002, L.SCALE_TENSOR, arr, 2, 1.0, 5, 256, N, K, out.data_ptr(), scratch.data_ptr(), scratch.numel(),
+                   torch.cuda.current_stream().cuda_stream) == 0
+        outs.append(out)
+    assert torch.equal(*outs) and not torch.equal(outs[0], w)
