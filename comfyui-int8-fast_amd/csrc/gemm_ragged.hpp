@@ -54,7 +54,11 @@ __device__ __forceinline__ void finish_one(const GemmArgs &g, int acc, int m, in
 // or a use near them (the compiler put a wait for all loads in flight at each join: 11.8 and 110 us before), and the
 // epilogue's operands come first instead of last.  Two waves to a SIMD is what the registers have to leave room for: with one
 // the larger shape takes 119 us.
-template <int OUT, int BM, int BN, bool TINY, int GROUPS = 1>
+// PAST: past the last K-tile (loads ahead, groups without one) every lane fetches the same 16 bytes; else the last K-tile again.
+// K-tiles that nobody needs are as many as needed ones where K is short, and with K odd their chunks cost as much as any: us, one group,
+// two without and with PAST, 30 x 301 x 17 5.0, 5.5 and 4.4, 35 x 967 x 257 5.8, 6.4 and 5.7, 512 x 2041 x 121 6.2, 6.5 and 5.5.  With K a
+// multiple of 4 they cost little and the selection of addresses as much: a layer of 333 x 1160 into 1001 in a row 10.20 without, 10.46 with it.
+template <int OUT, int BM, int BN, bool TINY, int GROUPS, bool PAST>
 __global__ __launch_bounds__((256 * GROUPS), (GROUPS < 2 ? 2 : GROUPS)) void gemm_i8_ragged_kernel(const GemmArgs g) {
     constexpr int AHEAD = 2;  // K-tiles in flight (4, 6 and 8 measured the same or slower)
     constexpr int BK = 128, MI = BM / 64, NJ = BN / 64;
@@ -100,9 +104,6 @@ __global__ __launch_bounds__((256 * GROUPS), (GROUPS < 2 ? 2 : GROUPS)) void gem
     }
     v4i reg[AHEAD][XC + WC];
     // A K-tile's loads and nothing else: no branch and no use of what they bring, or the compiler would wait for all of them here.
-    // Past the last K-tile every lane fetches the same 16 bytes: K-tiles that nobody needs are as many as needed ones where K is
-    // short, and with K odd their chunks cost as much as any (us, one group, two that fetch the last K-tile again, two as here: 30 x 301 x 17 5.0, 5.5
-    // and 4.4, 35 x 967 x 257 5.8, 6.4 and 5.7, 512 x 2041 x 121 6.2, 6.5 and 5.5; with K = 640, where a chunk is one line's, 5.8, 5.0 and 5.1).
     auto fetch = [&](int kt, v4i (&r)[XC + WC]) __attribute__((always_inline)) {
         if constexpr (TINY) {  // K < 16: the only chunk with bytes in it is the first
 #pragma unroll
@@ -114,8 +115,8 @@ __global__ __launch_bounds__((256 * GROUPS), (GROUPS < 2 ? 2 : GROUPS)) void gem
                 r[t] = v4i{(int)b[0], (int)b[1], (int)b[2], (int)b[3]};
             }
         } else {
-            const bool there = kt < KT;
-            const uint32_t pos = min((uint32_t)kt * BK + c * 16, (uint32_t)K - 16);
+            const bool there = !PAST || kt < KT;
+            const uint32_t pos = min((uint32_t)(PAST ? kt : min(kt, KT - 1)) * BK + c * 16, (uint32_t)K - 16);
 #pragma unroll
             for (int t = 0; t < XC + WC; ++t) __builtin_memcpy(&r[t], there ? src[t] + pos : g.w, 16);
         }
@@ -219,10 +220,15 @@ int launch_ragged(const GemmArgs &g, hipStream_t st) {
     // 128 x 128 tiles once there is one for every CU: half the bytes per product (1024 x 3001 x 3083, 192 tiles: 40.0 us
     // against 41.4 with 64 x 64 tiles; 2500 x 2501 x 1160, 400 tiles: 26.7 both; 2100 x 3001 x 3083, 408 tiles: 62 against
     // 83); below that they leave CUs idle (1500 x 1500 x 1500, 144 tiles: 21.9 against 16.2).
-    if (g.K < 16) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, true>), dim3((unsigned)t64), dim3(256), 0, st, g);
-    else if (t128 >= 256) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 128, 128, false>), dim3((unsigned)t128), dim3(256), 0, st, g);
-    else if (t64 <= 256) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, false, 2>), dim3((unsigned)t64), dim3(512), 0, st, g);
-    else hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, false>), dim3((unsigned)t64), dim3(256), 0, st, g);
+    auto launch = [&](auto PAST) {
+        constexpr bool P = decltype(PAST)::value;
+        if (t128 >= 256) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 128, 128, false, 1, P>), dim3((unsigned)t128), dim3(256), 0, st, g);
+        else if (t64 <= 256) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, false, 2, P>), dim3((unsigned)t64), dim3(512), 0, st, g);
+        else hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, false, 1, P>), dim3((unsigned)t64), dim3(256), 0, st, g);
+    };
+    if (g.K < 16) hipLaunchKernelGGL((gemm_i8_ragged_kernel<OUT, 64, 64, true, 1, false>), dim3((unsigned)t64), dim3(256), 0, st, g);
+    else if (g.K % 4) launch(std::true_type{});
+    else launch(std::false_type{});
     return check_launch();
 }
 
